@@ -22,6 +22,8 @@
 
 extern "C" __device__ uint32_t __ockl_wfred_min_u32(uint32_t);
 extern "C" __device__ uint32_t __ockl_wfred_max_u32(uint32_t);
+extern "C" __device__ uint32_t __ockl_wfred_or_u32(uint32_t);
+extern "C" __device__ uint32_t __ockl_wfscan_add_u32(uint32_t, bool);
 
 namespace rzd {
 
@@ -662,24 +664,28 @@ struct ItemLocal {
   uint64_t groups;  // bit k: aligned 64-quad group (quadBase >> 6) + k may touch the tile
 };
 
-constexpr uint32_t kItemWindow = 128;
 constexpr uint32_t kQuadChunk = 64;   // records staged in LDS at a time
 constexpr uint32_t kNoWinner = 0xFFFFFFFFu;  // pixel winner of labelled draws: none
 // A scan pass tests one quad per thread: 64 * NW quads.
 
 template <int TBX, int TBY>
 struct TileSmem {
+  // Sizes that let two work-groups share a CU's 160 KB: a 16x16-block tile's
+  // depth leaves less room than an 8x8-block tile's.  A chunk of 64 small
+  // quads has about two rows a quad in a tile; one that needs more rows than
+  // the fold table holds is drawn in several passes.
+  static constexpr uint32_t kItemWindow = TBX * TBY > 64 ? 64 : 128;  // items gathered at a time
+  static constexpr int kEntryRows = TBX * TBY > 64 ? 112 : 256;
   uint64_t cov[4096];              // coverage table (Rasterizer.cpp:547-604)
   uint16_t depth[TBX * TBY * 64];  // the tile's depth, block-linear
   uint16_t hiz[TBX * TBY];
   ItemLocal items[kItemWindow];    // this window's items that touch the tile
   QuadRec recs[kQuadChunk];        // setup records of the quads being drawn
-  uint32_t qid[kQuadChunk];        // their frame quad numbers (labelled draws)
-  // Block-major draw (8x8-block tiles): per staged quad its rectangle in the
-  // tile and origin, and per tile row the folded edge offsets and depth
-  // samples at the rectangle's first column in the tile.
-  uint32_t qinfo[kQuadChunk][4];
-  float entry[(TBX == 8 && TBY == 8) ? kQuadChunk * TBY * 12 : 1];
+  uint32_t qid[TBX * TBY > 64 ? 1 : kQuadChunk];  // their frame quad numbers (labelled draws, 8x8-block tiles)
+  // Per tile row of each staged quad's rectangle, the folded edge offsets and
+  // depth samples at the rectangle's first column in the tile.
+  float entry[kEntryRows * 12];
+  uint16_t pairs[8][64];  // per wave: the (block, quad) pairs being drawn
   uint32_t wcnt[8];
   uint32_t part[2][8];
   // Early query answers (query-gated launches): per window item, a bit when
@@ -694,14 +700,14 @@ struct TileSmem {
 };
 
 // Wave that owns tile-local block (lbx, lby) while a chunk of quads is drawn:
-// diagonals, so that any horizontal or vertical run of blocks is shared by all
-// four waves.
+// diagonals, so that any horizontal or vertical run of blocks is shared by
+// all waves.
 template <int NW>
 __device__ __forceinline__ uint32_t block_owner(int lbx, int lby) { return uint32_t(lbx + lby) & uint32_t(NW - 1); }
 
-// Adds `step` to `s` n times (uniform n), each add rounded: the reference's
-// per-row and per-block folds (Rasterizer.cpp:1130-1131, 1145-1146).  IEEE
-// addition commutes, so step + s and s + step are the same operation.
+// Adds `step` to `s` n times, each add rounded: the reference's per-row and
+// per-block folds (Rasterizer.cpp:1130-1131, 1145-1146).  IEEE addition
+// commutes, so step + s and s + step are the same operation.
 __device__ __forceinline__ float fold_n(float s, float step, int n) {
   for (; n >= 8; n -= 8) {
     s = s + step; s = s + step; s = s + step; s = s + step;
@@ -711,558 +717,353 @@ __device__ __forceinline__ float fold_n(float s, float step, int n) {
   return s;
 }
 
-struct QuadConst {
-  uint32_t mode, maxZ;
-  uint32_t sl[4];
-  float dDx, dDy;
-};
-
-// One block of one quad (Rasterizer.cpp:1148-1290): hiZ reject, coverage
-// mask from the four edge lookups (Convex: any offset >= 63 rejects the block;
-// other modes: an empty mask does), depth rows 0/1 and 8/9 from the plane
-// with rows 2-7 as rounding-up averages, max-merge unless the block is
-// fast-cleared (hiZ == 1), hiZ = min.  `s` holds the folded edge offsets and
-// depth samples in lanes 12g .. 12g+11 (offsets first).  The rejections come
-// first and each only waits for the LDS reads it needs: most visited blocks
-// end at the hiZ test.
-// Per-wave counters of the block loop (observability builds only): blocks
-// visited, rejected by hiZ or by the edge tests, and written.
+// Per-wave counters of the block loop (observability builds only): (quad,
+// block) pairs visited, rejected by hiZ or by the edge tests, and written.
 struct BlockCounters {
   uint32_t visited = 0, rejected = 0, written = 0, foldSteps = 0;
 };
-
-template <int TBX, int TBY, bool STATS>
-__device__ __forceinline__ void raster_block(TileSmem<TBX, TBY>& sm, int lb, float s, int g, uint32_t lane,
-                                             int kLane, const QuadConst& Q, BlockCounters& bc) {
-  if (STATS) bc.visited++;
-  const uint32_t hz = sm.hiz[lb];
-  if (hz >= Q.maxZ) {
-    if (STATS) bc.rejected++;
-    return;
-  }
-  // Lane L looks up edge (L & 3): its folded offset from lane 12g + (L & 3),
-  // one coverage read, and lanes 0-3's words back to the wave as scalars.
-  const uint32_t e = lane & 3u;
-  const float oe = __shfl(s, 12 * g + int(e));
-  const bool convex = Q.mode == kModeConvex;
-  if (convex && (__ballot(oe >= 63.0f) & 0xFull) != 0ull) {
-    if (STATS) bc.rejected++;
-    return;
-  }
-  const uint32_t sl = e == 0u ? Q.sl[0] : e == 1u ? Q.sl[1] : e == 2u ? Q.sl[2] : Q.sl[3];
-  const int32_t t = cvtt_x86(oe);
-  const uint32_t tc = convex ? uint32_t(max(t, 0)) : uint32_t(min(max(t, 0), 63));
-  const uint64_t word = sm.cov[(sl | tc) & 4095u];
-  const uint64_t A = readlane_u64(word, 0), B = readlane_u64(word, 1), C = readlane_u64(word, 2),
-                 D = readlane_u64(word, 3);
-  uint64_t mask;
-  if (Q.mode == kModeConvex) mask = (A & B) & (C & D);
-  else if (Q.mode == kModeTriangle0) mask = A & B & C;
-  else if (Q.mode == kModeTriangle1) mask = A & C & D;
-  else if (Q.mode == kModeConcaveRight) mask = (A | D) & (B & C);
-  else if (Q.mode == kModeConcaveCenter) mask = (A & B) | (C & D);
-  else mask = (A & D) & (B | C);
-  if (Q.mode != kModeConvex && mask == 0) {
-    if (STATS) bc.rejected++;
-    return;
-  }
-  if (STATS) bc.written++;
-
-  const uint32_t old = sm.depth[lb * 64 + int(lane)];
-  float v = __shfl(s, 12 * g + 4 + kLane);
-  const uint32_t px = lane & 7u, py = lane >> 3;
-  if (px >= 4u) v = fmaf(Q.dDx, 0.5f, v);
-  const uint32_t lo = pack_depth(v);
-  const uint32_t hi = pack_depth(Q.dDy + v);
-  const uint32_t mid = avg_u16(lo, hi);
-  const uint32_t q1 = avg_u16(lo, mid), q3 = avg_u16(mid, hi);
-  const uint32_t j = py >> 1;
-  const uint32_t a01 = (j & 1u) ? q1 : lo, a23 = (j & 1u) ? q3 : mid;
-  uint32_t d = (j & 2u) ? a23 : a01;
-  const uint32_t maskBit = 8u * px + ((py & 1u) ? (py >> 1) : 4u + (py >> 1));
-  d = ((mask >> maskBit) & 1ull) ? d : 0u;
-  if (hz != 1u) d = max(d, old);
-  sm.depth[lb * 64 + int(lane)] = uint16_t(d);
-  const uint32_t mn = __ockl_wfred_min_u32(d);
-  if (lane == 0) sm.hiz[lb] = uint16_t(mn);
-}
-
-// Draws the blocks of one quad that this wave owns in the tile
-// (Rasterizer.cpp:1095-1292).  Blocks are independent, so the order among a
-// quad's blocks does not matter; the order among quads is the caller's.  The
-// per-block values are the reference's folds: the edge offsets and the eight
-// depth samples of rows 0/1 start at the rectangle origin, add the row step
-// once per block row, then the column step once per block column, each add
-// rounded.  Lane 12g + e carries component e (4 offsets, 8 depth samples) for
-// the g-th of up to five rows handled together.
-template <int TBX, int TBY, int NW, bool STATS>
-__device__ __forceinline__ void raster_quad_wave(const QuadRec& R, TileSmem<TBX, TBY>& sm, int tbx0, int tbx1,
-                                                 int tby0, int tby1, int bX, float invBX, uint32_t wave,
-                                                 uint32_t lane, BlockCounters& bc) {
-  const int fb = int(R.fb);
-  const int rangeX = int(R.range & 0xFFFFu), rangeY = int(R.range >> 16);
-  QuadConst Q;
-  Q.mode = R.modeZ & 0xFFu;
-  Q.maxZ = R.modeZ >> 16;
-  Q.sl[0] = R.slope01 & 0xFFFFu;
-  Q.sl[1] = R.slope01 >> 16;
-  Q.sl[2] = R.slope23 & 0xFFFFu;
-  Q.sl[3] = R.slope23 >> 16;
-  Q.dDx = R.dDx;
-  Q.dDy = R.dDy;
-  const int minY = div_bx(fb, bX, invBX), minX = fb - minY * bX;
-  const int kLane = int(((lane & 7u) & 3u) + 4u * ((lane >> 3) & 1u));
-
-  const uint32_t g = lane / 12u, e = lane - 12u * g;
-  float base, stepY, stepX;
-  if (e < 4) {
-    base = e == 0 ? R.off[0] : e == 1 ? R.off[1] : e == 2 ? R.off[2] : R.off[3];
-    stepY = e == 0 ? R.ny[0] : e == 1 ? R.ny[1] : e == 2 ? R.ny[2] : R.ny[3];
-    stepX = e == 0 ? R.nx[0] : e == 1 ? R.nx[1] : e == 2 ? R.nx[2] : R.nx[3];
-  } else {
-    const uint32_t k = e - 4;
-    const float spx = -0.4375f + 0.125f * float(k & 3u);
-    const float spy = -0.4375f + 0.125f * float(k >> 2);
-    base = fmaf(Q.dDx, spx, fmaf(Q.dDy, spy, R.dp0));
-    stepY = Q.dDy;
-    stepX = Q.dDx;
-  }
-
-  if (minX + rangeX > bX) {
-    // The 16-bit multiply of the first block index wrapped (Rasterizer.cpp:1054):
-    // the quad's blocks fb + r*bX + c no longer form a screen rectangle, so
-    // each owned block finds its (r, c) and folds from the origin.
-    for (int by = tby0; by <= tby1; ++by)
-      for (int bx = tbx0; bx <= tbx1; ++bx) {
-        if (block_owner<NW>(bx - tbx0, by - tby0) != wave) continue;
-        const int d = by * bX + bx - fb;
-        if (d < 0) continue;
-        const int r = div_bx(d, bX, invBX), c = d - r * bX;
-        if (r >= rangeY || c >= rangeX) continue;
-        const float s = fold_n(fold_n(base, stepY, r), stepX, c);
-        raster_block<TBX, TBY, STATS>(sm, (by - tby0) * TBX + (bx - tbx0), s, 0, lane, kLane, Q, bc);
-      }
-    return;
-  }
-  const int x0 = max(tbx0, minX), x1 = min(tbx1, minX + rangeX - 1);
-  const int y0 = max(tby0, minY), y1 = min(tby1, minY + rangeY - 1);
-  if (x0 > x1 || y0 > y1) return;
-  // Skip quads none of whose blocks in the tile belong to this wave.
-  if ((x1 - x0) + (y1 - y0) < 3) {
-    bool mine = false;
-    for (int by = y0; by <= y1; ++by)
-      for (int bx = x0; bx <= x1; ++bx) mine |= block_owner<NW>(bx - tbx0, by - tby0) == wave;
-    if (!mine) return;
-  }
-  const int cLo = x0 - minX;
-  // Lane group g starts at quad row (y0 - minY) + g.
-  float line = fold_n(base, stepY, y0 - minY);
-#pragma unroll
-  for (uint32_t i = 0; i < 4; ++i)
-    if (i < g) line = line + stepY;
-  for (int py = y0; py <= y1; py += 5) {
-    float s = fold_n(line, stepX, cLo);
-    for (int bx = x0; bx <= x1; ++bx, s = stepX + s) {
-      for (int gg = 0; gg < 5 && py + gg <= y1; ++gg) {
-        const int lbx = bx - tbx0, lby = py + gg - tby0;
-        if (block_owner<NW>(lbx, lby) != wave) continue;
-        raster_block<TBX, TBY, STATS>(sm, lby * TBX + lbx, s, gg, lane, kLane, Q, bc);
-      }
-    }
-    line = fold_n(line, stepY, 5);
-  }
-}
-
-// One block of one quad in the block-major draw, the part that depends on
-// nothing the previous quads wrote (Rasterizer.cpp:1148-1290): the four edge
-// lookups and the coverage mask (Convex blocks with an offset >= 63 and other
-// modes' empty masks set `skip`, the same in every lane), depth rows 0/1 and
-// 8/9 from the plane, packed averages between, 0 outside the mask.  `o` holds
-// the block's four folded edge offsets (the same values in every lane) and
-// `v` the lane's row-0/1 depth sample (sample kLane of the eight), as
-// raster_block reads them from its lane groups.  The hiZ reject and the merge
-// are the caller's, in submission order.
-__device__ __forceinline__ void sample_block(const uint64_t* __restrict__ cov, const float (&o)[4], float v,
-                                             uint32_t lane, const QuadConst& Q, uint32_t& dOut, bool& skip) {
-  const bool convex = Q.mode == kModeConvex;
-  bool outside = false;
-  uint32_t idx[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int32_t t = cvtt_x86(o[e]);
-    outside |= o[e] >= 63.0f;
-    const uint32_t tc = convex ? uint32_t(max(t, 0)) : uint32_t(min(max(t, 0), 63));
-    idx[e] = (Q.sl[e] | tc) & 4095u;
-  }
-  const uint64_t A = cov[idx[0]], B = cov[idx[1]], C = cov[idx[2]], D = cov[idx[3]];
-  const uint64_t mConvex = (A & B) & (C & D);
-  const uint64_t mTri0 = A & B & C, mTri1 = A & C & D;
-  const uint64_t mRight = (A | D) & (B & C), mCenter = (A & B) | (C & D), mLeft = (A & D) & (B | C);
-  const uint64_t mask = convex ? mConvex
-                        : Q.mode == kModeTriangle0 ? mTri0
-                        : Q.mode == kModeTriangle1 ? mTri1
-                        : Q.mode == kModeConcaveRight ? mRight
-                        : Q.mode == kModeConcaveCenter ? mCenter
-                                                       : mLeft;
-  // Every lane computes the same test from the same values; the ballot
-  // makes it a wave-uniform value for the caller's branch.
-  skip = __ballot(convex ? outside : mask == 0ull) != 0ull;
-  const uint32_t px = lane & 7u, py = lane >> 3;
-  if (px >= 4u) v = fmaf(Q.dDx, 0.5f, v);
-  const uint32_t lo = pack_depth(v);
-  const uint32_t hi = pack_depth(Q.dDy + v);
-  const uint32_t mid = avg_u16(lo, hi);
-  const uint32_t q1 = avg_u16(lo, mid), q3 = avg_u16(mid, hi);
-  const uint32_t j = py >> 1;
-  const uint32_t a01 = (j & 1u) ? q1 : lo, a23 = (j & 1u) ? q3 : mid;
-  const uint32_t d = (j & 2u) ? a23 : a01;
-  const uint32_t maskBit = 8u * px + ((py & 1u) ? (py >> 1) : 4u + (py >> 1));
-  dOut = ((mask >> maskBit) & 1ull) ? d : 0u;
-}
-
-
-// sample_block with the four edge lookups spread over the lanes: lane L
-// holds edge (L & 3)'s folded offset in `oe` and looks up its coverage word;
-// lanes 0-3's words come back to the wave as scalars, where the mode's mask
-// logic runs.  `sl01` / `sl23` are the quad's packed slope lookups.  The
-// same values as sample_block, with one LDS lookup instead of four and the
-// per-edge index arithmetic done once for all four edges.
-__device__ __forceinline__ void sample_block_lanes(const uint64_t* __restrict__ cov, float oe, float v, uint32_t lane,
-                                                   const QuadConst& Q, uint32_t sl01, uint32_t sl23, uint32_t& dOut,
-                                                   bool& skip) {
-  const bool convex = Q.mode == kModeConvex;
-  const uint32_t e = lane & 3u;
-  const uint32_t slw = (e & 2u) ? sl23 : sl01;
-  const uint32_t sl = (e & 1u) ? (slw >> 16) : (slw & 0xFFFFu);
-  const int32_t t = cvtt_x86(oe);
-  const uint32_t tc = convex ? uint32_t(max(t, 0)) : uint32_t(min(max(t, 0), 63));
-  const uint64_t word = cov[(sl | tc) & 4095u];
-  const uint64_t A = readlane_u64(word, 0), B = readlane_u64(word, 1), C = readlane_u64(word, 2),
-                 D = readlane_u64(word, 3);
-  const bool outside = (__ballot(oe >= 63.0f) & 0xFull) != 0ull;
-  uint64_t mask;
-  if (convex) mask = (A & B) & (C & D);
-  else if (Q.mode == kModeTriangle0) mask = A & B & C;
-  else if (Q.mode == kModeTriangle1) mask = A & C & D;
-  else if (Q.mode == kModeConcaveRight) mask = (A | D) & (B & C);
-  else if (Q.mode == kModeConcaveCenter) mask = (A & B) | (C & D);
-  else mask = (A & D) & (B | C);
-  skip = convex ? outside : mask == 0ull;
-  const uint32_t px = lane & 7u, py = lane >> 3;
-  if (px >= 4u) v = fmaf(Q.dDx, 0.5f, v);
-  const uint32_t lo = pack_depth(v);
-  const uint32_t hi = pack_depth(Q.dDy + v);
-  const uint32_t mid = avg_u16(lo, hi);
-  const uint32_t q1 = avg_u16(lo, mid), q3 = avg_u16(mid, hi);
-  const uint32_t j = py >> 1;
-  const uint32_t a01 = (j & 1u) ? q1 : lo, a23 = (j & 1u) ? q3 : mid;
-  const uint32_t d = (j & 2u) ? a23 : a01;
-  const uint32_t maskBit = 8u * px + ((py & 1u) ? (py >> 1) : 4u + (py >> 1));
-  dOut = ((mask >> maskBit) & 1ull) ? d : 0u;
-}
-
-// s + step, n times (0 <= n <= 7), each add rounded, without branches.
-__device__ __forceinline__ float fold_upto7(float s, float step, int n) {
-#pragma unroll
-  for (int k = 0; k < 7; ++k) s = k < n ? s + step : s;
-  return s;
-}
-
-__device__ __forceinline__ QuadConst quad_const(const QuadRec& R) {
-  QuadConst Q;
-  Q.mode = R.modeZ & 0xFFu;
-  Q.maxZ = R.modeZ >> 16;
-  Q.sl[0] = R.slope01 & 0xFFFFu;
-  Q.sl[1] = R.slope01 >> 16;
-  Q.sl[2] = R.slope23 & 0xFFFFu;
-  Q.sl[3] = R.slope23 >> 16;
-  Q.dDx = R.dDx;
-  Q.dDy = R.dDy;
-  return Q;
-}
 
 // Component e of a quad's fold at its rectangle origin and its row and column
 // steps: e < 4 edge offset e, else depth sample e - 4 (rows 0/1 of a block).
 __device__ __forceinline__ void quad_component(const QuadRec& R, uint32_t e, float& base, float& stepY,
                                                float& stepX) {
-  if (e < 4) {
-    base = e == 0 ? R.off[0] : e == 1 ? R.off[1] : e == 2 ? R.off[2] : R.off[3];
-    stepY = e == 0 ? R.ny[0] : e == 1 ? R.ny[1] : e == 2 ? R.ny[2] : R.ny[3];
-    stepX = e == 0 ? R.nx[0] : e == 1 ? R.nx[1] : e == 2 ? R.nx[2] : R.nx[3];
-  } else {
-    const uint32_t k = e - 4;
-    const float spx = -0.4375f + 0.125f * float(k & 3u);
-    const float spy = -0.4375f + 0.125f * float(k >> 2);
-    base = fmaf(R.dDx, spx, fmaf(R.dDy, spy, R.dp0));
-    stepY = R.dDy;
-    stepX = R.dDx;
+  const bool edge = e < 4u;
+  const float* at = edge ? &R.off[e] : &R.dp0;
+  stepY = *(edge ? &R.ny[e] : &R.dDy);
+  stepX = *(edge ? &R.nx[e] : &R.dDx);
+  base = *at;
+  if (!edge) {
+    const uint32_t k = e - 4u;
+    base = fmaf(stepX, -0.4375f + 0.125f * float(k & 3u), fmaf(stepY, -0.4375f + 0.125f * float(k >> 2), base));
   }
 }
 
-// Block-major draw of a staged chunk of n quads in an 8x8-block tile.
-// Phase A: each quad's rectangle in the tile, and for each of its rows in the
-// tile the twelve folded components at the rectangle's first column (row
-// steps from the origin, then column steps, each add rounded, as the block
-// loop folds them); quads are split over the waves.  Phase B: each wave walks
-// its blocks; for a block, lane q tests staged quad q against the block
-// (inside its rectangle, and not below the block's hiZ unless the block is
-// fast-cleared, since hiZ only grows once written), and the survivors are
-// drawn in submission order with the block's hiZ and depth in registers,
-// each finishing its fold with the column steps left.
+// Orders this wave's LDS writes before its later reads of other lanes' words.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Draws a staged chunk of n quads (Rasterizer.cpp:1095-1292), in passes of as
+// many quads as the fold table holds rows for.
+//
+// Phase A: for each row of each quad's rectangle in the tile, the twelve
+// folded components (edge offsets and the eight depth samples of block rows
+// 0/1) at the rectangle's first column, twelve lanes a row and five rows a
+// wave at a time, each folded from the quad's origin: row steps, then column
+// steps, each add rounded.
+//
+// Phase B: each wave lists the (quad, block) pairs of the blocks it owns,
+// block by block and within a block in submission order, 64 at a time: lane q
+// tests staged quad q against a block's rectangle and hiZ (a block that is
+// not fast-cleared only grows), and the pairs are compacted by ballot.  Then
+// one lane per pair finishes the pair's four edge folds with the column steps
+// left, looks up the four coverage words and forms the 64-pixel mask by the
+// quad's mode (Convex: any offset >= 63 rejects; other modes: an empty mask
+// does).  None of that depends on what earlier pairs write, so 64 pairs cost
+// one pass of about 150 instructions where a wave per pair took about that
+// much for each.  What is left runs pair by pair, lane = pixel, with the open
+// block's depth in registers: the hiZ reject, the depth rows 0/1 and 8/9 from
+// the plane with rows 2-7 as rounding-up averages, and the max-merge
+// (replacing while the block is fast-cleared, hiZ == 1).
+//
+// A block's state: until its first write in this chunk, the hiZ it was
+// opened with; after it, hiZ is the minimum of the depth in registers, so the
+// reject test is a ballot over the depth (hiZ >= maxZ exactly when no pixel
+// is below maxZ) and the fast-clear test (hiZ == 1) a flag kept by two
+// ballots.  The minimum itself is taken once, when the block is closed.
+//
+// A quad whose first block index wrapped in the reference's 16-bit multiply
+// (Rasterizer.cpp:1054) covers blocks fb + r * bX + c that form no screen
+// rectangle: each block finds its (r, c) and folds from the quad's origin.
 //
 // LABELS: each block's pixel winners (`winner`, the view's block-linear
 // array) are loaded with its depth unless the block is cleared (its first
 // write sets them all) and stored with it; quad q's batch is qid[q] / 8.
 //
-// Returns (observability builds) the s_memrealtime stamp at which phase B
-// started.
+// What bounds it: the instruction and LDS latency of the one wave that owns a
+// block, not bandwidth.  It replaces a draw of 16x16-block tiles quad by quad
+// (every wave folding every quad) and one of 8x8-block tiles that formed each
+// pair's mask with a whole wave.  Measured, before and after: a 3840x2160
+// frame of 12,000 icospheres (16x16-block tiles) 8.35 and 1.76 ms; 128 city
+// frames in flight (the same tiles) 19.4 and 13.4 ms a step with its
+// readbacks; one 1080p city frame (8x8-block tiles) 0.25-0.32 and
+// 0.24-0.28 ms.
+//
+// Returns (observability builds) the s_memrealtime stamp at which the last
+// phase B started.
 template <int TBX, int TBY, int NW, bool STATS, bool LABELS>
-__device__ uint64_t draw_chunk_block_major(TileSmem<TBX, TBY>& sm, uint32_t n, int tbx0, int tbx1, int tby0, int tby1,
-                                           int bX, float invBX, uint32_t wave, uint32_t lane, BlockCounters& bc,
-                                           uint32_t* __restrict__ winner) {
-  // The wave index as a scalar, so that block indices and fold counts
-  // derived from it are wave-uniform.
+__device__ uint64_t draw_chunk(TileSmem<TBX, TBY>& sm, uint32_t n, int tbx0, int tbx1, int tby0, int tby1, int bX,
+                               float invBX, uint32_t wave, uint32_t lane, BlockCounters& bc,
+                               uint32_t* __restrict__ winner) {
+  static_assert(TBX % NW == 0, "diagonal block ownership");
+  constexpr int kPerRow = TBX / NW, kOwned = kPerRow * TBY;  // the wave's blocks, row by row
+  constexpr int kRows = TileSmem<TBX, TBY>::kEntryRows;
+  // The wave index as a scalar, so that block indices derived from it are
+  // wave-uniform.
   wave = __builtin_amdgcn_readfirstlane(wave);
-  const uint32_t g = lane / 12u, e = lane - 12u * g;
-  for (uint32_t q = wave; q < n; q += NW) {
-    const QuadRec& R = sm.recs[q];
-    const int fb = int(R.fb);
-    const int rangeX = int(R.range & 0xFFFFu), rangeY = int(R.range >> 16);
-    const int minY = div_bx(fb, bX, invBX), minX = fb - minY * bX;
-    const bool wrap = minX + rangeX > bX;
-    int x0 = 0, x1 = TBX - 1, y0 = 0, y1 = TBY - 1;
-    if (!wrap) {
-      x0 = max(tbx0, minX) - tbx0;
-      x1 = min(tbx1, minX + rangeX - 1) - tbx0;
-      y0 = max(tby0, minY) - tby0;
-      y1 = min(tby1, minY + rangeY - 1) - tby0;
-    }
-    const bool empty = x0 > x1 || y0 > y1;
-    if (lane == 0) {
-      sm.qinfo[q][0] = empty ? 0xFFu : uint32_t(x0) | uint32_t(x1) << 8 | uint32_t(y0) << 16 | uint32_t(y1) << 24;
-      sm.qinfo[q][1] = uint32_t(minX);
-      sm.qinfo[q][2] = uint32_t(minY);
-      sm.qinfo[q][3] = wrap ? 1u : 0u;
-    }
-    if (wrap || empty) continue;
-    float base, stepY, stepX;
-    quad_component(R, e, base, stepY, stepX);
-    const int cLo = x0 + tbx0 - minX;
-    if (STATS && lane == 0) bc.foldSteps += uint32_t(y0 + tby0 - minY + ((y1 - y0) / 5 + 1) * (cLo + 5));
-    float line = fold_n(base, stepY, y0 + tby0 - minY);
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i)
-      if (i < g) line = line + stepY;
-    for (int r0 = y0; r0 <= y1; r0 += 5) {
-      const float sv = fold_n(line, stepX, cLo);
-      const int row = r0 + int(g);
-      if (g < 5u && row <= y1) sm.entry[(q * TBY + uint32_t(row)) * 12u + e] = sv;
-      line = fold_n(line, stepY, 5);
-    }
-  }
-  __syncthreads();
-  const uint64_t tB = STATS ? __builtin_amdgcn_s_memrealtime() : 0;
+  uint64_t tB = 0;
+
+  // Lane q: staged quad q's rectangle in the tile and its constants.
+  const bool have = lane < n;
+  const QuadRec& RL = sm.recs[have ? lane : 0u];
+  const int rangeX = int(RL.range & 0xFFFFu), rangeY = int(RL.range >> 16);
+  const int minY = div_bx(int(RL.fb), bX, invBX), minX = int(RL.fb) - minY * bX;
+  const bool wrap = have && minX + rangeX > bX;
+  const int x0 = wrap ? 0 : max(tbx0, minX) - tbx0, x1 = wrap ? TBX - 1 : min(tbx1, minX + rangeX - 1) - tbx0;
+  const int y0 = wrap ? 0 : max(tby0, minY) - tby0, y1 = wrap ? TBY - 1 : min(tby1, minY + rangeY - 1) - tby0;
+  const bool drawn = have && x0 <= x1 && y0 <= y1;
+  const uint32_t rows = drawn && !wrap ? uint32_t(y1 - y0 + 1) : 0u;
+  const uint32_t incl = __ockl_wfscan_add_u32(rows, true);  // fold table rows of quads 0..lane
+  const uint32_t maxZq = RL.modeZ >> 16;
+  const float dDxq = RL.dDx, dDyq = RL.dDy;
+  // Row and column steps from the quad's origin to the rectangle's.
+  const uint32_t steps = uint32_t(y0 + tby0 - minY) | uint32_t(x0 + tbx0 - minX) << 16;
 
   const int kLane = int(((lane & 7u) & 3u) + 4u * ((lane >> 3) & 1u));
-  const bool valid = lane < n;
-  // Lane q holds staged quad q's constants for phase B (read with readlane):
-  // its rectangle in the tile, wrap flag, mode and packed maximum depth,
-  // slope lookups and depth gradients.
-  const uint32_t rect = valid ? sm.qinfo[lane][0] : 0xFFu;
-  const uint32_t wrapq = valid ? sm.qinfo[lane][3] : 0u;
-  const uint32_t modeZq = valid ? sm.recs[lane].modeZ : 0u;
-  const uint32_t maxZq = modeZq >> 16;
-  const uint32_t sl01q = valid ? sm.recs[lane].slope01 : 0u, sl23q = valid ? sm.recs[lane].slope23 : 0u;
-  const float dDxq = valid ? sm.recs[lane].dDx : 0.0f, dDyq = valid ? sm.recs[lane].dDy : 0.0f;
-  const int qx0 = int(rect & 0xFFu), qx1 = int((rect >> 8) & 0xFFu);
-  const int qy0 = int((rect >> 16) & 0xFFu), qy1 = int(rect >> 24);
-  const uint32_t ce = lane < 12u ? lane : 0u;
-  // The wave's blocks: (lbx + lby) & (NW - 1) == wave, TBX / NW per row.
-  static_assert(TBX % NW == 0, "diagonal block ownership");
-  constexpr int kPerRow = TBX / NW, kOwned = TBX * TBY / NW;
-  // Two blocks are drawn at a time, two candidates per step: the samples
-  // depend on nothing the merges change, so they are computed together and
-  // only the merges run in submission order.
-  //
-  // A block's state: until its first write in this chunk, the hiZ it was
-  // opened with (which the reject test and the fast-clear test read); after
-  // it, hiZ is the minimum of the depth in registers, so the reject test is a
-  // ballot over the depth (hiZ >= maxZ exactly when no pixel is below maxZ)
-  // and the fast-clear test (hiZ == 1) a flag kept by two ballots.  The
-  // minimum itself is taken once, when the block is closed.
-  struct Slot {
-    int lb = 0;  // lbx = lb % TBX, lby = lb / TBX
+  const uint32_t px = lane & 7u, py = lane >> 3;
+  const uint32_t maskBit = 8u * px + ((py & 1u) ? (py >> 1) : 4u + (py >> 1));
+
+  for (uint32_t q0 = 0; q0 < n;) {
+    // Quads q0..q1-1 fit the table (a quad has at most TBY rows).
+    const int before = q0 ? int(readlane_u(incl, q0 - 1u)) : 0;
+    const bool inPass = have && lane >= q0 && int(incl) - before <= kRows;
+    const uint32_t q1 = q0 + uint32_t(__popcll(__ballot(inPass)));
+    const int nRows = int(readlane_u(incl, q1 - 1u)) - before;
+    const int rowBase = int(incl - rows) - before;  // table row of the rectangle's first row
+
+    const uint32_t g = lane / 12u, e = lane - 12u * g;
+    for (int j0 = int(wave) * 5; j0 < nRows; j0 += 5 * NW) {
+      // The quad of table row j: the number of quads that end at or before it.
+      uint32_t q = 0;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        const uint32_t qk = uint32_t(__popcll(__ballot(int(incl) - before <= j0 + k)));
+        q = g == uint32_t(k) ? qk : q;
+      }
+      const int j = j0 + int(g);
+      const bool ok = g < 5u && j < nRows;
+      q = ok ? q : q0;
+      const uint32_t st = uint32_t(__shfl(int(steps), int(q)));
+      const int first = __shfl(rowBase, int(q));
+      const int r = ok ? int(st & 0xFFFFu) + (j - first) : 0, c = ok ? int(st >> 16) : 0;
+      float base, stepY, stepX;
+      quad_component(sm.recs[q], e, base, stepY, stepX);
+      const float s = fold_n(fold_n(base, stepY, r), stepX, c);
+      if (ok) sm.entry[j * 12 + int(e)] = s;
+      if (STATS) bc.foldSteps += __ockl_wfred_max_u32(uint32_t(r + c));
+    }
+    __syncthreads();
+    if (STATS) tB = __builtin_amdgcn_s_memrealtime();
+
+    const bool valid = drawn && inPass;
+    // Lane k: hiZ of the wave's k-th block (and of its k+64-th).
+    auto owned = [&](int k) -> int {
+      const int lby = k / kPerRow;
+      return lby * TBX + int((wave - uint32_t(lby)) & uint32_t(NW - 1)) + NW * (k % kPerRow);
+    };
+    const uint32_t hz0 = int(lane) < kOwned ? uint32_t(sm.hiz[owned(int(lane))]) : 0u;
+    const uint32_t hz1 = kOwned > 64 ? uint32_t(sm.hiz[owned(int(lane) + 64)]) : 0u;
+    // What a pair's lane needs of its quad: first column, wrap flag and table
+    // row of tile row 0 (biased: it can be negative).
+    const uint32_t pairInfo = uint32_t(x0) | (wrap ? 0x100u : 0u) | uint32_t(rowBase - y0 + 1024) << 16;
+
+    // The open block.
+    int cur = -1;
     uint32_t hz = 0, dval = 0, win = kNoWinner;
     bool dirty = false, one = false;
-    uint64_t m = 0;  // candidates left, in submission order
-  };
-  int nextK = 0;
-  // Next owned block with candidates into S (false when none is left).
-  auto open = [&](Slot& S) -> bool {
-    while (nextK < kOwned) {
-      const int k = nextK++;
-      const int lby = k / kPerRow;
-      const int lbx = int((wave - uint32_t(lby)) & uint32_t(NW - 1)) + NW * (k % kPerRow);
-      const int lb = lby * TBX + lbx;
-      const uint32_t hz = sm.hiz[lb];
-      const bool inRect = valid && lbx >= qx0 && lbx <= qx1 && lby >= qy0 && lby <= qy1;
-      const bool cand = inRect && !(hz != 1u && hz >= maxZq);
-      const uint64_t m = __ballot(cand);
-      if (STATS) {
-        const uint32_t pre = uint32_t(__popcll(__ballot(inRect) & ~m));
-        bc.visited += pre;
-        bc.rejected += pre;
+    auto close = [&]() {
+      if (!dirty) return;
+      sm.depth[cur * 64 + int(lane)] = uint16_t(dval);
+      const uint32_t mn = __ockl_wfred_min_u32(dval);
+      if (lane == 0) sm.hiz[cur] = uint16_t(mn);
+      if (LABELS)
+        winner[(size_t(tby0 + cur / TBX) * size_t(bX) + size_t(tbx0 + cur % TBX)) * 64u + lane] = win;
+    };
+
+    // Rows of the tile that some quad of the pass touches.
+    uint32_t rowsLeft =
+        __ockl_wfred_or_u32(valid ? (2u << uint32_t(y1 & 31)) - (1u << uint32_t(y0 & 31)) : 0u);
+    const bool anyWrap = __ballot(valid && wrap) != 0ull;
+    int kx = kPerRow, lby = 0, lb = 0;
+    uint64_t m = 0;  // candidates of block lb not yet listed
+    bool inRow = false;
+    while (true) {
+      // Up to 64 pairs, as block << 6 | quad.
+      uint32_t fill = 0;
+      while (fill < 64u) {
+        if (m == 0ull) {
+          if (kx == kPerRow) {
+            if (rowsLeft == 0u) break;
+            lby = int(__builtin_ctz(rowsLeft));
+            rowsLeft &= rowsLeft - 1u;
+            kx = 0;
+            inRow = valid && lby >= y0 && lby <= y1;
+          }
+          const int k = lby * kPerRow + kx++;
+          lb = owned(k);
+          const int lbx = lb % TBX;
+          const uint32_t bhz = k < 64 ? readlane_u(hz0, uint32_t(k)) : readlane_u(hz1, uint32_t(k - 64));
+          bool inRect = inRow && lbx >= x0 && lbx <= x1;
+          if (anyWrap) {
+            const int dd = (tby0 + lby) * bX + tbx0 + lbx - int(RL.fb);
+            const int r = div_bx(max(dd, 0), bX, invBX);
+            if (wrap) inRect = inRect && dd >= 0 && r < rangeY && dd - r * bX < rangeX;
+          }
+          m = __ballot(inRect && !(bhz != 1u && bhz >= maxZq));
+          if (STATS) {
+            const uint32_t pre = uint32_t(__popcll(__ballot(inRect) & ~m));
+            bc.visited += pre;
+            bc.rejected += pre;
+          }
+          if (m == 0ull) continue;
+        }
+        const uint32_t pos =
+            fill + __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
+        const bool bit = (m >> lane) & 1ull;
+        if (bit && pos < 64u) sm.pairs[wave][pos] = uint16_t(uint32_t(lb) << 6 | lane);
+        const uint32_t cnt = uint32_t(__popcll(m));
+        m = fill + cnt > 64u ? __ballot(bit && pos >= 64u) : 0ull;
+        fill = min(fill + cnt, 64u);
       }
-      if (m == 0ull) continue;
-      S.lb = lb;
-      S.hz = hz;
-      S.m = m;
-      S.dval = sm.depth[lb * 64 + int(lane)];
-      S.dirty = false;
-      S.one = false;
-      S.win = kNoWinner;
-      if (LABELS && hz != 1u) S.win = winner[(size_t(tby0 + lby) * size_t(bX) + size_t(tbx0 + lbx)) * 64u + lane];
-      return true;
-    }
-    return false;
-  };
-  auto close = [&](const Slot& S) {
-    if (!S.dirty) return;
-    sm.depth[S.lb * 64 + int(lane)] = uint16_t(S.dval);
-    const uint32_t mn = __ockl_wfred_min_u32(S.dval);
-    if (lane == 0) sm.hiz[S.lb] = uint16_t(mn);
-    if (LABELS)
-      winner[(size_t(tby0 + S.lb / TBX) * size_t(bX) + size_t(tbx0 + S.lb % TBX)) * 64u + lane] = S.win;
-  };
-  auto qconst = [&](uint32_t q) -> QuadConst {
-    QuadConst Q;
-    const uint32_t mz = readlane_u(modeZq, q), s01 = readlane_u(sl01q, q), s23 = readlane_u(sl23q, q);
-    Q.mode = mz & 0xFFu;
-    Q.maxZ = mz >> 16;
-    Q.sl[0] = s01 & 0xFFFFu;
-    Q.sl[1] = s01 >> 16;
-    Q.sl[2] = s23 & 0xFFFFu;
-    Q.sl[3] = s23 >> 16;
-    Q.dDx = readlane_f(dDxq, q);
-    Q.dDy = readlane_f(dDyq, q);
-    return Q;
-  };
-  // Staged quad q's sample for block lb when its first-block index did not
-  // wrap: phase A's components at the rectangle's first column in this row,
-  // folded with the column steps left; every lane folds the four edge
-  // offsets and its own depth sample.
-  auto sample_fast = [&](int lb, uint32_t q, uint32_t& d, bool& skip) {
-    const QuadConst Q = qconst(q);
-    const int c = lb % TBX - int(readlane_u(rect, q) & 0xFFu);
-    const float* E = &sm.entry[(q * TBY + uint32_t(lb / TBX)) * 12u];
-    const float step = sm.recs[q].nx[lane & 3u];
-    float oe = E[lane & 3u];
-    float v = E[4 + kLane];
-    // c is wave-uniform (0..7): a scalar loop of two adds a step, the lane's
-    // edge offset and its depth sample.
-    for (int k = 0; k < c; ++k) {
-      oe = oe + step;
-      v = v + Q.dDx;
-    }
-    sample_block_lanes(sm.cov, oe, v, lane, Q, readlane_u(sl01q, q), readlane_u(sl23q, q), d, skip);
-  };
-  // Any staged quad: false when a quad with a wrapped first-block index does
-  // not cover the block; such a quad's block (row, column) in its block
-  // numbering is found and its twelve components folded from the origin.
-  auto sample_any = [&](int lb, uint32_t q, uint32_t& d, bool& skip) -> bool {
-    if (!(readlane_u(wrapq, q) & 1u)) {
-      sample_fast(lb, q, d, skip);
-      return true;
-    }
-    const QuadRec& R = sm.recs[q];
-    const int dd = (tby0 + lb / TBX) * bX + tbx0 + lb % TBX - int(R.fb);
-    const int rangeX = int(R.range & 0xFFFFu), rangeY = int(R.range >> 16);
-    if (dd < 0) return false;
-    const int r = div_bx(dd, bX, invBX), c = dd - r * bX;
-    if (r >= rangeY || c >= rangeX) return false;
-    float base, stepY, stepX;
-    quad_component(R, ce, base, stepY, stepX);
-    const float s = fold_n(fold_n(base, stepY, r), stepX, c);
-    float o[4];
+      if (fill == 0u) break;
+      wave_lds_fence();
+
+      // One lane per pair: coverage.
+      const bool active = lane < fill;
+      const uint32_t pr = active ? uint32_t(sm.pairs[wave][lane]) : uint32_t(sm.pairs[wave][0]);
+      const uint32_t pq = pr & 63u, pb = pr >> 6;
+      const QuadRec& R = sm.recs[pq];
+      const uint32_t info = uint32_t(__shfl(int(pairInfo), int(pq)));
+      const int plx = int(pb % TBX), ply = int(pb / TBX);
+      const bool pwrap = info & 0x100u;
+      const int pc = plx - int(info & 0xFFu);
+      const int row = int(info >> 16) - 1024 + ply;
+      float o[4], nx[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) o[k] = readlane_f(s, k);
-    const float v = __shfl(s, 4 + kLane);
-    sample_block(sm.cov, o, v, lane, qconst(q), d, skip);
-    return true;
-  };
-  // Candidate q of slot S, in submission order: the hiZ reject, then the
-  // merge (max unless the block is fast-cleared), Rasterizer.cpp:1148-1290.
-  //
-  // LABELS: `win` is the lane's pixel's winner, the batch whose write
-  // produced its depth: the first write of a cleared block (hiZ == 1) sets it
-  // (none where the written depth is 0), later writes only where they raise
-  // the depth.
-  auto visit = [&](Slot& S, uint32_t q, uint32_t d, bool skip) {
-    const uint32_t maxZ = readlane_u(maxZq, q);
-    if (STATS) bc.visited++;
-    const bool rejected = S.dirty ? __ballot(S.dval < maxZ) == 0ull : S.hz >= maxZ;
-    if (rejected || skip) {
-      if (STATS) bc.rejected++;
-      return;
+      for (int i = 0; i < 4; ++i) nx[i] = R.nx[i];
+      if (!pwrap) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = sm.entry[row * 12 + i];
+        for (int t = 0; t < pc; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = o[i] + nx[i];
+      } else {
+        const int dd = (tby0 + ply) * bX + tbx0 + plx - int(R.fb);
+        const int r = div_bx(dd, bX, invBX);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = fold_n(fold_n(R.off[i], R.ny[i], r), nx[i], dd - r * bX);
+      }
+      const uint32_t modeZ = R.modeZ, mode = modeZ & 0xFFu, s01 = R.slope01, s23 = R.slope23;
+      const bool convex = mode == kModeConvex;
+      bool outside = false;
+      uint64_t word[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int32_t t = cvtt_x86(o[i]);
+        outside |= o[i] >= 63.0f;
+        const uint32_t tc = uint32_t(max(t, 0));
+        const uint32_t sl = i == 0 ? s01 & 0xFFFFu : i == 1 ? s01 >> 16 : i == 2 ? s23 & 0xFFFFu : s23 >> 16;
+        word[i] = sm.cov[(sl | (convex ? tc : min(tc, 63u))) & 4095u];
+      }
+      const uint64_t A = word[0], B = word[1], C = word[2], D = word[3];
+      uint64_t mask;
+      if (mode == kModeConvex) mask = (A & B) & (C & D);
+      else if (mode == kModeTriangle0) mask = A & B & C;
+      else if (mode == kModeTriangle1) mask = A & C & D;
+      else if (mode == kModeConcaveRight) mask = (A | D) & (B & C);
+      else if (mode == kModeConcaveCenter) mask = (A & B) | (C & D);
+      else mask = (A & D) & (B | C);
+      const bool skip = convex ? outside : mask == 0ull;
+      uint64_t live = __ballot(active && !skip);
+      if (STATS) {
+        bc.visited += fill;
+        bc.rejected += fill - uint32_t(__popcll(live));
+      }
+      const uint32_t maskLo = uint32_t(mask), maskHi = uint32_t(mask >> 32);
+      // Address of the pair's depth samples, and the column steps to them.
+      const uint32_t sampleAt = uint32_t(row * 12 + 4), wrapBit = pwrap ? 1u : 0u;
+
+      // The pairs that cover pixels, in order; the next one's depth sample
+      // and block are loaded while this one is merged.
+      uint32_t l = 0;
+      float vNext = 0.0f;
+      uint32_t dNext = 0;
+      auto fetch = [&](uint32_t at) {
+        if (!readlane_u(wrapBit, at)) vNext = sm.entry[readlane_u(sampleAt, at) + uint32_t(kLane)];
+        dNext = sm.depth[readlane_u(pb, at) * 64u + lane];
+      };
+      if (live) {
+        l = uint32_t(__builtin_ctzll(live));
+        fetch(l);
+      }
+      while (live) {
+        live &= live - 1ull;
+        float v = vNext;
+        const uint32_t dBlock = dNext;
+        const uint32_t at = l;
+        if (live) {
+          l = uint32_t(__builtin_ctzll(live));
+          fetch(l);
+        }
+        const int b = int(readlane_u(pb, at));
+        if (b != cur) {
+          if (cur >= 0) close();
+          cur = b;
+          const int lby = b / TBX, kk = lby * kPerRow + (b % TBX) / NW;
+          hz = kOwned <= 64 || kk < 64 ? readlane_u(hz0, uint32_t(kk)) : readlane_u(hz1, uint32_t(kk - 64));
+          dval = dBlock;
+          dirty = one = false;
+          win = kNoWinner;
+          if (LABELS && hz != 1u)
+            win = winner[(size_t(tby0 + lby) * size_t(bX) + size_t(tbx0 + b % TBX)) * 64u + lane];
+        }
+        const uint32_t mz = readlane_u(modeZ, at) >> 16;
+        if (dirty ? __ballot(dval < mz) == 0ull : hz >= mz) {
+          if (STATS) bc.rejected++;
+          continue;
+        }
+        if (STATS) bc.written++;
+        const uint32_t q = readlane_u(pq, at);
+        const float dDx = readlane_f(dDxq, int(q)), dDy = readlane_f(dDyq, int(q));
+        if (!readlane_u(wrapBit, at)) {
+          const int c = int(readlane_u(uint32_t(pc), at));
+          for (int t = 0; t < c; ++t) v = v + dDx;
+        } else {
+          const int dd = (tby0 + b / TBX) * bX + tbx0 + b % TBX - int(sm.recs[q].fb);
+          const int r = div_bx(dd, bX, invBX);
+          float base, stepY, stepX;
+          quad_component(sm.recs[q], 4u + uint32_t(kLane), base, stepY, stepX);
+          v = fold_n(fold_n(base, stepY, r), stepX, dd - r * bX);
+        }
+        if (px >= 4u) v = fmaf(dDx, 0.5f, v);
+        const uint32_t lo = pack_depth(v);
+        const uint32_t hi = pack_depth(dDy + v);
+        const uint32_t mid = avg_u16(lo, hi);
+        const uint32_t q1s = avg_u16(lo, mid), q3s = avg_u16(mid, hi);
+        const uint32_t jr = py >> 1;
+        const uint32_t a01 = (jr & 1u) ? q1s : lo, a23 = (jr & 1u) ? q3s : mid;
+        const uint64_t pm = uint64_t(readlane_u(maskLo, at)) | uint64_t(readlane_u(maskHi, at)) << 32;
+        uint32_t d = ((pm >> maskBit) & 1ull) ? ((jr & 2u) ? a23 : a01) : 0u;
+        const bool cleared = dirty ? one : hz == 1u;
+        if (LABELS) {
+          // The first write of a cleared block sets every pixel's winner
+          // (none where the written depth is 0), later ones only where they
+          // raise the depth.
+          const uint32_t batch = sm.qid[q] >> 3;
+          win = cleared ? (d != 0u ? batch : kNoWinner) : (d > dval ? batch : win);
+        }
+        if (!cleared) d = max(d, dval);
+        dval = d;
+        // hiZ == 1 after this write: no pixel at 0 and one at 1.
+        one = __ballot(d == 0u) == 0ull && __ballot(d == 1u) != 0ull;
+        dirty = true;
+      }
+      wave_lds_fence();  // the pair list is reused
     }
-    if (STATS) bc.written++;
-    const bool cleared = S.dirty ? S.one : S.hz == 1u;
-    if (LABELS) {
-      const uint32_t batch = sm.qid[q] >> 3;
-      S.win = cleared ? (d != 0u ? batch : kNoWinner) : (d > S.dval ? batch : S.win);
-    }
-    if (!cleared) d = max(d, S.dval);
-    S.dval = d;
-    // hiZ == 1 after this write: no pixel at 0 and one at 1.
-    S.one = __ballot(d == 0u) == 0ull && __ballot(d == 1u) != 0ull;
-    S.dirty = true;
-  };
-  // Two samples per step: the next candidates of both open blocks, or the
-  // next two of the only open one (kept in A).
-  Slot A, B;
-  bool aOn = open(A), bOn = open(B);
-  while (aOn || bOn) {
-    if (!aOn) {
-      A = B;
-      aOn = true;
-      bOn = false;
-    }
-    // An open slot has at least one candidate left.
-    const uint32_t qa = uint32_t(__builtin_ctzll(A.m));
-    A.m &= A.m - 1ull;
-    uint32_t qb = 0;
-    const bool second = bOn || A.m != 0ull;
-    if (bOn) {
-      qb = uint32_t(__builtin_ctzll(B.m));
-      B.m &= B.m - 1ull;
-    } else if (second) {
-      qb = uint32_t(__builtin_ctzll(A.m));
-      A.m &= A.m - 1ull;
-    }
-    const int lbb = bOn ? B.lb : A.lb;
-    uint32_t da = 0, db = 0;
-    bool ka = true, kb = true, ca = true, cb = second;
-    if (!((readlane_u(wrapq, qa) | readlane_u(wrapq, qb)) & 1u)) {
-      // Without a second candidate, quad 0 is sampled and not used.
-      sample_fast(A.lb, qa, da, ka);
-      sample_fast(lbb, qb, db, kb);
-    } else {
-      ca = sample_any(A.lb, qa, da, ka);
-      cb = cb && sample_any(lbb, qb, db, kb);
-    }
-    if (ca) visit(A, qa, da, ka);
-    if (cb) {
-      if (bOn) visit(B, qb, db, kb);
-      else visit(A, qb, db, kb);
-    }
-    if (A.m == 0ull) {
-      close(A);
-      aOn = open(A);
-    }
-    if (bOn && B.m == 0ull) {
-      close(B);
-      bOn = open(B);
-    }
+    if (cur >= 0) close();
+    q0 = q1;
+    if (q0 < n) __syncthreads();  // the fold table is reused
   }
   return tB;
 }
@@ -1456,7 +1257,7 @@ template <int TBX, int TBY, int NW, bool STATS, bool LABELS>
 __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY>& sm,
                                              const uint64_t* __restrict__ cov, bool& covLoaded,
                                              uint64_t (&ctr)[kFrameStatWords]) {
-  static_assert(!LABELS || (TBX == 8 && TBY == 8), "labelled draws use the block-major draw");
+  static_assert(!LABELS || (TBX == 8 && TBY == 8), "only 8x8-block tiles hold quad numbers");
   auto stamp = []() -> uint64_t { return STATS ? __builtin_amdgcn_s_memrealtime() : 0; };
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const uint32_t tX = J.tX, tY = J.tY;
@@ -1475,6 +1276,7 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
 
   int involved = 0;
   constexpr uint32_t NT = 64u * NW;
+  constexpr uint32_t kItemWindow = TileSmem<TBX, TBY>::kItemWindow;
   static_assert(NT >= kItemWindow, "the item window gathers one item per thread");
   if (J.list) involved = nList > 0u;
   else
@@ -1719,24 +1521,16 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
           }
           __syncthreads();
           const uint64_t tDraw = stamp();
-          uint64_t tB = 0;
-          if constexpr (TBX == 8 && TBY == 8) {
-            tB = draw_chunk_block_major<TBX, TBY, NW, STATS, LABELS>(sm, n, tbx0, tbx1, tby0, tby1, bX, invBX, wave,
-                                                                     lane, bc, J.winner);
-          } else {
-            for (uint32_t q = 0; q < n; ++q)
-              raster_quad_wave<TBX, TBY, NW, STATS>(sm.recs[q], sm, tbx0, tbx1, tby0, tby1, bX, invBX, wave, lane, bc);
-          }
+          const uint64_t tB = draw_chunk<TBX, TBY, NW, STATS, LABELS>(sm, n, tbx0, tbx1, tby0, tby1, bX, invBX, wave,
+                                                                      lane, bc, J.winner);
           if (STATS && tid == 0) ctr[kStatQuads] += n;
           __syncthreads();
           if (STATS && tid == 0) {
             const uint64_t t = stamp();
             ctr[kStatDrawTicks] += t - tDraw;
             ctr[kStatChunks]++;
-            if (TBX == 8 && TBY == 8) {
-              ctr[kStatPhaseATicks] += tB - tDraw;
-              ctr[kStatPhaseBTicks] += t - tB;
-            }
+            ctr[kStatPhaseATicks] += tB - tDraw;
+            ctr[kStatPhaseBTicks] += t - tB;
           }
         }
       }
