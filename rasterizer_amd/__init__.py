@@ -784,10 +784,9 @@ class Views:
 
     def queries(self, view: int):
         n = self._nq[view]
-        vis = np.zeros(max(n, 1), np.uint8)
-        clip = np.zeros(max(n, 1), np.uint8)
+        vis, clip = np.empty((2, n), np.bool_)  # the flags are bytes of 0 or 1
         _check(lib().rz_views_read_queries(self._v, view, _ptr(vis), _ptr(clip)), "rz_views_read_queries")
-        return vis[:n].astype(bool), clip[:n].astype(bool)
+        return vis, clip
 
     def status(self, view: int) -> np.ndarray:
         n = len(self._occ[view])
