@@ -50,7 +50,11 @@ const HostTables& host_tables() {
   static std::once_flag once;
   std::call_once(once, [] {
     if (!rzh::build_coverage_table(t.cov)) t.status = RZ_ERR_UNSUPPORTED_HOST;
-    else if (rzh::build_rcp_table(t.rcp) != 0) t.status = RZ_ERR_UNSUPPORTED_HOST;
+    for (int i = 0; i < 4096; ++i) {
+      t.covLanes[i] = 0;
+      for (uint32_t lane = 0; lane < 64; ++lane) t.covLanes[i] |= ((t.cov[i] >> cov_bit_of_lane(lane)) & 1ull) << lane;
+    }
+    if (t.status == RZ_OK && rzh::build_rcp_table(t.rcp) != 0) t.status = RZ_ERR_UNSUPPORTED_HOST;
     if (rzh::build_rsqrt_table(t.rsqrt) != 0) t.rsqrtStatus = RZ_ERR_UNSUPPORTED_HOST;
   });
   return t;
@@ -204,7 +208,7 @@ extern "C" int rz_create(uint32_t width, uint32_t height, rz_context** out) {
       hipMemset(c->d_hiz, 0, (nBlocks + 8) * sizeof(uint16_t)) != hipSuccess ||
       hipMemset(c->d_tileMin, 0, size_t(c->pyrX) * c->pyrY * sizeof(uint16_t)) != hipSuccess ||
       hipMemset(c->d_err, 0, sizeof(uint32_t)) != hipSuccess ||
-      hipMemcpy(c->d_cov, tabs.cov, sizeof tabs.cov, hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(c->d_cov, tabs.covLanes, sizeof tabs.covLanes, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(c->d_rcp, tabs.rcp, sizeof tabs.rcp, hipMemcpyHostToDevice) != hipSuccess)
     return fail(RZ_ERR_DEVICE);
 
@@ -832,7 +836,16 @@ extern "C" int rz_get_info(rz_context* ctx, uint32_t info[6]) {
 
 extern "C" int rz_get_tables(rz_context* ctx, uint64_t* coverage4096, uint32_t* rcp4096) {
   if (!ctx) return RZ_ERR_INVALID_ARGUMENT;
-  if (coverage4096) RZ_HIP(hipMemcpy(coverage4096, ctx->d_cov, 4096 * 8, hipMemcpyDeviceToHost));
+  if (coverage4096) {
+    // The device's words hold their bits in lane order.
+    std::vector<uint64_t> words(4096);
+    RZ_HIP(hipMemcpy(words.data(), ctx->d_cov, 4096 * 8, hipMemcpyDeviceToHost));
+    for (int i = 0; i < 4096; ++i) {
+      coverage4096[i] = 0;
+      for (uint32_t lane = 0; lane < 64; ++lane)
+        coverage4096[i] |= ((words[size_t(i)] >> lane) & 1ull) << rzi::cov_bit_of_lane(lane);
+    }
+  }
   if (rcp4096) RZ_HIP(hipMemcpy(rcp4096, ctx->d_rcp, 4096 * 4, hipMemcpyDeviceToHost));
   return RZ_OK;
 }

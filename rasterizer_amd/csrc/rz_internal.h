@@ -59,11 +59,19 @@ void report_hip_error(hipError_t error, const char* call, const char* file, int 
 struct HostTables {
   int status = RZ_OK;
   uint64_t cov[4096];
+  uint64_t covLanes[4096];  // the same, each word's bits in the kernels' lane order
   uint32_t rcp[4096];
   int rsqrtStatus = RZ_OK;  // the device bake needs this host's RSQRTPS structure
   uint32_t rsqrt[8192];
 };
 const HostTables& host_tables();
+
+// Bit of a coverage word (the reference's transposed layout, Rasterizer.cpp:
+// 527-604) that belongs to lane L, the block's pixel (L & 7, L >> 3).
+inline uint32_t cov_bit_of_lane(uint32_t lane) {
+  const uint32_t x = lane & 7u, y = lane >> 3;
+  return 8u * x + ((y & 1u) ? (y >> 1) : 4u + (y >> 1));
+}
 
 // Autotuning cache (rz_tune.cpp): "<device>,<shape>" -> configuration text.
 std::string device_key(int device);

@@ -676,7 +676,9 @@ struct TileSmem {
   // the fold table holds is drawn in several passes.
   static constexpr uint32_t kItemWindow = TBX * TBY > 64 ? 64 : 128;  // items gathered at a time
   static constexpr int kEntryRows = TBX * TBY > 64 ? 112 : 256;
-  uint64_t cov[4096];              // coverage table (Rasterizer.cpp:547-604)
+  // Coverage table (Rasterizer.cpp:547-604), each word's bits in lane order:
+  // bit L is pixel (L & 7, L >> 3) of the block.
+  uint64_t cov[4096];
   uint16_t depth[TBX * TBY * 64];  // the tile's depth, block-linear
   uint16_t hiz[TBX * TBY];
   ItemLocal items[kItemWindow];    // this window's items that touch the tile
@@ -736,6 +738,11 @@ __device__ __forceinline__ void quad_component(const QuadRec& R, uint32_t e, flo
     const uint32_t k = e - 4u;
     base = fmaf(stepX, -0.4375f + 0.125f * float(k & 3u), fmaf(stepY, -0.4375f + 0.125f * float(k >> 2), base));
   }
+}
+
+// x in the lanes whose bit of the wave-uniform mask is set, 0 in the others.
+__device__ __forceinline__ uint32_t lane_select(uint64_t mask, uint32_t x) {
+  return __builtin_amdgcn_inverse_ballot_w64(mask) ? x : 0u;
 }
 
 // Orders this wave's LDS writes before its later reads of other lanes' words.
@@ -816,13 +823,13 @@ __device__ uint64_t draw_chunk(TileSmem<TBX, TBY>& sm, uint32_t n, int tbx0, int
   const uint32_t rows = drawn && !wrap ? uint32_t(y1 - y0 + 1) : 0u;
   const uint32_t incl = __ockl_wfscan_add_u32(rows, true);  // fold table rows of quads 0..lane
   const uint32_t maxZq = RL.modeZ >> 16;
-  const float dDxq = RL.dDx, dDyq = RL.dDy;
   // Row and column steps from the quad's origin to the rectangle's.
   const uint32_t steps = uint32_t(y0 + tby0 - minY) | uint32_t(x0 + tbx0 - minX) << 16;
 
-  const int kLane = int(((lane & 7u) & 3u) + 4u * ((lane >> 3) & 1u));
-  const uint32_t px = lane & 7u, py = lane >> 3;
-  const uint32_t maskBit = 8u * px + ((py & 1u) ? (py >> 1) : 4u + (py >> 1));
+  // The lane's pixel: its depth sample of the eight, and how its row comes
+  // from rows 0/1 and 8/9.
+  const int kLane = int((lane & 3u) + 4u * ((lane >> 3) & 1u));
+  const bool right = (lane & 4u) != 0u, low = (lane & 32u) != 0u, odd = (lane & 16u) != 0u;
 
   for (uint32_t q0 = 0; q0 < n;) {
     // Quads q0..q1-1 fit the table (a quad has at most TBY rows).
@@ -868,14 +875,17 @@ __device__ uint64_t draw_chunk(TileSmem<TBX, TBY>& sm, uint32_t n, int tbx0, int
     // row of tile row 0 (biased: it can be negative).
     const uint32_t pairInfo = uint32_t(x0) | (wrap ? 0x100u : 0u) | uint32_t(rowBase - y0 + 1024) << 16;
 
-    // The open block.
+    // The open block.  `test` is what the hiZ reject compares with a quad's
+    // maximum depth in every lane: the block's hiZ until its first write here,
+    // then its depth.  `floor` is what a write is merged with: 0 while the
+    // block reads as fast-cleared, else its depth.
     int cur = -1;
-    uint32_t hz = 0, dval = 0, win = kNoWinner;
-    bool dirty = false, one = false;
+    uint32_t test = 0, floor = 0, win = kNoWinner;
+    bool dirty = false, cleared = false;
     auto close = [&]() {
       if (!dirty) return;
-      sm.depth[cur * 64 + int(lane)] = uint16_t(dval);
-      const uint32_t mn = __ockl_wfred_min_u32(dval);
+      sm.depth[cur * 64 + int(lane)] = uint16_t(test);
+      const uint32_t mn = __ockl_wfred_min_u32(test);
       if (lane == 0) sm.hiz[cur] = uint16_t(mn);
       if (LABELS)
         winner[(size_t(tby0 + cur / TBX) * size_t(bX) + size_t(tbx0 + cur % TBX)) * 64u + lane] = win;
@@ -955,113 +965,126 @@ __device__ uint64_t draw_chunk(TileSmem<TBX, TBY>& sm, uint32_t n, int tbx0, int
         for (int i = 0; i < 4; ++i) o[i] = fold_n(fold_n(R.off[i], R.ny[i], r), nx[i], dd - r * bX);
       }
       const uint32_t modeZ = R.modeZ, mode = modeZ & 0xFFu, s01 = R.slope01, s23 = R.slope23;
+      float pdDx = R.dDx, pdDy = R.dDy;
       const bool convex = mode == kModeConvex;
-      bool outside = false;
       uint64_t word[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int32_t t = cvtt_x86(o[i]);
-        outside |= o[i] >= 63.0f;
-        const uint32_t tc = uint32_t(max(t, 0));
+        const uint32_t tc = uint32_t(max(cvtt_x86(o[i]), 0));
         const uint32_t sl = i == 0 ? s01 & 0xFFFFu : i == 1 ? s01 >> 16 : i == 2 ? s23 & 0xFFFFu : s23 >> 16;
         word[i] = sm.cov[(sl | (convex ? tc : min(tc, 63u))) & 4095u];
       }
       const uint64_t A = word[0], B = word[1], C = word[2], D = word[3];
-      uint64_t mask;
-      if (mode == kModeConvex) mask = (A & B) & (C & D);
-      else if (mode == kModeTriangle0) mask = A & B & C;
-      else if (mode == kModeTriangle1) mask = A & C & D;
-      else if (mode == kModeConcaveRight) mask = (A | D) & (B & C);
-      else if (mode == kModeConcaveCenter) mask = (A & B) | (C & D);
-      else mask = (A & D) & (B | C);
-      const bool skip = convex ? outside : mask == 0ull;
-      uint64_t live = __ballot(active && !skip);
+      // Convex, or one triangle (which leaves an edge out); concave quads are
+      // rare enough for a branch of their own.
+      uint64_t mask = (A & C) & ((B | (mode == kModeTriangle1 ? ~0ull : 0ull)) & (D | (mode == kModeTriangle0 ? ~0ull : 0ull)));
+      const bool concave = mode >= kModeConcaveRight && mode <= kModeConcaveCenter;
+      if (__ballot(concave) != 0ull && concave)
+        mask = mode == kModeConcaveRight    ? (A | D) & (B & C)
+               : mode == kModeConcaveCenter ? (A & B) | (C & D)
+                                            : (A & D) & (B | C);
+      // Any offset >= 63 (a NaN is not): fmaxf leaves NaNs out.
+      const bool outside = fmaxf(fmaxf(o[0], o[1]), fmaxf(o[2], o[3])) >= 63.0f;
+      const uint64_t cm = __ballot(convex);
+      uint64_t live = __ballot(active) & ((cm & ~__ballot(outside)) | (~cm & __ballot(mask != 0ull)));
       if (STATS) {
         bc.visited += fill;
         bc.rejected += fill - uint32_t(__popcll(live));
       }
+      // What the pair's turn needs, as scalars by readlane: block, column steps
+      // to its samples, wrap flag and maximum depth; its depth gradients, its
+      // mask (one bit a lane) and where its samples are (any address when
+      // wrapped).
+      const uint32_t desc = pb | uint32_t(pwrap ? 0 : pc) << 8 | (pwrap ? 0x1000u : 0u) | (modeZ & 0xFFFF0000u);
       const uint32_t maskLo = uint32_t(mask), maskHi = uint32_t(mask >> 32);
-      // Address of the pair's depth samples, and the column steps to them.
-      const uint32_t sampleAt = uint32_t(row * 12 + 4), wrapBit = pwrap ? 1u : 0u;
+      const uint32_t sampleAt = pwrap ? 0u : uint32_t(row * 12 + 4);
+      // Loaded before the loop, whose waits would otherwise cover its prefetches.
+      asm volatile("" : "+v"(pdDx), "+v"(pdDy));
 
       // The pairs that cover pixels, in order; the next one's depth sample
       // and block are loaded while this one is merged.
-      uint32_t l = 0;
+      uint32_t at = 0, ds = 0, dNext = 0;
       float vNext = 0.0f;
-      uint32_t dNext = 0;
-      auto fetch = [&](uint32_t at) {
-        if (!readlane_u(wrapBit, at)) vNext = sm.entry[readlane_u(sampleAt, at) + uint32_t(kLane)];
-        dNext = sm.depth[readlane_u(pb, at) * 64u + lane];
+      auto fetch = [&]() {
+        at = uint32_t(__builtin_ctzll(live));
+        ds = readlane_u(desc, at);
+        vNext = sm.entry[readlane_u(sampleAt, at) + uint32_t(kLane)];
+        dNext = sm.depth[(ds & 0xFFu) * 64u + lane];
       };
-      if (live) {
-        l = uint32_t(__builtin_ctzll(live));
-        fetch(l);
-      }
+      if (live) fetch();
       while (live) {
         live &= live - 1ull;
+        const uint32_t turn = at, dsc = ds, dBlock = dNext;
         float v = vNext;
-        const uint32_t dBlock = dNext;
-        const uint32_t at = l;
-        if (live) {
-          l = uint32_t(__builtin_ctzll(live));
-          fetch(l);
-        }
-        const int b = int(readlane_u(pb, at));
+        if (live) fetch();
+        const int b = int(dsc & 0xFFu);
         if (b != cur) {
-          if (cur >= 0) close();
+          close();
           cur = b;
-          const int lby = b / TBX, kk = lby * kPerRow + (b % TBX) / NW;
-          hz = kOwned <= 64 || kk < 64 ? readlane_u(hz0, uint32_t(kk)) : readlane_u(hz1, uint32_t(kk - 64));
-          dval = dBlock;
-          dirty = one = false;
-          win = kNoWinner;
-          if (LABELS && hz != 1u)
-            win = winner[(size_t(tby0 + lby) * size_t(bX) + size_t(tbx0 + b % TBX)) * 64u + lane];
+          const int by = b / TBX, kk = by * kPerRow + (b % TBX) / NW;
+          const uint32_t hz = kOwned <= 64 || kk < 64 ? readlane_u(hz0, uint32_t(kk)) : readlane_u(hz1, uint32_t(kk - 64));
+          dirty = false;
+          cleared = hz == 1u;
+          test = hz;
+          floor = cleared ? 0u : dBlock;
+          if (LABELS) {
+            win = kNoWinner;
+            if (!cleared) win = winner[(size_t(tby0 + by) * size_t(bX) + size_t(tbx0 + b % TBX)) * 64u + lane];
+          }
         }
-        const uint32_t mz = readlane_u(modeZ, at) >> 16;
-        if (dirty ? __ballot(dval < mz) == 0ull : hz >= mz) {
+        if (__ballot(test < (dsc >> 16)) == 0ull) {
           if (STATS) bc.rejected++;
           continue;
         }
         if (STATS) bc.written++;
-        const uint32_t q = readlane_u(pq, at);
-        const float dDx = readlane_f(dDxq, int(q)), dDy = readlane_f(dDyq, int(q));
-        if (!readlane_u(wrapBit, at)) {
-          const int c = int(readlane_u(uint32_t(pc), at));
-          for (int t = 0; t < c; ++t) v = v + dDx;
+        const float dDx = readlane_f(pdDx, int(turn)), dDy = readlane_f(pdDy, int(turn));
+        if (__builtin_expect(!(dsc & 0x1000u), 1)) {
+          if (TBX > 8 && (dsc & 0x800u)) {
+            v = v + dDx; v = v + dDx; v = v + dDx; v = v + dDx;
+            v = v + dDx; v = v + dDx; v = v + dDx; v = v + dDx;
+          }
+          if (dsc & 0x400u) {
+            v = v + dDx; v = v + dDx; v = v + dDx; v = v + dDx;
+          }
+          if (dsc & 0x200u) {
+            v = v + dDx; v = v + dDx;
+          }
+          if (dsc & 0x100u) v = v + dDx;
         } else {
-          const int dd = (tby0 + b / TBX) * bX + tbx0 + b % TBX - int(sm.recs[q].fb);
+          const QuadRec& W = sm.recs[readlane_u(pq, turn)];
+          const int dd = (tby0 + b / TBX) * bX + tbx0 + b % TBX - int(W.fb);
           const int r = div_bx(dd, bX, invBX);
           float base, stepY, stepX;
-          quad_component(sm.recs[q], 4u + uint32_t(kLane), base, stepY, stepX);
+          quad_component(W, 4u + uint32_t(kLane), base, stepY, stepX);
           v = fold_n(fold_n(base, stepY, r), stepX, dd - r * bX);
         }
-        if (px >= 4u) v = fmaf(dDx, 0.5f, v);
-        const uint32_t lo = pack_depth(v);
-        const uint32_t hi = pack_depth(dDy + v);
-        const uint32_t mid = avg_u16(lo, hi);
-        const uint32_t q1s = avg_u16(lo, mid), q3s = avg_u16(mid, hi);
-        const uint32_t jr = py >> 1;
-        const uint32_t a01 = (jr & 1u) ? q1s : lo, a23 = (jr & 1u) ? q3s : mid;
-        const uint64_t pm = uint64_t(readlane_u(maskLo, at)) | uint64_t(readlane_u(maskHi, at)) << 32;
-        uint32_t d = ((pm >> maskBit) & 1ull) ? ((jr & 2u) ? a23 : a01) : 0u;
-        const bool cleared = dirty ? one : hz == 1u;
+        // Rows 0/1 and 8/9 from the plane, rows 2-7 as PAVGW of them.
+        if (right) v = fmaf(dDx, 0.5f, v);
+        const uint32_t top = pack_depth(v), bottom = pack_depth(dDy + v);
+        const uint32_t mid = avg_u16(top, bottom), mean = avg_u16(low ? bottom : top, mid);
+        const uint32_t row = odd ? mean : (low ? mid : top);
+        const uint64_t pm = uint64_t(readlane_u(maskLo, turn)) | uint64_t(readlane_u(maskHi, turn)) << 32;
+        const uint32_t drawnDepth = lane_select(pm, row);
         if (LABELS) {
           // The first write of a cleared block sets every pixel's winner
           // (none where the written depth is 0), later ones only where they
           // raise the depth.
-          const uint32_t batch = sm.qid[q] >> 3;
-          win = cleared ? (d != 0u ? batch : kNoWinner) : (d > dval ? batch : win);
+          const uint32_t batch = sm.qid[readlane_u(pq, turn)] >> 3;
+          win = cleared ? (drawnDepth != 0u ? batch : kNoWinner) : (drawnDepth > floor ? batch : win);
         }
-        if (!cleared) d = max(d, dval);
-        dval = d;
-        // hiZ == 1 after this write: no pixel at 0 and one at 1.
-        one = __ballot(d == 0u) == 0ull && __ballot(d == 1u) != 0ull;
+        test = floor = max(drawnDepth, floor);
         dirty = true;
+        cleared = false;
+        // hiZ == 1 after this write (no pixel at 0 and one at 1) reads as
+        // fast-cleared to the next one.
+        if (__ballot(test == 0u) == 0ull && __ballot(test == 1u) != 0ull) {
+          cleared = true;
+          floor = 0u;
+        }
       }
       wave_lds_fence();  // the pair list is reused
     }
-    if (cur >= 0) close();
+    close();
     q0 = q1;
     if (q0 < n) __syncthreads();  // the fold table is reused
   }

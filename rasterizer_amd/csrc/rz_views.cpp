@@ -301,7 +301,7 @@ extern "C" int rz_views_create(uint32_t nViews, const uint32_t* widths, const ui
   if (hipHostGetDevicePointer(reinterpret_cast<void**>(&v->d_hErr), v->h_err, 0) != hipSuccess)
     return fail(RZ_ERR_DEVICE);
   if (const char* mode = std::getenv("RZ_FRAME_LAUNCH")) v->cooperative = std::strcmp(mode, "plain") != 0;
-  if (hipMemcpy(v->d_cov, tabs.cov, sizeof tabs.cov, hipMemcpyHostToDevice) != hipSuccess ||
+  if (hipMemcpy(v->d_cov, tabs.covLanes, sizeof tabs.covLanes, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(v->d_rcp, tabs.rcp, sizeof tabs.rcp, hipMemcpyHostToDevice) != hipSuccess)
     return fail(RZ_ERR_DEVICE);
   v->views.resize(nViews);

@@ -133,6 +133,6 @@ __device__ __forceinline__ uint32_t pack_depth(float d) {
   return v < 0 ? 0u : (v > 65535 ? 65535u : uint32_t(v));
 }
 
-__device__ __forceinline__ uint32_t avg_u16(uint32_t a, uint32_t b) { return (a + b + 1u) >> 1; }
+__device__ __forceinline__ uint32_t avg_u16(uint32_t a, uint32_t b) { return __builtin_amdgcn_ubfe(a + b + 1u, 1u, 16u); }
 
 }  // namespace rzd
