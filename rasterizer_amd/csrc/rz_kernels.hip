@@ -22,6 +22,7 @@
 
 extern "C" __device__ uint32_t __ockl_wfred_min_u32(uint32_t);
 extern "C" __device__ uint32_t __ockl_wfred_max_u32(uint32_t);
+extern "C" __device__ uint32_t __ockl_wfred_add_u32(uint32_t);
 extern "C" __device__ uint32_t __ockl_wfred_or_u32(uint32_t);
 extern "C" __device__ uint32_t __ockl_wfscan_add_u32(uint32_t, bool);
 
@@ -760,25 +761,26 @@ __device__ __forceinline__ void wave_lds_fence() {
 // wave at a time, each folded from the quad's origin: row steps, then column
 // steps, each add rounded.
 //
-// Phase B: each wave lists the (quad, block) pairs of the blocks it owns,
-// block by block and within a block in submission order, 64 at a time: lane q
-// tests staged quad q against a block's rectangle and hiZ (a block that is
-// not fast-cleared only grows), and the pairs are compacted by ballot.  Then
-// one lane per pair finishes the pair's four edge folds with the column steps
-// left, looks up the four coverage words and forms the 64-pixel mask by the
-// quad's mode (Convex: any offset >= 63 rejects; other modes: an empty mask
-// does).  None of that depends on what earlier pairs write, so 64 pairs cost
-// one pass of about 150 instructions where a wave per pair took about that
-// much for each.  What is left runs pair by pair, lane = pixel, with the open
+// Phase B: each wave lists the (quad, block) pairs of the blocks it owns, up
+// to 64 at a time in submission order: lane q turns quad q's rectangle into
+// one bit per owned block and writes its pairs behind those of the quads
+// before it.  Then one lane per pair tests the block's hiZ, finishes the
+// pair's four edge folds with the column steps left, looks up the four
+// coverage words and forms the 64-pixel mask by the quad's mode (Convex: any
+// offset >= 63 rejects; other modes: an empty mask does).  None of that
+// depends on what earlier pairs write (a block that is not fast-cleared only
+// grows), so 64 pairs cost one pass of about 150 instructions where a wave
+// per pair took about that much for each.  What is left runs block by block
+// and within a block pair by pair in submission order, lane = pixel, with the
 // block's depth in registers: the hiZ reject, the depth rows 0/1 and 8/9 from
 // the plane with rows 2-7 as rounding-up averages, and the max-merge
 // (replacing while the block is fast-cleared, hiZ == 1).
 //
-// A block's state: until its first write in this chunk, the hiZ it was
-// opened with; after it, hiZ is the minimum of the depth in registers, so the
-// reject test is a ballot over the depth (hiZ >= maxZ exactly when no pixel
-// is below maxZ) and the fast-clear test (hiZ == 1) a flag kept by two
-// ballots.  The minimum itself is taken once, when the block is closed.
+// A block's state: until its first write, the hiZ it was opened with; after
+// it, hiZ is the minimum of the depth in registers, so the reject test is a
+// ballot over the depth (hiZ >= maxZ exactly when no pixel is below maxZ) and
+// the fast-clear test (hiZ == 1) two ballots.  The minimum itself is taken
+// once, when the block is closed.
 //
 // A quad whose first block index wrapped in the reference's 16-bit multiply
 // (Rasterizer.cpp:1054) covers blocks fb + r * bX + c that form no screen
@@ -788,14 +790,13 @@ __device__ __forceinline__ void wave_lds_fence() {
 // array) are loaded with its depth unless the block is cleared (its first
 // write sets them all) and stored with it; quad q's batch is qid[q] / 8.
 //
-// What bounds it: the instruction and LDS latency of the one wave that owns a
-// block, not bandwidth.  It replaces a draw of 16x16-block tiles quad by quad
-// (every wave folding every quad) and one of 8x8-block tiles that formed each
-// pair's mask with a whole wave.  Measured, before and after: a 3840x2160
-// frame of 12,000 icospheres (16x16-block tiles) 8.35 and 1.76 ms; 128 city
-// frames in flight (the same tiles) 19.4 and 13.4 ms a step with its
-// readbacks; one 1080p city frame (8x8-block tiles) 0.25-0.32 and
-// 0.24-0.28 ms.
+// What bounds it: instruction issue and LDS latency of the waves that own a
+// busy tile's blocks, not bandwidth.  Before, 16x16-block tiles drew quad by
+// quad (every wave folding every quad) and 8x8-block tiles formed each pair's
+// mask with a whole wave.  Measured, before and after: a 3840x2160 frame of
+// 12,000 icospheres (16x16-block tiles) 8.40 and 1.35 ms; the raster launch
+// of 128 city frames in flight (the same tiles) 11.0 and 5.0 ms; one 1080p
+// city frame (8x8-block tiles) 0.32 and 0.26 ms.
 //
 // Returns (observability builds) the s_memrealtime stamp at which the last
 // phase B started.
@@ -804,7 +805,8 @@ __device__ uint64_t draw_chunk(TileSmem<TBX, TBY>& sm, uint32_t n, int tbx0, int
                                float invBX, uint32_t wave, uint32_t lane, BlockCounters& bc,
                                uint32_t* __restrict__ winner) {
   static_assert(TBX % NW == 0, "diagonal block ownership");
-  constexpr int kPerRow = TBX / NW, kOwned = kPerRow * TBY;  // the wave's blocks, row by row
+  constexpr int kPerRow = TBX / NW;  // the wave's blocks in a row
+  constexpr int kGroupRows = kPerRow * TBY <= 32 ? TBY : 32 / kPerRow;
   constexpr int kRows = TileSmem<TBX, TBY>::kEntryRows;
   // The wave index as a scalar, so that block indices derived from it are
   // wave-uniform.
@@ -864,227 +866,235 @@ __device__ uint64_t draw_chunk(TileSmem<TBX, TBY>& sm, uint32_t n, int tbx0, int
     if (STATS) tB = __builtin_amdgcn_s_memrealtime();
 
     const bool valid = drawn && inPass;
-    // Lane k: hiZ of the wave's k-th block (and of its k+64-th).
-    auto owned = [&](int k) -> int {
-      const int lby = k / kPerRow;
-      return lby * TBX + int((wave - uint32_t(lby)) & uint32_t(NW - 1)) + NW * (k % kPerRow);
-    };
-    const uint32_t hz0 = int(lane) < kOwned ? uint32_t(sm.hiz[owned(int(lane))]) : 0u;
-    const uint32_t hz1 = kOwned > 64 ? uint32_t(sm.hiz[owned(int(lane) + 64)]) : 0u;
+    const bool anyWrap = __ballot(valid && wrap) != 0ull;
     // What a pair's lane needs of its quad: first column, wrap flag and table
     // row of tile row 0 (biased: it can be negative).
     const uint32_t pairInfo = uint32_t(x0) | (wrap ? 0x100u : 0u) | uint32_t(rowBase - y0 + 1024) << 16;
+    const uint32_t colBits = valid ? (2u << (uint32_t(x1) & 31u)) - (1u << (uint32_t(x0) & 31u)) : 0u;
+    const uint32_t rowBits = valid ? (2u << (uint32_t(y1) & 31u)) - (1u << (uint32_t(y0) & 31u)) : 0u;
 
-    // The open block.  `test` is what the hiZ reject compares with a quad's
-    // maximum depth in every lane: the block's hiZ until its first write here,
-    // then its depth.  `floor` is what a write is merged with: 0 while the
-    // block reads as fast-cleared, else its depth.
-    int cur = -1;
-    uint32_t test = 0, floor = 0, win = kNoWinner;
-    bool dirty = false, cleared = false;
-    auto close = [&]() {
-      if (!dirty) return;
-      sm.depth[cur * 64 + int(lane)] = uint16_t(test);
-      const uint32_t mn = __ockl_wfred_min_u32(test);
-      if (lane == 0) sm.hiz[cur] = uint16_t(mn);
-      if (LABELS)
-        winner[(size_t(tby0 + cur / TBX) * size_t(bX) + size_t(tbx0 + cur % TBX)) * 64u + lane] = win;
-    };
-
-    // Rows of the tile that some quad of the pass touches.
-    uint32_t rowsLeft =
-        __ockl_wfred_or_u32(valid ? (2u << uint32_t(y1 & 31)) - (1u << uint32_t(y0 & 31)) : 0u);
-    const bool anyWrap = __ballot(valid && wrap) != 0ull;
-    int kx = kPerRow, lby = 0, lb = 0;
-    uint64_t m = 0;  // candidates of block lb not yet listed
-    bool inRow = false;
-    while (true) {
-      // Up to 64 pairs, as block << 6 | quad.
-      uint32_t fill = 0;
-      while (fill < 64u) {
-        if (m == 0ull) {
-          if (kx == kPerRow) {
-            if (rowsLeft == 0u) break;
-            lby = int(__builtin_ctz(rowsLeft));
-            rowsLeft &= rowsLeft - 1u;
-            kx = 0;
-            inRow = valid && lby >= y0 && lby <= y1;
-          }
-          const int k = lby * kPerRow + kx++;
-          lb = owned(k);
-          const int lbx = lb % TBX;
-          const uint32_t bhz = k < 64 ? readlane_u(hz0, uint32_t(k)) : readlane_u(hz1, uint32_t(k - 64));
-          bool inRect = inRow && lbx >= x0 && lbx <= x1;
-          if (anyWrap) {
-            const int dd = (tby0 + lby) * bX + tbx0 + lbx - int(RL.fb);
-            const int r = div_bx(max(dd, 0), bX, invBX);
-            if (wrap) inRect = inRect && dd >= 0 && r < rangeY && dd - r * bX < rangeX;
-          }
-          m = __ballot(inRect && !(bhz != 1u && bhz >= maxZq));
-          if (STATS) {
-            const uint32_t pre = uint32_t(__popcll(__ballot(inRect) & ~m));
-            bc.visited += pre;
-            bc.rejected += pre;
-          }
-          if (m == 0ull) continue;
-        }
-        const uint32_t pos =
-            fill + __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
-        const bool bit = (m >> lane) & 1ull;
-        if (bit && pos < 64u) sm.pairs[wave][pos] = uint16_t(uint32_t(lb) << 6 | lane);
-        const uint32_t cnt = uint32_t(__popcll(m));
-        m = fill + cnt > 64u ? __ballot(bit && pos >= 64u) : 0ull;
-        fill = min(fill + cnt, 64u);
-      }
-      if (fill == 0u) break;
-      wave_lds_fence();
-
-      // One lane per pair: coverage.
-      const bool active = lane < fill;
-      const uint32_t pr = active ? uint32_t(sm.pairs[wave][lane]) : uint32_t(sm.pairs[wave][0]);
-      const uint32_t pq = pr & 63u, pb = pr >> 6;
-      const QuadRec& R = sm.recs[pq];
-      const uint32_t info = uint32_t(__shfl(int(pairInfo), int(pq)));
-      const int plx = int(pb % TBX), ply = int(pb / TBX);
-      const bool pwrap = info & 0x100u;
-      const int pc = plx - int(info & 0xFFu);
-      const int row = int(info >> 16) - 1024 + ply;
-      float o[4], nx[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) nx[i] = R.nx[i];
-      if (!pwrap) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = sm.entry[row * 12 + i];
-        for (int t = 0; t < pc; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = o[i] + nx[i];
-      } else {
-        const int dd = (tby0 + ply) * bX + tbx0 + plx - int(R.fb);
-        const int r = div_bx(dd, bX, invBX);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = fold_n(fold_n(R.off[i], R.ny[i], r), nx[i], dd - r * bX);
-      }
-      const uint32_t modeZ = R.modeZ, mode = modeZ & 0xFFu, s01 = R.slope01, s23 = R.slope23;
-      float pdDx = R.dDx, pdDy = R.dDy;
-      const bool convex = mode == kModeConvex;
-      uint64_t word[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t tc = uint32_t(max(cvtt_x86(o[i]), 0));
-        const uint32_t sl = i == 0 ? s01 & 0xFFFFu : i == 1 ? s01 >> 16 : i == 2 ? s23 & 0xFFFFu : s23 >> 16;
-        word[i] = sm.cov[(sl | (convex ? tc : min(tc, 63u))) & 4095u];
-      }
-      const uint64_t A = word[0], B = word[1], C = word[2], D = word[3];
-      // Convex, or one triangle (which leaves an edge out); concave quads are
-      // rare enough for a branch of their own.
-      uint64_t mask = (A & C) & ((B | (mode == kModeTriangle1 ? ~0ull : 0ull)) & (D | (mode == kModeTriangle0 ? ~0ull : 0ull)));
-      const bool concave = mode >= kModeConcaveRight && mode <= kModeConcaveCenter;
-      if (__ballot(concave) != 0ull && concave)
-        mask = mode == kModeConcaveRight    ? (A | D) & (B & C)
-               : mode == kModeConcaveCenter ? (A & B) | (C & D)
-                                            : (A & D) & (B | C);
-      // Any offset >= 63 (a NaN is not): fmaxf leaves NaNs out.
-      const bool outside = fmaxf(fmaxf(o[0], o[1]), fmaxf(o[2], o[3])) >= 63.0f;
-      const uint64_t cm = __ballot(convex);
-      uint64_t live = __ballot(active) & ((cm & ~__ballot(outside)) | (~cm & __ballot(mask != 0ull)));
-      if (STATS) {
-        bc.visited += fill;
-        bc.rejected += fill - uint32_t(__popcll(live));
-      }
-      // What the pair's turn needs, as scalars by readlane: block, column steps
-      // to its samples, wrap flag and maximum depth; its depth gradients, its
-      // mask (one bit a lane) and where its samples are (any address when
-      // wrapped).
-      const uint32_t desc = pb | uint32_t(pwrap ? 0 : pc) << 8 | (pwrap ? 0x1000u : 0u) | (modeZ & 0xFFFF0000u);
-      const uint32_t maskLo = uint32_t(mask), maskHi = uint32_t(mask >> 32);
-      const uint32_t sampleAt = pwrap ? 0u : uint32_t(row * 12 + 4);
-      // Loaded before the loop, whose waits would otherwise cover its prefetches.
-      asm volatile("" : "+v"(pdDx), "+v"(pdDy));
-
-      // The pairs that cover pixels, in order; the next one's depth sample
-      // and block are loaded while this one is merged.
-      uint32_t at = 0, ds = 0, dNext = 0;
-      float vNext = 0.0f;
-      auto fetch = [&]() {
-        at = uint32_t(__builtin_ctzll(live));
-        ds = readlane_u(desc, at);
-        vNext = sm.entry[readlane_u(sampleAt, at) + uint32_t(kLane)];
-        dNext = sm.depth[(ds & 0xFFu) * 64u + lane];
+    // The wave's blocks, at most 32 at a time: block k of a group is in row
+    // yg + k % kGroupRows, in the (k / kGroupRows)-th of the row's columns.
+    for (int yg = 0; yg < TBY; yg += kGroupRows) {
+      auto block_of = [&](uint32_t k) -> uint32_t {
+        const uint32_t y = uint32_t(yg) + k % uint32_t(kGroupRows);
+        return y * TBX + ((wave - y) & uint32_t(NW - 1)) + NW * (k / uint32_t(kGroupRows));
       };
-      if (live) fetch();
-      while (live) {
-        live &= live - 1ull;
-        const uint32_t turn = at, dsc = ds, dBlock = dNext;
-        float v = vNext;
-        if (live) fetch();
-        const int b = int(dsc & 0xFFu);
-        if (b != cur) {
-          close();
-          cur = b;
-          const int by = b / TBX, kk = by * kPerRow + (b % TBX) / NW;
-          const uint32_t hz = kOwned <= 64 || kk < 64 ? readlane_u(hz0, uint32_t(kk)) : readlane_u(hz1, uint32_t(kk - 64));
-          dirty = false;
-          cleared = hz == 1u;
-          test = hz;
-          floor = cleared ? 0u : dBlock;
-          if (LABELS) {
-            win = kNoWinner;
-            if (!cleared) win = winner[(size_t(tby0 + by) * size_t(bX) + size_t(tbx0 + b % TBX)) * 64u + lane];
-          }
-        }
-        if (__ballot(test < (dsc >> 16)) == 0ull) {
-          if (STATS) bc.rejected++;
-          continue;
-        }
-        if (STATS) bc.written++;
-        const float dDx = readlane_f(pdDx, int(turn)), dDy = readlane_f(pdDy, int(turn));
-        if (__builtin_expect(!(dsc & 0x1000u), 1)) {
-          if (TBX > 8 && (dsc & 0x800u)) {
-            v = v + dDx; v = v + dDx; v = v + dDx; v = v + dDx;
-            v = v + dDx; v = v + dDx; v = v + dDx; v = v + dDx;
-          }
-          if (dsc & 0x400u) {
-            v = v + dDx; v = v + dDx; v = v + dDx; v = v + dDx;
-          }
-          if (dsc & 0x200u) {
-            v = v + dDx; v = v + dDx;
-          }
-          if (dsc & 0x100u) v = v + dDx;
-        } else {
-          const QuadRec& W = sm.recs[readlane_u(pq, turn)];
-          const int dd = (tby0 + b / TBX) * bX + tbx0 + b % TBX - int(W.fb);
-          const int r = div_bx(dd, bX, invBX);
-          float base, stepY, stepX;
-          quad_component(W, 4u + uint32_t(kLane), base, stepY, stepX);
-          v = fold_n(fold_n(base, stepY, r), stepX, dd - r * bX);
-        }
-        // Rows 0/1 and 8/9 from the plane, rows 2-7 as PAVGW of them.
-        if (right) v = fmaf(dDx, 0.5f, v);
-        const uint32_t top = pack_depth(v), bottom = pack_depth(dDy + v);
-        const uint32_t mid = avg_u16(top, bottom), mean = avg_u16(low ? bottom : top, mid);
-        const uint32_t row = odd ? mean : (low ? mid : top);
-        const uint64_t pm = uint64_t(readlane_u(maskLo, turn)) | uint64_t(readlane_u(maskHi, turn)) << 32;
-        const uint32_t drawnDepth = lane_select(pm, row);
-        if (LABELS) {
-          // The first write of a cleared block sets every pixel's winner
-          // (none where the written depth is 0), later ones only where they
-          // raise the depth.
-          const uint32_t batch = sm.qid[readlane_u(pq, turn)] >> 3;
-          win = cleared ? (drawnDepth != 0u ? batch : kNoWinner) : (drawnDepth > floor ? batch : win);
-        }
-        test = floor = max(drawnDepth, floor);
-        dirty = true;
-        cleared = false;
-        // hiZ == 1 after this write (no pixel at 0 and one at 1) reads as
-        // fast-cleared to the next one.
-        if (__ballot(test == 0u) == 0ull && __ballot(test == 1u) != 0ull) {
-          cleared = true;
-          floor = 0u;
-        }
+      // Lane q: which of them quad q's rectangle holds.  Row y's columns are
+      // (wave - y) mod NW and every NW-th after it: the column bits, repeated,
+      // reversed and rotated, give one bit a row.
+      uint32_t own = 0;
+#pragma unroll
+      for (int kx = 0; kx < kPerRow; ++kx) {
+        const uint32_t field = (colBits >> (NW * kx)) & uint32_t((1 << NW) - 1);
+        const uint32_t byRow = __builtin_bitreverse32(field * (NW == 8 ? 0x01010101u : NW == 4 ? 0x11111111u : 0x55555555u));
+        const uint32_t turn = (31u - wave + uint32_t(yg)) & 31u;
+        own |= (__builtin_amdgcn_alignbit(byRow, byRow, turn) & (rowBits >> yg) & uint32_t((1 << kGroupRows) - 1))
+               << (kx * kGroupRows);
       }
-      wave_lds_fence();  // the pair list is reused
+      if (anyWrap) {
+        uint32_t w = 0;
+        for (uint32_t k = 0; k < uint32_t(kPerRow * kGroupRows); ++k) {
+          const int b = int(block_of(k));
+          const int dd = (tby0 + b / TBX) * bX + tbx0 + b % TBX - int(RL.fb);
+          const int r = div_bx(max(dd, 0), bX, invBX);
+          if (dd >= 0 && r < rangeY && dd - r * bX < rangeX && tbx0 + b % TBX <= tbx1 && tby0 + b / TBX <= tby1)
+            w |= 1u << k;
+        }
+        if (valid && wrap) own = w;
+      }
+      uint32_t count = uint32_t(__popc(own));
+      uint32_t upTo = __ockl_wfscan_add_u32(count, true);  // pairs of quads 0..lane
+      uint32_t total = readlane_u(upTo, 63u);
+      if (total > 64u) {
+        // More than one round of pairs: drop those below their block's hiZ
+        // first (one block at a time; a block that is not fast-cleared only
+        // grows).
+        const uint32_t hz = lane < uint32_t(kPerRow * kGroupRows) ? uint32_t(sm.hiz[block_of(lane)]) : 0u;
+        for (uint32_t left = __ockl_wfred_or_u32(own); left; left &= left - 1u) {
+          const uint32_t k = uint32_t(__builtin_ctz(left)), bhz = readlane_u(hz, k);
+          if (bhz != 1u) own &= maxZq <= bhz ? ~(1u << k) : ~0u;
+        }
+        if (STATS) {
+          const uint32_t dropped = __ockl_wfred_add_u32(count - uint32_t(__popc(own)));
+          bc.visited += dropped;
+          bc.rejected += dropped;
+        }
+        count = uint32_t(__popc(own));
+        upTo = __ockl_wfscan_add_u32(count, true);
+        total = readlane_u(upTo, 63u);
+      }
+
+      for (uint32_t taken = 0; taken < total;) {
+        // The next quads' pairs, 64 or fewer (a quad has at most 32), as
+        // block << 6 | quad in submission order.
+        const bool inRound = upTo > taken && upTo - taken <= 64u;
+        const uint32_t last = 63u - uint32_t(__builtin_clzll(__ballot(inRound)));
+        const uint32_t fill = readlane_u(upTo, last) - taken;
+        uint32_t pos = upTo - count - taken;
+        for (uint32_t mine = inRound ? own : 0u; mine; mine &= mine - 1u)
+          sm.pairs[wave][pos++] = uint16_t(block_of(uint32_t(__builtin_ctz(mine))) << 6 | lane);
+        taken += fill;
+        wave_lds_fence();
+
+        // One lane per pair: coverage.
+        const bool active = lane < fill;
+        const uint32_t pr = active ? uint32_t(sm.pairs[wave][lane]) : uint32_t(sm.pairs[wave][0]);
+        const uint32_t pq = pr & 63u, pb = pr >> 6;
+        const QuadRec& R = sm.recs[pq];
+        const uint32_t info = uint32_t(__shfl(int(pairInfo), int(pq)));
+        const int plx = int(pb % TBX), ply = int(pb / TBX);
+        const uint32_t phz = sm.hiz[pb];
+        const bool pwrap = info & 0x100u;
+        const int pc = plx - int(info & 0xFFu);
+        const int row = int(info >> 16) - 1024 + ply;
+        float o[4], nx[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) nx[i] = R.nx[i];
+        if (!pwrap) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = sm.entry[row * 12 + i];
+          for (int t = 0; t < pc; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = o[i] + nx[i];
+        } else {
+          const int dd = (tby0 + ply) * bX + tbx0 + plx - int(R.fb);
+          const int r = div_bx(dd, bX, invBX);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = fold_n(fold_n(R.off[i], R.ny[i], r), nx[i], dd - r * bX);
+        }
+        const uint32_t modeZ = R.modeZ, mode = modeZ & 0xFFu, s01 = R.slope01, s23 = R.slope23;
+        float pdDx = R.dDx, pdDy = R.dDy;
+        const bool convex = mode == kModeConvex;
+        uint64_t word[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t tc = uint32_t(max(cvtt_x86(o[i]), 0));
+          const uint32_t sl = i == 0 ? s01 & 0xFFFFu : i == 1 ? s01 >> 16 : i == 2 ? s23 & 0xFFFFu : s23 >> 16;
+          word[i] = sm.cov[(sl | (convex ? tc : min(tc, 63u))) & 4095u];
+        }
+        const uint64_t A = word[0], B = word[1], C = word[2], D = word[3];
+        // Convex, or one triangle (which leaves an edge out); concave quads are
+        // rare enough for a branch of their own.
+        uint64_t mask = (A & C) & ((B | (mode == kModeTriangle1 ? ~0ull : 0ull)) & (D | (mode == kModeTriangle0 ? ~0ull : 0ull)));
+        const bool concave = mode >= kModeConcaveRight && mode <= kModeConcaveCenter;
+        if (__ballot(concave) != 0ull && concave)
+          mask = mode == kModeConcaveRight    ? (A | D) & (B & C)
+                 : mode == kModeConcaveCenter ? (A & B) | (C & D)
+                                              : (A & D) & (B | C);
+        // Any offset >= 63 (a NaN is not): fmaxf leaves NaNs out.
+        const bool outside = fmaxf(fmaxf(o[0], o[1]), fmaxf(o[2], o[3])) >= 63.0f;
+        const uint64_t cm = __ballot(convex);
+        uint64_t live = __ballot(active && !(phz != 1u && phz >= (modeZ >> 16))) &
+                        ((cm & ~__ballot(outside)) | (~cm & __ballot(mask != 0ull)));
+        if (STATS) {
+          bc.visited += fill;
+          bc.rejected += fill - uint32_t(__popcll(live));
+        }
+        // What the pair's turn needs, as scalars by readlane: column steps to
+        // its samples, wrap flag and maximum depth; its depth gradients, its
+        // mask (one bit a lane) and where its samples are (any address when
+        // wrapped).
+        const uint32_t desc = uint32_t(pwrap ? 0 : pc) | (pwrap ? 0x10u : 0u) | (modeZ & 0xFFFF0000u);
+        const uint32_t maskLo = uint32_t(mask), maskHi = uint32_t(mask >> 32);
+        const uint32_t sampleAt = pwrap ? 0u : uint32_t(row * 12 + 4);
+        // Loaded before the loop, whose waits would otherwise cover its prefetches.
+        asm volatile("" : "+v"(pdDx), "+v"(pdDy));
+
+        // The pairs that cover pixels, block by block, a block's in submission
+        // order; the next block's depth and the next pair's depth sample are
+        // loaded while a pair is merged.
+        uint32_t head = 0, b = 0, dNext = 0;
+        auto fetch_block = [&]() {
+          head = uint32_t(__builtin_ctzll(live));
+          b = readlane_u(pb, head);
+          dNext = sm.depth[b * 64u + lane];
+        };
+        if (live) fetch_block();
+        while (live) {
+          const uint32_t block = b, hz = readlane_u(phz, head);
+          uint64_t same = live & __ballot(pb == block);
+          live &= ~same;
+          // `test` is what the hiZ reject compares with a quad's maximum depth
+          // in every lane: the block's hiZ until its first write here, then its
+          // depth.  `floor` is what a write is merged with: 0 while the block
+          // reads as fast-cleared, else its depth.
+          bool dirty = false, cleared = hz == 1u;
+          uint32_t test = hz, floor = cleared ? 0u : dNext, win = kNoWinner;
+          uint32_t* const winners =
+              LABELS ? winner + ((size_t(tby0) + block / TBX) * size_t(bX) + size_t(tbx0) + block % TBX) * 64u + lane
+                     : nullptr;
+          if (LABELS && !cleared) win = *winners;
+          uint32_t at = uint32_t(__builtin_ctzll(same));
+          float vNext = sm.entry[readlane_u(sampleAt, at) + uint32_t(kLane)];
+          if (live) fetch_block();
+          do {
+            const uint32_t turn = at, dsc = readlane_u(desc, turn);
+            float v = vNext;
+            same &= same - 1ull;
+            if (same) {
+              at = uint32_t(__builtin_ctzll(same));
+              vNext = sm.entry[readlane_u(sampleAt, at) + uint32_t(kLane)];
+            }
+            if (__ballot(test < (dsc >> 16)) == 0ull) {
+              if (STATS) bc.rejected++;
+              continue;
+            }
+            if (STATS) bc.written++;
+            const float dDx = readlane_f(pdDx, int(turn)), dDy = readlane_f(pdDy, int(turn));
+            if (__builtin_expect(!(dsc & 0x10u), 1)) {
+              if (TBX > 8 && (dsc & 8u)) {
+                v = v + dDx; v = v + dDx; v = v + dDx; v = v + dDx;
+                v = v + dDx; v = v + dDx; v = v + dDx; v = v + dDx;
+              }
+              if (dsc & 4u) {
+                v = v + dDx; v = v + dDx; v = v + dDx; v = v + dDx;
+              }
+              if (dsc & 2u) {
+                v = v + dDx; v = v + dDx;
+              }
+              if (dsc & 1u) v = v + dDx;
+            } else {
+              const QuadRec& W = sm.recs[readlane_u(pq, turn)];
+              const int dd = (tby0 + int(block) / TBX) * bX + tbx0 + int(block) % TBX - int(W.fb);
+              const int r = div_bx(dd, bX, invBX);
+              float base, stepY, stepX;
+              quad_component(W, 4u + uint32_t(kLane), base, stepY, stepX);
+              v = fold_n(fold_n(base, stepY, r), stepX, dd - r * bX);
+            }
+            // Rows 0/1 and 8/9 from the plane, rows 2-7 as PAVGW of them.
+            if (right) v = fmaf(dDx, 0.5f, v);
+            const uint32_t top = pack_depth(v), bottom = pack_depth(dDy + v);
+            const uint32_t mid = avg_u16(top, bottom), mean = avg_u16(low ? bottom : top, mid);
+            const uint64_t pm = uint64_t(readlane_u(maskLo, turn)) | uint64_t(readlane_u(maskHi, turn)) << 32;
+            const uint32_t d = lane_select(pm, odd ? mean : (low ? mid : top));
+            if (LABELS) {
+              // The first write of a cleared block sets every pixel's winner
+              // (none where the written depth is 0), later ones only where they
+              // raise the depth.
+              const uint32_t batch = sm.qid[readlane_u(pq, turn)] >> 3;
+              win = cleared ? (d != 0u ? batch : kNoWinner) : (d > floor ? batch : win);
+            }
+            test = floor = max(d, floor);
+            dirty = true;
+            cleared = false;
+            // hiZ == 1 after this write (no pixel at 0 and one at 1) reads as
+            // fast-cleared to the next one.
+            if (__ballot(test == 0u) == 0ull && __ballot(test == 1u) != 0ull) {
+              cleared = true;
+              floor = 0u;
+            }
+          } while (same);
+          if (dirty) {
+            sm.depth[block * 64u + lane] = uint16_t(test);
+            const uint32_t mn = __ockl_wfred_min_u32(test);
+            if (lane == 0) sm.hiz[block] = uint16_t(mn);
+            if (LABELS) *winners = win;
+          }
+        }
+        wave_lds_fence();  // the pair list is reused
+      }
     }
-    close();
     q0 = q1;
     if (q0 < n) __syncthreads();  // the fold table is reused
   }
