@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstddef>
 
 #include "rz_x86.h"
 
@@ -1183,48 +1184,72 @@ __device__ __forceinline__ bool box_touches(uint64_t bb, int tbx0, int tbx1, int
   return c0 <= c1 && c0 <= tbx1 && c1 >= tbx0 && r0 <= tby1 && r1 >= tby0;
 }
 
-// True when no pixel of the tile can be covered by the quad because some edge
-// is outside for every block of the tile.  The block loop folds each edge
-// offset as off + nY + ... + nY (row steps) + nX + ... + nX (column steps) in
-// float; after k steps the fold differs from the exact off + r*nY + c*nX by at
-// most k * max|partial sum| * 2^-24 (each rounding is within half an ulp), so
-// an exact minimum at least 63 + that bound proves the offset test
-// (Rasterizer.cpp:1158) or the clamped lookup of bucket 63, whose table entry
-// is empty (:599), rejects every block.  For the non-convex modes the offset
-// must also stay below 2^31, where the truncation would wrap to bucket 0.
-// Quads whose block index wrapped in the 16-bit multiply are never rejected.
-__device__ bool quad_misses_tile(const QuadRec& R, int tbx0, int tbx1, int tby0, int tby1, int bX) {
-  const int fb = int(R.fb), rangeX = int(R.range & 0xFFFFu), rangeY = int(R.range >> 16);
-  const int minX = fb % bX, minY = fb / bX;
-  if (minX + rangeX > bX) return false;
-  const int c0 = max(tbx0, minX) - minX, c1 = min(tbx1, minX + rangeX - 1) - minX;
-  const int r0 = max(tby0, minY) - minY, r1 = min(tby1, minY + rangeY - 1) - minY;
-  if (c0 > c1 || r0 > r1) return true;
-  const uint32_t mode = R.modeZ & 0xFFu;
+// A setup record as five 16-byte words, each loaded whole and all before any
+// is used (taken field by field, the compiler loads some only once a test on
+// the others has passed).
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+struct RecWords {
+  u32x4 w[5];
+};
+static_assert(sizeof(QuadRec) == sizeof(RecWords) && offsetof(QuadRec, ny) == 16 && offsetof(QuadRec, off) == 32 &&
+                  offsetof(QuadRec, fb) == 60 && offsetof(QuadRec, range) == 64 && offsetof(QuadRec, modeZ) == 68,
+              "QuadRec layout");
+__device__ __forceinline__ RecWords load_rec(const QuadRec* __restrict__ at) {
+  const u32x4* p = reinterpret_cast<const u32x4*>(at);
+  RecWords r = {{p[0], p[1], p[2], p[3], p[4]}};
+  asm volatile("" : "+v"(r.w[0]), "+v"(r.w[1]), "+v"(r.w[2]), "+v"(r.w[3]), "+v"(r.w[4]));
+  return r;
+}
+
+// Whether a quad may cover a pixel of the tile: its blocks touch the tile,
+// and no edge is outside for every block they share.  The block loop folds
+// each edge offset as off + nY + ... + nY (row steps) + nX + ... + nX (column
+// steps) in float; after k steps the fold differs from the exact off + r*nY +
+// c*nX by at most k * max|partial sum| * 2^-24 (each rounding is within half
+// an ulp), and the corner values below by a few roundings more, so a minimum
+// over the corners of at least 63 + that bound (taken more than twice over)
+// proves the offset test (Rasterizer.cpp:1158) or the clamped lookup of
+// bucket 63, whose table entry is empty (:599), rejects every block.  For the
+// non-convex modes the offset must also stay below 2^31, where the truncation
+// would wrap to bucket 0.  Infinities and NaNs make the bound infinite or NaN,
+// which proves nothing.  Quads whose block index wrapped in the 16-bit
+// multiply span whole rows and are never rejected by an edge.  A pass is bound
+// by its loads' latency and then by these instructions: with double arithmetic
+// and integer divisions the scans of 128 city frames in flight took 185 ms of
+// work-group time, with these 145 ms.
+__device__ __forceinline__ bool quad_touches_tile(const RecWords& R, int tbx0, int tbx1, int tby0, int tby1, int bX,
+                                                  float invBX) {
+  const int fb = int(R.w[3].w), rangeX = int(R.w[4].x & 0xFFFFu), rangeY = int(R.w[4].x >> 16);
+  if (rangeX == 0) return false;  // not drawn
+  const int minY = div_bx(fb, bX, invBX), minX = fb - minY * bX;
+  if (minX + rangeX > bX) return minY <= tby1 && minY + rangeY >= tby0;
+  const int c0 = max(tbx0 - minX, 0), c1 = min(tbx1 - minX, rangeX - 1);
+  const int r0 = max(tby0 - minY, 0), r1 = min(tby1 - minY, rangeY - 1);
+  if (c0 > c1 || r0 > r1) return false;
+  const uint32_t mode = R.w[4].y & 0xFFu;
+  const float fr0 = float(r0), fr1 = float(r1), fc0 = float(c0), fc1 = float(c1);
+  const float steps = fr1 + fc1 + 8.0f;
   bool out[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const double o = R.off[e], nx = R.nx[e], ny = R.ny[e];
-    const double v00 = o + r0 * ny + c0 * nx, v01 = o + r0 * ny + c1 * nx;
-    const double v10 = o + r1 * ny + c0 * nx, v11 = o + r1 * ny + c1 * nx;
-    const double lo = fmin(fmin(v00, v01), fmin(v10, v11));
-    const double hi = fmax(fmax(v00, v01), fmax(v10, v11));
-    const double steps = double(r1 + c1);
-    const double bound = fabs(o) + r1 * fabs(ny) + c1 * fabs(nx);
-    const double err = steps * (bound * 0x1p-23 + 0x1p-126);
-    const bool finite = isfinite(o) && isfinite(nx) && isfinite(ny) && isfinite(bound);
-    const bool below31 = hi + err < 2147483648.0;
-    out[e] = finite && lo - err >= 63.0 && (mode == kModeConvex || below31);
+    const float o = bitsf(R.w[2][e]), nx = bitsf(R.w[0][e]), ny = bitsf(R.w[1][e]);
+    const float a = fmaf(fr0, ny, o), b = fmaf(fr1, ny, o);
+    const float loX = fminf(fc0 * nx, fc1 * nx), hiX = fmaxf(fc0 * nx, fc1 * nx);
+    const float bound = fmaf(fr1, __builtin_fabsf(ny), fmaf(fc1, __builtin_fabsf(nx), __builtin_fabsf(o)));
+    const float err = steps * fmaf(bound, 0x1p-22f, 0x1p-120f);
+    out[e] = (fminf(a, b) + loX) - err >= 63.0f &&
+             (mode == kModeConvex || (fmaxf(a, b) + hiX) + err < 2147483648.0f);
   }
+  bool misses = false;
   switch (mode) {
-    case kModeConvex: return out[0] || out[1] || out[2] || out[3];
-    case kModeTriangle0: return out[0] || out[1] || out[2];
-    case kModeTriangle1: return out[0] || out[2] || out[3];
-    case kModeConcaveRight: return out[1] || out[2] || (out[0] && out[3]);
-    case kModeConcaveLeft: return out[0] || out[3] || (out[1] && out[2]);
-    case kModeConcaveCenter: return (out[0] || out[1]) && (out[2] || out[3]);
-    default: return false;
+    case kModeConvex: misses = out[0] || out[1] || out[2] || out[3]; break;
+    case kModeTriangle0: misses = out[0] || out[1] || out[2]; break;
+    case kModeTriangle1: misses = out[0] || out[2] || out[3]; break;
+    case kModeConcaveRight: misses = out[1] || out[2] || (out[0] && out[3]); break;
+    case kModeConcaveLeft: misses = out[0] || out[3] || (out[1] && out[2]); break;
+    case kModeConcaveCenter: misses = (out[0] || out[1]) && (out[2] || out[3]); break;
   }
+  return !misses;
 }
 
 // Tile-overlap tests shared by the prep kernel's tile count and the frame
@@ -1515,17 +1540,12 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
         if (STATS && tid == 0) ctr[kStatPasses]++;
         const uint32_t waveFirst = base + wave * 64u;
         bool hit = false;
-        QuadRec rec;
         if (waveFirst < L.quadCount) {
           const uint32_t wg0 = ((L.quadBase + waveFirst) >> 6) - gBase;
           const uint32_t wg1 = ((L.quadBase + min(waveFirst + 63u, L.quadCount - 1u)) >> 6) - gBase;
           const bool groupHit = wg1 >= 64 || ((L.groups >> wg0) & 1ull) || ((L.groups >> wg1) & 1ull);
-          if (groupHit && base + tid < L.quadCount) {
-            rec = J.recs[L.quadBase + base + tid];
-            const uint32_t rx = rec.range & 0xFFFFu, ry = rec.range >> 16;
-            hit = rx != 0u && box_touches(quad_box(rec.fb, rx, ry, uint32_t(bX), uint32_t(bY)), tbx0, tbx1, tby0, tby1) &&
-                  !quad_misses_tile(rec, tbx0, tbx1, tby0, tby1, bX);
-          }
+          if (groupHit && base + tid < L.quadCount)
+            hit = quad_touches_tile(load_rec(&J.recs[L.quadBase + base + tid]), tbx0, tbx1, tby0, tby1, bX, invBX);
         }
         const uint64_t hm = __ballot(hit);
         const uint32_t hpre =
