@@ -4,22 +4,46 @@
 // The reference recurses depth first; each call sorts its index range stably
 // by box centre along x, then y, then z, scores every split position that is
 // a multiple of the granularity with prefix and suffix box areas, and sorts
-// the range once more along the winning axis.  Here one level of the
-// recursion is one round over all open ranges ("segments") at once:
-//   - each stable sort is one device-wide radix sort on (segment, centre
-//     key), so segments stay where they are and sort independently;
-//   - prefix and suffix boxes are segmented scans over the boxes of chunks
-//     of gran positions, since every split falls between chunks (min and max
-//     are exact, so neither the chunking nor the scan order changes them);
-//   - the winning (cost, axis, index) of a segment is a 64-bit atomicMin,
-//     which keeps the reference's first strict minimum in (axis, index) order.
-// Segments stay in the index array in the order the depth-first recursion
-// would emit them, so the batches are the final segments, left to right.
+// the range once more along the winning axis.
+//
+// Nothing is sorted per call here: every order that a call can see is the
+// restriction of one of a few orders of the whole set, which are sorted once.
+// Write (x, z, y) for the lexicographic order by those centres, ties by input
+// index.  A range sorted along a winning axis is in (x, z, y), (y, z, x) or
+// (z, y, x), since that last sort is stable over the z sort, which is stable
+// over the y sort, which is stable over the x sort; equal centres never
+// change places.  Its child calls then see, for the x scoring, (x, z, y) (or
+// (x, y, z) when the range was last sorted along y), for the y scoring
+// (y, x, z) and for the z scoring (z, y, x).  Only the first call sees the
+// input order: (x, index) and (y, x, index).  So the five orders are kept as
+// five index arrays, and a split is a stable partition of each.
+//
+// One level of the recursion is one round over all open ranges ("segments")
+// at once, without the host:
+//   - the boxes of chunks of gran positions, since every split falls between
+//     chunks, in the three scoring orders;
+//   - per segment and axis one work-group: prefix and suffix areas over the
+//     chunks (min and max are exact, so the order in which boxes are merged
+//     does not change them) and the split costs.  The best (cost, axis, index)
+//     is a 64-bit minimum, which keeps the reference's first strict minimum in
+//     (axis, index) order; the last of the segment's three work-groups splits
+//     it;
+//   - a flag per element (right of the split or not) from the winning order,
+//     one prefix sum of those flags over all five arrays, and the partition.
+// Segments stay in the arrays where the depth-first recursion would emit
+// them, so the batches are the final segments, left to right.
+//
+// What bounds it: launches and latency (six short launches a level, 12 levels
+// for 286,000 quads), then the random reads of the boxes.  Four device sorts
+// and four scans by key per axis and level, as the reference's sorts would
+// translate to, took 6.2 ms of kernels for 240,000 box quads; this takes
+// 1.4 ms.
 #include <hip/hip_runtime.h>
 
-#include <cstring>
 #include <rocprim/device/device_radix_sort.hpp>
-#include <rocprim/device/device_scan_by_key.hpp>
+#include <rocprim/device/device_scan.hpp>
+#include <rocprim/iterator/counting_iterator.hpp>
+#include <rocprim/iterator/transform_iterator.hpp>
 
 #include <algorithm>
 #include <cstdint>
@@ -92,61 +116,95 @@ __global__ void __launch_bounds__(256) sah_iota_kernel(uint32_t* __restrict__ id
   if (i < n) idx[i] = i;
 }
 
-// Segment of every position: the last segment start at or before it.
-__global__ void __launch_bounds__(256) sah_segof_kernel(const uint32_t* __restrict__ segStart, uint32_t nSeg,
-                                                        uint32_t n, uint32_t* __restrict__ segOf) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// The five orders, and the three the winning axis chooses from.
+enum Order : int { kXzy = 0, kYzx = 1, kZyx = 2, kXyz = 3, kYxz = 4, kOrders = 5 };
+
+// One array of a sorting round: the elements in the order they come in (null:
+// input order) and the axis of the centre to sort by.
+struct SortPart {
+  const uint32_t* in;
+  int axis;
+};
+struct SortRound {
+  SortPart part[3];
+};
+
+// Radix keys (part << 32 | centre key) and values of a round's parts, one
+// after another: one stable sort then sorts each part by itself.
+__global__ void __launch_bounds__(256) sah_round_keys_kernel(SortRound r, const float* __restrict__ boxes, uint32_t n,
+                                                             uint64_t* __restrict__ keys,
+                                                             uint32_t* __restrict__ values) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, p = blockIdx.y;
   if (i >= n) return;
-  uint32_t lo = 0, hi = nSeg - 1;
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi + 1) >> 1;
-    if (segStart[mid] <= i) lo = mid;
-    else hi = mid - 1;
-  }
-  segOf[i] = lo;
+  const uint32_t e = r.part[p].in ? r.part[p].in[i] : i;
+  const int a = r.part[p].axis;
+  const float c = boxes[8 * size_t(e) + a] + boxes[8 * size_t(e) + 4 + a];  // Aabb::getCenter
+  keys[size_t(p) * n + i] = uint64_t(p) << 32 | centre_key(c);
+  values[size_t(p) * n + i] = e;
 }
 
-// Radix keys (segment << 32 | centre key along the axis).  Closed segments
-// get a constant key and keep their order; axis < 0 takes each open
-// segment's winning axis.
-__global__ void __launch_bounds__(256) sah_keys_kernel(const float* __restrict__ boxes, const uint32_t* __restrict__ idx,
-                                                       const uint32_t* __restrict__ segOf,
-                                                       const uint32_t* __restrict__ segOpen,
-                                                       const uint64_t* __restrict__ segBest, int axis, uint32_t n,
-                                                       uint64_t* __restrict__ keys) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t s = segOf[i];
-  uint32_t low = 0;
-  if (segOpen[s]) {
-    const int a = axis >= 0 ? axis : int((segBest[s] >> 30) & 3u);
-    const uint32_t e = idx[i];
-    low = centre_key(boxes[8 * size_t(e) + a] + boxes[8 * size_t(e) + 4 + a]);  // Aabb::getCenter
-  }
-  keys[i] = (uint64_t(s) << 32) | low;
+constexpr uint32_t kClosed = ~0u;
+
+// An open segment of a level: its positions and the axis its elements were
+// last sorted along (3: the whole set in input order).
+struct Segment {
+  uint32_t start, len, axis;
+};
+// Its split: left part's length, winning axis, and its children's numbers in
+// the next level (kClosed: a batch).
+struct Split {
+  uint32_t k, axis, child[2];
+};
+
+struct SahLevel {
+  const float* boxes;
+  uint32_t n, nChunks, gran, target;
+  uint32_t* orders;       // kOrders arrays of n
+  uint32_t* nextOrders;   // the same after the level's splits
+  const uint32_t* rootX;  // (x, index) and (y, x, index), for the first level
+  const uint32_t* rootY;
+  uint32_t* chunkSeg;     // per chunk: open segment or kClosed
+  uint32_t* nextChunkSeg;
+  Segment* segs;
+  Segment* nextSegs;
+  unsigned long long* best;      // per open segment
+  unsigned long long* nextBest;
+  uint32_t* arrived;             // work-groups of the segment that are done
+  uint32_t* nextArrived;
+  uint32_t* nOpen;
+  uint32_t* nextNOpen;
+  Split* splits;
+  Ext6* chunkBox;        // per axis and chunk, in the axis's scoring order
+  float* rightArea;      // per axis and chunk: area of the boxes from the chunk to the segment's end
+  uint8_t* side;         // per element: right of its segment's split
+  const uint32_t* lefts; // per order and position: elements left of their split before it
+  uint8_t* starts;       // per chunk: a batch starts here
+  uint8_t* batchAxis;    // per chunk: the axis its batch was last sorted along
+  uint32_t* err;
+};
+
+__device__ __forceinline__ const uint32_t* scoring_order(const SahLevel& L, uint32_t axis, uint32_t lastAxis) {
+  if (axis == 2u) return L.orders + size_t(kZyx) * L.n;
+  if (lastAxis == 3u) return axis == 0u ? L.rootX : L.rootY;
+  if (axis == 1u) return L.orders + size_t(kYxz) * L.n;
+  return L.orders + size_t(lastAxis == 1u ? kXyz : kXzy) * L.n;
 }
 
-// Boxes of each chunk of gran consecutive positions, in sorted order,
-// forwards and reversed (the suffix scan runs over the reversed array).
-// Every segment starts at a multiple of gran (the root at 0, each split gran
-// times an integer further on), so no chunk spans two segments.
-__global__ void __launch_bounds__(256) sah_chunks_kernel(const float* __restrict__ boxes,
-                                                         const uint32_t* __restrict__ idx,
-                                                         const uint32_t* __restrict__ segOf, uint32_t n,
-                                                         uint32_t gran, uint32_t nChunks, Ext6* __restrict__ fwd,
-                                                         Ext6* __restrict__ rev, uint32_t* __restrict__ chunkSeg,
-                                                         uint32_t* __restrict__ revSeg) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nChunks) return;
-  const uint32_t i0 = c * gran, i1 = min(i0 + gran, n);
-  Ext6 b = load_ext(boxes, idx[i0]);
+// Boxes of each open segment's chunks of gran positions, in the three scoring
+// orders (blockIdx.y).  Every segment starts at a multiple of gran (the root
+// at 0, each split gran times an integer further on), so no chunk spans two
+// segments.
+__global__ void __launch_bounds__(256) sah_chunks_kernel(SahLevel L) {
+  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x, axis = blockIdx.y;
+  if (c >= L.nChunks) return;
+  const uint32_t s = L.chunkSeg[c];
+  if (s == kClosed) return;
+  const uint32_t* order = scoring_order(L, axis, L.segs[s].axis);
+  const uint32_t i0 = c * L.gran, i1 = min(i0 + L.gran, L.n);
+  Ext6 b = load_ext(L.boxes, order[i0]);
   const MergeExt merge;
-  for (uint32_t i = i0 + 1; i < i1; ++i) b = merge(b, load_ext(boxes, idx[i]));
-  const uint32_t sg = segOf[i0];
-  fwd[c] = b;
-  rev[nChunks - 1 - c] = b;
-  chunkSeg[c] = sg;
-  revSeg[nChunks - 1 - c] = sg;
+  for (uint32_t i = i0 + 1; i < i1; ++i) b = merge(b, load_ext(L.boxes, order[i]));
+  L.chunkBox[size_t(axis) * L.nChunks + c] = b;
 }
 
 __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
@@ -160,94 +218,175 @@ __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
   return v;
 }
 
-// sahSplit's cost loop (SurfaceAreaHeuristic.cpp:46-64) for one axis: split
-// position k of a segment of len items costs area(items [0, k)) * k +
-// area(items [k, len)) * (len - k), for k = gran, 2 gran, ... < len - gran.
-// The key orders by cost (non-negative, -0 folded into +0), then axis, then
-// k, so the minimum is the reference's first strict minimum.  Keys are
-// reduced per wave and per work-group while they share a segment, so a large
-// segment takes one atomic per work-group rather than one per candidate.
-__global__ void __launch_bounds__(256) sah_cost_kernel(const Ext6* __restrict__ fwdScan,
-                                                       const Ext6* __restrict__ revScan,
-                                                       const uint32_t* __restrict__ chunkSeg,
-                                                       const uint32_t* __restrict__ segStart,
-                                                       const uint32_t* __restrict__ segLen,
-                                                       const uint32_t* __restrict__ segOpen, uint32_t nChunks,
-                                                       uint32_t gran, uint32_t axis, uint64_t* __restrict__ segBest) {
-  __shared__ uint64_t waveBest[4];
-  __shared__ uint32_t waveSeg[4];
-  // One thread per chunk c: the split before position c * gran, whose left
-  // part ends with chunk c - 1 and whose right part starts with chunk c.
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  const bool inRange = c < nChunks;
-  const uint32_t s = inRange ? chunkSeg[c] : 0u;
-  uint64_t key = ~0ull;
-  if (inRange && segOpen[s]) {
-    const uint32_t k = c * gran - segStart[s], len = segLen[s];
-    if (k >= gran && k + gran < len) {
-      const float left = surface_area(fwdScan[c - 1]) * float(int(k));
-      const float right = surface_area(revScan[nChunks - 1 - c]) * float(int(len - k));
-      float cost = left + right;
-      if (cost == 0.0f) cost = 0.0f;
-      key = (uint64_t(__float_as_uint(cost)) << 32) | (uint64_t(axis) << 30) | k;
-    }
-  }
-  // Lanes are consecutive chunks, so lane 0 is in range whenever any is.
-  const uint32_t s0 = uint32_t(__builtin_amdgcn_readfirstlane(int(s)));
-  const bool uniform = __ballot(inRange && s != s0) == 0ull;
-  uint64_t wk = ~0ull;
-  if (uniform) {
-    wk = wave_min_u64(key);
-  } else if (key != ~0ull) {
-    atomicMin(reinterpret_cast<unsigned long long*>(&segBest[s]), static_cast<unsigned long long>(key));
-  }
-  if (lane == 0) {
-    waveBest[wave] = wk;
-    waveSeg[wave] = s0;
-  }
+// sahSplit's cost loop (SurfaceAreaHeuristic.cpp:46-64) for one open segment
+// and axis, by one work-group: split position k of a segment of len items
+// costs area(items [0, k)) * k + area(items [k, len)) * (len - k), for k =
+// gran, 2 gran, ... < len - gran.  Each thread takes a run of consecutive
+// chunks; the runs' boxes are scanned in both directions in LDS, then each
+// thread walks its run backwards for the right areas and forwards for the left
+// ones and the costs.  The key orders by cost (non-negative, -0 folded into
+// +0), then axis, then k, so the minimum is the reference's first strict
+// minimum.  The last of the segment's three work-groups splits it.
+//
+// NT threads: the first levels' few long segments take 1024, so that a run is
+// short; later ones 256, so that many segments share a CU.
+template <uint32_t NT>
+__global__ void __launch_bounds__(NT) sah_split_kernel(SahLevel L) {
+  const uint32_t s = blockIdx.x, axis = blockIdx.y, t = threadIdx.x;
+  if (s >= *L.nOpen) return;
+  __shared__ Ext6 pre[2][NT], suf[2][NT];
+  __shared__ uint64_t waveBest[NT / 64];
+  const Segment S = L.segs[s];
+  const uint32_t c0 = S.start / L.gran, nc = (S.len + L.gran - 1) / L.gran;
+  const uint32_t per = (nc + NT - 1) / NT, r0 = min(t * per, nc), r1 = min(r0 + per, nc);
+  const Ext6* box = L.chunkBox + size_t(axis) * L.nChunks + c0;
+  float* right = L.rightArea + size_t(axis) * L.nChunks + c0;
+  const MergeExt merge;
+  const float inf = __builtin_inff();
+  const Ext6 empty = {{inf, inf, inf}, {-inf, -inf, -inf}};
+  Ext6 run = empty;
+  for (uint32_t c = r0; c < r1; ++c) run = merge(run, box[c]);
+  pre[0][t] = suf[0][t] = run;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    uint64_t cur = ~0ull;
-    uint32_t curSeg = 0;
-    for (uint32_t w = 0; w < 4; ++w) {
-      if (waveBest[w] == ~0ull) continue;
-      if (cur != ~0ull && waveSeg[w] != curSeg) {
-        atomicMin(reinterpret_cast<unsigned long long*>(&segBest[curSeg]), static_cast<unsigned long long>(cur));
-        cur = ~0ull;
-      }
-      curSeg = waveSeg[w];
-      cur = waveBest[w] < cur ? waveBest[w] : cur;
-    }
-    if (cur != ~0ull)
-      atomicMin(reinterpret_cast<unsigned long long*>(&segBest[curSeg]), static_cast<unsigned long long>(cur));
+  uint32_t cur = 0;
+  for (uint32_t d = 1; d < NT; d <<= 1) {
+    pre[cur ^ 1][t] = t >= d ? merge(pre[cur][t - d], pre[cur][t]) : pre[cur][t];
+    suf[cur ^ 1][t] = t + d < NT ? merge(suf[cur][t], suf[cur][t + d]) : suf[cur][t];
+    cur ^= 1;
+    __syncthreads();
   }
+  run = t + 1 < NT ? suf[cur][t + 1] : empty;
+  for (uint32_t c = r1; c > r0; --c) {
+    run = merge(run, box[c - 1]);
+    right[c - 1] = surface_area(run);
+  }
+  run = t > 0 ? pre[cur][t - 1] : empty;
+  uint64_t key = ~0ull;
+  for (uint32_t c = r0; c < r1; ++c) {
+    const uint32_t k = c * L.gran;
+    if (k >= L.gran && k + L.gran < S.len) {
+      float cost = surface_area(run) * float(int(k)) + right[c] * float(int(S.len - k));
+      if (cost == 0.0f) cost = 0.0f;
+      const uint64_t mine = (uint64_t(__float_as_uint(cost)) << 32) | (uint64_t(axis) << 30) | k;
+      key = mine < key ? mine : key;
+    }
+    run = merge(run, box[c]);
+  }
+  key = wave_min_u64(key);
+  if ((t & 63u) == 0u) waveBest[t >> 6] = key;
+  __syncthreads();
+  if (t != 0u) return;
+  for (uint32_t w = 1; w < NT / 64; ++w) key = waveBest[w] < key ? waveBest[w] : key;
+  atomicMin(&L.best[s], static_cast<unsigned long long>(key));
+  if (__hip_atomic_fetch_add(&L.arrived[s], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != 2u) return;
+  // All three axes are in.
+  const uint64_t best = __hip_atomic_load(&L.best[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  Split P = {uint32_t(best & 0x3FFFFFFFu), uint32_t(best >> 30) & 3u, {kClosed, kClosed}};
+  if (best == ~0ull) {
+    // Every open segment has a split position: the root holds more than 2 gran
+    // items and a child stays open only with target > 2 gran items.
+    atomicOr(L.err, 1u);
+    P = {S.len, 0u, {kClosed, kClosed}};
+  }
+  const uint32_t start[2] = {S.start, S.start + P.k}, len[2] = {P.k, S.len - P.k};
+  for (int i = 0; i < 2; ++i) {
+    // A child recurses when it holds target items or more
+    // (SurfaceAreaHeuristic.cpp:81-92).
+    if (len[i] >= L.target && best != ~0ull) {
+      const uint32_t id = atomicAdd(L.nextNOpen, 1u);
+      P.child[i] = id;
+      L.nextSegs[id] = {start[i], len[i], P.axis};
+      L.nextBest[id] = ~0ull;
+      L.nextArrived[id] = 0u;
+    }
+  }
+  if (best != ~0ull) L.starts[start[1] / L.gran] = 1;
+  L.splits[s] = P;
+}
+
+// Which elements lie right of their segment's split, in the winning order.
+__global__ void __launch_bounds__(256) sah_sides_kernel(SahLevel L) {
+  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= L.n) return;
+  const uint32_t s = L.chunkSeg[p / L.gran];
+  if (s == kClosed) return;
+  const Split P = L.splits[s];
+  L.side[L.orders[size_t(P.axis) * L.n + p]] = p - L.segs[s].start >= P.k;
+}
+
+// 1 for an element left of its split, 0 right of it or in a batch: the input
+// of the prefix sum over all five arrays.
+struct IsLeft {
+  const uint32_t* orders;
+  const uint32_t* chunkSeg;
+  const uint8_t* side;
+  uint32_t n, gran;
+  __device__ uint32_t operator()(uint32_t i) const {
+    const uint32_t a = i / n, p = i - a * n;
+    if (chunkSeg[p / gran] == kClosed) return 0u;
+    return side[orders[i]] ? 0u : 1u;
+  }
+};
+
+// The stable partition of every open segment in each order (blockIdx.y), and
+// the next level's segment of every chunk.
+__global__ void __launch_bounds__(256) sah_partition_kernel(SahLevel L) {
+  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x, a = blockIdx.y;
+  if (p == 0u && a == 0u) *L.nOpen = 0u;  // this level's count is the one after next's
+  if (p >= L.n) return;
+  const uint32_t* in = L.orders + size_t(a) * L.n;
+  uint32_t* out = L.nextOrders + size_t(a) * L.n;
+  const uint32_t c = p / L.gran, s = L.chunkSeg[c], e = in[p];
+  const bool first = a == 0u && p == c * L.gran;
+  if (s == kClosed) {
+    out[p] = e;
+    if (first) L.nextChunkSeg[c] = kClosed;
+    return;
+  }
+  const Split P = L.splits[s];
+  const uint32_t start = L.segs[s].start, at = p - start;
+  const uint32_t* lefts = L.lefts + size_t(a) * L.n;
+  const uint32_t l = lefts[p] - lefts[start];
+  out[start + (L.side[e] ? P.k + (at - l) : l)] = e;
+  if (first) {
+    const uint32_t child = P.child[at >= P.k ? 1 : 0];
+    L.nextChunkSeg[c] = child;
+    if (child == kClosed) L.batchAxis[c] = uint8_t(P.axis);
+  }
+}
+
+// The batches' elements: each batch in the order it was last sorted in.
+__global__ void __launch_bounds__(256) sah_emit_kernel(const uint32_t* __restrict__ orders,
+                                                       const uint8_t* __restrict__ batchAxis, uint32_t n,
+                                                       uint32_t gran, uint32_t* __restrict__ out) {
+  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < n) out[p] = orders[size_t(batchAxis[p / gran]) * n + p];
 }
 
 uint32_t grid_of(uint32_t n) { return (n + 255u) / 256u; }
 
-template <typename T>
-hipError_t alloc(T** p, size_t count) {
-  *p = nullptr;
-  return hipMalloc(reinterpret_cast<void**>(p), (count ? count : 1) * sizeof(T));
-}
-
-struct SahBuffers {
-  uint32_t* idx[2] = {nullptr, nullptr};
-  uint64_t* keys[2] = {nullptr, nullptr};
-  uint32_t *segOf = nullptr, *chunkSeg = nullptr, *revSeg = nullptr, *segStart = nullptr, *segLen = nullptr,
-           *segOpen = nullptr;
-  uint32_t* bad = nullptr;
-  uint64_t* segBest = nullptr;
-  Ext6 *fwd = nullptr, *fwdScan = nullptr, *rev = nullptr, *revScan = nullptr;
-  void* temp = nullptr;
-  ~SahBuffers() {
-    for (void* p : {(void*)idx[0], (void*)idx[1], (void*)keys[0], (void*)keys[1], (void*)segOf, (void*)chunkSeg,
-                    (void*)revSeg,
-                    (void*)segStart, (void*)segLen, (void*)segOpen, (void*)bad, (void*)segBest, (void*)fwd,
-                    (void*)fwdScan, (void*)rev, (void*)revScan, temp})
-      if (p) (void)hipFree(p);
+// One device allocation, handed out in 256-byte aligned parts.
+class Arena {
+ public:
+  ~Arena() {
+    if (base_) (void)hipFree(base_);
   }
+  // First pass (nothing allocated): adds up the parts' sizes.
+  template <typename T>
+  void take(T** p, size_t count) {
+    *p = base_ ? reinterpret_cast<T*>(base_ + used_) : nullptr;
+    used_ += (count * sizeof(T) + 255) & ~size_t(255);
+  }
+  hipError_t allocate() {
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&base_), used_ ? used_ : 1);
+    used_ = 0;
+    if (e != hipSuccess) base_ = nullptr;
+    return e;
+  }
+
+ private:
+  unsigned char* base_ = nullptr;
+  size_t used_ = 0;
 };
 
 }  // namespace
@@ -266,18 +405,76 @@ int sah_batches_run(hipStream_t stream, uint32_t n, const float* d_boxes, uint32
     *nBatches = 0;
     return RZ_OK;
   }
-  SahBuffers B;
-  if (alloc(&B.bad, 1) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
-  uint32_t bad = 0;
-  SAH_HIP(hipMemsetAsync(B.bad, 0, 4, stream));
-  sah_check_kernel<<<grid_of(n), 256, 0, stream>>>(d_boxes, n, B.bad);
+  const bool whole = n <= 2 * gran;  // no split position (see below)
+  const uint32_t nChunks = (n + gran - 1) / gran;
+  const uint32_t maxOpen = n / target + 1;  // every open segment but the root holds target items or more
+  const size_t n3 = size_t(3) * n;
+  SahLevel A{}, B{};  // the levels' two views of the buffers
+  uint64_t *keys = nullptr, *keysOut = nullptr;
+  uint32_t *values = nullptr, *round1 = nullptr, *round2 = nullptr, *lefts = nullptr;
+  unsigned char* temp = nullptr;
+  size_t sortBytes = 0, scanBytes = 0;
+  auto left_iterator = [&](const SahLevel& L) {
+    return rocprim::make_transform_iterator(rocprim::counting_iterator<uint32_t>(0u),
+                                            IsLeft{L.orders, L.chunkSeg, L.side, n, gran});
+  };
+  if (!whole) {
+    for (uint32_t parts = 2; parts <= 3; ++parts) {
+      size_t bytes = 0;
+      SAH_HIP(rocprim::radix_sort_pairs(nullptr, bytes, keys, keysOut, values, values, size_t(parts) * n, 0u, 34u,
+                                        stream));
+      sortBytes = std::max(sortBytes, bytes);
+    }
+    SAH_HIP(rocprim::exclusive_scan(nullptr, scanBytes, left_iterator(A), lefts, 0u, size_t(kOrders) * n,
+                                    rocprim::plus<uint32_t>(), stream));
+  }
+  const size_t tempBytes = std::max(sortBytes, scanBytes);
+  Arena arena;
+  for (int pass = 0; pass < 2; ++pass) {
+    if (pass == 1 && arena.allocate() != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
+    // A word for the range check, the two open counts and the error word.
+    uint32_t* words = nullptr;
+    arena.take(&words, 4);
+    if (words) {
+      A.err = words;
+      A.nOpen = words + 2;
+      A.nextNOpen = words + 3;
+    }
+    if (whole) continue;
+    arena.take(&A.orders, size_t(kOrders) * n);
+    arena.take(&A.nextOrders, size_t(kOrders) * n);
+    arena.take(&keys, n3);
+    arena.take(&keysOut, n3);
+    arena.take(&values, n3);
+    arena.take(&round1, size_t(2) * n);
+    arena.take(&round2, n3);
+    arena.take(&lefts, size_t(kOrders) * n);
+    arena.take(&temp, tempBytes);
+    arena.take(&A.chunkSeg, nChunks);
+    arena.take(&A.nextChunkSeg, nChunks);
+    arena.take(&A.segs, maxOpen);
+    arena.take(&A.nextSegs, maxOpen);
+    arena.take(&A.best, maxOpen);
+    arena.take(&A.nextBest, maxOpen);
+    arena.take(&A.arrived, maxOpen);
+    arena.take(&A.nextArrived, maxOpen);
+    arena.take(&A.splits, maxOpen);
+    arena.take(&A.chunkBox, size_t(3) * nChunks);
+    arena.take(&A.rightArea, size_t(3) * nChunks);
+    arena.take(&A.side, n);
+    arena.take(&A.starts, nChunks);
+    arena.take(&A.batchAxis, nChunks);
+  }
+  uint32_t words[4] = {0, 0, 1, 0};
+  SAH_HIP(hipMemcpyAsync(A.err, words, sizeof words, hipMemcpyHostToDevice, stream));
+  sah_check_kernel<<<grid_of(n), 256, 0, stream>>>(d_boxes, n, A.err + 1);
   SAH_HIP(hipGetLastError());
-  SAH_HIP(hipMemcpyAsync(&bad, B.bad, 4, hipMemcpyDeviceToHost, stream));
-  SAH_HIP(hipStreamSynchronize(stream));
-  if (bad) return RZ_ERR_INVALID_ARGUMENT;
-  if (n <= 2 * gran) {
+  if (whole) {
     // No split position exists, so the reference's recursion is undefined
     // here (bestIndex stays -1); the whole set is one batch in input order.
+    SAH_HIP(hipMemcpyAsync(words, A.err, sizeof words, hipMemcpyDeviceToHost, stream));
+    SAH_HIP(hipStreamSynchronize(stream));
+    if (words[1]) return RZ_ERR_INVALID_ARGUMENT;
     sah_iota_kernel<<<grid_of(n), 256, 0, stream>>>(d_indices, n);
     SAH_HIP(hipGetLastError());
     SAH_HIP(hipStreamSynchronize(stream));
@@ -285,100 +482,97 @@ int sah_batches_run(hipStream_t stream, uint32_t n, const float* d_boxes, uint32
     *nBatches = 1;
     return RZ_OK;
   }
-  // At most n / gran + 1 segments: every closed piece holds gran items or more.
-  const size_t maxSeg = size_t(n) / gran + 2;
-  const uint32_t nChunks = (n + gran - 1) / gran;
-  if (alloc(&B.idx[0], n) != hipSuccess || alloc(&B.idx[1], n) != hipSuccess || alloc(&B.keys[0], n) != hipSuccess ||
-      alloc(&B.keys[1], n) != hipSuccess || alloc(&B.segOf, n) != hipSuccess ||
-      alloc(&B.chunkSeg, nChunks) != hipSuccess || alloc(&B.revSeg, nChunks) != hipSuccess ||
-      alloc(&B.segStart, maxSeg) != hipSuccess || alloc(&B.segLen, maxSeg) != hipSuccess ||
-      alloc(&B.segOpen, maxSeg) != hipSuccess || alloc(&B.segBest, maxSeg) != hipSuccess ||
-      alloc(&B.fwd, nChunks) != hipSuccess || alloc(&B.fwdScan, nChunks) != hipSuccess ||
-      alloc(&B.rev, nChunks) != hipSuccess || alloc(&B.revScan, nChunks) != hipSuccess)
-    return RZ_ERR_OUT_OF_MEMORY;
-  size_t sortBytes = 0, scanBytes = 0;
-  SAH_HIP(rocprim::radix_sort_pairs(nullptr, sortBytes, B.keys[0], B.keys[1], B.idx[0], B.idx[1], n, 0u, 64u,
-                                    stream));
-  SAH_HIP(rocprim::inclusive_scan_by_key(nullptr, scanBytes, B.chunkSeg, B.fwd, B.fwdScan, size_t(nChunks), MergeExt(),
-                                         rocprim::equal_to<uint32_t>(), stream));
-  size_t tempBytes = std::max(sortBytes, scanBytes);
-  if (alloc(reinterpret_cast<uint8_t**>(&B.temp), tempBytes) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
 
-  sah_iota_kernel<<<grid_of(n), 256, 0, stream>>>(B.idx[0], n);
-  SAH_HIP(hipGetLastError());
-  int cur = 0;
-  // The root is split whatever its size (generateBatches calls the
-  // recursion on it directly); a child recurses when it holds target items
-  // or more (SurfaceAreaHeuristic.cpp:81-92).
-  std::vector<uint32_t> start{0}, len{n}, open{1};
-  std::vector<uint64_t> best;
+  // The orders, in four rounds of stable sorts, each sorting two or three
+  // arrays at once:
+  //   (x)        (z)
+  //   (y, x)     (y, z)     (x, z)
+  //   (z, y, x)  (x, y, z)  (y, x, z)
+  //   (x, z, y)  (y, z, x)
+  auto sort_round = [&](const SortRound& r, uint32_t parts, uint32_t* out) -> hipError_t {
+    sah_round_keys_kernel<<<dim3(grid_of(n), parts), 256, 0, stream>>>(r, d_boxes, n, keys, values);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    size_t bytes = tempBytes;
+    return rocprim::radix_sort_pairs(temp, bytes, keys, keysOut, values, out, size_t(parts) * n, 0u, 34u, stream);
+  };
+  auto order = [&](int o) { return A.orders + size_t(o) * n; };
+  // The third round's results are not neighbours in `orders`: it goes through
+  // nextOrders, which the levels only write.
+  uint32_t* round3 = A.nextOrders;
+  SAH_HIP(sort_round({{{nullptr, 0}, {nullptr, 2}, {nullptr, 0}}}, 2, round1));
+  SAH_HIP(sort_round({{{round1, 1}, {round1 + n, 1}, {round1 + n, 0}}}, 3, round2));
+  SAH_HIP(sort_round({{{round2, 2}, {round2 + n, 0}, {round2 + 2 * size_t(n), 1}}}, 3, round3));
+  static_assert(kYzx == kXzy + 1 && kXyz == kZyx + 1 && kYxz == kZyx + 2, "the rounds write neighbouring orders");
+  SAH_HIP(sort_round({{{round3, 0}, {round3, 1}, {nullptr, 0}}}, 2, order(kXzy)));
+  SAH_HIP(hipMemcpyAsync(order(kZyx), round3, n3 * 4, hipMemcpyDeviceToDevice, stream));
+
+  // The root is split whatever its size (generateBatches calls the recursion
+  // on it directly).
+  const Segment root = {0u, n, 3u};
+  const unsigned long long none = ~0ull;
+  SAH_HIP(hipMemcpyAsync(A.segs, &root, sizeof root, hipMemcpyHostToDevice, stream));
+  SAH_HIP(hipMemcpyAsync(A.best, &none, sizeof none, hipMemcpyHostToDevice, stream));
+  SAH_HIP(hipMemsetAsync(A.arrived, 0, 4, stream));
+  SAH_HIP(hipMemsetAsync(A.chunkSeg, 0, size_t(nChunks) * 4, stream));
+  SAH_HIP(hipMemsetAsync(A.starts, 0, nChunks, stream));
+  SAH_HIP(hipMemsetAsync(A.starts, 1, 1, stream));
+  A.boxes = d_boxes;
+  A.n = n;
+  A.nChunks = nChunks;
+  A.gran = gran;
+  A.target = target;
+  A.rootX = round1;
+  A.rootY = round2;
+  A.lefts = lefts;
+  B = A;
+  std::swap(B.orders, B.nextOrders);
+  std::swap(B.chunkSeg, B.nextChunkSeg);
+  std::swap(B.segs, B.nextSegs);
+  std::swap(B.best, B.nextBest);
+  std::swap(B.arrived, B.nextArrived);
+  std::swap(B.nOpen, B.nextNOpen);
+  // Levels until none is open: the host looks after as many as even splits
+  // need, then after every second one (a level without open segments only
+  // copies the orders).
+  uint32_t level = 0, look = 1;
+  while ((uint64_t(target) << look) <= n) ++look;
   while (true) {
-    const uint32_t S = uint32_t(start.size());
-    uint32_t bits = 0;
-    while ((1ull << bits) < S) ++bits;
-    SAH_HIP(hipMemcpyAsync(B.segStart, start.data(), S * 4, hipMemcpyHostToDevice, stream));
-    SAH_HIP(hipMemcpyAsync(B.segLen, len.data(), S * 4, hipMemcpyHostToDevice, stream));
-    SAH_HIP(hipMemcpyAsync(B.segOpen, open.data(), S * 4, hipMemcpyHostToDevice, stream));
-    SAH_HIP(hipMemsetAsync(B.segBest, 0xFF, S * 8, stream));
-    sah_segof_kernel<<<grid_of(n), 256, 0, stream>>>(B.segStart, S, n, B.segOf);
+    const SahLevel& L = level & 1u ? B : A;
+    sah_chunks_kernel<<<dim3(grid_of(nChunks), 3), 256, 0, stream>>>(L);
     SAH_HIP(hipGetLastError());
-    for (int axis = 0; axis <= 3; ++axis) {
-      // Axes 0-2 score the splits; the fourth pass re-sorts along the winner.
-      sah_keys_kernel<<<grid_of(n), 256, 0, stream>>>(d_boxes, B.idx[cur], B.segOf, B.segOpen, B.segBest,
-                                                      axis < 3 ? axis : -1, n, B.keys[0]);
-      SAH_HIP(hipGetLastError());
-      size_t bytes = tempBytes;
-      SAH_HIP(rocprim::radix_sort_pairs(B.temp, bytes, B.keys[0], B.keys[1], B.idx[cur], B.idx[cur ^ 1], n, 0u,
-                                        32u + bits, stream));
-      cur ^= 1;
-      if (axis == 3) break;
-      sah_chunks_kernel<<<grid_of(nChunks), 256, 0, stream>>>(d_boxes, B.idx[cur], B.segOf, n, gran, nChunks,
-                                                              B.fwd, B.rev, B.chunkSeg, B.revSeg);
-      SAH_HIP(hipGetLastError());
-      bytes = tempBytes;
-      SAH_HIP(rocprim::inclusive_scan_by_key(B.temp, bytes, B.chunkSeg, B.fwd, B.fwdScan, size_t(nChunks), MergeExt(),
-                                             rocprim::equal_to<uint32_t>(), stream));
-      bytes = tempBytes;
-      SAH_HIP(rocprim::inclusive_scan_by_key(B.temp, bytes, B.revSeg, B.rev, B.revScan, size_t(nChunks), MergeExt(),
-                                             rocprim::equal_to<uint32_t>(), stream));
-      sah_cost_kernel<<<grid_of(nChunks), 256, 0, stream>>>(B.fwdScan, B.revScan, B.chunkSeg, B.segStart, B.segLen,
-                                                            B.segOpen, nChunks, gran, uint32_t(axis), B.segBest);
-      SAH_HIP(hipGetLastError());
-    }
-    best.resize(S);
-    SAH_HIP(hipMemcpyAsync(best.data(), B.segBest, S * 8, hipMemcpyDeviceToHost, stream));
+    const uint32_t open = level < 31u ? std::min(maxOpen, 1u << level) : maxOpen;
+    if (level < 4u)
+      sah_split_kernel<1024><<<dim3(open, 3), 1024, 0, stream>>>(L);
+    else
+      sah_split_kernel<256><<<dim3(open, 3), 256, 0, stream>>>(L);
+    SAH_HIP(hipGetLastError());
+    sah_sides_kernel<<<grid_of(n), 256, 0, stream>>>(L);
+    SAH_HIP(hipGetLastError());
+    size_t bytes = tempBytes;
+    SAH_HIP(rocprim::exclusive_scan(temp, bytes, left_iterator(L), lefts, 0u, size_t(kOrders) * n,
+                                    rocprim::plus<uint32_t>(), stream));
+    sah_partition_kernel<<<dim3(grid_of(n), kOrders), 256, 0, stream>>>(L);
+    SAH_HIP(hipGetLastError());
+    ++level;
+    if (level < look) continue;
+    look = level + 2;
+    SAH_HIP(hipMemcpyAsync(words, A.err, sizeof words, hipMemcpyDeviceToHost, stream));
     SAH_HIP(hipStreamSynchronize(stream));
-    std::vector<uint32_t> nStart, nLen, nOpen;
-    bool any = false;
-    for (uint32_t s = 0; s < S; ++s) {
-      if (!open[s]) {
-        nStart.push_back(start[s]);
-        nLen.push_back(len[s]);
-        nOpen.push_back(0);
-        continue;
-      }
-      // Every open segment has a split position: the root holds more than
-      // 2 gran items and a child stays open only with target > 2 gran items.
-      if (best[s] == ~0ull) return RZ_ERR_DEVICE;
-      const uint32_t k = uint32_t(best[s] & 0x3FFFFFFFu);
-      const uint32_t parts[2][2] = {{start[s], k}, {start[s] + k, len[s] - k}};
-      for (const auto& part : parts) {
-        const uint32_t o = part[1] >= target ? 1u : 0u;
-        nStart.push_back(part[0]);
-        nLen.push_back(part[1]);
-        nOpen.push_back(o);
-        any = any || o;
-      }
-    }
-    start.swap(nStart);
-    len.swap(nLen);
-    open.swap(nOpen);
-    if (!any) break;
+    if (words[1]) return RZ_ERR_INVALID_ARGUMENT;
+    if (words[0]) return RZ_ERR_DEVICE;
+    if (words[2] == 0 && words[3] == 0) break;
   }
-  SAH_HIP(hipMemcpyAsync(d_indices, B.idx[cur], size_t(n) * 4, hipMemcpyDeviceToDevice, stream));
+  sah_emit_kernel<<<grid_of(n), 256, 0, stream>>>(level & 1u ? B.orders : A.orders, A.batchAxis, n, gran, d_indices);
+  SAH_HIP(hipGetLastError());
+  std::vector<uint8_t> starts(nChunks);
+  SAH_HIP(hipMemcpyAsync(starts.data(), A.starts, nChunks, hipMemcpyDeviceToHost, stream));
   SAH_HIP(hipStreamSynchronize(stream));
-  for (size_t s = 0; s < start.size(); ++s) batchOffsets[s + 1] = start[s] + len[s];
-  *nBatches = uint32_t(start.size());
+  uint32_t count = 0;
+  for (uint32_t c = 1; c < nChunks; ++c)
+    if (starts[c]) batchOffsets[++count] = c * gran;
+  batchOffsets[++count] = n;
+  *nBatches = count;
   return RZ_OK;
 }
 
