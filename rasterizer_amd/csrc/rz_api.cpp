@@ -73,6 +73,7 @@ struct rz_context {
   uint32_t pyrX = 0, pyrY = 0;
   uint64_t* d_cov = nullptr;
   uint32_t* d_rcp = nullptr;
+  uint32_t* d_rsqrt = nullptr;  // RSQRTPS table, for scene preparation (ensure_rsqrt)
   uint32_t* d_err = nullptr;
   Mvp mvp{};
   // per-draw buffers
@@ -143,6 +144,7 @@ static void free_context(rz_context* c) {
   hipFree(c->d_tileMin);
   hipFree(c->d_cov);
   hipFree(c->d_rcp);
+  hipFree(c->d_rsqrt);
   hipFree(c->d_err);
   hipFree(c->d_items);
   hipFree(c->d_state);
@@ -865,6 +867,19 @@ extern "C" int rz_bake(const float* vertices, uint32_t n, const float refMin[4],
                                                                                              : RZ_ERR_INVALID_ARGUMENT;
 }
 
+// This host's RSQRTPS table on the context's device, uploaded by the first
+// call that needs it (the caller has checked that the host has one).
+static int ensure_rsqrt(rz_context* c) {
+  if (c->d_rsqrt) return RZ_OK;
+  if (dev_alloc(&c->d_rsqrt, 8192) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
+  if (hipMemcpy(c->d_rsqrt, rzi::host_tables().rsqrt, 8192 * 4, hipMemcpyHostToDevice) != hipSuccess) {
+    hipFree(c->d_rsqrt);
+    c->d_rsqrt = nullptr;
+    return RZ_ERR_DEVICE;
+  }
+  return RZ_OK;
+}
+
 extern "C" int rz_bake_device(rz_context* ctx, uint32_t n, const uint32_t* vertexOffsets, const float* d_vertices,
                               const float* refMinMax, uint32_t* d_packets, float* d_bounds) {
   if (!ctx || (n && (!vertexOffsets || !d_vertices || !refMinMax || !d_packets || !d_bounds)))
@@ -877,40 +892,33 @@ extern "C" int rz_bake_device(rz_context* ctx, uint32_t n, const uint32_t* verte
   if (vertexOffsets[n] >= (1u << 31)) return RZ_ERR_TOO_LARGE;
   const rzi::HostTables& tabs = rzi::host_tables();
   if (tabs.rsqrtStatus != RZ_OK) return tabs.rsqrtStatus;
-  const size_t quads = vertexOffsets[n] / 4;
+  const int status = ensure_rsqrt(ctx);
+  if (status != RZ_OK) return status;
+  uint32_t largest = 0;
+  for (uint32_t i = 0; i < n; ++i) largest = std::max(largest, (vertexOffsets[i + 1] - vertexOffsets[i]) / 4);
+  const size_t quads = largest > kBakeLdsQuads ? vertexOffsets[n] / 4 : 0;
+  // One allocation: reference boxes, then normals (both 16-byte aligned),
+  // cluster, order and the offsets.
+  unsigned char* d_all = nullptr;
+  const size_t refBytes = size_t(n) * 32, offsetBytes = (size_t(n) + 1) * 4;
+  if (dev_alloc(&d_all, refBytes + quads * 24 + offsetBytes) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
   BakeParams p{};
-  uint32_t* d_offsets = nullptr;
-  float* d_ref = nullptr;
-  uint32_t* d_rsqrt = nullptr;
-  int status = RZ_OK;
-  if (dev_alloc(&d_offsets, size_t(n) + 1) != hipSuccess || dev_alloc(&d_ref, size_t(n) * 8) != hipSuccess ||
-      dev_alloc(&d_rsqrt, 8192) != hipSuccess || dev_alloc(&p.normals, quads) != hipSuccess ||
-      dev_alloc(&p.cluster, quads) != hipSuccess || dev_alloc(&p.order, quads) != hipSuccess) {
-    status = RZ_ERR_OUT_OF_MEMORY;
-  } else if (hipMemcpyAsync(d_offsets, vertexOffsets, (size_t(n) + 1) * 4, hipMemcpyHostToDevice, ctx->stream) !=
-                 hipSuccess ||
-             hipMemcpyAsync(d_ref, refMinMax, size_t(n) * 32, hipMemcpyHostToDevice, ctx->stream) != hipSuccess ||
-             hipMemcpyAsync(d_rsqrt, tabs.rsqrt, sizeof tabs.rsqrt, hipMemcpyHostToDevice, ctx->stream) !=
-                 hipSuccess) {
-    status = RZ_ERR_DEVICE;
-  } else {
-    p.vertices = d_vertices;
-    p.offsets = d_offsets;
-    p.ref = d_ref;
-    p.packets = d_packets;
-    p.bounds = d_bounds;
-    p.rsqrt = d_rsqrt;
-    if (launch_bake(p, n, ctx->stream) != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess)
-      status = RZ_ERR_DEVICE;
-  }
-  (void)hipStreamSynchronize(ctx->stream);
-  hipFree(d_offsets);
-  hipFree(d_ref);
-  hipFree(d_rsqrt);
-  hipFree(p.normals);
-  hipFree(p.cluster);
-  hipFree(p.order);
-  return status;
+  p.vertices = d_vertices;
+  p.packets = d_packets;
+  p.bounds = d_bounds;
+  p.rsqrt = ctx->d_rsqrt;
+  p.normals = reinterpret_cast<float4*>(d_all + refBytes);
+  p.cluster = reinterpret_cast<uint32_t*>(d_all + refBytes + quads * 16);
+  p.order = p.cluster + quads;
+  uint32_t* d_offsets = p.order + quads;
+  p.offsets = d_offsets;
+  p.ref = reinterpret_cast<float*>(d_all);
+  bool ok = hipMemcpyAsync(d_offsets, vertexOffsets, offsetBytes, hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
+            hipMemcpyAsync(d_all, refMinMax, refBytes, hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
+            launch_bake(p, n, ctx->stream) == hipSuccess;
+  ok = hipStreamSynchronize(ctx->stream) == hipSuccess && ok;
+  hipFree(d_all);
+  return ok ? RZ_OK : RZ_ERR_DEVICE;
 }
 
 extern "C" int rz_quad_decompose_device(rz_context* ctx, uint32_t nTriangles, const uint32_t* d_indices,
@@ -922,7 +930,9 @@ extern "C" int rz_quad_decompose_device(rz_context* ctx, uint32_t nTriangles, co
   if (nTriangles == 0) return RZ_OK;
   const rzi::HostTables& tabs = rzi::host_tables();
   if (tabs.rsqrtStatus != RZ_OK) return tabs.rsqrtStatus;
-  return quad_decompose_run(ctx->stream, nTriangles, d_indices, d_vertices, nVertices, tabs.rsqrt, d_out, nOut);
+  const int status = ensure_rsqrt(ctx);
+  if (status != RZ_OK) return status;
+  return quad_decompose_run(ctx->stream, nTriangles, d_indices, d_vertices, nVertices, ctx->d_rsqrt, d_out, nOut);
 }
 
 extern "C" int rz_sah_batches(rz_context* ctx, uint32_t n, const float* d_boxes, uint32_t targetSize,
@@ -942,22 +952,21 @@ int prepare_scene(rz_context* ctx, uint32_t nQuads, const float* d_vertices, con
                   uint32_t nBox, uint32_t targetSize, uint32_t splitGranularity, uint32_t* d_packets,
                   float* d_bounds, uint32_t* quadOffsets, uint32_t* nOccluders, float refMinMax[8]) {
   const uint32_t nPad = (nQuads + 7u) & ~7u;  // Main.cpp:90-94
-  float* d_boxes = nullptr;
+  // One allocation: the vertices in batch order (16-byte aligned), the padded
+  // quads' boxes, their order, and the scene box with its scratch.
   float* d_sorted = nullptr;
-  uint32_t* d_order = nullptr;
-  uint32_t* d_keys = nullptr;
   int status = RZ_OK;
-  // Scene box as ordered-float keys (min xyzw, max xyzw), then a word that
-  // the boxes kernel sets when a vertex is not finite or exceeds 2^40.
-  uint32_t keys[9] = {~0u, ~0u, ~0u, ~0u, 0u, 0u, 0u, 0u, 0u};
-  if (dev_alloc(&d_boxes, size_t(nPad) * 8) != hipSuccess || dev_alloc(&d_sorted, size_t(nPad) * 16) != hipSuccess ||
-      dev_alloc(&d_order, nPad) != hipSuccess || dev_alloc(&d_keys, 9) != hipSuccess) {
-    status = RZ_ERR_OUT_OF_MEMORY;
-  } else if (hipMemcpyAsync(d_keys, keys, sizeof keys, hipMemcpyHostToDevice, ctx->stream) != hipSuccess ||
-             launch_scene_boxes(d_vertices, nQuads, nPad, d_boxes, d_keys, ctx->stream) != hipSuccess ||
-             (d_boxVertices && launch_vertex_keys(d_boxVertices, nBox, d_keys, ctx->stream) != hipSuccess) ||
-             hipMemcpyAsync(keys, d_keys, sizeof keys, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
-             hipStreamSynchronize(ctx->stream) != hipSuccess) {
+  // Scene box as ordered-float keys (min xyzw, max xyzw), then a word that is
+  // set when a vertex is not finite or exceeds 2^40.
+  uint32_t keys[9];
+  if (dev_alloc(&d_sorted, size_t(nPad) * 25 + 9 + size_t(kSceneParts) * 9) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
+  float* d_boxes = d_sorted + size_t(nPad) * 16;
+  uint32_t* d_order = reinterpret_cast<uint32_t*>(d_boxes + size_t(nPad) * 8);
+  uint32_t* d_keys = d_order + nPad;
+  if (launch_scene_boxes(d_vertices, nQuads, nPad, d_boxVertices, nBox, d_boxes, d_keys + 9, d_keys, ctx->stream) !=
+          hipSuccess ||
+      hipMemcpyAsync(keys, d_keys, sizeof keys, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+      hipStreamSynchronize(ctx->stream) != hipSuccess) {
     status = RZ_ERR_DEVICE;
   } else if (keys[8] != 0u) {
     status = RZ_ERR_INVALID_ARGUMENT;
@@ -983,10 +992,7 @@ int prepare_scene(rz_context* ctx, uint32_t nQuads, const float* d_vertices, con
     }
   }
   (void)hipStreamSynchronize(ctx->stream);
-  hipFree(d_boxes);
   hipFree(d_sorted);
-  hipFree(d_order);
-  hipFree(d_keys);
   return status;
 }
 
@@ -1029,11 +1035,12 @@ extern "C" int rz_prepare_mesh_device(rz_context* ctx, uint32_t nTriangles, cons
   uint32_t* d_quadIdx = nullptr;
   float* d_quadVertices = nullptr;
   uint32_t nWords = 0;
-  int status = RZ_OK;
+  int status = ensure_rsqrt(ctx);
   // Main.cpp:86: the quads' indices, then their vertices in quad order.
+  if (status != RZ_OK) return status;
   if (dev_alloc(&d_quadIdx, size_t(nTriangles) * 4) != hipSuccess) status = RZ_ERR_OUT_OF_MEMORY;
   else
-    status = quad_decompose_run(ctx->stream, nTriangles, d_indices, d_vertices, nVertices, tabs.rsqrt, d_quadIdx,
+    status = quad_decompose_run(ctx->stream, nTriangles, d_indices, d_vertices, nVertices, ctx->d_rsqrt, d_quadIdx,
                                 &nWords);
   if (status == RZ_OK && nWords > 0) {
     if (dev_alloc(&d_quadVertices, size_t(nWords) * 4) != hipSuccess)

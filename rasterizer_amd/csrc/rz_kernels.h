@@ -287,7 +287,10 @@ uint32_t mlp_forward_max_groups();
 // vertices[offsets[o] .. offsets[o + 1]) (4 floats each, a multiple of 32),
 // its reference box ref[8o .. 8o + 8) (min xyzw, max xyzw); packets get one
 // word per vertex at the same offsets, bounds 12 floats per occluder
-// (boundsMin, boundsMax, centre).  Scratch per quad: normals, cluster, order.
+// (boundsMin, boundsMax, centre).  Scratch per quad (normals, cluster, order)
+// is used by occluders of more than kBakeLdsQuads quads only, and may be null
+// without any.
+constexpr uint32_t kBakeLdsQuads = 1024;  // 40 KB of LDS an occluder, four to a CU
 struct BakeParams {
   const float* vertices;
   const uint32_t* offsets;
@@ -308,19 +311,19 @@ int sah_batches_run(hipStream_t stream, uint32_t n, const float* d_boxes, uint32
 // writes the quads' indices to d_out and their word count to *nOut.  An
 // RZ_* status.
 int quad_decompose_run(hipStream_t stream, uint32_t nTri, const uint32_t* d_idx, const float* d_vertices,
-                       uint32_t nVertices, const uint32_t* hostRsqrt, uint32_t* d_out, uint32_t* nOut);
-// Scene preparation around it (rz_sah.hip): boxes of nPad padded quads and
-// the scene box as ordered-float keys (min xyzw, max xyzw; the caller sets
-// them to ~0 and 0 first) and sceneKeys[8] set non-zero when a vertex has a
-// coordinate (x, y, z) that is not finite or exceeds 2^40 (zero it first);
-// the padded quads' vertices gathered in `order`.
-hipError_t launch_scene_boxes(const float* vertices, uint32_t nQuads, uint32_t nPad, float* boxes,
-                              uint32_t* sceneKeys, hipStream_t stream);
+                       uint32_t nVertices, const uint32_t* d_rsqrt, uint32_t* d_out, uint32_t* nOut);
+// Scene preparation around it (rz_sah.hip): boxes of nPad padded quads; the
+// scene box over the padded quads' vertices and, when given, nBox more
+// vertices, as ordered-float keys (min xyzw, max xyzw) in sceneKeys[0..8);
+// sceneKeys[8] is 1 when a vertex has a coordinate (x, y, z) that is not
+// finite or exceeds 2^40, else 0.  partials: kSceneParts * 9 words of scratch.
+constexpr uint32_t kSceneParts = 512;
+hipError_t launch_scene_boxes(const float* vertices, uint32_t nQuads, uint32_t nPad, const float* boxVertices,
+                              uint32_t nBox, float* boxes, uint32_t* partials, uint32_t* sceneKeys,
+                              hipStream_t stream);
+// The padded quads' vertices gathered in `order`.
 hipError_t launch_scene_gather(const float* vertices, uint32_t nQuads, uint32_t nPad, const uint32_t* order,
                                float* out, hipStream_t stream);
-// The scene box's ordered keys (and the bad-vertex word) over a whole vertex
-// buffer of n xyzw vertices, folded into sceneKeys.
-hipError_t launch_vertex_keys(const float* vertices, uint32_t n, uint32_t* sceneKeys, hipStream_t stream);
 // Quad q's four vertices, vertices[quadIdx[4q + j]], for nWords / 4 quads.
 hipError_t launch_quad_gather(const float* vertices, const uint32_t* quadIdx, uint32_t nWords, float* out,
                               hipStream_t stream);

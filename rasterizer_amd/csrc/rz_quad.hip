@@ -239,28 +239,20 @@ hipError_t launch_quad_gather(const float* vertices, const uint32_t* quadIdx, ui
 }
 
 int quad_decompose_run(hipStream_t stream, uint32_t nTri, const uint32_t* d_idx, const float* d_vertices,
-                       uint32_t nVertices, const uint32_t* hostRsqrt, uint32_t* d_out, uint32_t* nOut) {
+                       uint32_t nVertices, const uint32_t* d_rsqrt, uint32_t* d_out, uint32_t* nOut) {
   *nOut = 0;
   if (nTri == 0) return RZ_OK;
   if (nTri > 0x7FFFFFFFu / 3u) return RZ_ERR_TOO_LARGE;
   const uint32_t nHalf = 3u * nTri;
   QdBuffers B;
-  uint32_t* d_rsq = nullptr;
   if (qd_alloc(&B.keys[0], nHalf) != hipSuccess || qd_alloc(&B.keys[1], nHalf) != hipSuccess ||
       qd_alloc(&B.seqs[0], nHalf) != hipSuccess || qd_alloc(&B.seqs[1], nHalf) != hipSuccess ||
       qd_alloc(&B.revFirst, nHalf) != hipSuccess || qd_alloc(&B.linkCount, size_t(nHalf) + 1) != hipSuccess ||
       qd_alloc(&B.linkOff, size_t(nHalf) + 1) != hipSuccess || qd_alloc(&B.degree, size_t(nTri) + 1) != hipSuccess ||
       qd_alloc(&B.start, size_t(nTri) + 1) != hipSuccess || qd_alloc(&B.bad, 1) != hipSuccess ||
       qd_alloc(&B.writes, size_t(nTri) + 1) != hipSuccess || qd_alloc(&B.pos, size_t(nTri) + 1) != hipSuccess ||
-      qd_alloc(&B.mate, nTri) != hipSuccess || qd_alloc(&d_rsq, 8192) != hipSuccess) {
-    if (d_rsq) (void)hipFree(d_rsq);
+      qd_alloc(&B.mate, nTri) != hipSuccess)
     return RZ_ERR_OUT_OF_MEMORY;
-  }
-  struct RsqGuard {
-    uint32_t* p;
-    ~RsqGuard() { (void)hipFree(p); }
-  } rsqGuard{d_rsq};
-  QD_HIP(hipMemcpyAsync(d_rsq, hostRsqrt, 8192 * 4, hipMemcpyHostToDevice, stream));
   QD_HIP(hipMemsetAsync(B.bad, 0, 4, stream));
 
   // Half-edges, sorted by (key, insertion number).
@@ -288,7 +280,7 @@ int quad_decompose_run(hipStream_t stream, uint32_t nTri, const uint32_t* d_idx,
   P.keys = B.keys[1];
   P.seqs = B.seqs[1];
   P.revFirst = B.revFirst;
-  P.rsq = d_rsq;
+  P.rsq = d_rsqrt;
   P.linkCount = B.linkCount;
   P.linkOff = B.linkOff;
   P.degree = B.degree;

@@ -595,70 +595,88 @@ __device__ __forceinline__ float4 padded_vertex(const float4* __restrict__ v, ui
   return j < nQuads ? v[4 * size_t(j) + k] : v[0];
 }
 
-__global__ void __launch_bounds__(256) scene_boxes_kernel(const float4* __restrict__ vertices, uint32_t nQuads,
-                                                          uint32_t nPad, float4* __restrict__ boxes,
-                                                          uint32_t* __restrict__ sceneKeys) {
-  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  float4 mn = make_float4(INFINITY, INFINITY, INFINITY, INFINITY);
-  float4 mx = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-  uint32_t kmn[4] = {~0u, ~0u, ~0u, ~0u}, kmx[4] = {0u, 0u, 0u, 0u};
+// A thread's share of the scene box (Main.cpp:109-113) as ordered keys, and
+// whether it met a vertex that the SAH costs cannot take (they need finite
+// boxes of bounded size, as rz_sah_batches checks; NaN would also escape the
+// fminf/fmaxf boxes).
+struct SceneShare {
+  uint32_t mn[4] = {~0u, ~0u, ~0u, ~0u}, mx[4] = {0u, 0u, 0u, 0u};
   bool bad = false;
-  if (j < nPad) {
-    // Main.cpp:96-105: the quad's Aabb over its four vertices (all lanes).
+  __device__ void add(float4 v) {
+    const float c[4] = {v.x, v.y, v.z, v.w};
+    bad = bad || !(fabsf(v.x) <= 0x1p40f) || !(fabsf(v.y) <= 0x1p40f) || !(fabsf(v.z) <= 0x1p40f);
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+      mn[l] = min(mn[l], ordered_key(c[l]));
+      mx[l] = max(mx[l], ordered_key(c[l]));
+    }
+  }
+};
+
+// The work-group's (256 threads) share as nine words: minima, maxima, bad.
+__device__ void reduce_share(const SceneShare& s, uint32_t* __restrict__ out) {
+  __shared__ uint32_t part[4][9];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int l = 0; l < 4; ++l) {
+    const uint32_t a = __ockl_wfred_min_u32(s.mn[l]), b = __ockl_wfred_max_u32(s.mx[l]);
+    if (lane == 0u) {
+      part[wave][l] = a;
+      part[wave][4 + l] = b;
+    }
+  }
+  const uint64_t bad = __ballot(s.bad);
+  if (lane == 0u) part[wave][8] = bad != 0ull ? 1u : 0u;
+  __syncthreads();
+  if (threadIdx.x < 9u) {
+    uint32_t v = part[0][threadIdx.x];
+    for (int w = 1; w < 4; ++w) v = threadIdx.x < 4u ? min(v, part[w][threadIdx.x]) : max(v, part[w][threadIdx.x]);
+    out[threadIdx.x] = v;
+  }
+}
+
+// Main.cpp:96-105: the quads' Aabbs over their four vertices (all lanes), and
+// the scene box over those vertices and boxVertices (a whole vertex buffer can
+// hold vertices no quad references).  Each work-group writes its share of the
+// scene box; one atomic per wave and word on the same eight words took 0.83 ms
+// of the city mesh's preparation.
+__global__ void __launch_bounds__(256) scene_boxes_kernel(const float4* __restrict__ vertices, uint32_t nQuads,
+                                                          uint32_t nPad, const float4* __restrict__ boxVertices,
+                                                          uint32_t nBox, float4* __restrict__ boxes,
+                                                          uint32_t* __restrict__ partials) {
+  const uint32_t first = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+  SceneShare s;
+  for (uint32_t j = first; j < nPad; j += step) {
+    float4 mn = make_float4(INFINITY, INFINITY, INFINITY, INFINITY);
+    float4 mx = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
       const float4 v = padded_vertex(vertices, nQuads, j, k);
       mn = make_float4(fminf(mn.x, v.x), fminf(mn.y, v.y), fminf(mn.z, v.z), fminf(mn.w, v.w));
       mx = make_float4(fmaxf(mx.x, v.x), fmaxf(mx.y, v.y), fmaxf(mx.z, v.z), fmaxf(mx.w, v.w));
-      const float c[4] = {v.x, v.y, v.z, v.w};
-      // The SAH costs need finite boxes of bounded size (as rz_sah_batches
-      // checks); NaN would also escape the fminf/fmaxf boxes.
-      bad = bad || !(fabsf(v.x) <= 0x1p40f) || !(fabsf(v.y) <= 0x1p40f) || !(fabsf(v.z) <= 0x1p40f);
-#pragma unroll
-      for (int l = 0; l < 4; ++l) {
-        kmn[l] = min(kmn[l], ordered_key(c[l]));
-        kmx[l] = max(kmx[l], ordered_key(c[l]));
-      }
+      s.add(v);
     }
     boxes[2 * size_t(j)] = mn;
     boxes[2 * size_t(j) + 1] = mx;
   }
-  if (__ballot(bad) != 0ull && (threadIdx.x & 63u) == 0u) atomicOr(&sceneKeys[8], 1u);
-  // Main.cpp:109-113: the scene box over every vertex, as ordered keys.
-#pragma unroll
-  for (int l = 0; l < 4; ++l) {
-    const uint32_t a = __ockl_wfred_min_u32(kmn[l]), b = __ockl_wfred_max_u32(kmx[l]);
-    if ((threadIdx.x & 63u) == 0u) {
-      atomicMin(&sceneKeys[l], a);
-      atomicMax(&sceneKeys[4 + l], b);
-    }
-  }
+  for (uint32_t j = first; j < nBox; j += step) s.add(boxVertices[j]);
+  reduce_share(s, partials + 9 * size_t(blockIdx.x));
 }
 
-// Main.cpp:109-113 over a whole vertex buffer (which can hold vertices no
-// quad references): the scene box as ordered keys, and sceneKeys[8] set when
-// a vertex's x, y or z is not finite or exceeds 2^40.
-__global__ void __launch_bounds__(256) vertex_keys_kernel(const float4* __restrict__ vertices, uint32_t n,
-                                                          uint32_t* __restrict__ sceneKeys) {
-  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  uint32_t kmn[4] = {~0u, ~0u, ~0u, ~0u}, kmx[4] = {0u, 0u, 0u, 0u};
-  bool bad = false;
-  if (j < n) {
-    const float4 v = vertices[j];
-    const float c[4] = {v.x, v.y, v.z, v.w};
-    bad = !(fabsf(v.x) <= 0x1p40f) || !(fabsf(v.y) <= 0x1p40f) || !(fabsf(v.z) <= 0x1p40f);
+// The scene box from the work-groups' shares.
+__global__ void __launch_bounds__(256) scene_keys_kernel(const uint32_t* __restrict__ partials, uint32_t parts,
+                                                         uint32_t* __restrict__ sceneKeys) {
+  SceneShare s;
+  for (uint32_t p = threadIdx.x; p < parts; p += blockDim.x) {
+    const uint32_t* w = partials + 9 * size_t(p);
 #pragma unroll
-    for (int l = 0; l < 4; ++l) kmn[l] = kmx[l] = ordered_key(c[l]);
-  }
-  if (__ballot(bad) != 0ull && (threadIdx.x & 63u) == 0u) atomicOr(&sceneKeys[8], 1u);
-#pragma unroll
-  for (int l = 0; l < 4; ++l) {
-    const uint32_t a = __ockl_wfred_min_u32(kmn[l]), b = __ockl_wfred_max_u32(kmx[l]);
-    if ((threadIdx.x & 63u) == 0u) {
-      atomicMin(&sceneKeys[l], a);
-      atomicMax(&sceneKeys[4 + l], b);
+    for (int l = 0; l < 4; ++l) {
+      s.mn[l] = min(s.mn[l], w[l]);
+      s.mx[l] = max(s.mx[l], w[4 + l]);
     }
+    s.bad = s.bad || w[8] != 0u;
   }
+  reduce_share(s, sceneKeys);
 }
 
 __global__ void __launch_bounds__(256) scene_gather_kernel(const float4* __restrict__ vertices, uint32_t nQuads,
@@ -671,16 +689,16 @@ __global__ void __launch_bounds__(256) scene_gather_kernel(const float4* __restr
 
 }  // namespace
 
-hipError_t launch_scene_boxes(const float* vertices, uint32_t nQuads, uint32_t nPad, float* boxes,
-                              uint32_t* sceneKeys, hipStream_t stream) {
-  scene_boxes_kernel<<<grid_of(nPad), 256, 0, stream>>>(reinterpret_cast<const float4*>(vertices), nQuads, nPad,
-                                                        reinterpret_cast<float4*>(boxes), sceneKeys);
-  return hipGetLastError();
-}
-
-hipError_t launch_vertex_keys(const float* vertices, uint32_t n, uint32_t* sceneKeys, hipStream_t stream) {
-  if (n == 0) return hipSuccess;
-  vertex_keys_kernel<<<grid_of(n), 256, 0, stream>>>(reinterpret_cast<const float4*>(vertices), n, sceneKeys);
+hipError_t launch_scene_boxes(const float* vertices, uint32_t nQuads, uint32_t nPad, const float* boxVertices,
+                              uint32_t nBox, float* boxes, uint32_t* partials, uint32_t* sceneKeys,
+                              hipStream_t stream) {
+  const uint32_t parts = std::min(grid_of(std::max(nPad, boxVertices ? nBox : 0u)), kSceneParts);
+  scene_boxes_kernel<<<parts, 256, 0, stream>>>(reinterpret_cast<const float4*>(vertices), nQuads, nPad,
+                                                reinterpret_cast<const float4*>(boxVertices), boxVertices ? nBox : 0u,
+                                                reinterpret_cast<float4*>(boxes), partials);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  scene_keys_kernel<<<1, 256, 0, stream>>>(partials, parts, sceneKeys);
   return hipGetLastError();
 }
 
