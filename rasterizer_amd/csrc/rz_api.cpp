@@ -15,6 +15,7 @@
 #include "rz_host.h"
 #include "rz_internal.h"
 #include "rz_kernels.h"
+#include "rz_scratch.h"
 
 using namespace rzd;
 
@@ -73,6 +74,7 @@ struct rz_context {
   uint32_t pyrX = 0, pyrY = 0;
   uint64_t* d_cov = nullptr;
   uint32_t* d_rcp = nullptr;
+  Scratch scratch;              // scene preparation's working memory
   uint32_t* d_rsqrt = nullptr;  // RSQRTPS table, for scene preparation (ensure_rsqrt)
   uint32_t* d_err = nullptr;
   Mvp mvp{};
@@ -897,27 +899,25 @@ extern "C" int rz_bake_device(rz_context* ctx, uint32_t n, const uint32_t* verte
   uint32_t largest = 0;
   for (uint32_t i = 0; i < n; ++i) largest = std::max(largest, (vertexOffsets[i + 1] - vertexOffsets[i]) / 4);
   const size_t quads = largest > kBakeLdsQuads ? vertexOffsets[n] / 4 : 0;
-  // One allocation: reference boxes, then normals (both 16-byte aligned),
-  // cluster, order and the offsets.
-  unsigned char* d_all = nullptr;
-  const size_t refBytes = size_t(n) * 32, offsetBytes = (size_t(n) + 1) * 4;
-  if (dev_alloc(&d_all, refBytes + quads * 24 + offsetBytes) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
+  Scratch::Frame frame(ctx->scratch);
+  float* d_ref = ctx->scratch.take<float>(size_t(n) * 8);
+  uint32_t* d_offsets = ctx->scratch.take<uint32_t>(size_t(n) + 1);
   BakeParams p{};
   p.vertices = d_vertices;
   p.packets = d_packets;
   p.bounds = d_bounds;
   p.rsqrt = ctx->d_rsqrt;
-  p.normals = reinterpret_cast<float4*>(d_all + refBytes);
-  p.cluster = reinterpret_cast<uint32_t*>(d_all + refBytes + quads * 16);
-  p.order = p.cluster + quads;
-  uint32_t* d_offsets = p.order + quads;
+  p.normals = ctx->scratch.take<float4>(quads);
+  p.cluster = ctx->scratch.take<uint32_t>(quads);
+  p.order = ctx->scratch.take<uint32_t>(quads);
   p.offsets = d_offsets;
-  p.ref = reinterpret_cast<float*>(d_all);
-  bool ok = hipMemcpyAsync(d_offsets, vertexOffsets, offsetBytes, hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
-            hipMemcpyAsync(d_all, refMinMax, refBytes, hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
+  p.ref = d_ref;
+  if (!d_ref || !d_offsets || !p.normals || !p.cluster || !p.order) return RZ_ERR_OUT_OF_MEMORY;
+  bool ok = hipMemcpyAsync(d_offsets, vertexOffsets, (size_t(n) + 1) * 4, hipMemcpyHostToDevice, ctx->stream) ==
+                hipSuccess &&
+            hipMemcpyAsync(d_ref, refMinMax, size_t(n) * 32, hipMemcpyHostToDevice, ctx->stream) == hipSuccess &&
             launch_bake(p, n, ctx->stream) == hipSuccess;
   ok = hipStreamSynchronize(ctx->stream) == hipSuccess && ok;
-  hipFree(d_all);
   return ok ? RZ_OK : RZ_ERR_DEVICE;
 }
 
@@ -932,7 +932,8 @@ extern "C" int rz_quad_decompose_device(rz_context* ctx, uint32_t nTriangles, co
   if (tabs.rsqrtStatus != RZ_OK) return tabs.rsqrtStatus;
   const int status = ensure_rsqrt(ctx);
   if (status != RZ_OK) return status;
-  return quad_decompose_run(ctx->stream, nTriangles, d_indices, d_vertices, nVertices, ctx->d_rsqrt, d_out, nOut);
+  return quad_decompose_run(ctx->stream, ctx->scratch, nTriangles, d_indices, d_vertices, nVertices, ctx->d_rsqrt,
+                            d_out, nOut);
 }
 
 extern "C" int rz_sah_batches(rz_context* ctx, uint32_t n, const float* d_boxes, uint32_t targetSize,
@@ -940,7 +941,8 @@ extern "C" int rz_sah_batches(rz_context* ctx, uint32_t n, const float* d_boxes,
                               uint32_t* nBatches) {
   if (!ctx || !batchOffsets || !nBatches || (n && (!d_boxes || !d_indices))) return RZ_ERR_INVALID_ARGUMENT;
   if (reinterpret_cast<uintptr_t>(d_boxes) % 16u != 0u) return RZ_ERR_INVALID_ARGUMENT;  // read as float4
-  return sah_batches_run(ctx->stream, n, d_boxes, targetSize, splitGranularity, d_indices, batchOffsets, nBatches);
+  return sah_batches_run(ctx->stream, ctx->scratch, n, d_boxes, targetSize, splitGranularity, d_indices, batchOffsets,
+                         nBatches);
 }
 
 namespace {
@@ -952,17 +954,18 @@ int prepare_scene(rz_context* ctx, uint32_t nQuads, const float* d_vertices, con
                   uint32_t nBox, uint32_t targetSize, uint32_t splitGranularity, uint32_t* d_packets,
                   float* d_bounds, uint32_t* quadOffsets, uint32_t* nOccluders, float refMinMax[8]) {
   const uint32_t nPad = (nQuads + 7u) & ~7u;  // Main.cpp:90-94
-  // One allocation: the vertices in batch order (16-byte aligned), the padded
-  // quads' boxes, their order, and the scene box with its scratch.
-  float* d_sorted = nullptr;
+  // The vertices in batch order, the padded quads' boxes, their order, and the
+  // scene box with its partial results.
+  Scratch::Frame frame(ctx->scratch);
+  float* d_sorted = ctx->scratch.take<float>(size_t(nPad) * 16);
+  float* d_boxes = ctx->scratch.take<float>(size_t(nPad) * 8);
+  uint32_t* d_order = ctx->scratch.take<uint32_t>(nPad);
+  uint32_t* d_keys = ctx->scratch.take<uint32_t>(9 + size_t(kSceneParts) * 9);
+  if (!d_sorted || !d_boxes || !d_order || !d_keys) return RZ_ERR_OUT_OF_MEMORY;
   int status = RZ_OK;
   // Scene box as ordered-float keys (min xyzw, max xyzw), then a word that is
   // set when a vertex is not finite or exceeds 2^40.
   uint32_t keys[9];
-  if (dev_alloc(&d_sorted, size_t(nPad) * 25 + 9 + size_t(kSceneParts) * 9) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
-  float* d_boxes = d_sorted + size_t(nPad) * 16;
-  uint32_t* d_order = reinterpret_cast<uint32_t*>(d_boxes + size_t(nPad) * 8);
-  uint32_t* d_keys = d_order + nPad;
   if (launch_scene_boxes(d_vertices, nQuads, nPad, d_boxVertices, nBox, d_boxes, d_keys + 9, d_keys, ctx->stream) !=
           hipSuccess ||
       hipMemcpyAsync(keys, d_keys, sizeof keys, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
@@ -977,7 +980,8 @@ int prepare_scene(rz_context* ctx, uint32_t nQuads, const float* d_vertices, con
       std::memcpy(&refMinMax[l], &u, 4);
     }
     uint32_t nOcc = 0;
-    status = sah_batches_run(ctx->stream, nPad, d_boxes, targetSize, splitGranularity, d_order, quadOffsets, &nOcc);
+    status = sah_batches_run(ctx->stream, ctx->scratch, nPad, d_boxes, targetSize, splitGranularity, d_order,
+                             quadOffsets, &nOcc);
     if (status == RZ_OK) {
       if (launch_scene_gather(d_vertices, nQuads, nPad, d_order, d_sorted, ctx->stream) != hipSuccess) {
         status = RZ_ERR_DEVICE;
@@ -992,7 +996,6 @@ int prepare_scene(rz_context* ctx, uint32_t nQuads, const float* d_vertices, con
     }
   }
   (void)hipStreamSynchronize(ctx->stream);
-  hipFree(d_sorted);
   return status;
 }
 
@@ -1032,18 +1035,18 @@ extern "C" int rz_prepare_mesh_device(rz_context* ctx, uint32_t nTriangles, cons
   if (nTriangles > (1u << 28)) return RZ_ERR_TOO_LARGE;
   const rzi::HostTables& tabs = rzi::host_tables();
   if (tabs.rsqrtStatus != RZ_OK) return tabs.rsqrtStatus;
-  uint32_t* d_quadIdx = nullptr;
-  float* d_quadVertices = nullptr;
-  uint32_t nWords = 0;
   int status = ensure_rsqrt(ctx);
-  // Main.cpp:86: the quads' indices, then their vertices in quad order.
   if (status != RZ_OK) return status;
-  if (dev_alloc(&d_quadIdx, size_t(nTriangles) * 4) != hipSuccess) status = RZ_ERR_OUT_OF_MEMORY;
-  else
-    status = quad_decompose_run(ctx->stream, nTriangles, d_indices, d_vertices, nVertices, ctx->d_rsqrt, d_quadIdx,
-                                &nWords);
+  // Main.cpp:86: the quads' indices, then their vertices in quad order.
+  Scratch::Frame frame(ctx->scratch);
+  uint32_t* d_quadIdx = ctx->scratch.take<uint32_t>(size_t(nTriangles) * 4);
+  if (!d_quadIdx) return RZ_ERR_OUT_OF_MEMORY;
+  uint32_t nWords = 0;
+  status = quad_decompose_run(ctx->stream, ctx->scratch, nTriangles, d_indices, d_vertices, nVertices, ctx->d_rsqrt,
+                              d_quadIdx, &nWords);
   if (status == RZ_OK && nWords > 0) {
-    if (dev_alloc(&d_quadVertices, size_t(nWords) * 4) != hipSuccess)
+    float* d_quadVertices = ctx->scratch.take<float>(size_t(nWords) * 4);
+    if (!d_quadVertices)
       status = RZ_ERR_OUT_OF_MEMORY;
     else if (launch_quad_gather(d_vertices, d_quadIdx, nWords, d_quadVertices, ctx->stream) != hipSuccess)
       status = RZ_ERR_DEVICE;
@@ -1052,8 +1055,6 @@ extern "C" int rz_prepare_mesh_device(rz_context* ctx, uint32_t nTriangles, cons
                              d_packets, d_bounds, quadOffsets, nOccluders, refMinMax);
   }
   (void)hipStreamSynchronize(ctx->stream);
-  hipFree(d_quadIdx);
-  hipFree(d_quadVertices);
   return status;
 }
 

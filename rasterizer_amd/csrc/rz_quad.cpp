@@ -71,14 +71,15 @@ inline uint64_t edge_key(uint32_t a, uint32_t b) { return (uint64_t(a) << 32) | 
 // --- maximum matching (QuadDecomposition.cpp:28-309) ------------------------
 class Matcher {
  public:
-  Matcher(int n, const uint32_t* adjStart, const int* adj)
-      : start_(adjStart), adj_(adj), n_(n), mate_(size_t(n_), -1), bridge_(size_t(n_)),
-        depth_(size_t(n_), 0), parent_(size_t(n_), -1), blossom_(size_t(n_), 0), token_(size_t(n_), 0) {}
+  // Writes each vertex's partner, or -1, to mate[0 .. n).
+  Matcher(int n, const uint32_t* adjStart, const int* adj, int* mate)
+      : start_(adjStart), adj_(adj), n_(n), mate_(mate) {}
 
   // Greedy maximal matching in vertex and adjacency order (:34-54), then an
   // augmenting-path search from each vertex the greedy pass left single
   // (:56-67).
   void run() {
+    std::fill(mate_, mate_ + n_, -1);
     std::vector<int> single;
     for (int v = 0; v < n_; ++v) {
       if (mate_[v] != -1) continue;
@@ -93,6 +94,13 @@ class Matcher {
       }
       if (!found) single.push_back(v);
     }
+    if (single.empty()) return;
+    // The search's state, which a perfect greedy matching never needs.
+    bridge_.resize(size_t(n_));
+    depth_.resize(size_t(n_), 0);
+    parent_.resize(size_t(n_), -1);
+    blossom_.resize(size_t(n_), 0);
+    token_.resize(size_t(n_), 0);
     std::vector<int> path;
     for (int v : single) {
       if (mate_[v] != -1) continue;
@@ -102,8 +110,6 @@ class Matcher {
       }
     }
   }
-
-  int mate(int v) const { return mate_[v]; }
 
  private:
   void pair(int v, int w) {
@@ -234,7 +240,7 @@ class Matcher {
   const uint32_t* start_;
   const int* adj_;
   int n_;
-  std::vector<int> mate_;
+  int* mate_;
   std::vector<std::pair<int, int>> bridge_;
   std::vector<int> depth_, parent_, blossom_, token_;
   int round_ = 0;
@@ -246,9 +252,8 @@ class Matcher {
 namespace rzq {
 
 void match(uint32_t n, const uint32_t* start, const int* adj, int* mate) {
-  Matcher m(int(n), start, adj);
+  Matcher m(int(n), start, adj, mate);
   m.run();
-  for (uint32_t v = 0; v < n; ++v) mate[v] = m.mate(int(v));
 }
 
 }  // namespace rzq
@@ -316,7 +321,8 @@ extern "C" int rz_quad_decompose(const uint32_t* indices, size_t nIndices, const
     std::vector<uint32_t>().swap(linkA);
     std::vector<uint32_t>().swap(linkB);
 
-    Matcher m(int(T), start.data(), adj.data());
+    std::vector<int> mate(T);
+    Matcher m(int(T), start.data(), adj.data(), mate.data());
     m.run();
 
     // Quads in triangle order (:392-441): a single triangle becomes the
@@ -326,7 +332,7 @@ extern "C" int rz_quad_decompose(const uint32_t* indices, size_t nIndices, const
     size_t w = 0;
     for (uint32_t t = 0; t < T; ++t) {
       const uint32_t* i = indices + 3 * size_t(t);
-      const int nb = m.mate(int(t));
+      const int nb = mate[t];
       if (nb == -1) {
         out[w++] = i[0];
         out[w++] = i[2];

@@ -1,28 +1,36 @@
 // QuadDecomposition::decompose (QuadDecomposition.cpp:311-445) for meshes
 // that live in HBM.  Its data-parallel half runs on the device:
-//   - the half-edges (QuadDecomposition.cpp:355-365): one 64-bit key
-//     (from << 32 | to) per triangle edge, radix-sorted stably with the
+//   - the half-edges (QuadDecomposition.cpp:355-365): one key (from, to) per
+//     triangle edge, radix-sorted stably over its significant bits with the
 //     insertion number 3t + k as the value, so each directed edge's list is
 //     contiguous and in the order the reference appends to it;
 //   - per half-edge, the start of its reverse edge's list (a binary search);
-//   - the candidate graph (:366-384): per half-edge of triangle t, the
-//     triangles already listed on the reverse edge (those inserted up to t's
-//     last edge), each through the 0.5-unit plane test (:326-343) with the
-//     host CPU's RSQRTPS (from its table) and DPPS's summation order.  A count
-//     pass and a scan give every link its position in the reference's
-//     global link order; a fill pass writes the links, two adjacency entries
-//     each, and a stable radix sort by triangle turns them into flat
-//     adjacency lists in that order;
+//   - the candidate graph (:366-384): the reference links triangle t, edge by
+//     edge, with the triangles already listed on the reverse edge (those
+//     inserted up to t's last edge) that pass the 0.5-unit plane test
+//     (:326-343, with the host CPU's RSQRTPS from its table and DPPS's
+//     summation order).  A link enters both triangles' lists, so t's list
+//     holds first its own links and then those that later triangles make with
+//     it, by their insertion numbers: exactly the entries of its three reverse
+//     lists from there on, merged.  One thread per triangle gathers its list in
+//     that order (a count pass, a scan, a fill pass), so nothing is sorted;
 //   - the quads (:392-441), once the matching is known: one thread per
 //     triangle, positions from a scan of which triangles write.
 // The matching itself (:28-309) is a sequential augmenting-path search with
 // blossom shrinking; it runs on the host (rz_quad.cpp) over the adjacency
 // lists copied back, and the partners are copied to the device.
+//
+// Bound by the host: 1.3 ms of matching for the city mesh's 807 k list
+// entries, then the copies (pinned, so 57 GB/s) and the key sort.  Emitting the
+// links in order and sorting them by (triangle, place) took a second 64-bit
+// radix sort and its buffers; with it, and with every buffer allocated per
+// call, rz_prepare_mesh_device took 12.3 ms for that mesh, and takes 3.2 ms.
 #include <hip/hip_runtime.h>
 
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 
+#include <algorithm>
 #include <cstdint>
 #include <new>
 #include <vector>
@@ -30,6 +38,7 @@
 #include "rasterizer_amd.h"
 #include "rz_kernels.h"
 #include "rz_quad.h"
+#include "rz_scratch.h"
 #include "rz_x86.h"
 
 namespace rzd {
@@ -43,18 +52,20 @@ struct QdParams {
   const uint32_t* idx;  // 3 per triangle
   const float4* vertices;
   uint32_t nTri, nHalf;
+  uint32_t bits;         // of a vertex number: key = from << bits | to
   const uint64_t* keys;  // sorted half-edge keys
   const uint32_t* seqs;  // their insertion numbers
   const uint32_t* revFirst;  // per insertion number: first entry of the reverse edge's list
   const uint32_t* rsq;       // 8192-entry RSQRTPS table
-  uint32_t* linkCount;       // count pass: links per half-edge
-  const uint32_t* linkOff;   // fill pass: their first position in link order
-  uint32_t* adjKey;          // fill pass: 2 entries per link (triangle, neighbour)
-  uint32_t* adjVal;
-  uint32_t* degree;
+  uint32_t* degree;          // count pass: entries of each triangle's list
+  const uint32_t* start;     // fill pass: its first entry
+  int* adj;                  // fill pass: the lists
   uint32_t* bad;
 };
 
+__device__ __forceinline__ uint64_t edge_key(uint32_t from, uint32_t to, uint32_t bits) {
+  return (uint64_t(from) << bits) | to;
+}
 __device__ __forceinline__ uint32_t next3(uint32_t k) { return k == 2u ? 0u : k + 1u; }
 __device__ __forceinline__ uint32_t prev3(uint32_t k) { return k == 0u ? 2u : k - 1u; }
 
@@ -73,24 +84,25 @@ __device__ bool mergeable(float4 v0, float4 v1, float4 v2, float4 v3, const uint
 // Half-edge h = 3t + k runs from i[k] to i[(k + 1) % 3].  Every index is
 // the origin of one half-edge, so this is where indices are checked.
 __global__ void __launch_bounds__(kQdBlock) qd_half_edges_kernel(const uint32_t* __restrict__ idx, uint32_t nTri,
-                                                                 uint32_t nVertices, uint64_t* __restrict__ keys,
+                                                                 uint32_t nVertices, uint32_t bits,
+                                                                 uint64_t* __restrict__ keys,
                                                                  uint32_t* __restrict__ seqs, uint32_t* __restrict__ bad) {
   const uint32_t h = blockIdx.x * blockDim.x + threadIdx.x;
   if (h >= 3u * nTri) return;
   const uint32_t t = h / 3u, k = h - 3u * t;
   const uint32_t a = idx[h], b = idx[3u * t + next3(k)];
   if (a >= nVertices) atomicOr(bad, 1u);
-  keys[h] = (uint64_t(a) << 32) | b;
+  keys[h] = edge_key(a, b, bits);
   seqs[h] = h;
 }
 
 __global__ void __launch_bounds__(kQdBlock) qd_reverse_kernel(const uint64_t* __restrict__ keys,
                                                               const uint32_t* __restrict__ seqs, uint32_t nHalf,
-                                                              uint32_t* __restrict__ revFirst) {
+                                                              uint32_t bits, uint32_t* __restrict__ revFirst) {
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= nHalf) return;
   const uint64_t key = keys[p];
-  const uint64_t rev = (key << 32) | (key >> 32);
+  const uint64_t rev = ((key & ((uint64_t(1) << bits) - 1u)) << bits) | (key >> bits);
   uint32_t lo = 0, hi = nHalf;  // first entry >= rev
   while (lo < hi) {
     const uint32_t mid = (lo + hi) >> 1;
@@ -100,38 +112,62 @@ __global__ void __launch_bounds__(kQdBlock) qd_reverse_kernel(const uint64_t* __
   revFirst[seqs[p]] = lo;
 }
 
-// The candidate links of half-edge h = 3t + k (QuadDecomposition.cpp:366-
-// 384): the reverse edge's list entries inserted up to t's last edge (t
-// itself included), in list order.
+// Triangle t's adjacency list (QuadDecomposition.cpp:366-384): its own links,
+// edge by edge, each with the reverse list's entries inserted up to t's last
+// edge (t itself included, which enters twice), in list order; then the links
+// of later triangles with t, by their half-edges' insertion numbers, which is
+// the order of the rest of t's three reverse lists merged.  A later triangle's
+// plane test runs over its own edge, as when the reference reaches it.
 template <bool FILL>
-__global__ void __launch_bounds__(kQdBlock) qd_links_kernel(QdParams p) {
-  const uint32_t h = blockIdx.x * blockDim.x + threadIdx.x;
-  if (h >= p.nHalf) return;
-  const uint32_t t = h / 3u, k = h - 3u * t;
+__global__ void __launch_bounds__(kQdBlock) qd_adjacency_kernel(QdParams p) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= p.nTri) return;
   const uint32_t* i = p.idx + 3u * size_t(t);
-  const uint32_t a = i[k], b = i[next3(k)], c = i[prev3(k)];
-  const uint64_t rev = (uint64_t(b) << 32) | a;
-  const float4 v0 = p.vertices[a], v2 = p.vertices[b], v3 = p.vertices[c];
+  const uint32_t v[3] = {i[0], i[1], i[2]};
+  const float4 x[3] = {p.vertices[v[0]], p.vertices[v[1]], p.vertices[v[2]]};
   uint32_t n = 0;
-  const uint32_t base = FILL ? p.linkOff[h] : 0u;
-  for (uint32_t j = p.revFirst[h]; j < p.nHalf && p.keys[j] == rev; ++j) {
-    const uint32_t s = p.seqs[j];
-    if (s > 3u * t + 2u) break;  // listed after t
-    const uint32_t nb = s / 3u, kk = s - 3u * nb;
-    const uint32_t apex = p.idx[3u * size_t(nb) + prev3(kk)];
-    if (!mergeable(v0, p.vertices[apex], v2, v3, p.rsq)) continue;
-    if (FILL) {
-      const size_t q = size_t(base) + n;
-      p.adjKey[2 * q] = t;
-      p.adjVal[2 * q] = nb;
-      p.adjKey[2 * q + 1] = nb;
-      p.adjVal[2 * q + 1] = t;
-      atomicAdd(&p.degree[t], 1u);
-      atomicAdd(&p.degree[nb], 1u);
-    }
+  int* out = FILL ? p.adj + p.start[t] : nullptr;
+  auto push = [&](uint32_t nb) {
+    if (FILL) out[n] = int(nb);
     ++n;
+  };
+  uint64_t rev[3];
+  uint32_t at[3];
+#pragma unroll
+  for (uint32_t k = 0; k < 3; ++k) {
+    rev[k] = edge_key(v[next3(k)], v[k], p.bits);
+    uint32_t j = p.revFirst[3u * t + k];
+    for (; j < p.nHalf && p.keys[j] == rev[k]; ++j) {
+      const uint32_t s = p.seqs[j];
+      if (s > 3u * t + 2u) break;  // listed after t
+      const uint32_t nb = s / 3u;
+      const uint32_t apex = p.idx[3u * size_t(nb) + prev3(s - 3u * nb)];
+      if (!mergeable(x[k], p.vertices[apex], x[next3(k)], x[prev3(k)], p.rsq)) continue;
+      push(nb);
+      if (nb == t) push(nb);
+    }
+    at[k] = j;
   }
-  if (!FILL) p.linkCount[h] = n;
+  while (true) {
+    uint32_t s = 0xFFFFFFFFu, from = 3u;
+#pragma unroll
+    for (uint32_t k = 0; k < 3; ++k)
+      if (at[k] < p.nHalf && p.keys[at[k]] == rev[k] && p.seqs[at[k]] < s) {
+        s = p.seqs[at[k]];
+        from = k;
+      }
+    if (from == 3u) break;
+#pragma unroll
+    for (uint32_t k = 0; k < 3; ++k)
+      if (k == from) {
+        ++at[k];
+        const uint32_t nb = s / 3u, kk = s - 3u * nb;
+        const uint32_t* o = p.idx + 3u * size_t(nb);
+        // The later triangle's edge runs from v[next3(k)] to v[k].
+        if (mergeable(x[next3(k)], x[prev3(k)], x[k], p.vertices[o[prev3(kk)]], p.rsq)) push(nb);
+      }
+  }
+  if (!FILL) p.degree[t] = n;
 }
 
 // Which triangles write a quad: a single one (its degenerate quad) and the
@@ -168,7 +204,7 @@ __global__ void __launch_bounds__(kQdBlock) qd_emit_kernel(QdParams p, const int
     return;
   }
   for (uint32_t k = 0; k < 3u; ++k) {
-    const uint64_t rev = (uint64_t(i[next3(k)]) << 32) | i[k];
+    const uint64_t rev = edge_key(i[next3(k)], i[k], p.bits);
     for (uint32_t j = p.revFirst[3u * t + k]; j < p.nHalf && p.keys[j] == rev; ++j) {
       const uint32_t s = p.seqs[j];
       if (s / 3u != uint32_t(nb)) continue;
@@ -189,38 +225,9 @@ __global__ void __launch_bounds__(kQdBlock) qd_gather_kernel(const float4* __res
   if (w < nWords) out[w] = vertices[quadIdx[w]];
 }
 
-template <typename T>
-hipError_t qd_alloc(T** p, size_t count) {
-  *p = nullptr;
-  return hipMalloc(reinterpret_cast<void**>(p), (count ? count : 1) * sizeof(T));
-}
-
-struct QdBuffers {
-  uint64_t* keys[2] = {nullptr, nullptr};
-  uint32_t* seqs[2] = {nullptr, nullptr};
-  uint32_t *revFirst = nullptr, *linkCount = nullptr, *linkOff = nullptr, *degree = nullptr, *start = nullptr,
-           *bad = nullptr, *writes = nullptr, *pos = nullptr;
-  uint32_t *adjKey[2] = {nullptr, nullptr}, *adjVal[2] = {nullptr, nullptr};
-  int* mate = nullptr;
-  void* temp = nullptr;
-  ~QdBuffers() {
-    for (void* q : {(void*)keys[0], (void*)keys[1], (void*)seqs[0], (void*)seqs[1], (void*)revFirst,
-                    (void*)linkCount, (void*)linkOff, (void*)degree, (void*)start, (void*)bad, (void*)writes,
-                    (void*)pos, (void*)adjKey[0], (void*)adjKey[1], (void*)adjVal[0], (void*)adjVal[1], (void*)mate,
-                    temp})
-      if (q) (void)hipFree(q);
-  }
-  // Temporary storage of at least `bytes` for one rocPRIM call.
-  size_t tempBytes = 0;
-  hipError_t reserve(size_t bytes) {
-    if (bytes <= tempBytes) return hipSuccess;
-    if (temp) (void)hipFree(temp);
-    temp = nullptr;
-    tempBytes = 0;
-    const hipError_t e = hipMalloc(&temp, bytes ? bytes : 1);
-    if (e == hipSuccess) tempBytes = bytes;
-    return e;
-  }
+// List lengths add up without wrapping, so that too many links are refused.
+struct SatPlus {
+  __host__ __device__ uint32_t operator()(uint32_t a, uint32_t b) const { return a + b < a ? 0xFFFFFFFFu : a + b; }
 };
 
 }  // namespace
@@ -238,123 +245,108 @@ hipError_t launch_quad_gather(const float* vertices, const uint32_t* quadIdx, ui
   return hipGetLastError();
 }
 
-int quad_decompose_run(hipStream_t stream, uint32_t nTri, const uint32_t* d_idx, const float* d_vertices,
-                       uint32_t nVertices, const uint32_t* d_rsqrt, uint32_t* d_out, uint32_t* nOut) {
+int quad_decompose_run(hipStream_t stream, Scratch& scratch, uint32_t nTri, const uint32_t* d_idx,
+                       const float* d_vertices, uint32_t nVertices, const uint32_t* d_rsqrt, uint32_t* d_out,
+                       uint32_t* nOut) {
   *nOut = 0;
   if (nTri == 0) return RZ_OK;
   if (nTri > 0x7FFFFFFFu / 3u) return RZ_ERR_TOO_LARGE;
   const uint32_t nHalf = 3u * nTri;
-  QdBuffers B;
-  if (qd_alloc(&B.keys[0], nHalf) != hipSuccess || qd_alloc(&B.keys[1], nHalf) != hipSuccess ||
-      qd_alloc(&B.seqs[0], nHalf) != hipSuccess || qd_alloc(&B.seqs[1], nHalf) != hipSuccess ||
-      qd_alloc(&B.revFirst, nHalf) != hipSuccess || qd_alloc(&B.linkCount, size_t(nHalf) + 1) != hipSuccess ||
-      qd_alloc(&B.linkOff, size_t(nHalf) + 1) != hipSuccess || qd_alloc(&B.degree, size_t(nTri) + 1) != hipSuccess ||
-      qd_alloc(&B.start, size_t(nTri) + 1) != hipSuccess || qd_alloc(&B.bad, 1) != hipSuccess ||
-      qd_alloc(&B.writes, size_t(nTri) + 1) != hipSuccess || qd_alloc(&B.pos, size_t(nTri) + 1) != hipSuccess ||
-      qd_alloc(&B.mate, nTri) != hipSuccess)
+  uint32_t bits = 1;
+  while (bits < 32 && (uint64_t(1) << bits) < nVertices) ++bits;
+  size_t sortBytes = 0, scanBytes = 0;
+  QD_HIP(rocprim::radix_sort_pairs(nullptr, sortBytes, static_cast<uint64_t*>(nullptr), static_cast<uint64_t*>(nullptr),
+                                   static_cast<uint32_t*>(nullptr), static_cast<uint32_t*>(nullptr), nHalf, 0u,
+                                   2u * bits, stream));
+  QD_HIP(rocprim::exclusive_scan(nullptr, scanBytes, static_cast<uint32_t*>(nullptr), static_cast<uint32_t*>(nullptr),
+                                 0u, size_t(nTri) + 1, SatPlus(), stream));
+  Scratch::Frame frame(scratch);
+  uint64_t* keys = scratch.take<uint64_t>(nHalf);
+  uint64_t* sortedKeys = scratch.take<uint64_t>(nHalf);
+  uint32_t* seqs = scratch.take<uint32_t>(nHalf);
+  uint32_t* sortedSeqs = scratch.take<uint32_t>(nHalf);
+  uint32_t* revFirst = scratch.take<uint32_t>(nHalf);
+  uint32_t* degree = scratch.take<uint32_t>(size_t(nTri) + 1);  // then: which triangles write a quad
+  uint32_t* start = scratch.take<uint32_t>(size_t(nTri) + 1);   // then: the quads' positions
+  int* mates = scratch.take<int>(nTri);
+  uint32_t* words = scratch.take<uint32_t>(1);
+  unsigned char* temp = scratch.take<unsigned char>(std::max(sortBytes, scanBytes));
+  if (!keys || !sortedKeys || !seqs || !sortedSeqs || !revFirst || !degree || !start || !mates || !words || !temp)
     return RZ_ERR_OUT_OF_MEMORY;
-  QD_HIP(hipMemsetAsync(B.bad, 0, 4, stream));
+  QD_HIP(hipMemsetAsync(words, 0, 4, stream));
 
   // Half-edges, sorted by (key, insertion number).
-  qd_half_edges_kernel<<<qd_grid(nHalf), kQdBlock, 0, stream>>>(d_idx, nTri, nVertices, B.keys[0], B.seqs[0], B.bad);
+  qd_half_edges_kernel<<<qd_grid(nHalf), kQdBlock, 0, stream>>>(d_idx, nTri, nVertices, bits, keys, seqs, words);
   QD_HIP(hipGetLastError());
   uint32_t bad = 0;
-  QD_HIP(hipMemcpyAsync(&bad, B.bad, 4, hipMemcpyDeviceToHost, stream));
+  QD_HIP(hipMemcpyAsync(&bad, words, 4, hipMemcpyDeviceToHost, stream));
   QD_HIP(hipStreamSynchronize(stream));
   if (bad) return RZ_ERR_INVALID_ARGUMENT;
-  size_t bytes = 0;
-  QD_HIP(rocprim::radix_sort_pairs(nullptr, bytes, B.keys[0], B.keys[1], B.seqs[0], B.seqs[1], nHalf, 0u, 64u,
-                                   stream));
-  if (B.reserve(bytes) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
-  QD_HIP(rocprim::radix_sort_pairs(B.temp, bytes, B.keys[0], B.keys[1], B.seqs[0], B.seqs[1], nHalf, 0u, 64u,
-                                   stream));
-  qd_reverse_kernel<<<qd_grid(nHalf), kQdBlock, 0, stream>>>(B.keys[1], B.seqs[1], nHalf, B.revFirst);
+  size_t bytes = sortBytes;
+  QD_HIP(rocprim::radix_sort_pairs(temp, bytes, keys, sortedKeys, seqs, sortedSeqs, nHalf, 0u, 2u * bits, stream));
+  qd_reverse_kernel<<<qd_grid(nHalf), kQdBlock, 0, stream>>>(sortedKeys, sortedSeqs, nHalf, bits, revFirst);
   QD_HIP(hipGetLastError());
 
-  // Candidate links: count, scan, fill.
+  // Adjacency lists: count, scan, fill.
   QdParams P{};
   P.idx = d_idx;
   P.vertices = reinterpret_cast<const float4*>(d_vertices);
   P.nTri = nTri;
   P.nHalf = nHalf;
-  P.keys = B.keys[1];
-  P.seqs = B.seqs[1];
-  P.revFirst = B.revFirst;
+  P.bits = bits;
+  P.keys = sortedKeys;
+  P.seqs = sortedSeqs;
+  P.revFirst = revFirst;
   P.rsq = d_rsqrt;
-  P.linkCount = B.linkCount;
-  P.linkOff = B.linkOff;
-  P.degree = B.degree;
-  P.bad = B.bad;
-  QD_HIP(hipMemsetAsync(B.linkCount + nHalf, 0, 4, stream));
-  qd_links_kernel<false><<<qd_grid(nHalf), kQdBlock, 0, stream>>>(P);
+  P.degree = degree;
+  P.start = start;
+  P.bad = words;
+  QD_HIP(hipMemsetAsync(degree + nTri, 0, 4, stream));
+  qd_adjacency_kernel<false><<<qd_grid(nTri), kQdBlock, 0, stream>>>(P);
   QD_HIP(hipGetLastError());
-  bytes = 0;
-  QD_HIP(rocprim::exclusive_scan(nullptr, bytes, B.linkCount, B.linkOff, 0u, size_t(nHalf) + 1,
-                                 rocprim::plus<uint32_t>(), stream));
-  if (B.reserve(bytes) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
-  QD_HIP(rocprim::exclusive_scan(B.temp, bytes, B.linkCount, B.linkOff, 0u, size_t(nHalf) + 1,
-                                 rocprim::plus<uint32_t>(), stream));
-  uint32_t nLinks = 0;
-  QD_HIP(hipMemcpyAsync(&nLinks, B.linkOff + nHalf, 4, hipMemcpyDeviceToHost, stream));
+  bytes = scanBytes;
+  QD_HIP(rocprim::exclusive_scan(temp, bytes, degree, start, 0u, size_t(nTri) + 1, SatPlus(), stream));
+  uint32_t nAdj = 0;
+  QD_HIP(hipMemcpyAsync(&nAdj, start + nTri, 4, hipMemcpyDeviceToHost, stream));
   QD_HIP(hipStreamSynchronize(stream));
-  if (nLinks > 0x7FFFFFFFu / 2u) return RZ_ERR_TOO_LARGE;
-  const uint32_t nAdj = 2u * nLinks;
-  if (qd_alloc(&B.adjKey[0], nAdj) != hipSuccess || qd_alloc(&B.adjKey[1], nAdj) != hipSuccess ||
-      qd_alloc(&B.adjVal[0], nAdj) != hipSuccess || qd_alloc(&B.adjVal[1], nAdj) != hipSuccess)
-    return RZ_ERR_OUT_OF_MEMORY;
-  P.adjKey = B.adjKey[0];
-  P.adjVal = B.adjVal[0];
-  QD_HIP(hipMemsetAsync(B.degree, 0, (size_t(nTri) + 1) * 4, stream));
-  qd_links_kernel<true><<<qd_grid(nHalf), kQdBlock, 0, stream>>>(P);
+  if (nAdj > 0x7FFFFFFFu) return RZ_ERR_TOO_LARGE;
+  P.adj = scratch.take<int>(nAdj);
+  if (!P.adj) return RZ_ERR_OUT_OF_MEMORY;
+  qd_adjacency_kernel<true><<<qd_grid(nTri), kQdBlock, 0, stream>>>(P);
   QD_HIP(hipGetLastError());
-  // Adjacency lists: entries stably sorted by triangle keep link order.
-  if (nAdj > 0) {
-    uint32_t bits = 1;
-    while (bits < 32 && (uint64_t(1) << bits) < nTri) ++bits;
-    bytes = 0;
-    QD_HIP(rocprim::radix_sort_pairs(nullptr, bytes, B.adjKey[0], B.adjKey[1], B.adjVal[0], B.adjVal[1], nAdj, 0u,
-                                     bits, stream));
-    if (B.reserve(bytes) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
-    QD_HIP(rocprim::radix_sort_pairs(B.temp, bytes, B.adjKey[0], B.adjKey[1], B.adjVal[0], B.adjVal[1], nAdj, 0u,
-                                     bits, stream));
-  }
-  bytes = 0;
-  QD_HIP(rocprim::exclusive_scan(nullptr, bytes, B.degree, B.start, 0u, size_t(nTri) + 1, rocprim::plus<uint32_t>(),
-                                 stream));
-  if (B.reserve(bytes) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
-  QD_HIP(rocprim::exclusive_scan(B.temp, bytes, B.degree, B.start, 0u, size_t(nTri) + 1, rocprim::plus<uint32_t>(),
-                                 stream));
 
-  // The matching, on the host.
-  std::vector<int> mate;
+  // The matching, on the host: the lists come and the partners go through
+  // pinned memory where it can be had.
+  const size_t hostWords = size_t(nTri) + 1 + nAdj + nTri;
   try {
-    std::vector<uint32_t> start(size_t(nTri) + 1);
-    std::vector<int> adj(nAdj);
-    QD_HIP(hipMemcpyAsync(start.data(), B.start, start.size() * 4, hipMemcpyDeviceToHost, stream));
-    if (nAdj) QD_HIP(hipMemcpyAsync(adj.data(), B.adjVal[1], size_t(nAdj) * 4, hipMemcpyDeviceToHost, stream));
+    std::vector<uint32_t> pageable;
+    uint32_t* h = static_cast<uint32_t*>(scratch.host(hostWords * 4));
+    if (!h) {
+      pageable.resize(hostWords);
+      h = pageable.data();
+    }
+    int* adj = reinterpret_cast<int*>(h + size_t(nTri) + 1);
+    int* mate = adj + nAdj;
+    QD_HIP(hipMemcpyAsync(h, start, (size_t(nTri) + 1) * 4, hipMemcpyDeviceToHost, stream));
+    if (nAdj) QD_HIP(hipMemcpyAsync(adj, P.adj, size_t(nAdj) * 4, hipMemcpyDeviceToHost, stream));
     QD_HIP(hipStreamSynchronize(stream));
-    if (start[nTri] != nAdj) return RZ_ERR_DEVICE;
-    mate.resize(nTri);
-    rzq::match(nTri, start.data(), adj.data(), mate.data());
+    rzq::match(nTri, h, adj, mate);
+    QD_HIP(hipMemcpyAsync(mates, mate, size_t(nTri) * 4, hipMemcpyHostToDevice, stream));
+    if (!pageable.empty()) QD_HIP(hipStreamSynchronize(stream));
   } catch (const std::bad_alloc&) {
     return RZ_ERR_OUT_OF_MEMORY;
   }
-  QD_HIP(hipMemcpyAsync(B.mate, mate.data(), size_t(nTri) * 4, hipMemcpyHostToDevice, stream));
 
   // The quads.
-  qd_writers_kernel<<<qd_grid(size_t(nTri) + 1), kQdBlock, 0, stream>>>(B.mate, nTri, B.writes);
+  qd_writers_kernel<<<qd_grid(size_t(nTri) + 1), kQdBlock, 0, stream>>>(mates, nTri, degree);
   QD_HIP(hipGetLastError());
-  bytes = 0;
-  QD_HIP(rocprim::exclusive_scan(nullptr, bytes, B.writes, B.pos, 0u, size_t(nTri) + 1, rocprim::plus<uint32_t>(),
-                                 stream));
-  if (B.reserve(bytes) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
-  QD_HIP(rocprim::exclusive_scan(B.temp, bytes, B.writes, B.pos, 0u, size_t(nTri) + 1, rocprim::plus<uint32_t>(),
-                                 stream));
-  qd_emit_kernel<<<qd_grid(nTri), kQdBlock, 0, stream>>>(P, B.mate, B.pos, d_out);
+  bytes = scanBytes;
+  QD_HIP(rocprim::exclusive_scan(temp, bytes, degree, start, 0u, size_t(nTri) + 1, SatPlus(), stream));
+  qd_emit_kernel<<<qd_grid(nTri), kQdBlock, 0, stream>>>(P, mates, start, d_out);
   QD_HIP(hipGetLastError());
   uint32_t quads = 0;
-  QD_HIP(hipMemcpyAsync(&quads, B.pos + nTri, 4, hipMemcpyDeviceToHost, stream));
-  QD_HIP(hipMemcpyAsync(&bad, B.bad, 4, hipMemcpyDeviceToHost, stream));
+  QD_HIP(hipMemcpyAsync(&quads, start + nTri, 4, hipMemcpyDeviceToHost, stream));
+  QD_HIP(hipMemcpyAsync(&bad, words, 4, hipMemcpyDeviceToHost, stream));
   QD_HIP(hipStreamSynchronize(stream));
   if (bad) return RZ_ERR_DEVICE;
   *nOut = 4u * quads;

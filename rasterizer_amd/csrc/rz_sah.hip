@@ -47,10 +47,12 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "rasterizer_amd.h"
 #include "rz_kernels.h"
+#include "rz_scratch.h"
 
 extern "C" __device__ uint32_t __ockl_wfred_min_u32(uint32_t);
 extern "C" __device__ uint32_t __ockl_wfred_max_u32(uint32_t);
@@ -365,30 +367,6 @@ __global__ void __launch_bounds__(256) sah_emit_kernel(const uint32_t* __restric
 
 uint32_t grid_of(uint32_t n) { return (n + 255u) / 256u; }
 
-// One device allocation, handed out in 256-byte aligned parts.
-class Arena {
- public:
-  ~Arena() {
-    if (base_) (void)hipFree(base_);
-  }
-  // First pass (nothing allocated): adds up the parts' sizes.
-  template <typename T>
-  void take(T** p, size_t count) {
-    *p = base_ ? reinterpret_cast<T*>(base_ + used_) : nullptr;
-    used_ += (count * sizeof(T) + 255) & ~size_t(255);
-  }
-  hipError_t allocate() {
-    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&base_), used_ ? used_ : 1);
-    used_ = 0;
-    if (e != hipSuccess) base_ = nullptr;
-    return e;
-  }
-
- private:
-  unsigned char* base_ = nullptr;
-  size_t used_ = 0;
-};
-
 }  // namespace
 
 #define SAH_HIP(call)                                  \
@@ -396,8 +374,8 @@ class Arena {
     if ((call) != hipSuccess) return RZ_ERR_DEVICE;    \
   } while (0)
 
-int sah_batches_run(hipStream_t stream, uint32_t n, const float* d_boxes, uint32_t target, uint32_t gran,
-                    uint32_t* d_indices, uint32_t* batchOffsets, uint32_t* nBatches) {
+int sah_batches_run(hipStream_t stream, Scratch& scratch, uint32_t n, const float* d_boxes, uint32_t target,
+                    uint32_t gran, uint32_t* d_indices, uint32_t* batchOffsets, uint32_t* nBatches) {
   if (gran == 0 || target <= 2 * uint64_t(gran)) return RZ_ERR_INVALID_ARGUMENT;
   if (n > kMaxSahItems) return RZ_ERR_TOO_LARGE;
   batchOffsets[0] = 0;
@@ -429,42 +407,41 @@ int sah_batches_run(hipStream_t stream, uint32_t n, const float* d_boxes, uint32
                                     rocprim::plus<uint32_t>(), stream));
   }
   const size_t tempBytes = std::max(sortBytes, scanBytes);
-  Arena arena;
-  for (int pass = 0; pass < 2; ++pass) {
-    if (pass == 1 && arena.allocate() != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
-    // A word for the range check, the two open counts and the error word.
-    uint32_t* words = nullptr;
-    arena.take(&words, 4);
-    if (words) {
-      A.err = words;
-      A.nOpen = words + 2;
-      A.nextNOpen = words + 3;
-    }
-    if (whole) continue;
-    arena.take(&A.orders, size_t(kOrders) * n);
-    arena.take(&A.nextOrders, size_t(kOrders) * n);
-    arena.take(&keys, n3);
-    arena.take(&keysOut, n3);
-    arena.take(&values, n3);
-    arena.take(&round1, size_t(2) * n);
-    arena.take(&round2, n3);
-    arena.take(&lefts, size_t(kOrders) * n);
-    arena.take(&temp, tempBytes);
-    arena.take(&A.chunkSeg, nChunks);
-    arena.take(&A.nextChunkSeg, nChunks);
-    arena.take(&A.segs, maxOpen);
-    arena.take(&A.nextSegs, maxOpen);
-    arena.take(&A.best, maxOpen);
-    arena.take(&A.nextBest, maxOpen);
-    arena.take(&A.arrived, maxOpen);
-    arena.take(&A.nextArrived, maxOpen);
-    arena.take(&A.splits, maxOpen);
-    arena.take(&A.chunkBox, size_t(3) * nChunks);
-    arena.take(&A.rightArea, size_t(3) * nChunks);
-    arena.take(&A.side, n);
-    arena.take(&A.starts, nChunks);
-    arena.take(&A.batchAxis, nChunks);
+  Scratch::Frame frame(scratch);
+  bool ok = true;
+  auto take = [&](auto** p, size_t count) {
+    *p = scratch.take<std::remove_pointer_t<std::remove_pointer_t<decltype(p)>>>(count);
+    ok = ok && *p != nullptr;
+  };
+  take(&A.err, 4);  // the error word, the range check's, and the two open counts
+  if (!whole) {
+    take(&A.orders, size_t(kOrders) * n);
+    take(&A.nextOrders, size_t(kOrders) * n);
+    take(&keys, n3);
+    take(&keysOut, n3);
+    take(&values, n3);
+    take(&round1, size_t(2) * n);
+    take(&round2, n3);
+    take(&lefts, size_t(kOrders) * n);
+    take(&temp, tempBytes);
+    take(&A.chunkSeg, nChunks);
+    take(&A.nextChunkSeg, nChunks);
+    take(&A.segs, maxOpen);
+    take(&A.nextSegs, maxOpen);
+    take(&A.best, maxOpen);
+    take(&A.nextBest, maxOpen);
+    take(&A.arrived, maxOpen);
+    take(&A.nextArrived, maxOpen);
+    take(&A.splits, maxOpen);
+    take(&A.chunkBox, size_t(3) * nChunks);
+    take(&A.rightArea, size_t(3) * nChunks);
+    take(&A.side, n);
+    take(&A.starts, nChunks);
+    take(&A.batchAxis, nChunks);
   }
+  if (!ok) return RZ_ERR_OUT_OF_MEMORY;
+  A.nOpen = A.err + 2;
+  A.nextNOpen = A.err + 3;
   uint32_t words[4] = {0, 0, 1, 0};
   SAH_HIP(hipMemcpyAsync(A.err, words, sizeof words, hipMemcpyHostToDevice, stream));
   sah_check_kernel<<<grid_of(n), 256, 0, stream>>>(d_boxes, n, A.err + 1);

@@ -1,0 +1,125 @@
+// Working memory of a context's scene preparation (rz_sah_batches,
+// rz_quad_decompose_device, rz_bake_device, rz_prepare_*), kept between calls:
+// allocating and freeing a buffer of some megabytes takes about 0.3 ms, more
+// than most of the kernels that use it.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+
+namespace rzd {
+
+// Device memory handed out in 256-byte aligned parts, released in the reverse
+// order (Frame).  A call that needs more than is there gets further blocks;
+// after it they are given back and the next call allocates one block of the
+// size that was in use, and a block above kKeepDevice is not kept either.
+// Used by one context's calls, on its stream, by one thread at a time, so a
+// part is only handed on to work that the stream orders behind its last use;
+// everything is freed with the context.
+class Scratch {
+ public:
+  static constexpr size_t kKeepDevice = size_t(256) << 20;
+  static constexpr size_t kMaxHost = size_t(64) << 20;
+
+  ~Scratch() {
+    free_blocks();
+    if (host_) (void)hipHostFree(host_);
+  }
+
+  // Device memory until the enclosing Frame ends; null when there is none.
+  template <typename T>
+  T* take(size_t count) {
+    size_t bytes = (count * sizeof(T) + 255) & ~size_t(255);
+    if (bytes == 0) bytes = 256;
+    while (cur_ < nBlocks_ && used_ + bytes > blocks_[cur_].size) {
+      before_ += blocks_[cur_++].size;
+      used_ = 0;
+    }
+    if (cur_ == nBlocks_) {
+      if (nBlocks_ == kMaxBlocks) return nullptr;
+      Block b;
+      if (nBlocks_ == 0 && want_ > bytes && hipMalloc(&b.base, want_) == hipSuccess) {
+        b.size = want_;
+      } else {
+        (void)hipGetLastError();
+        if (hipMalloc(&b.base, bytes) != hipSuccess) {
+          (void)hipGetLastError();
+          return nullptr;
+        }
+        b.size = bytes;
+      }
+      blocks_[nBlocks_++] = b;
+      used_ = 0;
+    }
+    T* p = reinterpret_cast<T*>(static_cast<unsigned char*>(blocks_[cur_].base) + used_);
+    used_ += bytes;
+    peak_ = peak_ > before_ + used_ ? peak_ : before_ + used_;
+    return p;
+  }
+
+  // Pinned host memory (one user at a time), or null when it cannot be had or
+  // would exceed kMaxHost.
+  void* host(size_t bytes) {
+    if (bytes > kMaxHost) return nullptr;
+    if (bytes > hostBytes_) {
+      if (host_) (void)hipHostFree(host_);
+      host_ = nullptr;
+      hostBytes_ = 0;
+      if (hipHostMalloc(&host_, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        host_ = nullptr;
+        return nullptr;
+      }
+      hostBytes_ = bytes;
+    }
+    return host_;
+  }
+
+  // Parts taken while a Frame lives are released when it ends.
+  class Frame {
+   public:
+    explicit Frame(Scratch& s) : s_(s), cur_(s.cur_), used_(s.used_), before_(s.before_) { ++s_.depth_; }
+    ~Frame() {
+      s_.cur_ = cur_;
+      s_.used_ = used_;
+      s_.before_ = before_;
+      if (--s_.depth_ == 0) s_.trim();
+    }
+    Frame(const Frame&) = delete;
+    Frame& operator=(const Frame&) = delete;
+
+   private:
+    Scratch& s_;
+    size_t cur_, used_, before_;
+  };
+
+ private:
+  struct Block {
+    void* base = nullptr;
+    size_t size = 0;
+  };
+
+  void free_blocks() {
+    for (size_t i = 0; i < nBlocks_; ++i) (void)hipFree(blocks_[i].base);  // waits for the work that uses it
+    nBlocks_ = cur_ = used_ = before_ = 0;
+  }
+  void trim() {
+    if (nBlocks_ > 1 || (nBlocks_ == 1 && blocks_[0].size > kKeepDevice)) free_blocks();
+    want_ = peak_;
+    peak_ = 0;
+  }
+
+  // A call takes at most 40 parts (rz_prepare_mesh_device).
+  static constexpr size_t kMaxBlocks = 64;
+  Block blocks_[kMaxBlocks];
+  size_t nBlocks_ = 0;
+  size_t cur_ = 0, used_ = 0;  // the next part starts at blocks_[cur_].base + used_
+  size_t before_ = 0;          // the sizes of the blocks before it
+  size_t peak_ = 0, want_ = 0;
+  int depth_ = 0;
+  void* host_ = nullptr;
+  size_t hostBytes_ = 0;
+};
+
+}  // namespace rzd
