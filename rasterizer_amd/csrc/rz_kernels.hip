@@ -164,6 +164,49 @@ __device__ QueryPre query_pre(const Mvp& M, const float* bmin, const float* bmax
   return out;
 }
 
+// One buffer's depth as the query kernels read it from device memory.
+struct QueryBufs {
+  const uint16_t* __restrict__ depth;
+  const uint16_t* __restrict__ hiz;
+  const uint16_t* __restrict__ tileMin;
+  uint32_t bX, pyrX;
+};
+
+// Whether block (bx, by) has a pixel of the rectangle nearer than maxZ.  Pixels
+// outside it are set to the largest depth, so the test is one packed minimum
+// over the rows; four rows' loads are issued before their use.
+typedef unsigned short U16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ bool block_pixels_hit(const QueryBufs& B, uint32_t bx, uint32_t by, uint32_t minX,
+                                                 uint32_t maxX, uint32_t minY, uint32_t maxY, uint32_t maxZ) {
+  const int32_t sy = int32_t(minY - 8 * by), ey = int32_t(maxY - 8 * by);
+  const int32_t sx = int32_t(minX - 8 * bx), ex = int32_t(maxX - 8 * bx);
+  const uint32_t startY = uint32_t(sy > 0 ? sy : 0), endY = uint32_t(ey < 7 ? ey : 7);
+  const uint32_t startX = uint32_t(sx > 0 ? sx : 0), endX = uint32_t(ex < 7 ? ex : 7);
+  const uint32_t in = (0xFFu << startX) & (0xFFu >> (7u - endX));
+  uint32_t outside[4];
+#pragma unroll
+  for (uint32_t x = 0; x < 4; ++x)
+    outside[x] = ((in >> (2 * x)) & 1u ? 0u : 0xFFFFu) | ((in >> (2 * x + 1)) & 1u ? 0u : 0xFFFF0000u);
+  const uint4* rows = reinterpret_cast<const uint4*>(B.depth + (size_t(by) * B.bX + bx) * 64);
+  U16x2 least = {0xFFFF, 0xFFFF};
+  for (uint32_t h = startY & ~3u; h <= endY; h += 4) {
+    uint4 r[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      r[j] = make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu);
+      if (h + j >= startY && h + j <= endY) r[j] = rows[h + j];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+      const uint32_t w[4] = {r[j].x, r[j].y, r[j].z, r[j].w};
+#pragma unroll
+      for (uint32_t x = 0; x < 4; ++x)
+        least = __builtin_elementwise_min(least, __builtin_bit_cast(U16x2, w[x] | outside[x]));
+    }
+  }
+  return uint32_t(least.x < least.y ? least.x : least.y) < maxZ;
+}
+
 // query2D (Rasterizer.cpp:283-349) by one wave on the buffers in device
 // memory.  The result is the OR over the rectangle's blocks of "maxZ > hiZ
 // and (block interior to the rectangle, or a pixel in range nearer than
@@ -171,14 +214,13 @@ __device__ QueryPre query_pre(const Mvp& M, const float* bmin, const float* bmax
 // whose minimum hiZ is below maxZ (other tiles hold no candidate block), then
 // one block per lane inside each candidate tile.
 __device__ bool query2d_wave(uint32_t minX, uint32_t maxX, uint32_t minY, uint32_t maxY, uint32_t maxZ,
-                             const uint16_t* __restrict__ depth, const uint16_t* __restrict__ hiz,
-                             const uint16_t* __restrict__ tileMin, uint32_t bX, uint32_t pyrX, uint32_t lane) {
+                             const QueryBufs& B, uint32_t lane) {
   const uint32_t bx0 = minX >> 3, bx1 = maxX >> 3, by0 = minY >> 3, by1 = maxY >> 3;
   const uint32_t tx0 = bx0 >> 3, tx1 = bx1 >> 3, ty0 = by0 >> 3, ty1 = by1 >> 3;
   const uint32_t ntx = tx1 - tx0 + 1, nt = ntx * (ty1 - ty0 + 1);
   for (uint32_t tb = 0; tb < nt; tb += 64) {
     const uint32_t t = tb + lane;
-    const bool cand = t < nt && uint32_t(tileMin[(ty0 + t / ntx) * pyrX + tx0 + t % ntx]) < maxZ;
+    const bool cand = t < nt && uint32_t(B.tileMin[(ty0 + t / ntx) * B.pyrX + tx0 + t % ntx]) < maxZ;
     uint64_t cm = __ballot(cand);
     while (cm) {
       const uint32_t k = uint32_t(__builtin_ctzll(cm));
@@ -187,43 +229,114 @@ __device__ bool query2d_wave(uint32_t minX, uint32_t maxX, uint32_t minY, uint32
       const uint32_t bx = (tx0 + tt % ntx) * 8 + (lane & 7u), by = (ty0 + tt / ntx) * 8 + (lane >> 3);
       bool v = false;
       if (bx >= bx0 && bx <= bx1 && by >= by0 && by <= by1) {
-        const uint32_t b = by * bX + bx;
-        if (maxZ > uint32_t(hiz[b])) {
-          const int32_t sy = int32_t(minY - 8 * by), ey = int32_t(maxY - 8 * by);
-          const int32_t sx = int32_t(minX - 8 * bx), ex = int32_t(maxX - 8 * bx);
-          const uint32_t startY = uint32_t(sy > 0 ? sy : 0), endY = uint32_t(ey < 7 ? ey : 7);
-          const uint32_t startX = uint32_t(sx > 0 ? sx : 0), endX = uint32_t(ex < 7 ? ex : 7);
-          if (startY == 0 && endY == 7 && startX == 0 && endX == 7) {
-            v = true;
-          } else {
-            // The rectangle's rows of the block, four rows' loads issued
-            // before their tests (a row-by-row loop with an early exit would
-            // wait for each load in turn).
-            const uint4* rows = reinterpret_cast<const uint4*>(depth + size_t(b) * 64);
-            for (uint32_t h = startY & ~3u; h <= endY && !v; h += 4) {
-              uint4 r[4];
-#pragma unroll
-              for (uint32_t j = 0; j < 4; ++j) {
-                r[j] = make_uint4(0, 0, 0, 0);
-                if (h + j >= startY && h + j <= endY) r[j] = rows[h + j];
-              }
-#pragma unroll
-              for (uint32_t j = 0; j < 4; ++j) {
-                const uint32_t y = h + j;
-                const uint32_t w[4] = {r[j].x, r[j].y, r[j].z, r[j].w};
-#pragma unroll
-                for (uint32_t x = 0; x < 8; ++x)
-                  v |= y >= startY && y <= endY && x >= startX && x <= endX &&
-                       ((w[x >> 1] >> (16 * (x & 1))) & 0xFFFFu) < maxZ;
-              }
-            }
-          }
+        if (maxZ > uint32_t(B.hiz[by * B.bX + bx])) {
+          v = (minX <= 8 * bx && maxX >= 8 * bx + 7 && minY <= 8 * by && maxY >= 8 * by + 7) ||
+              block_pixels_hit(B, bx, by, minX, maxX, minY, maxY, maxZ);
         }
       }
       if (__ballot(v) != 0ull) return true;
     }
   }
   return false;
+}
+
+// query2D of the wave's boxes, one rectangle per lane with `test` set; returns
+// the lane's answer.
+//   - A rectangle of at most 4x4 tiles first takes its tiles' minima alone, one
+//     lane per box: what they cover is answered here, for 64 boxes at once.
+//   - The rest go eight at a time, eight lanes each, a lane to a column of
+//     blocks: a candidate tile's 64 hiZ values are one load per row and lane,
+//     all in flight together, and only where no interior block is open do the
+//     blocks at the rectangle's border read their pixels.
+//   - Wider rectangles take the whole wave, one after another.
+// Bound by latency (box, reciprocal table, tile minima, hiZ, pixels in turn)
+// and instructions: a city query's rectangle has some tens of blocks, so a
+// whole wave for each box in turn left most lanes idle.  A batch of 1,000,003
+// city boxes, together with launch_query's rule: 180 us before, 28 us now.
+__device__ bool query2d_boxes(const QueryPre& Q, bool test, const QueryBufs& B, uint32_t lane) {
+  const uint32_t tx0 = Q.minX >> 6, ty0 = Q.minY >> 6;
+  const uint32_t ntx = (Q.maxX >> 6) - tx0 + 1, nty = (Q.maxY >> 6) - ty0 + 1;
+  const bool narrow = test && ntx <= 4u && nty <= 4u;
+  bool vis = false;
+  uint32_t cand = 0;  // bit 4 y + x: tile (tx0 + x, ty0 + y) may hold an open block
+  if (narrow) {
+    const uint16_t* row = B.tileMin + ty0 * B.pyrX + tx0;
+    for (uint32_t y = 0; y < nty; ++y, row += B.pyrX) {
+      uint32_t z[4];
+#pragma unroll
+      for (uint32_t x = 0; x < 4; ++x) z[x] = x < ntx ? uint32_t(row[x]) : 0xFFFFu;
+#pragma unroll
+      for (uint32_t x = 0; x < 4; ++x) cand |= z[x] < Q.maxZ ? 1u << (4 * y + x) : 0u;
+    }
+  }
+  uint64_t m = __ballot(cand != 0u);
+  const uint32_t group = lane >> 3, shift = lane & ~7u;
+  while (m) {
+    uint32_t from[8], src = 64;
+#pragma unroll
+    for (uint32_t g = 0; g < 8; ++g) {
+      from[g] = m ? uint32_t(__builtin_ctzll(m)) : 64u;
+      m &= m - 1ull;
+      src = group == g ? from[g] : src;
+    }
+    const int j = int(src & 63u);
+    const uint32_t minX = __shfl(Q.minX, j), maxX = __shfl(Q.maxX, j);
+    const uint32_t minY = __shfl(Q.minY, j), maxY = __shfl(Q.maxY, j);
+    const uint32_t maxZ = __shfl(Q.maxZ, j);
+    uint32_t c = __shfl(cand, j);
+    if (src == 64u) c = 0;
+    bool hit = false;
+    while (c) {
+      const uint32_t t = uint32_t(__builtin_ctz(c));
+      c &= c - 1u;
+      const uint32_t bx = ((minX >> 6) + (t & 3u)) * 8 + (lane & 7u), y0 = ((minY >> 6) + (t >> 2)) * 8;
+      const bool inX = bx >= minX >> 3 && bx <= maxX >> 3;
+      uint32_t z[8];
+#pragma unroll
+      for (uint32_t r = 0; r < 8; ++r) {
+        z[r] = 0xFFFFu;
+        if (inX && y0 + r >= minY >> 3 && y0 + r <= maxY >> 3) z[r] = B.hiz[(y0 + r) * B.bX + bx];
+      }
+      const bool wholeX = minX <= 8 * bx && maxX >= 8 * bx + 7;
+      uint32_t border = 0;
+      bool v = false;
+#pragma unroll
+      for (uint32_t r = 0; r < 8; ++r) {
+        const bool whole = wholeX && minY <= 8 * (y0 + r) && maxY >= 8 * (y0 + r) + 7;
+        if (z[r] < maxZ) {
+          if (whole) v = true;
+          else border |= 1u << r;
+        }
+      }
+      hit = ((__ballot(v) >> shift) & 0xFFull) != 0ull;
+      while (!hit && ((__ballot(border != 0u) >> shift) & 0xFFull) != 0ull) {
+        if (border) {
+          const uint32_t by = y0 + uint32_t(__builtin_ctz(border));
+          border &= border - 1u;
+          v = block_pixels_hit(B, bx, by, minX, maxX, minY, maxY, maxZ);
+        }
+        hit = ((__ballot(v) >> shift) & 0xFFull) != 0ull;
+      }
+      if (hit) c = 0;
+    }
+    const uint64_t hits = __ballot(hit);
+#pragma unroll
+    for (uint32_t g = 0; g < 8; ++g)
+      if (lane == from[g]) vis = ((hits >> (8 * g)) & 1ull) != 0ull;
+  }
+  m = __ballot(test && !narrow);
+  while (m) {
+    const int j = int(__builtin_ctzll(m));
+    m &= m - 1ull;
+    const uint32_t minX = uint32_t(__builtin_amdgcn_readlane(int(Q.minX), j));
+    const uint32_t maxX = uint32_t(__builtin_amdgcn_readlane(int(Q.maxX), j));
+    const uint32_t minY = uint32_t(__builtin_amdgcn_readlane(int(Q.minY), j));
+    const uint32_t maxY = uint32_t(__builtin_amdgcn_readlane(int(Q.maxY), j));
+    const uint32_t maxZ = uint32_t(__builtin_amdgcn_readlane(int(Q.maxZ), j));
+    const bool v = query2d_wave(minX, maxX, minY, maxY, maxZ, B, lane);
+    if (int(lane) == j) vis = v;
+  }
+  return vis;
 }
 
 // ---------------------------------------------------------------------------
@@ -1931,15 +2044,10 @@ __global__ void rz_status_kernel(const ItemState* __restrict__ state, const uint
 // ---------------------------------------------------------------------------
 // Queries, readback, clear.
 // ---------------------------------------------------------------------------
-// queryVisibility (Rasterizer.cpp:123-281), one wave per box.
 // queryVisibility (Rasterizer.cpp:123-281) of a batch: lanes 0..BPW-1 of a
 // wave each take one box for the depth-independent part (projection,
-// frustum, near plane, rectangle), and the wave then runs query2D for its
-// boxes that need it, one after another.  A frame's 65,536 boxes are too few
-// to give each wave 64 of them (one wave per SIMD, long serial query2D
-// chains), and too many for one wave per box (the wave launches dominate):
-// four boxes per wave take 20 us per 65,536-box city batch, one 33 us, eight
-// 28 us.
+// frustum, near plane, rectangle), then the wave runs query2D for those that
+// need it (query2d_boxes).  launch_query chooses BPW.
 template <uint32_t BPW>
 __global__ void __launch_bounds__(256) rz_query_kernel(QueryParams p) {
   const uint32_t lane = threadIdx.x & 63u;
@@ -1952,20 +2060,9 @@ __global__ void __launch_bounds__(256) rz_query_kernel(QueryParams p) {
     const float bmax[4] = {b[4], b[5], b[6], b[7]};
     Q = query_pre(p.mvp, bmin, bmax, p.width, p.height, p.rcp);
   }
-  uint32_t vis = Q.kind == 1 ? 1u : 0u;
-  const uint32_t clip = vis;
-  uint64_t m = __ballot(valid && Q.kind == 3);
-  while (m) {
-    const int j = int(__builtin_ctzll(m));
-    m &= m - 1ull;
-    const uint32_t minX = uint32_t(__builtin_amdgcn_readlane(int(Q.minX), j));
-    const uint32_t maxX = uint32_t(__builtin_amdgcn_readlane(int(Q.maxX), j));
-    const uint32_t minY = uint32_t(__builtin_amdgcn_readlane(int(Q.minY), j));
-    const uint32_t maxY = uint32_t(__builtin_amdgcn_readlane(int(Q.maxY), j));
-    const uint32_t maxZ = uint32_t(__builtin_amdgcn_readlane(int(Q.maxZ), j));
-    const bool v = query2d_wave(minX, maxX, minY, maxY, maxZ, p.depth, p.hiz, p.tileMin, p.bX, p.pyrX, lane);
-    if (int(lane) == j) vis = v ? 1u : 0u;
-  }
+  const uint32_t clip = Q.kind == 1 ? 1u : 0u;
+  const QueryBufs B = {p.depth, p.hiz, p.tileMin, p.bX, p.pyrX};
+  const uint32_t vis = query2d_boxes(Q, valid && Q.kind == 3, B, lane) ? 1u : clip;
   if (valid) {
     p.visible[q] = uint8_t(vis);
     if (p.needsClipping) p.needsClipping[q] = uint8_t(clip);
@@ -1977,9 +2074,7 @@ __global__ void __launch_bounds__(256) rz_query_kernel(QueryParams p) {
 // queryVisibility over the queries of every view of a multi-view launch;
 // blockIdx.y is the view.  A step holds many boxes, so one lane per box does
 // the depth-independent part (projection, frustum, near plane, rectangle)
-// and the wave then runs query2D for its boxes that need it.  (The
-// single-view kernel gives each wave four boxes: its batches are too small
-// to fill the GPU with 64 boxes per wave.)
+// and the wave then runs query2D for its boxes that need it.
 __global__ void __launch_bounds__(256) rz_views_query_kernel(ViewsQueryParams p) {
   // The raster launch that sets the error word has completed.
   if (p.errOut && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *p.errOut = *p.err;
@@ -1994,21 +2089,9 @@ __global__ void __launch_bounds__(256) rz_views_query_kernel(ViewsQueryParams p)
     const float bmax[4] = {b[4], b[5], b[6], b[7]};
     Q = query_pre(V.mvp, bmin, bmax, V.width, V.height, p.rcp);
   }
-  uint32_t vis = Q.kind == 1 ? 1u : 0u;
-  const uint32_t clip = vis;
-  // The boxes that need query2D, one after another, each by the whole wave.
-  uint64_t m = __ballot(valid && Q.kind == 3);
-  while (m) {
-    const int j = int(__builtin_ctzll(m));
-    m &= m - 1ull;
-    const uint32_t minX = uint32_t(__builtin_amdgcn_readlane(int(Q.minX), j));
-    const uint32_t maxX = uint32_t(__builtin_amdgcn_readlane(int(Q.maxX), j));
-    const uint32_t minY = uint32_t(__builtin_amdgcn_readlane(int(Q.minY), j));
-    const uint32_t maxY = uint32_t(__builtin_amdgcn_readlane(int(Q.maxY), j));
-    const uint32_t maxZ = uint32_t(__builtin_amdgcn_readlane(int(Q.maxZ), j));
-    const bool v = query2d_wave(minX, maxX, minY, maxY, maxZ, V.depth, V.hiz, V.tileMin, V.bX, V.pyrX, lane);
-    if (int(lane) == j) vis = v ? 1u : 0u;
-  }
+  const uint32_t clip = Q.kind == 1 ? 1u : 0u;
+  const QueryBufs B = {V.depth, V.hiz, V.tileMin, V.bX, V.pyrX};
+  const uint32_t vis = query2d_boxes(Q, valid && Q.kind == 3, B, lane) ? 1u : clip;
   if (valid) {
     V.queryVisible[k] = uint8_t(vis);
     V.queryClip[k] = uint8_t(clip);
@@ -2034,7 +2117,7 @@ __global__ void rz_views_clear_kernel(const ViewDesc* __restrict__ src, ViewDesc
 
 __global__ void rz_query2d_kernel(uint32_t minX, uint32_t maxX, uint32_t minY, uint32_t maxY, uint32_t maxZ,
                                   QueryParams p, uint8_t* out) {
-  const bool v = query2d_wave(minX, maxX, minY, maxY, maxZ, p.depth, p.hiz, p.tileMin, p.bX, p.pyrX, threadIdx.x);
+  const bool v = query2d_wave(minX, maxX, minY, maxY, maxZ, {p.depth, p.hiz, p.tileMin, p.bX, p.pyrX}, threadIdx.x);
   if (threadIdx.x == 0) *out = v ? 1 : 0;
 }
 
@@ -2406,9 +2489,20 @@ hipError_t launch_status(const ItemState* state, const uint32_t* visible, uint32
 
 hipError_t launch_query(const QueryParams& p, hipStream_t stream) {
   if (p.n == 0) return hipSuccess;
-  constexpr uint32_t kBoxesPerWave = 4;  // measured over 1, 2, 4, 8, 16 and 32 on the city frames' batches
-  hipLaunchKernelGGL(rz_query_kernel<kBoxesPerWave>, dim3(groups(groups(p.n, kBoxesPerWave), 4)), dim3(256), 0, stream,
-                     p);
+  // As many boxes per wave as fill the chip's 8,192 wave slots once: fewer leave
+  // most lanes of the projection idle, more leave slots idle and make longer
+  // waves.  Device batches of city boxes over the 1080p buffer, us per call
+  // with 8 / 16 / 32 / 64 boxes per wave: 65,536 boxes 16.3 / 17.1 / 18.6 /
+  // 19.1, 131,072 boxes 20.5 / 17.6 / 18.4 / 19.4, 262,144 boxes 32.8 / 21.8 /
+  // 17.8 / 19.8, 1,000,003 boxes 106 / 64 / 40 / 28 (four: 18, 29, 50, 182).
+  constexpr uint32_t kWaves = 8192;
+  auto go = [&](auto kernel, uint32_t bpw) {
+    hipLaunchKernelGGL(kernel, dim3(groups(groups(p.n, bpw), 4)), dim3(256), 0, stream, p);
+  };
+  if (p.n <= 8 * kWaves) go(rz_query_kernel<8>, 8);
+  else if (p.n <= 16 * kWaves) go(rz_query_kernel<16>, 16);
+  else if (p.n <= 32 * kWaves) go(rz_query_kernel<32>, 32);
+  else go(rz_query_kernel<64>, 64);
   return hipGetLastError();
 }
 

@@ -1,0 +1,59 @@
+"""Batches of visibility queries against the oracle, bit for bit, on random
+depth: sizes around a wave's share of boxes and around the changes of that
+share, and screen rectangles that touch no more than 4x4 tiles of 64x64
+pixels, just more, and the buffer's whole width, over buffers whose tiles are
+all covered, all open, or decided by the pixels at the rectangles' borders."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from rasterizer_amd import Rasterizer, scenes
+
+pytestmark = pytest.mark.gpu
+
+W, H = 712, 648
+
+
+def _pair(oracle_mod, open_share, seed):
+    rng = np.random.default_rng(seed)
+    m = scenes.config1(seed=1).meta
+    g, o = Rasterizer(W, H), oracle_mod.OracleRasterizer(W, H)
+    depth = rng.integers(0, 65536, (H // 8 * (W // 8), 64), dtype=np.uint16)
+    depth[rng.random(depth.shape) > open_share] = 0xFFFF
+    hiz = np.ones(H // 8 * (W // 8) + 8, np.uint16)
+    hiz[:-8] = depth.min(axis=1)
+    for r in (g, o):
+        r.setModelViewProjection(m["mvp"])
+    g.upload_raw(depth, hiz)
+    o.set_raw(depth, hiz)
+    return g, o, m, rng
+
+
+def _boxes(rng, m, n):
+    """Boxes around the eye at log-uniform distances and sizes."""
+    d = rng.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    c = np.asarray(m["eye"], np.float64)[:3] + d * np.exp(rng.uniform(0.0, 6.0, (n, 1)))
+    return scenes.aabb_bounds(c.astype(np.float32), np.exp(rng.uniform(-3.0, 4.0, (n, 3))).astype(np.float32))
+
+
+@pytest.mark.parametrize("open_share", [0.0, 0.002, 0.02, 1.0])
+def test_batches_match_oracle(oracle_mod, open_share):
+    g, o, m, rng = _pair(oracle_mod, open_share, int(open_share * 1000))
+    for n in (1, 7, 8, 9, 63, 64, 65, 511, 3001):
+        b = _boxes(rng, m, n)
+        for got, want in zip(g.query_batch(b), o.query_batch(b)):
+            assert np.array_equal(got, want), f"{n} boxes: {int((got != want).sum())} differ"
+
+
+@pytest.mark.parametrize("n", [65536, 65537, 131072, 131073, 262144, 262145])
+def test_share_of_boxes(oracle_mod, n):
+    """The same boxes over and over: every wave of a large batch answers them as
+    a small one does."""
+    g, o, m, rng = _pair(oracle_mod, 0.01, 5)
+    b = _boxes(rng, m, 1021)
+    want = o.query_batch(b)
+    for got, w in zip(g.query_batch(np.resize(b, (n, 8))), want):
+        assert np.array_equal(got, np.resize(w, n))
