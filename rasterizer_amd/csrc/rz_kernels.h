@@ -157,6 +157,19 @@ enum FrameStat : int {
   kFrameStatWords = 22,
 };
 
+// Two words of pinned host memory that a blocking call's last kernel writes,
+// through their device mapping, instead of copies after it: [0] the context's
+// error word (err), [1] the answer of a single query.
+struct HostWords {
+  const uint32_t* err;
+  uint32_t* out;
+};
+
+// A query's box, passed with the launch.
+struct QueryBox {
+  float lo[4], hi[4];
+};
+
 struct QueryParams {
   const float* bounds;  // n x 8 floats
   uint32_t n;
@@ -168,7 +181,7 @@ struct QueryParams {
   const uint32_t* rcp;
   uint8_t* visible;
   uint8_t* needsClipping;  // may be null
-  uint8_t* code;           // may be null: visible | clip << 1 | clipWritten << 2
+  HostWords words;         // may be null
   Mvp mvp;
 };
 
@@ -186,13 +199,18 @@ hipError_t frame_max_groups(int tileW, int waves, int* maxGroups);
 hipError_t launch_status(const ItemState* state, const uint32_t* visible, uint32_t n, uint8_t* out,
                          hipStream_t stream);
 hipError_t launch_query(const QueryParams& p, hipStream_t stream);
+// One box; words.out[1] = visible | clip << 1 | clipWritten << 2.
+hipError_t launch_query_one(const QueryParams& p, const QueryBox& box, hipStream_t stream);
+// words.out[1] = query2D of the rectangle.
 hipError_t launch_query2d(uint32_t minX, uint32_t maxX, uint32_t minY, uint32_t maxY, uint32_t maxZ,
-                          const QueryParams& p, uint8_t* out, hipStream_t stream);
+                          const QueryParams& p, hipStream_t stream);
+// words.out[0] = the error word, nothing else.
+hipError_t launch_host_words(const HostWords& words, hipStream_t stream);
 // Recomputes the min-hiZ of every 8x8-block tile from hiz.
 hipError_t launch_tile_min(const uint16_t* hiz, uint32_t bX, uint32_t bY, uint16_t* tileMin, uint32_t pyrX,
                            uint32_t pyrY, hipStream_t stream);
 hipError_t launch_readback(const uint16_t* depth, const uint16_t* hiz, uint32_t width, uint32_t height, uint32_t bX,
-                           uint32_t* rgba, hipStream_t stream);
+                           uint32_t* rgba, const HostWords& words, hipStream_t stream);
 hipError_t launch_clear(uint16_t* hiz, uint32_t nHiz, uint16_t* tileMin, uint32_t nMin, hipStream_t stream);
 // Multi-view: grid of `groups` persistent work-groups over p.nUnits units of
 // 8x8-block tiles.

@@ -2066,10 +2066,32 @@ __global__ void __launch_bounds__(256) rz_query_kernel(QueryParams p) {
   if (valid) {
     p.visible[q] = uint8_t(vis);
     if (p.needsClipping) p.needsClipping[q] = uint8_t(clip);
+  }
+  // The draws that set the error word have completed.
+  if (p.words.out && blockIdx.x == 0 && threadIdx.x == 0) p.words.out[0] = *p.words.err;
+}
+
+// queryVisibility of one box, by one wave: the box comes with the launch and
+// the answer goes straight to host memory, so a blocking call is one launch
+// and one wait.  Latency bound: rz_query takes 15 us on an idle stream.  (With
+// a copy of the box before it, and copies of the answer and of the error word
+// after it, it took 41 us.)
+__global__ void __launch_bounds__(64) rz_query_one_kernel(QueryParams p, QueryBox box) {
+  const QueryPre Q = query_pre(p.mvp, box.lo, box.hi, p.width, p.height, p.rcp);
+  const uint32_t clip = Q.kind == 1 ? 1u : 0u;
+  uint32_t vis = clip;
+  if (Q.kind == 3) {  // the same in every lane
+    const QueryBufs B = {p.depth, p.hiz, p.tileMin, p.bX, p.pyrX};
+    vis = query2d_wave(Q.minX, Q.maxX, Q.minY, Q.maxY, Q.maxZ, B, threadIdx.x) ? 1u : 0u;
+  }
+  if (threadIdx.x == 0) {
     // bit 0 visible, bit 1 needsClipping, bit 2 needsClipping was written
-    if (p.code) p.code[q] = uint8_t(vis | (clip << 1) | (Q.kind != 0 ? 4u : 0u));
+    p.words.out[1] = vis | (clip << 1) | (Q.kind != 0 ? 4u : 0u);
+    p.words.out[0] = *p.words.err;
   }
 }
+
+__global__ void rz_host_words_kernel(HostWords words) { words.out[0] = *words.err; }
 
 // queryVisibility over the queries of every view of a multi-view launch;
 // blockIdx.y is the view.  A step holds many boxes, so one lane per box does
@@ -2116,9 +2138,12 @@ __global__ void rz_views_clear_kernel(const ViewDesc* __restrict__ src, ViewDesc
 }
 
 __global__ void rz_query2d_kernel(uint32_t minX, uint32_t maxX, uint32_t minY, uint32_t maxY, uint32_t maxZ,
-                                  QueryParams p, uint8_t* out) {
+                                  QueryParams p) {
   const bool v = query2d_wave(minX, maxX, minY, maxY, maxZ, {p.depth, p.hiz, p.tileMin, p.bX, p.pyrX}, threadIdx.x);
-  if (threadIdx.x == 0) *out = v ? 1 : 0;
+  if (threadIdx.x == 0) {
+    p.words.out[1] = v ? 1u : 0u;
+    p.words.out[0] = *p.words.err;
+  }
 }
 
 // Min of hiZ over each 8x8-block tile, one wave per tile.
@@ -2136,7 +2161,9 @@ __global__ void rz_tile_min_kernel(const uint16_t* __restrict__ hiz, uint32_t bX
 // readBackDepth (Rasterizer.cpp:351-399), one pixel per thread.
 __global__ void __launch_bounds__(256) rz_readback_kernel(const uint16_t* __restrict__ depth,
                                                           const uint16_t* __restrict__ hiz, uint32_t width,
-                                                          uint32_t height, uint32_t bX, uint32_t* __restrict__ rgba) {
+                                                          uint32_t height, uint32_t bX, uint32_t* __restrict__ rgba,
+                                                          HostWords words) {
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) words.out[0] = *words.err;
   const uint32_t px = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t py = blockIdx.y;
   if (px >= width || py >= height) return;
@@ -2506,9 +2533,19 @@ hipError_t launch_query(const QueryParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+hipError_t launch_query_one(const QueryParams& p, const QueryBox& box, hipStream_t stream) {
+  hipLaunchKernelGGL(rz_query_one_kernel, dim3(1), dim3(64), 0, stream, p, box);
+  return hipGetLastError();
+}
+
 hipError_t launch_query2d(uint32_t minX, uint32_t maxX, uint32_t minY, uint32_t maxY, uint32_t maxZ,
-                          const QueryParams& p, uint8_t* out, hipStream_t stream) {
-  hipLaunchKernelGGL(rz_query2d_kernel, dim3(1), dim3(64), 0, stream, minX, maxX, minY, maxY, maxZ, p, out);
+                          const QueryParams& p, hipStream_t stream) {
+  hipLaunchKernelGGL(rz_query2d_kernel, dim3(1), dim3(64), 0, stream, minX, maxX, minY, maxY, maxZ, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_host_words(const HostWords& words, hipStream_t stream) {
+  hipLaunchKernelGGL(rz_host_words_kernel, dim3(1), dim3(1), 0, stream, words);
   return hipGetLastError();
 }
 
@@ -2520,9 +2557,9 @@ hipError_t launch_tile_min(const uint16_t* hiz, uint32_t bX, uint32_t bY, uint16
 }
 
 hipError_t launch_readback(const uint16_t* depth, const uint16_t* hiz, uint32_t width, uint32_t height, uint32_t bX,
-                           uint32_t* rgba, hipStream_t stream) {
+                           uint32_t* rgba, const HostWords& words, hipStream_t stream) {
   hipLaunchKernelGGL(rz_readback_kernel, dim3(groups(width, 256), height), dim3(256), 0, stream, depth, hiz, width,
-                     height, bX, rgba);
+                     height, bX, rgba, words);
   return hipGetLastError();
 }
 
