@@ -42,6 +42,10 @@ struct rz_mlp {
   uint32_t* d_pairs = nullptr;
   uint32_t capPairs = 0;
   float* d_loss = nullptr;
+  float* d_partial = nullptr;  // backward's rows, for capPartial work-groups
+  uint32_t capPartial = 0;
+  float* h_result = nullptr;   // pinned: the gradient, then the loss
+  float* d_hResult = nullptr;  // its device mapping
   uint32_t step = 0;
   // The model reads feature 10, the previous step's label of the batch; when
   // it does not (trained with that feature held at 0), multi-view steps

@@ -295,8 +295,14 @@ struct MlpParams {
   const uint32_t* nRows;
   float* scores;        // forward output
   const float* dscore;  // backward input: dLoss/dscore per sample
-  float* grad;          // backward output, accumulated (zero it first)
+  float* clear;         // optional (forward): n words set to 0, and *clearLoss
+  float* clearLoss;
+  float* partial;       // backward: kMlpParams words per mlp_backward_rows(n)
+  float* grad;          // backward output
+  const float* loss;    // with host
+  float* host;          // optional (backward): grad, then *loss, in mapped host memory
 };
+uint32_t mlp_backward_rows(uint32_t n);
 hipError_t launch_mlp_forward(const MlpParams& p, hipStream_t stream);
 // Work-groups of the scoring kernel resident on the current device at once
 // (queried once per process; call outside stream capture before the first

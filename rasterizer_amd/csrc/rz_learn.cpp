@@ -40,6 +40,8 @@ void mlp_free(rz_mlp* m) {
   hipFree(m->d_ds);
   hipFree(m->d_pairs);
   hipFree(m->d_loss);
+  hipFree(m->d_partial);
+  if (m->h_result) (void)hipHostFree(m->h_result);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
 }
@@ -69,6 +71,32 @@ int ensure_pairs(rz_mlp* m, uint32_t n) {
   return RZ_OK;
 }
 
+// Backward's partial sums, and the result that its last kernel writes to host
+// memory.
+int ensure_backward(rz_mlp* m, uint32_t n) {
+  if (!m->h_result) {
+    void* h = nullptr;
+    if (hipHostMalloc(&h, (kMlpParams + 1) * sizeof(float), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+      return RZ_ERR_OUT_OF_MEMORY;
+    void* d = nullptr;
+    if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+      (void)hipHostFree(h);
+      return RZ_ERR_DEVICE;
+    }
+    m->h_result = static_cast<float*>(h);
+    m->d_hResult = static_cast<float*>(d);
+  }
+  const uint32_t rows = mlp_backward_rows(n);
+  if (rows <= m->capPartial) return RZ_OK;
+  hipFree(m->d_partial);
+  m->d_partial = nullptr;
+  m->capPartial = 0;
+  if (hipMalloc(reinterpret_cast<void**>(&m->d_partial), size_t(rows) * kMlpParams * sizeof(float)) != hipSuccess)
+    return RZ_ERR_OUT_OF_MEMORY;
+  m->capPartial = rows;
+  return RZ_OK;
+}
+
 MlpParams params_of(const rz_mlp* m, uint32_t n) {
   MlpParams p{};
   p.w = m->d_w;
@@ -81,7 +109,8 @@ MlpParams params_of(const rz_mlp* m, uint32_t n) {
   return p;
 }
 
-// Loss and gradients of the pairs on the uploaded samples into d_grad.
+// Loss and gradients of the pairs on the uploaded samples into d_grad and
+// h_result.
 int run_gradients(rz_mlp* m, uint32_t n, const float* x, uint32_t nPairs, const uint32_t* pairs) {
   for (uint32_t k = 0; k < 2 * nPairs; ++k)
     if (pairs[k] >= n) return RZ_ERR_INVALID_ARGUMENT;
@@ -89,12 +118,16 @@ int run_gradients(rz_mlp* m, uint32_t n, const float* x, uint32_t nPairs, const 
   if (s != RZ_OK) return s;
   s = ensure_pairs(m, std::max(nPairs, 1u));
   if (s != RZ_OK) return s;
+  s = ensure_backward(m, n);
+  if (s != RZ_OK) return s;
   RZ_HIP(hipMemcpyAsync(m->d_x, x, size_t(n) * kMlpIn * 4, hipMemcpyHostToDevice, m->stream));
   if (nPairs) RZ_HIP(hipMemcpyAsync(m->d_pairs, pairs, size_t(nPairs) * 8, hipMemcpyHostToDevice, m->stream));
-  const MlpParams p = params_of(m, n);
-  RZ_HIP(launch_fill_f32(m->d_grad, kMlpParams, 0.0f, m->stream));
-  RZ_HIP(launch_fill_f32(m->d_ds, n, 0.0f, m->stream));
-  RZ_HIP(launch_fill_f32(m->d_loss, 1, 0.0f, m->stream));
+  MlpParams p = params_of(m, n);
+  p.clear = m->d_ds;
+  p.clearLoss = m->d_loss;
+  p.partial = m->d_partial;
+  p.loss = m->d_loss;
+  p.host = m->d_hResult;
   RZ_HIP(launch_mlp_forward(p, m->stream));
   RZ_HIP(launch_mlp_pair_loss(m->d_scores, m->d_pairs, nPairs, m->d_ds, m->d_loss, m->stream));
   RZ_HIP(launch_mlp_backward(p, m->stream));
@@ -193,9 +226,9 @@ extern "C" int rz_mlp_gradients(rz_mlp* m, uint32_t n, const float* x, uint32_t 
   if (!m || !x || (nPairs && !pairs) || n == 0) return RZ_ERR_INVALID_ARGUMENT;
   int s = run_gradients(m, n, x, nPairs, pairs);
   if (s != RZ_OK) return s;
-  if (grad) RZ_HIP(hipMemcpyAsync(grad, m->d_grad, kMlpParams * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-  if (loss) RZ_HIP(hipMemcpyAsync(loss, m->d_loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
   RZ_HIP(hipStreamSynchronize(m->stream));
+  if (grad) std::memcpy(grad, m->h_result, kMlpParams * sizeof(float));
+  if (loss) *loss = m->h_result[kMlpParams];
   return RZ_OK;
 }
 
@@ -208,7 +241,7 @@ extern "C" int rz_mlp_train_step(rz_mlp* m, uint32_t n, const float* x, uint32_t
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.0f - std::pow(b1, float(m->step)), c2 = 1.0f - std::pow(b2, float(m->step));
   RZ_HIP(launch_mlp_adam(m->d_w, m->d_grad, m->d_m, m->d_v, kMlpParams, lr, b1, b2, 1e-8f, c1, c2, m->stream));
-  if (loss) RZ_HIP(hipMemcpyAsync(loss, m->d_loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
   RZ_HIP(hipStreamSynchronize(m->stream));
+  if (loss) *loss = m->h_result[kMlpParams];
   return RZ_OK;
 }
