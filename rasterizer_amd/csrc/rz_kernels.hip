@@ -1390,7 +1390,12 @@ __device__ __forceinline__ uint32_t tile_relevance(const ItemState& S, uint32_t 
 
 // done[i] packs, over the tiles of item i's query rectangle, the number of
 // tiles that have contributed (bits 0-15) and how many found a visible pixel
-// (bits 16-31).
+// (bits 16-31).  The word is all that passes between tiles (each reads and
+// writes its own depth, hiZ and winners only), so its additions and loads are
+// relaxed: a release writes the XCD's L2 back before each addition and an
+// acquire drops the cached records after each load.  With those, one 1080p city
+// frame took 250 us, the raster launches of 20 and 128 city frames in flight
+// 1.55 and 5.05 ms; without, 217 us, 0.82 and 3.08 ms.
 constexpr uint32_t kDoneCountMask = 0xFFFFu;
 constexpr uint32_t kDoneVisibleOne = 0x10000u;
 
@@ -1495,7 +1500,7 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
 #pragma unroll
       for (int w = 0; w < NW; ++w) any |= sm.spart[sPar][w];
       if (any == 0u) {
-        __hip_atomic_fetch_add(&J.done[L.index], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(&J.done[L.index], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         sm.spec[c >> 5] |= 1u << (c & 31u);
       } else {
         sm.tried[c] = drawVersion;
@@ -1584,7 +1589,7 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
           uint32_t part = 0;
 #pragma unroll
           for (int w = 0; w < NW; ++w) part |= sm.part[qPar][w];
-          __hip_atomic_fetch_add(&J.done[item], 1u + (part ? kDoneVisibleOne : 0u), __ATOMIC_RELEASE,
+          __hip_atomic_fetch_add(&J.done[item], 1u + (part ? kDoneVisibleOne : 0u), __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
         }
         qPar ^= 1u;
@@ -1603,7 +1608,7 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
         bool vis;
         while (true) {
           if (tid == 0) {
-            const uint32_t d = __hip_atomic_load(&J.done[item], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+            const uint32_t d = __hip_atomic_load(&J.done[item], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             uint32_t st = 0;
             if ((d & kDoneCountMask) >= L.expected || d >= kDoneVisibleOne) {
               st = d >= kDoneVisibleOne ? 2u : 1u;
