@@ -756,6 +756,16 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
+// A value that is the same in every lane, as a scalar.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint64_t uniform(uint64_t v) {
+  return uniform(uint32_t(v)) | uint64_t(uniform(uint32_t(v >> 32))) << 32;
+}
+template <typename T>
+__device__ __forceinline__ T* uniform(T* p) {
+  return reinterpret_cast<T*>(uniform(reinterpret_cast<uint64_t>(p)));
+}
+
 __device__ __forceinline__ uint32_t readlane_u(uint32_t v, uint32_t l) { return __builtin_amdgcn_readlane(v, l); }
 
 __device__ __forceinline__ uint64_t readlane_u64(uint64_t v, uint32_t l) {
@@ -772,11 +782,12 @@ __device__ __forceinline__ int div_bx(int d, int bX, float invBX) {
 // What a tile needs of one item, gathered once per item window.
 struct ItemLocal {
   uint32_t index;
-  uint32_t flags;  // bit 0: query rectangle overlaps the tile, bit 1: footprint does, bits 2-3: status
+  uint32_t flags;  // bit 0: query rectangle overlaps the tile, bit 1: footprint does, bits 2-3: status, 16-31: tiles
+                   // of the rectangle
   uint32_t qMinX, qMaxX, qMinY, qMaxY, qMaxZ;
-  uint32_t expected;
   uint32_t quadBase, quadCount;
-  uint64_t groups;  // bit k: aligned 64-quad group (quadBase >> 6) + k may touch the tile
+  uint32_t nGroups;  // its groups that may touch the tile (all when they exceed 64)
+  uint64_t groups;   // bit k: aligned 64-quad group (quadBase >> 6) + k may touch the tile
 };
 
 constexpr uint32_t kQuadChunk = 64;   // records staged in LDS at a time
@@ -803,15 +814,9 @@ struct TileSmem {
   // depth samples at the rectangle's first column in the tile.
   float entry[kEntryRows * 12];
   uint16_t pairs[8][64];  // per wave: the (block, quad) pairs being drawn
-  uint32_t wcnt[8];
-  uint32_t part[2][8];
-  // Early query answers (query-gated launches): per window item, a bit when
-  // this tile has already contributed its partial, and the tile's draw count
-  // at which an early evaluation last failed; per-wave results; wait state.
-  uint32_t spec[kItemWindow / 32];
-  uint32_t tried[kItemWindow];
-  uint32_t spart[2][8];
-  uint32_t wstate[2];
+  uint32_t wcnt[2][8];
+  // Where a round's run of items ends, and the mask of its visible query items.
+  uint4 run[2];
   uint32_t wnext;          // candidate position where the next item window starts
   uint32_t blockStats[4];  // observability builds: visited, rejected, written, fold steps
 };
@@ -1215,79 +1220,54 @@ __device__ uint64_t draw_chunk(TileSmem<TBX, TBY>& sm, uint32_t n, int tbx0, int
   return tB;
 }
 
-// One row of blocks of query2D inside the tile, one lane per block:
-// returns 1 if the wave finds a visible pixel in row lr, and with SPEC 2 if
-// a block of the rectangle in that row has hiZ 0 or 1; 0 otherwise.  The
-// hiZ tests of the row's blocks run together; only blocks that pass them are
-// tested pixel by pixel.
-template <int TBX, int TBY, bool SPEC>
-__device__ __forceinline__ uint32_t query_row(const ItemLocal& S, const TileSmem<TBX, TBY>& sm, int lr, int by,
-                                              int tbx0, int tbx1, uint32_t lane) {
-  static_assert(TBX <= 64, "one lane per block of a tile row");
-  const uint32_t maxZ = S.qMaxZ;
-  const int qbx0 = int(S.qMinX >> 3), qbx1 = int(S.qMaxX >> 3);
-  const int startY = max(int(S.qMinY) - 8 * by, 0), endY = min(int(S.qMaxY) - 8 * by, 7);
-  const int cx0 = max(tbx0, qbx0), cx1 = min(tbx1, qbx1);
-  const int n = cx1 - cx0 + 1;
-  bool cleared = false, cand = false, full = false;
-  if (int(lane) < n) {
-    const int bx = cx0 + int(lane);
-    const uint32_t hz = sm.hiz[lr * TBX + (bx - tbx0)];
-    cleared = hz <= 1u;
-    cand = maxZ > hz;
-    full = cand && startY == 0 && endY == 7 && int(S.qMinX) <= 8 * bx && int(S.qMaxX) >= 8 * bx + 7;
+// query2D restricted to the tile (Rasterizer.cpp:283-349), by one wave: 1 if a
+// pixel of the rectangle in the tile is visible, and with EARLY 2 if a block
+// of the rectangle in it has hiZ 0 or 1; 0 otherwise.  One lane per block for
+// the hiZ tests, then, where no interior block is visible, one lane per pixel
+// for each block at the rectangle's border that passed, four at a time.  Any
+// order of the blocks gives the same answer.
+//
+// EARLY: query2D evaluated ahead of the item's turn.  A block with hiZ >= 2
+// can never read as cleared (hiZ == 1) again, since its minimum only grows:
+// every later write max-merges, so its depth and hiZ only grow, and every test
+// of query2D (the hiZ skip and the row test) can only move from visible to not
+// visible.  So a result of 0 is the answer the tile gives at the item's turn.
+// A cleared block's next write replaces its stale depth, and a block at hiZ 0
+// could reach exactly 1, so neither proves anything.
+template <int TBX, int TBY, bool EARLY>
+__device__ __forceinline__ uint32_t query_tile(const ItemLocal& S, const TileSmem<TBX, TBY>& sm, int tbx0, int tbx1,
+                                               int tby0, int tby1, uint32_t lane) {
+  constexpr int kSteps = TBX * TBY / 64;  // 64 blocks a step
+  const int x0 = int(uniform(S.qMinX)), x1 = int(uniform(S.qMaxX));
+  const int y0 = int(uniform(S.qMinY)), y1 = int(uniform(S.qMaxY));
+  const uint32_t maxZ = uniform(S.qMaxZ);
+  uint64_t border[kSteps];
+#pragma unroll
+  for (int t = 0; t < kSteps; ++t) {
+    const int lb = 64 * t + int(lane), bx = tbx0 + lb % TBX, by = tby0 + lb / TBX;
+    const bool in = bx >= x0 >> 3 && bx <= x1 >> 3 && by >= y0 >> 3 && by <= y1 >> 3 && bx <= tbx1 && by <= tby1;
+    const uint32_t hz = sm.hiz[lb];
+    if (EARLY && __ballot(in && hz <= 1u) != 0ull) return 2u;
+    const bool open = in && maxZ > hz;
+    const bool whole = x0 <= 8 * bx && x1 >= 8 * bx + 7 && y0 <= 8 * by && y1 >= 8 * by + 7;
+    if (__ballot(open && whole) != 0ull) return 1u;
+    border[t] = __ballot(open);
   }
-  if (SPEC && __ballot(cleared) != 0ull) return 2u;
-  if (__ballot(full) != 0ull) return 1u;
-  uint64_t m = __ballot(cand);
   const int px = int(lane & 7u), py = int(lane >> 3);
-  while (m) {
-    const int bx = cx0 + int(__builtin_ctzll(m));
-    m &= m - 1ull;
-    const int lb = lr * TBX + (bx - tbx0);
-    const int startX = max(int(S.qMinX) - 8 * bx, 0), endX = min(int(S.qMaxX) - 8 * bx, 7);
-    const bool mine = py >= startY && py <= endY && px >= startX && px <= endX &&
-                      uint32_t(sm.depth[lb * 64 + int(lane)]) < maxZ;
-    if (__ballot(mine) != 0ull) return 1u;
-  }
-  return 0u;
-}
-
-// query2D restricted to this wave's rows of the tile (Rasterizer.cpp:283-349):
-// true if a pixel of the rectangle in those rows is visible.  Any order of
-// the blocks gives the same answer.
-template <int TBX, int TBY, int NW>
-__device__ __forceinline__ bool query_wave(const ItemLocal& S, TileSmem<TBX, TBY>& sm, int tbx0, int tbx1,
-                                           int tby0, int tby1, uint32_t wave, uint32_t lane) {
-  const int qby0 = int(S.qMinY >> 3), qby1 = int(S.qMaxY >> 3);
-  for (int lr = int(wave); lr < TBY; lr += NW) {
-    const int by = tby0 + lr;
-    if (by > tby1) break;
-    if (by < qby0 || by > qby1) continue;
-    if (query_row<TBX, TBY, false>(S, sm, lr, by, tbx0, tbx1, lane)) return true;
-  }
-  return false;
-}
-
-// query2D of this wave's rows evaluated ahead of the item's turn: bit 0 when
-// a pixel is visible, bit 1 when a block of the rectangle has hiZ 0 or 1.
-// A block with hiZ >= 2 can never read as cleared (hiZ == 1) again, since its
-// minimum only grows: every later write max-merges, so its depth and hiZ only
-// grow, and every test of query2D (the hiZ skip and the row test) can only
-// move from visible to not visible.  So a result of 0 from every wave is the
-// answer the tile gives at the item's turn.  A cleared block's next write
-// replaces its stale depth, and a block at hiZ 0 could reach exactly 1, so
-// neither proves anything.
-template <int TBX, int TBY, int NW>
-__device__ __forceinline__ uint32_t spec_query_wave(const ItemLocal& S, TileSmem<TBX, TBY>& sm, int tbx0, int tbx1,
-                                                    int tby0, int tby1, uint32_t wave, uint32_t lane) {
-  const int qby0 = int(S.qMinY >> 3), qby1 = int(S.qMaxY >> 3);
-  for (int lr = int(wave); lr < TBY; lr += NW) {
-    const int by = tby0 + lr;
-    if (by > tby1) break;
-    if (by < qby0 || by > qby1) continue;
-    const uint32_t r = query_row<TBX, TBY, true>(S, sm, lr, by, tbx0, tbx1, lane);
-    if (r) return r;
+#pragma unroll
+  for (int t = 0; t < kSteps; ++t) {
+    for (uint64_t m = border[t]; m;) {
+      bool hit = false;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int lb = 64 * t + (m ? __builtin_ctzll(m) : 0);
+        const bool some = m != 0ull;
+        m &= m - 1ull;
+        const int x = 8 * (tbx0 + lb % TBX) + px, y = 8 * (tby0 + lb / TBX) + py;
+        hit |= some && x >= x0 && x <= x1 && y >= y0 && y <= y1 && uint32_t(sm.depth[lb * 64 + int(lane)]) < maxZ;
+      }
+      if (__ballot(hit) != 0ull) return 1u;
+    }
   }
   return 0u;
 }
@@ -1435,7 +1415,12 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
                                              uint64_t (&ctr)[kFrameStatWords]) {
   static_assert(!LABELS || (TBX == 8 && TBY == 8), "only 8x8-block tiles hold quad numbers");
   auto stamp = []() -> uint64_t { return STATS ? __builtin_amdgcn_s_memrealtime() : 0; };
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  // Opaque, so that what a tile derives from it is not held in registers across
+  // the multi-view kernel's loop over tiles (at 128 registers that spilled).
+  uint32_t tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  tid &= 64u * NW - 1u;
+  const uint32_t lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t tX = J.tX, tY = J.tY;
   const int bX = J.bX, bY = J.bY;
   const int tbx0 = int(tX) * TBX, tby0 = int(tY) * TBY;
@@ -1478,40 +1463,17 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
     sm.hiz[lb] = (gx <= tbx1 && gy <= tby1) ? J.hiz[size_t(gy) * bX + gx] : uint16_t(0xFFFF);
   }
 
-  uint32_t qPar = 0;
   BlockCounters bc;
-  // Early "not visible" answers for later query items of the window, tried
-  // while the tile waits (see spec_query_wave), in query-gated launches only.
-  const bool gated = J.done != nullptr;
-  uint32_t drawVersion = 1, sPar = 0, wPar = 0, nRelW = 0;
-  auto answered_early = [&](uint32_t k) -> bool { return (sm.spec[k >> 5] >> (k & 31u)) & 1u; };
-  auto next_early = [&](uint32_t from) -> uint32_t {
-    for (uint32_t c = from; c < nRelW; ++c)
-      if ((sm.items[c].flags & 1u) && !answered_early(c) && sm.tried[c] != drawVersion) return c;
-    return nRelW;
-  };
-  auto try_early = [&](uint32_t c) {
-    const ItemLocal& L = sm.items[c];
-    const uint32_t r = spec_query_wave<TBX, TBY, NW>(L, sm, tbx0, tbx1, tby0, tby1, wave, lane);
-    if (lane == 0) sm.spart[sPar][wave] = r;
-    __syncthreads();
-    if (tid == 0) {
-      uint32_t any = 0;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) any |= sm.spart[sPar][w];
-      if (any == 0u) {
-        __hip_atomic_fetch_add(&J.done[L.index], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        sm.spec[c >> 5] |= 1u << (c & 31u);
-      } else {
-        sm.tried[c] = drawVersion;
-      }
-      if (STATS) {
-        ctr[kStatEarlyTried]++;
-        if (any == 0u) ctr[kStatEarlyAnswered]++;
-      }
-    }
-    sPar ^= 1u;
-  };
+  uint32_t rPar = 0, wPar = 0;
+  uint32_t fill = 0;  // quads staged in sm.recs and not yet drawn
+  // The window's current block of 64 slots: the lane's item, its flags and the
+  // groups it is drawn with; masks of the items with a share of query2D in the
+  // tile, with quads in it and with quads in it that need a decision.
+  uint32_t block = 0, laneIndex = 0, laneFlags = 0, laneGroups = 0;
+  uint64_t shares = 0, quads = 0, waits = 0;
+  // Wave 0: whose share was given, which of those with quads are decided and
+  // which of those visible; whose early evaluation failed since the last draw.
+  uint64_t given = 0, decided = 0, visible = 0, tried = 0;
   if (STATS) {
     if (tid < 4) sm.blockStats[tid] = 0;
     __syncthreads();
@@ -1528,172 +1490,257 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
     const uint32_t rel = inWin ? relevance(i) : 0u;
     const uint64_t m = __ballot(rel != 0u);
     const uint32_t pre = __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
-    if (lane == 0) sm.wcnt[wave] = uint32_t(__popcll(m));
+    if (lane == 0) sm.wcnt[wPar][wave] = uint32_t(__popcll(m));
     if (tid == 0) sm.wnext = min(wbase + NT, nList);
     __syncthreads();
     uint32_t off = 0, nRel = 0;
 #pragma unroll
     for (uint32_t w = 0; w < NW; ++w) {
-      off += w < wave ? sm.wcnt[w] : 0u;
-      nRel += sm.wcnt[w];
+      off += w < wave ? sm.wcnt[wPar][w] : 0u;
+      nRel += sm.wcnt[wPar][w];
     }
+    wPar ^= 1u;
     if (rel && off + pre == kItemWindow) sm.wnext = wbase + tid;
     nRel = min(nRel, kItemWindow);
     if (rel && off + pre < kItemWindow) {
       const ItemState& S = J.state[i];
       ItemLocal& L = sm.items[off + pre];
       L.index = i;
-      L.flags = rel;
+      L.flags = rel | S.expected << 16;
       L.qMinX = S.qMinX;
       L.qMaxX = S.qMaxX;
       L.qMinY = S.qMinY;
       L.qMaxY = S.qMaxY;
       L.qMaxZ = S.qMaxZ;
-      L.expected = S.expected;
       const uint32_t qb = J.items[i].quadBase, qc = J.items[i].quadCount;
       L.quadBase = qb;
       L.quadCount = qc;
       uint64_t groups = ~0ull;
+      uint32_t nGroups = 0;
       if ((rel & 2u) && qc > 0) {
         const uint32_t g0 = qb >> 6, g1 = (qb + qc - 1) >> 6;
-        if (g1 - g0 < 64) {
+        nGroups = g1 - g0 + 1;
+        if (nGroups <= 64) {
           groups = 0;
           for (uint32_t gi = g0; gi <= g1; ++gi)
             if (box_touches(J.groupBox[gi], tbx0, tbx1, tby0, tby1)) groups |= 1ull << (gi - g0);
+          nGroups = uint32_t(__popcll(groups));
         }
       }
       L.groups = groups;
-    }
-    if (gated) {
-      if (tid < kItemWindow / 32) sm.spec[tid] = 0u;
-      if (tid < kItemWindow) sm.tried[tid] = 0u;
+      L.nGroups = nGroups;
     }
     __syncthreads();
-    nRelW = nRel;
-    const uint32_t wnext = sm.wnext;
-    // Later query items are answered early only while the tile waits: a
-    // pass over the window's query items at its start delays the tiles with
-    // the longest lists, which other tiles' waits depend on.
+    nRel = uniform(nRel);
+    const uint32_t wnext = uniform(sm.wnext);
 
-    for (uint32_t k = 0; k < nRel; ++k) {
-      const ItemLocal& L = sm.items[k];
-      const uint32_t item = L.index, flags = L.flags, status = flags >> 2;
-      if (STATS && tid == 0) ctr[kStatItems]++;
-      if ((flags & 1u) && !(gated && answered_early(k))) {
-        // This tile's share of query2D for the item, at its exact turn.
-        const uint64_t tq = stamp();
-        const bool found = query_wave<TBX, TBY, NW>(L, sm, tbx0, tbx1, tby0, tby1, wave, lane);
-        if (lane == 0) sm.part[qPar][wave] = found ? 1u : 0u;
-        __syncthreads();
-        if (tid == 0) {
-          uint32_t part = 0;
-#pragma unroll
-          for (int w = 0; w < NW; ++w) part |= sm.part[qPar][w];
-          __hip_atomic_fetch_add(&J.done[item], 1u + (part ? kDoneVisibleOne : 0u), __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
+    // The window's items in draw order, in rounds.  Wave 0 goes over the items
+    // from k on: it gives the tile's share of query2D where one is due, reads
+    // the decisions of query items and waits for them, up to an item that needs
+    // what is to be drawn before it to be drawn (or the block's end).  All waves
+    // then scan the quads of the round's visible items together and stage them
+    // behind those already staged; 64 are drawn at a time, what is left before
+    // wave 0 goes on if it needs it, else with the next round's.
+    //
+    // What bounds it: the latency of this chain, tile after tile, and the issue
+    // slots that it takes from the work-group on the same CU.  So the seven
+    // other waves are at a barrier meanwhile, and small items share scans and
+    // draws.  (With the eight waves sharing every query2D and every poll, two
+    // barriers an item, and each item scanned and drawn by itself, a 4K frame
+    // of 12,000 icospheres took 1.20 ms, and takes 0.72 ms; the raster launches
+    // of 20 and 128 city frames in flight took 0.83 and 3.09 ms, and take 0.78 and
+    // 3.01 ms, that of 64 mixed views 0.61 and 0.51 ms.)
+    bool arrived = true;  // at a block of 64 slots
+    uint32_t upTo = 0;    // lane i: groups of the round's drawn items up to item block + i
+    for (uint32_t k = 0;;) {
+      bool drain = false;
+      uint64_t draw = 0;
+      if (k == nRel) {
+        if (fill == 0u || wnext < nList) break;
+        drain = true;
+      } else {
+        if (arrived) {
+          arrived = false;
+          block = k;
+          const bool in = k + lane < nRel;
+          const ItemLocal& I = sm.items[in ? k + lane : k];
+          laneIndex = I.index;
+          laneFlags = in ? I.flags : 0u;
+          laneGroups = I.nGroups;
+          shares = __ballot((laneFlags & 1u) != 0u);
+          quads = __ballot((laneFlags & 2u) != 0u);
+          waits = __ballot((laneFlags & 2u) && ((laneFlags >> 2) & 3u) == uint32_t(kStatusTest));
+          given = decided = visible = tried = 0;
         }
-        qPar ^= 1u;
-        if (STATS) {
-          ctr[kStatQueryTicks] += stamp() - tq;
-          ctr[kStatQueries]++;
-        }
-      }
-      if (!(flags & 2u)) continue;
-      if (status == kStatusTest) {
-        // Wait until every tile of the rectangle has answered, or one of them
-        // has already seen a visible pixel; meanwhile answer later items of
-        // the window early where the tile's state already proves them.
-        const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-        uint32_t c = k + 1;
-        bool vis;
-        while (true) {
-          if (tid == 0) {
-            const uint32_t d = __hip_atomic_load(&J.done[item], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            uint32_t st = 0;
-            if ((d & kDoneCountMask) >= L.expected || d >= kDoneVisibleOne) {
-              st = d >= kDoneVisibleOne ? 2u : 1u;
-            } else if (__builtin_amdgcn_s_memrealtime() - t0 > J.timeoutTicks ||
-                       __hip_atomic_load(J.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
-              // After one wait of the launch has timed out, the others stop
-              // waiting too (the launch's result is reported as an error).
-              __hip_atomic_fetch_or(J.err, uint32_t(kErrTimeout), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-              st = d >= kDoneVisibleOne ? 2u : 1u;
+        if (wave == 0) {
+          uint32_t at = k - block;
+          while (true) {
+            // The next item with a share due or a decision open; those before it
+            // are decided.
+            const uint64_t rest = ~0ull << at, open = waits & ~decided & rest;
+            uint64_t due = shares & ~given & rest;
+            const uint64_t events = due | open;
+            at = events ? uint32_t(__builtin_ctzll(events)) : min(nRel - block, 64u);
+            draw |= quads & (visible | ~waits) & rest & ((1ull << (at & 63u)) - (at < 64u ? 1ull : 2ull));
+            if (events == 0ull) break;
+            const uint64_t turn = 1ull << at;
+            const bool pending = draw != 0ull || fill != 0u;
+            if (due & turn) {
+              // This tile's share of query2D for the item, at its exact turn.
+              if (pending) {
+                drain = true;
+                break;
+              }
+              const uint64_t tq = stamp();
+              const bool found = query_tile<TBX, TBY, false>(sm.items[block + at], sm, tbx0, tbx1, tby0, tby1, lane);
+              if (lane == at)
+                __hip_atomic_fetch_add(&J.done[laneIndex], 1u + (found ? kDoneVisibleOne : 0u), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+              given |= turn;
+              if (found || readlane_u(laneFlags, at) >> 16 == 1u) {
+                // It decides: a pixel is visible, or no other tile has a share.
+                decided |= turn;
+                visible |= found ? turn : 0ull;
+              }
+              if (STATS && lane == 0) {
+                ctr[kStatQueryTicks] += stamp() - tq;
+                ctr[kStatQueries]++;
+              }
+              continue;
             }
-            sm.wstate[wPar] = st;
+            // A query item is decided when every tile of its rectangle has given
+            // its share, or one of them has seen a visible pixel: the counters of
+            // the items up to the next share, together.
+            const uint64_t ask = open & (due ? (due & (0ull - due)) - 1ull : ~0ull);
+            uint32_t d = 0;
+            if (__builtin_amdgcn_inverse_ballot_w64(ask))
+              d = __hip_atomic_load(&J.done[laneIndex], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint64_t seen = __ballot(d >= kDoneVisibleOne) & ask;
+            visible |= seen;
+            decided |= seen | (__ballot((d & kDoneCountMask) >= laneFlags >> 16) & ask);
+            if (decided & turn) continue;
+            if (pending) {
+              drain = true;
+              break;
+            }
+            // Wait for it.  Meanwhile give later items' shares early where the
+            // tile's state already proves that they see nothing.
+            const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
+            if (STATS && lane == 0) ctr[kStatWaits]++;
+            const uint32_t expected = readlane_u(laneFlags, at) >> 16;
+            const uint32_t* counter = &J.done[readlane_u(laneIndex, at)];
+            while (true) {
+              d = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              const uint32_t err = __hip_atomic_load(J.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              const uint64_t later = due & ~tried;
+              if (later != 0ull) {
+                const uint32_t c = uint32_t(__builtin_ctzll(later));
+                const uint64_t bit = 1ull << c;
+                const bool none = query_tile<TBX, TBY, true>(sm.items[block + c], sm, tbx0, tbx1, tby0, tby1, lane) == 0u;
+                if (none) {
+                  if (lane == c) __hip_atomic_fetch_add(&J.done[laneIndex], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                  given |= bit;
+                  due &= ~bit;
+                  if (readlane_u(laneFlags, c) >> 16 == 1u) decided |= bit;
+                } else {
+                  tried |= bit;
+                }
+                if (STATS && lane == 0) {
+                  ctr[kStatEarlyTried]++;
+                  if (none) ctr[kStatEarlyAnswered]++;
+                }
+              } else {
+                __builtin_amdgcn_s_sleep(1);
+              }
+              const uint32_t now = uniform(d);
+              if (now >= kDoneVisibleOne) visible |= turn;
+              if (now >= kDoneVisibleOne || (now & kDoneCountMask) >= expected) break;
+              if (__builtin_amdgcn_s_memrealtime() - t0 > J.timeoutTicks || uniform(err) != 0u) {
+                // After one wait of the launch has timed out, the others stop
+                // waiting too (the launch's result is reported as an error).
+                if (lane == 0)
+                  __hip_atomic_fetch_or(J.err, uint32_t(kErrTimeout), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+              }
+            }
+            decided |= turn;
+            if (STATS && lane == 0) ctr[kStatWaitTicks] += __builtin_amdgcn_s_memrealtime() - t0;
           }
-          __syncthreads();
-          const uint32_t st = sm.wstate[wPar];
-          wPar ^= 1u;
-          if (st != 0u) {
-            vis = st == 2u;
-            break;
-          }
-          c = next_early(c);
-          if (c < nRel) {
-            try_early(c);
-            ++c;
-          } else if (tid == 0) {
-            __builtin_amdgcn_s_sleep(1);
-          }
+          if (lane == 0)
+            sm.run[rPar] = make_uint4(at, drain ? 1u : 0u, uint32_t(draw), uint32_t(draw >> 32));
+          if (STATS && lane == 0) ctr[kStatItems] += at - (k - block);
         }
-        if (STATS && tid == 0) {
-          ctr[kStatWaitTicks] += stamp() - t0;
-          ctr[kStatWaits]++;
-        }
-        if (!vis) continue;
-      }
-      // Draw the item's quads that touch the tile, in submission order: each
-      // pass tests 64 * NW quads (one per thread; passes and waves whose
-      // 64-quad groups miss the tile are skipped); hits are staged into LDS
-      // and drawn 64 at a time.
-      const uint64_t tr = stamp();
-      const uint32_t gBase = L.quadBase >> 6;
-      for (uint32_t base = 0; base < L.quadCount; base += NT) {
-        // groups overlapping this pass, relative to gBase
-        const uint32_t pg0 = ((L.quadBase + base) >> 6) - gBase;
-        const uint32_t pg1 = ((L.quadBase + min(base + NT, L.quadCount) - 1) >> 6) - gBase;
-        const uint64_t passMask = (pg1 - pg0 >= 63) ? ~0ull : (((2ull << (pg1 - pg0)) - 1) << pg0);
-        if (pg0 < 64 && (L.groups & passMask) == 0) continue;
-        const uint64_t tScan = stamp();
-        if (STATS && tid == 0) ctr[kStatPasses]++;
-        const uint32_t waveFirst = base + wave * 64u;
-        bool hit = false;
-        if (waveFirst < L.quadCount) {
-          const uint32_t wg0 = ((L.quadBase + waveFirst) >> 6) - gBase;
-          const uint32_t wg1 = ((L.quadBase + min(waveFirst + 63u, L.quadCount - 1u)) >> 6) - gBase;
-          const bool groupHit = wg1 >= 64 || ((L.groups >> wg0) & 1ull) || ((L.groups >> wg1) & 1ull);
-          if (groupHit && base + tid < L.quadCount)
-            hit = quad_touches_tile(load_rec(&J.recs[L.quadBase + base + tid]), tbx0, tbx1, tby0, tby1, bX, invBX);
-        }
-        const uint64_t hm = __ballot(hit);
-        const uint32_t hpre =
-            __builtin_amdgcn_mbcnt_hi(uint32_t(hm >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(hm), 0u));
-        if (lane == 0) sm.wcnt[wave] = uint32_t(__popcll(hm));
         __syncthreads();
-        uint32_t hoff = 0, total = 0;
+        const uint4 r = sm.run[rPar];
+        rPar ^= 1u;
+        const uint32_t end = uniform(r.x);
+        drain = uniform(r.y) != 0u;
+        draw = uniform(r.z) | uint64_t(uniform(r.w)) << 32;
+        k = block + end;
+        arrived = end == 64u;
+      }
+      uint32_t nGroups = 0;
+      if (draw != 0ull) {
+        upTo = __ockl_wfscan_add_u32(lane_select(draw, laneGroups), true);
+        nGroups = readlane_u(upTo, 63u);
+      }
+      // Scan the run, one 64-quad group that may touch the tile per wave and
+      // pass, and draw.
+      const uint64_t tr = stamp();
+      for (uint32_t f0 = 0; f0 < nGroups || (drain && fill != 0u); f0 += NW) {
+        uint32_t total = fill, pos = 0, quad = 0;
+        bool hit = false;
+        if (f0 < nGroups) {
+          const uint64_t tScan = stamp();
+          if (STATS && tid == 0) ctr[kStatPasses]++;
+          const uint32_t f = f0 + wave;
+          if (f < nGroups) {
+            const uint32_t r = uint32_t(__popcll(__ballot(upTo <= f)));
+            const uint32_t j = f - (r ? readlane_u(upTo, r - 1u) : 0u);  // the item's j-th group
+            const ItemLocal& L = sm.items[block + r];
+            const uint64_t groups = L.groups;
+            const uint32_t first = L.quadBase, past = first + L.quadCount;
+            uint32_t g = j;
+            if (((past - 1u) >> 6) - (first >> 6) < 64u) {
+              const bool set = (groups >> lane) & 1ull;
+              const uint32_t rank = uint32_t(__popcll(groups & ((1ull << lane) - 1ull)));
+              g = uint32_t(__builtin_ctzll(__ballot(set && rank == j)));
+            }
+            quad = ((first >> 6) + g) * 64u + lane;
+            if (quad >= first && quad < past)
+              hit = quad_touches_tile(load_rec(&J.recs[quad]), tbx0, tbx1, tby0, tby1, bX, invBX);
+          }
+          const uint64_t hm = __ballot(hit);
+          const uint32_t hpre =
+              __builtin_amdgcn_mbcnt_hi(uint32_t(hm >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(hm), 0u));
+          if (lane == 0) sm.wcnt[wPar][wave] = uint32_t(__popcll(hm));
+          __syncthreads();
+          pos = fill + hpre;
 #pragma unroll
-        for (uint32_t w = 0; w < NW; ++w) {
-          hoff += w < wave ? sm.wcnt[w] : 0u;
-          total += sm.wcnt[w];
-        }
-        const uint32_t pos = hoff + hpre;
-        if (STATS && tid == 0) ctr[kStatScanTicks] += stamp() - tScan;
-        // Hits reload their record (just read, so from cache) rather than
-        // hold it across the compaction, which made the compiler spill it.
-        if (hit && pos < kQuadChunk) {
-          sm.recs[pos] = J.recs[L.quadBase + base + tid];
-          if (LABELS) sm.qid[pos] = L.quadBase + base + tid;
+          for (uint32_t w = 0; w < NW; ++w) {
+            pos += w < wave ? sm.wcnt[wPar][w] : 0u;
+            total += sm.wcnt[wPar][w];
+          }
+          total = uniform(total);
+          wPar ^= 1u;
+          if (STATS && tid == 0) ctr[kStatScanTicks] += stamp() - tScan;
         }
         for (uint32_t k0 = 0; k0 < total; k0 += kQuadChunk) {
           const uint32_t n = min(kQuadChunk, total - k0);
-          if (k0 > 0 && hit && pos >= k0 && pos < k0 + n) {
-            sm.recs[pos - k0] = J.recs[L.quadBase + base + tid];
-            if (LABELS) sm.qid[pos - k0] = L.quadBase + base + tid;
+          // Hits reload their record (just read, so from cache) rather than
+          // hold it across the compaction, which made the compiler spill it.
+          if (hit && pos >= k0 && pos < k0 + n) {
+            sm.recs[pos - k0] = J.recs[quad];
+            if (LABELS) sm.qid[pos - k0] = quad;
           }
+          fill = n;
+          if (n < kQuadChunk && !(drain && f0 + NW >= nGroups)) break;
           __syncthreads();
           const uint64_t tDraw = stamp();
           const uint64_t tB = draw_chunk<TBX, TBY, NW, STATS, LABELS>(sm, n, tbx0, tbx1, tby0, tby1, bX, invBX, wave,
                                                                       lane, bc, J.winner);
+          fill = 0;
+          tried = 0;  // the tile's state changed: early evaluations that failed may now succeed
           if (STATS && tid == 0) ctr[kStatQuads] += n;
           __syncthreads();
           if (STATS && tid == 0) {
@@ -1706,7 +1753,6 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
         }
       }
       if (STATS && tid == 0) ctr[kStatRasterTicks] += stamp() - tr;
-      ++drawVersion;  // the tile's state changed: early answers that failed may now succeed
     }
     __syncthreads();
     wbase = wnext;
@@ -1837,7 +1883,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) rz_views_kernel(View
       unitSh = u >= nHanded ? 0xFFFFFFFFu : p.unitList ? p.unitList[u] : u;
     }
     __syncthreads();
-    const uint32_t entry = unitSh;
+    const uint32_t entry = __builtin_amdgcn_readfirstlane(unitSh);
     __syncthreads();
     if (entry == 0xFFFFFFFFu) break;
     uint32_t lo = 0, t = 0;
@@ -1854,29 +1900,31 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) rz_views_kernel(View
       t = entry - p.views[lo].unitBase;
     }
     const ViewDesc& V = p.views[lo];
-    const uint32_t unit = V.unitBase + t;
+    const uint32_t unit = uniform(V.unitBase) + t, tilesX = uniform(V.tilesX);
     TileJob J;
     J.items = p.items;
     J.state = p.state;
-    J.itemBegin = p.batchItems ? V.batchBase : V.itemBase;
-    J.itemEnd = p.batchItems ? V.batchBase + V.nBatches : V.itemBase + V.nItems;
-    J.bX = int(V.bX);
-    J.bY = int(V.bY);
-    J.tX = t % V.tilesX;
-    J.tY = t / V.tilesX;
+    const uint32_t first = uniform(p.batchItems ? V.batchBase : V.itemBase);
+    const uint32_t count = uniform(p.batchItems ? V.nBatches : V.nItems);
+    J.itemBegin = first;
+    J.itemEnd = first + count;
+    J.bX = int(uniform(V.bX));
+    J.bY = int(uniform(V.bY));
+    J.tX = t % tilesX;
+    J.tY = t / tilesX;
     J.recs = p.recs;
     J.groupBox = p.groupBox;
-    J.depth = V.depth;
-    J.hiz = V.hiz;
-    J.tileMin = V.tileMin;
-    J.pyrX = V.pyrX;
+    J.depth = uniform(V.depth);
+    J.hiz = uniform(V.hiz);
+    J.tileMin = uniform(V.tileMin);
+    J.pyrX = uniform(V.pyrX);
     J.done = p.done;
     J.err = p.err;
     J.timeoutTicks = p.timeoutTicks;
-    J.winner = V.winner;
+    J.winner = uniform(V.winner);
     J.labels = p.labels;
-    J.list = p.lists ? p.lists + V.listBase + size_t(t) * (J.itemEnd - J.itemBegin) : nullptr;
-    J.listLen = p.lists ? p.listLen[unit] : 0u;
+    J.list = p.lists ? p.lists + uniform(V.listBase) + size_t(t) * count : nullptr;
+    J.listLen = p.lists ? uniform(p.listLen[unit]) : 0u;
     process_tile<TBX, TBY, NW, STATS, LABELS>(J, sm, p.cov, covLoaded, ctr);
     __syncthreads();
   }
