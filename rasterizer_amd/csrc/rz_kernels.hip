@@ -1345,6 +1345,40 @@ __device__ __forceinline__ bool quad_touches_tile(const RecWords& R, int tbx0, i
   return !misses;
 }
 
+// Whether every block that a quad may write in the tile already rejects it (hiZ
+// at or above its largest depth), for a quad of at most kHiddenBlocks blocks in
+// the tile.  Only blocks with hiZ >= 2 count: their minimum only grows, so they
+// still reject it at its turn (a block at hiZ 0 could come to read as cleared).
+// Where most quads are hidden this spares them the staging and the draw's two
+// phases: a 4K frame of 12,000 icospheres 0.70 ms without, 0.50 ms with it.
+constexpr int kHiddenBlocks = 64;
+template <int TBX, int TBY>
+__device__ __forceinline__ bool quad_hidden(const RecWords& R, const TileSmem<TBX, TBY>& sm, int tbx0, int tbx1,
+                                            int tby0, int tby1, int bX, float invBX) {
+  const int fb = int(R.w[3].w), rangeX = int(R.w[4].x & 0xFFFFu), rangeY = int(R.w[4].x >> 16);
+  const uint32_t maxZ = R.w[4].y >> 16;
+  const int minY = div_bx(fb, bX, invBX), minX = fb - minY * bX;
+  const int x0 = max(tbx0, minX) - tbx0, x1 = min(tbx1, minX + rangeX - 1) - tbx0;
+  const int y0 = max(tby0, minY) - tby0, y1 = min(tby1, minY + rangeY - 1) - tby0;
+  const int n = (x1 - x0 + 1) * (y1 - y0 + 1);
+  if (minX + rangeX > bX || n > kHiddenBlocks) return false;
+  bool open = false;
+  int x = x0, lb = y0 * TBX + x0;
+  for (int i = 0; i < n && !open; i += 4) {
+    uint32_t hz[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      hz[j] = i + j < n ? uint32_t(sm.hiz[lb]) : 0xFFFFu;
+      const bool wrap = x == x1;
+      lb += wrap ? TBX - (x1 - x0) : 1;
+      x = wrap ? x0 : x + 1;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) open |= hz[j] < 2u || hz[j] < maxZ;
+  }
+  return !open;
+}
+
 // Tile-overlap tests shared by the prep kernel's tile count and the frame
 // kernel (they must agree exactly).
 template <int TBX, int TBY>
@@ -1466,6 +1500,7 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
   BlockCounters bc;
   uint32_t rPar = 0, wPar = 0;
   uint32_t fill = 0;  // quads staged in sm.recs and not yet drawn
+  bool drew = false;  // before the first draw there is little to hide a quad
   // The window's current block of 64 slots: the lane's item, its flags and the
   // groups it is drawn with; masks of the items with a share of query2D in the
   // tile, with quads in it and with quads in it that need a decision.
@@ -1707,8 +1742,11 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
               g = uint32_t(__builtin_ctzll(__ballot(set && rank == j)));
             }
             quad = ((first >> 6) + g) * 64u + lane;
-            if (quad >= first && quad < past)
-              hit = quad_touches_tile(load_rec(&J.recs[quad]), tbx0, tbx1, tby0, tby1, bX, invBX);
+            if (quad >= first && quad < past) {
+              const RecWords rec = load_rec(&J.recs[quad]);
+              hit = quad_touches_tile(rec, tbx0, tbx1, tby0, tby1, bX, invBX) &&
+                    !(drew && quad_hidden<TBX, TBY>(rec, sm, tbx0, tbx1, tby0, tby1, bX, invBX));
+            }
           }
           const uint64_t hm = __ballot(hit);
           const uint32_t hpre =
@@ -1740,6 +1778,7 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
           const uint64_t tB = draw_chunk<TBX, TBY, NW, STATS, LABELS>(sm, n, tbx0, tbx1, tby0, tby1, bX, invBX, wave,
                                                                       lane, bc, J.winner);
           fill = 0;
+          drew = true;
           tried = 0;  // the tile's state changed: early evaluations that failed may now succeed
           if (STATS && tid == 0) ctr[kStatQuads] += n;
           __syncthreads();

@@ -71,3 +71,27 @@ def test_rounds_match_oracle(oracle_mod, report, n, tile_w, waves):
     v.draw_frame(items, gated=False)
     want = v.raw()
     assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0])
+
+
+@pytest.mark.parametrize("tile_w", [8, 16])
+@pytest.mark.parametrize("low", [0, 1, 2, 3, 40000])
+def test_quads_behind_what_is_there(oracle_mod, report, low, tile_w):
+    """Small quads over a buffer whose blocks' smallest depth is 0, 1 (which
+    reads as cleared), 2, 3 or nearer than most of them, drawn after others: the
+    tests that leave out quads that every block rejects."""
+    rng = np.random.default_rng(low)
+    occ = _occluders(300, rng)
+    mvp = scenes.view_projection((0.0, 0.0, 0.0), np.array([0.0, 0.0, 1.0]), (0, 1, 0), math.pi / 8, W / H)
+    depth = rng.integers(low, 50000, (W // 8 * (H // 8), 64)).astype(np.uint16)
+    depth[:, 0] = low
+    hiz = np.concatenate([depth.min(axis=1), np.zeros(8, np.uint16)]).astype(np.uint16)
+    g, o = Rasterizer(W, H), oracle_mod.OracleRasterizer(W, H)
+    g.set_config(tile_w, 8)
+    g.upload_raw(depth, hiz)
+    o.set_raw(depth, hiz)
+    for r in (g, o):
+        r.setModelViewProjection(mvp)
+    assert np.array_equal(g.draw_frame(occ), o.draw_frame(occ))
+    (dg, hg), (do, ho) = g.raw(), o.raw()
+    assert np.array_equal(hg, ho), f"hiZ {report(hg, ho)}"
+    assert np.array_equal(dg, do), f"depth {report(dg, do)}"
