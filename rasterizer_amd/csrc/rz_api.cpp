@@ -485,9 +485,11 @@ static void fill_items(ItemDesc* items, uint32_t n, const rz_occluder* const* oc
 // Enqueues the prep, setup and frame kernels of one draw whose item
 // descriptors are already in b.items (or enqueued before them), or, with
 // hostItems, in mapped host memory from which prep copies them to b.items.
-// prof: optional event quadruple (prep, setup, frame, end).
+// prof: optional event quadruple (prep, setup, frame, end).  gated: items may
+// wait for other tiles' answers, so the tiles must be co-resident whatever else
+// runs: a cooperative launch, which takes about 18 us more than a plain one.
 static int enqueue_kernels(rz_context* c, uint32_t n, uint32_t totalQuads, const DrawBufs& b, hipEvent_t* prof,
-                           const ItemDesc* hostItems = nullptr) {
+                           bool gated, const ItemDesc* hostItems = nullptr) {
   if (prof) RZ_HIP(hipEventRecord(prof[0], c->stream));
   PrepParams pp{};
   pp.items = b.items;
@@ -543,7 +545,7 @@ static int enqueue_kernels(rz_context* c, uint32_t n, uint32_t totalQuads, const
   fp.tileMin = c->d_tileMin;
   fp.pyrX = c->pyrX;
   fp.stats = c->d_frameStats;
-  RZ_HIP(launch_frame(fp, c->tileW, c->stream, c->cooperative, c->waves));
+  RZ_HIP(launch_frame(fp, c->tileW, c->stream, c->cooperative && gated, c->waves));
   if (prof) RZ_HIP(hipEventRecord(prof[3], c->stream));
   return RZ_OK;
 }
@@ -598,7 +600,8 @@ static int enqueue_draw(rz_context* c, uint32_t n, const rz_occluder* const* occ
   fill_items(c->h_items[slot], n, occ, kinds);
   const DrawBufs bufs{c->d_items, c->d_state,    c->d_done,     c->d_visible,
                       c->d_recs,  c->d_bbox,     c->d_groupBox, c->d_groupItem};
-  s = enqueue_kernels(c, n, uint32_t(totalQuads), bufs, profile_slot(c, 0), c->d_hItems[slot]);
+  // Items of given kinds (rz_rasterize) are drawn without a query.
+  s = enqueue_kernels(c, n, uint32_t(totalQuads), bufs, profile_slot(c, 0), kinds == nullptr, c->d_hItems[slot]);
   if (s != RZ_OK) return s;
   if (d % kDrawsPerEvent == kDrawsPerEvent - 1)
     RZ_HIP(hipEventRecord(c->ev_items[(d / kDrawsPerEvent) & 1], c->stream));
@@ -694,7 +697,7 @@ extern "C" int rz_draw_frame_noalloc(rz_context* ctx, uint32_t n, const rz_occlu
   // The prep kernel writes every state, done and visibility word of items
   // 0..n-1 and the setup kernel every record and box of their quads, so
   // nothing left in scratch by an earlier call is read.
-  s = enqueue_kernels(ctx, n, uint32_t(totalQuads), bufs, nullptr);
+  s = enqueue_kernels(ctx, n, uint32_t(totalQuads), bufs, nullptr, true);
   if (s != RZ_OK) return s;
   if (d_statusOut) RZ_HIP(launch_status(bufs.state, bufs.done, n, d_statusOut, ctx->stream));
   return RZ_OK;
