@@ -118,6 +118,7 @@ struct FrameParams {
   const QuadRec* recs;
   const uint64_t* bbox;
   const uint64_t* groupBox;
+  const uint64_t* itemBox;  // optional (launch_item_boxes): what each item may touch
   uint32_t* done;
   uint32_t* visible;
   uint16_t* depth;
@@ -188,6 +189,9 @@ struct QueryParams {
 // Launchers (defined with the kernels); all enqueue on `stream`.
 hipError_t launch_prep(const PrepParams& p, hipStream_t stream);
 hipError_t launch_setup(const SetupParams& p, hipStream_t stream);
+// Box of the blocks that item i's query rectangle and quads touch, after setup:
+// u16 min column, max column, min row, max row (empty: 0xFFFF, 0, 0, 0).
+hipError_t launch_item_boxes(const ItemState* state, uint32_t n, uint64_t* out, hipStream_t stream);
 // tileW x tileH must be 8x8 or 16x16; the grid is tilesX * tilesY
 // cooperative work-groups.
 // cooperative == false launches the same grid as a plain dispatch (for tools

@@ -1427,6 +1427,7 @@ struct TileJob {
   uint32_t tX, tY;
   const QuadRec* recs;
   const uint64_t* groupBox;
+  const uint64_t* itemBox;  // optional: what each item may touch
   uint16_t* depth;
   uint16_t* hiz;
   uint16_t* tileMin;
@@ -1443,7 +1444,9 @@ struct TileJob {
 // LABELS (8x8-block tiles): the draw tracks each pixel's winning batch, and
 // once the tile is final every written block adds one to the label of each
 // distinct batch that wins one of its pixels.
-template <int TBX, int TBY, int NW, bool STATS, bool LABELS>
+//
+// BOXED: with item boxes (TileJob::itemBox), which a thread tests four at a time.
+template <int TBX, int TBY, int NW, bool STATS, bool LABELS, bool BOXED>
 __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY>& sm,
                                              const uint64_t* __restrict__ cov, bool& covLoaded,
                                              uint64_t (&ctr)[kFrameStatWords]) {
@@ -1473,7 +1476,13 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
   constexpr uint32_t NT = 64u * NW;
   constexpr uint32_t kItemWindow = TileSmem<TBX, TBY>::kItemWindow;
   static_assert(NT >= kItemWindow, "the item window gathers one item per thread");
+  constexpr uint32_t kPerThread = BOXED ? 4 : 1;
   if (J.list) involved = nList > 0u;
+  else if (BOXED)
+    for (uint32_t i = 4u * tid; i < nList && !involved; i += 4u * NT)
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j)
+        involved |= i + j < nList && box_touches(J.itemBox[J.itemBegin + i + j], tbx0, tbx1, tby0, tby1);
   else
     for (uint32_t i = J.itemBegin + tid; i < J.itemEnd && !involved; i += NT) involved = relevance(i) != 0u;
   if (!__syncthreads_or(involved)) return;
@@ -1517,29 +1526,52 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
   const uint64_t tLoop = stamp();
   for (uint32_t wbase = 0; wbase < nList;) {
     // Gather this window's items that touch the tile, in draw order: every
-    // thread tests one candidate, the first kItemWindow relevant ones are
-    // kept, and the next window starts at the first relevant candidate not
-    // kept (or after the last candidate tested).
-    const bool inWin = wbase + tid < nList;
-    const uint32_t i = inWin ? item_at(wbase + tid) : 0u;
-    const uint32_t rel = inWin ? relevance(i) : 0u;
-    const uint64_t m = __ballot(rel != 0u);
-    const uint32_t pre = __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
-    if (lane == 0) sm.wcnt[wPar][wave] = uint32_t(__popcll(m));
-    if (tid == 0) sm.wnext = min(wbase + NT, nList);
+    // thread tests one candidate (four in turn with item boxes, of which few
+    // touch the tile), the first kItemWindow relevant ones are kept, and the
+    // next window starts at the first relevant candidate not kept (or after the
+    // last candidate tested).
+    const uint32_t pos0 = wbase + kPerThread * tid;
+    uint32_t rels = 0, count = 0;  // four bits a candidate
+#pragma unroll
+    for (uint32_t j = 0; j < kPerThread; ++j) {
+      uint32_t rel = 0;
+      if (pos0 + j < nList &&
+          (!BOXED || box_touches(J.itemBox[J.itemBegin + pos0 + j], tbx0, tbx1, tby0, tby1)))
+        rel = relevance(item_at(pos0 + j));
+      rels |= rel << (4 * j);
+      count += rel != 0u;
+    }
+    uint32_t off, sum;  // relevant candidates of the lanes before this one, and of the wave
+    if constexpr (BOXED) {
+      off = __ockl_wfscan_add_u32(count, true);
+      sum = readlane_u(off, 63u);
+      off -= count;
+    } else {
+      const uint64_t m = __ballot(rels != 0u);
+      off = __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
+      sum = uint32_t(__popcll(m));
+    }
+    if (lane == 0) sm.wcnt[wPar][wave] = sum;
+    if (tid == 0) sm.wnext = min(wbase + kPerThread * NT, nList);
     __syncthreads();
-    uint32_t off = 0, nRel = 0;
+    uint32_t nRel = 0;
 #pragma unroll
     for (uint32_t w = 0; w < NW; ++w) {
       off += w < wave ? sm.wcnt[wPar][w] : 0u;
       nRel += sm.wcnt[wPar][w];
     }
     wPar ^= 1u;
-    if (rel && off + pre == kItemWindow) sm.wnext = wbase + tid;
     nRel = min(nRel, kItemWindow);
-    if (rel && off + pre < kItemWindow) {
+    for (uint32_t j = 0; j < kPerThread; ++j) {
+      const uint32_t rel = (rels >> (4 * j)) & 15u;
+      if (!rel) continue;
+      if (off >= kItemWindow) {
+        if (off == kItemWindow) sm.wnext = pos0 + j;
+        break;
+      }
+      const uint32_t i = item_at(pos0 + j);
       const ItemState& S = J.state[i];
-      ItemLocal& L = sm.items[off + pre];
+      ItemLocal& L = sm.items[off++];
       L.index = i;
       L.flags = rel | S.expected << 16;
       L.qMinX = S.qMinX;
@@ -1858,7 +1890,7 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
 
 // Two work-groups per CU, as the multi-view kernel (at most 128 VGPRs with
 // eight waves per group).
-template <int TBX, int TBY, int NW, bool STATS>
+template <int TBX, int TBY, int NW, bool STATS, bool BOXED>
 __global__ void __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) rz_frame_kernel(FrameParams p) {
   __shared__ TileSmem<TBX, TBY> sm;
   // Observability counters, kept in LDS by thread 0 (unused unless STATS).
@@ -1876,6 +1908,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) rz_frame_kernel(Fram
   J.tY = blockIdx.x / p.tilesX;
   J.recs = p.recs;
   J.groupBox = p.groupBox;
+  J.itemBox = p.itemBox;
   J.depth = p.depth;
   J.hiz = p.hiz;
   J.tileMin = p.tileMin;
@@ -1888,7 +1921,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) rz_frame_kernel(Fram
   J.list = nullptr;
   J.listLen = 0;
   bool covLoaded = false;
-  process_tile<TBX, TBY, NW, STATS, false>(J, sm, p.cov, covLoaded, ctr);
+  process_tile<TBX, TBY, NW, STATS, false, BOXED>(J, sm, p.cov, covLoaded, ctr);
   if (STATS && threadIdx.x == 0) {
     ctr[kStatTotalTicks] = __builtin_amdgcn_s_memrealtime() - tEntry;
     for (int k = 0; k < kFrameStatWords; ++k) p.stats[size_t(blockIdx.x) * kFrameStatWords + k] = ctr[k];
@@ -1953,6 +1986,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) rz_views_kernel(View
     J.tY = t / tilesX;
     J.recs = p.recs;
     J.groupBox = p.groupBox;
+    J.itemBox = nullptr;
     J.depth = uniform(V.depth);
     J.hiz = uniform(V.hiz);
     J.tileMin = uniform(V.tileMin);
@@ -1964,7 +1998,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 4 : 2) rz_views_kernel(View
     J.labels = p.labels;
     J.list = p.lists ? p.lists + uniform(V.listBase) + size_t(t) * count : nullptr;
     J.listLen = p.lists ? uniform(p.listLen[unit]) : 0u;
-    process_tile<TBX, TBY, NW, STATS, LABELS>(J, sm, p.cov, covLoaded, ctr);
+    process_tile<TBX, TBY, NW, STATS, LABELS, false>(J, sm, p.cov, covLoaded, ctr);
     __syncthreads();
   }
   if (STATS) {
@@ -2031,6 +2065,29 @@ __global__ void __launch_bounds__(256) rz_views_gather_kernel(ViewsParams p, con
   const uint32_t src = p.views[v].unitBase;
   for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) p.unitList[off + k] = unitTmp[src + k];
   if (v == p.nViews - 1 && threadIdx.x == 0) *p.nActive = off + n;
+}
+
+__global__ void __launch_bounds__(256) rz_item_boxes_kernel(const ItemState* __restrict__ state, uint32_t n,
+                                                            uint64_t* __restrict__ out) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const ItemState& S = state[i];
+  uint32_t c0 = 0xFFFFu, c1 = 0u, r0 = 0xFFFFu, r1 = 0u;
+  if (S.status != kStatusSkip) {
+    if (S.fp[0] <= S.fp[1]) {
+      c0 = S.fp[0];
+      c1 = S.fp[1];
+      r0 = S.fp[2];
+      r1 = S.fp[3];
+    }
+    if (S.status == kStatusTest) {
+      c0 = min(c0, S.qMinX >> 3);
+      c1 = max(c1, S.qMaxX >> 3);
+      r0 = min(r0, S.qMinY >> 3);
+      r1 = max(r1, S.qMaxY >> 3);
+    }
+  }
+  out[i] = c0 <= c1 ? uint64_t(c0) | uint64_t(c1) << 16 | uint64_t(r0) << 32 | uint64_t(r1) << 48 : kEmptyBox;
 }
 
 // Per item of a multi-view launch, the box in 8x8-block tiles (u16 x0, x1,
@@ -2534,21 +2591,22 @@ hipError_t launch_setup(const SetupParams& p, hipStream_t stream) {
 }
 
 template <int T, int NW>
-static const void* frame_fn(bool stats) {
-  return stats ? reinterpret_cast<const void*>(&rz_frame_kernel<T, T, NW, true>)
-               : reinterpret_cast<const void*>(&rz_frame_kernel<T, T, NW, false>);
+static const void* frame_fn(bool stats, bool boxed) {
+  return stats ? reinterpret_cast<const void*>(&rz_frame_kernel<T, T, NW, true, false>)
+         : boxed ? reinterpret_cast<const void*>(&rz_frame_kernel<T, T, NW, false, true>)
+                 : reinterpret_cast<const void*>(&rz_frame_kernel<T, T, NW, false, false>);
 }
 
-static const void* frame_kernel_fn(int tileW, int waves, bool stats) {
+static const void* frame_kernel_fn(int tileW, int waves, bool stats, bool boxed) {
   if (tileW == 8)
-    return waves == 8 ? frame_fn<8, 8>(stats)
-           : waves == 4 ? frame_fn<8, 4>(stats)
-           : waves == 2 ? frame_fn<8, 2>(stats)
+    return waves == 8 ? frame_fn<8, 8>(stats, boxed)
+           : waves == 4 ? frame_fn<8, 4>(stats, boxed)
+           : waves == 2 ? frame_fn<8, 2>(stats, boxed)
                         : nullptr;
   if (tileW == 16)
-    return waves == 8 ? frame_fn<16, 8>(stats)
-           : waves == 4 ? frame_fn<16, 4>(stats)
-           : waves == 2 ? frame_fn<16, 2>(stats)
+    return waves == 8 ? frame_fn<16, 8>(stats, boxed)
+           : waves == 4 ? frame_fn<16, 4>(stats, boxed)
+           : waves == 2 ? frame_fn<16, 2>(stats, boxed)
                         : nullptr;
   return nullptr;
 }
@@ -2575,7 +2633,8 @@ hipError_t launch_frame(const FrameParams& p, int tileW, hipStream_t stream, boo
   FrameParams local = p;
   void* args[] = {&local};
   const dim3 grid(p.tilesX * p.tilesY), block(64 * waves);
-  const void* fn = frame_kernel_fn(tileW, waves, p.stats != nullptr);
+  // The counting variant tests every item's record.
+  const void* fn = frame_kernel_fn(tileW, waves, p.stats != nullptr, p.itemBox != nullptr);
   if (!fn) return hipErrorInvalidValue;
   return launch_coresident(fn, grid, block, args, stream, cooperative);
 }
@@ -2587,8 +2646,8 @@ hipError_t frame_max_groups(int tileW, int waves, int* maxGroups) {
   e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   if (e != hipSuccess) return e;
   int perCU = 1 << 30;
-  for (bool stats : {false, true}) {
-    const void* fn = frame_kernel_fn(tileW, waves, stats);
+  for (int variant = 0; variant < 3; ++variant) {
+    const void* fn = frame_kernel_fn(tileW, waves, variant == 1, variant == 2);
     if (!fn) return hipErrorInvalidValue;
     int n = 0;
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, 64 * waves, 0);
@@ -2597,6 +2656,12 @@ hipError_t frame_max_groups(int tileW, int waves, int* maxGroups) {
   }
   *maxGroups = perCU * cus;
   return hipSuccess;
+}
+
+hipError_t launch_item_boxes(const ItemState* state, uint32_t n, uint64_t* out, hipStream_t stream) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(rz_item_boxes_kernel, dim3(groups(n, 256)), dim3(256), 0, stream, state, n, out);
+  return hipGetLastError();
 }
 
 hipError_t launch_status(const ItemState* state, const uint32_t* visible, uint32_t n, uint8_t* out,

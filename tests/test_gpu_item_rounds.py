@@ -95,3 +95,24 @@ def test_quads_behind_what_is_there(oracle_mod, report, low, tile_w):
     (dg, hg), (do, ho) = g.raw(), o.raw()
     assert np.array_equal(hg, ho), f"hiZ {report(hg, ho)}"
     assert np.array_equal(dg, do), f"depth {report(dg, do)}"
+
+
+@pytest.mark.parametrize("tile_w,waves", [(8, 8), (16, 8), (16, 2)])
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 4300])
+def test_many_items(oracle_mod, report, n, tile_w, waves):
+    """Around the number of items from which a tile tests their boxes, four a
+    thread, with most of them outside any one tile."""
+    rng = np.random.default_rng(n)
+    kinds = _occluders(40, rng)
+    occ = [kinds[i] for i in rng.integers(0, len(kinds), n)]
+    occ[::50] = occ[: len(occ[::50])]
+    mvp = scenes.view_projection((0.0, 0.0, 0.0), np.array([0.0, 0.0, 1.0]), (0, 1, 0), math.pi / 8, 4 * W / H)
+    g, o = Rasterizer(4 * W, H), oracle_mod.OracleRasterizer(4 * W, H)
+    g.set_config(tile_w, waves)
+    for r in (g, o):
+        r.clear()
+        r.setModelViewProjection(mvp)
+    assert np.array_equal(g.draw_frame(occ), o.draw_frame(occ))
+    (dg, hg), (do, ho) = g.raw(), o.raw()
+    assert np.array_equal(hg, ho), f"hiZ {report(hg, ho)}"
+    assert np.array_equal(dg, do), f"depth {report(dg, do)}"
