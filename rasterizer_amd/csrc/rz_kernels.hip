@@ -248,15 +248,17 @@ __device__ bool query2d_wave(uint32_t minX, uint32_t maxX, uint32_t minY, uint32
 //     blocks: a candidate tile's 64 hiZ values are one load per row and lane,
 //     all in flight together, and only where no interior block is open do the
 //     blocks at the rectangle's border read their pixels.
-//   - Wider rectangles take the whole wave, one after another.
+//   - Wider rectangles take the whole wave, one after another; so do all with
+//     WHOLE.
 // Bound by latency (box, reciprocal table, tile minima, hiZ, pixels in turn)
 // and instructions: a city query's rectangle has some tens of blocks, so a
 // whole wave for each box in turn left most lanes idle.  A batch of 1,000,003
 // city boxes, together with launch_query's rule: 180 us before, 28 us now.
+template <bool WHOLE>
 __device__ bool query2d_boxes(const QueryPre& Q, bool test, const QueryBufs& B, uint32_t lane) {
   const uint32_t tx0 = Q.minX >> 6, ty0 = Q.minY >> 6;
   const uint32_t ntx = (Q.maxX >> 6) - tx0 + 1, nty = (Q.maxY >> 6) - ty0 + 1;
-  const bool narrow = test && ntx <= 4u && nty <= 4u;
+  const bool narrow = !WHOLE && test && ntx <= 4u && nty <= 4u;
   bool vis = false;
   uint32_t cand = 0;  // bit 4 y + x: tile (tx0 + x, ty0 + y) may hold an open block
   if (narrow) {
@@ -2196,8 +2198,8 @@ __global__ void rz_status_kernel(const ItemState* __restrict__ state, const uint
 // queryVisibility (Rasterizer.cpp:123-281) of a batch: lanes 0..BPW-1 of a
 // wave each take one box for the depth-independent part (projection,
 // frustum, near plane, rectangle), then the wave runs query2D for those that
-// need it (query2d_boxes).  launch_query chooses BPW.
-template <uint32_t BPW>
+// need it (query2d_boxes).  launch_query chooses BPW and WHOLE.
+template <uint32_t BPW, bool WHOLE>
 __global__ void __launch_bounds__(256) rz_query_kernel(QueryParams p) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t q = ((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * BPW + lane;
@@ -2211,7 +2213,7 @@ __global__ void __launch_bounds__(256) rz_query_kernel(QueryParams p) {
   }
   const uint32_t clip = Q.kind == 1 ? 1u : 0u;
   const QueryBufs B = {p.depth, p.hiz, p.tileMin, p.bX, p.pyrX};
-  const uint32_t vis = query2d_boxes(Q, valid && Q.kind == 3, B, lane) ? 1u : clip;
+  const uint32_t vis = query2d_boxes<WHOLE>(Q, valid && Q.kind == 3, B, lane) ? 1u : clip;
   if (valid) {
     p.visible[q] = uint8_t(vis);
     if (p.needsClipping) p.needsClipping[q] = uint8_t(clip);
@@ -2262,7 +2264,7 @@ __global__ void __launch_bounds__(256) rz_views_query_kernel(ViewsQueryParams p)
   }
   const uint32_t clip = Q.kind == 1 ? 1u : 0u;
   const QueryBufs B = {V.depth, V.hiz, V.tileMin, V.bX, V.pyrX};
-  const uint32_t vis = query2d_boxes(Q, valid && Q.kind == 3, B, lane) ? 1u : clip;
+  const uint32_t vis = query2d_boxes<false>(Q, valid && Q.kind == 3, B, lane) ? 1u : clip;
   if (valid) {
     V.queryVisible[k] = uint8_t(vis);
     V.queryClip[k] = uint8_t(clip);
@@ -2673,20 +2675,28 @@ hipError_t launch_status(const ItemState* state, const uint32_t* visible, uint32
 
 hipError_t launch_query(const QueryParams& p, hipStream_t stream) {
   if (p.n == 0) return hipSuccess;
-  // As many boxes per wave as fill the chip's 8,192 wave slots once: fewer leave
-  // most lanes of the projection idle, more leave slots idle and make longer
-  // waves.  Device batches of city boxes over the 1080p buffer, us per call
-  // with 8 / 16 / 32 / 64 boxes per wave: 65,536 boxes 16.3 / 17.1 / 18.6 /
-  // 19.1, 131,072 boxes 20.5 / 17.6 / 18.4 / 19.4, 262,144 boxes 32.8 / 21.8 /
-  // 17.8 / 19.8, 1,000,003 boxes 106 / 64 / 40 / 28 (four: 18, 29, 50, 182).
+  // Small batches leave wave slots (8,192) idle: a wave a box or four, each with
+  // the whole wave, is the shortest chain.  Larger ones get as many boxes per
+  // wave as fill the slots once, eight rectangles at a time: fewer leave most
+  // lanes of the projection idle, more leave slots idle and make longer waves.
+  // Device batches of city boxes over the 1080p buffer, us per call:
+  //   boxes      1 whole  4 whole  8 boxes  16    32    64
+  //   1,000      7.7      8.3      12.7
+  //   8,192      9.2      8.0      12.6
+  //   32,768     16.8     10.7     12.9
+  //   65,536     27       15.9     15.9     17    19    19
+  //   131,072    48       25       20.5     17.6  18.4  19.4
+  //   262,144                      33       22    18    20
+  //   1,000,003                    106      64    40    28
   constexpr uint32_t kWaves = 8192;
   auto go = [&](auto kernel, uint32_t bpw) {
     hipLaunchKernelGGL(kernel, dim3(groups(groups(p.n, bpw), 4)), dim3(256), 0, stream, p);
   };
-  if (p.n <= 8 * kWaves) go(rz_query_kernel<8>, 8);
-  else if (p.n <= 16 * kWaves) go(rz_query_kernel<16>, 16);
-  else if (p.n <= 32 * kWaves) go(rz_query_kernel<32>, 32);
-  else go(rz_query_kernel<64>, 64);
+  if (p.n <= kWaves / 2) go(rz_query_kernel<1, true>, 1);
+  else if (p.n <= 8 * kWaves) go(rz_query_kernel<4, true>, 4);
+  else if (p.n <= 16 * kWaves) go(rz_query_kernel<16, false>, 16);
+  else if (p.n <= 32 * kWaves) go(rz_query_kernel<32, false>, 32);
+  else go(rz_query_kernel<64, false>, 64);
   return hipGetLastError();
 }
 

@@ -48,7 +48,7 @@ def test_batches_match_oracle(oracle_mod, open_share):
             assert np.array_equal(got, want), f"{n} boxes: {int((got != want).sum())} differ"
 
 
-@pytest.mark.parametrize("n", [65536, 65537, 131072, 131073, 262144, 262145])
+@pytest.mark.parametrize("n", [4096, 4097, 65536, 65537, 131072, 131073, 262144, 262145])
 def test_share_of_boxes(oracle_mod, n):
     """The same boxes over and over: every wave of a large batch answers them as
     a small one does."""
