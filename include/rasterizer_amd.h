@@ -292,7 +292,8 @@ int rz_profile_read(rz_context* ctx, double ms[4], uint32_t counts[2]);
  * counting variant of the kernel.  rz_frame_stats_read blocks and copies
  * tilesX*tilesY records of 22 u64 into out (when out is non-NULL and *count
  * is large enough) and sets *count to the number of records: total ticks,
- * ticks waiting on other tiles, waits, ticks in local query2D work, query2D
+ * ticks waiting on other tiles, waits (items undecided when the tile reached
+ * them), ticks in local query2D work, query2D
  * contributions, ticks drawing (scan + draw), quads drawn, items touching the
  * tile, scan ticks, scan passes, tile load ticks, item-loop ticks, draw
  * ticks, (quad, block) pairs visited, of which rejected, of which written,

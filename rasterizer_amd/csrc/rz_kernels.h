@@ -135,14 +135,14 @@ struct FrameParams {
 enum FrameStat : int {
   kStatTotalTicks = 0,   // kernel entry to exit
   kStatWaitTicks = 1,    // spinning on another tile's query contribution
-  kStatWaits = 2,
+  kStatWaits = 2,        // items undecided when the tile reached them
   kStatQueryTicks = 3,   // local query2D contributions
   kStatQueries = 4,
   kStatRasterTicks = 5,  // quad list build + block loop
   kStatQuads = 6,        // quads drawn into this tile
   kStatItems = 7,        // items touching this tile
   kStatScanTicks = 8,    // overlap tests and quad compaction
-  kStatPasses = 9,       // 256-quad scan passes run
+  kStatPasses = 9,       // scan passes run (one 64-quad group a wave)
   kStatLoadTicks = 10,   // table, depth and hiZ staging at entry
   kStatLoopTicks = 11,   // the whole item loop
   kStatDrawTicks = 12,   // staged-quad drawing (inside raster ticks)

@@ -9,9 +9,10 @@
 //                    the tile's depth and hiZ live in LDS; items are walked in
 //                    draw order; a query2D is reduced across the tiles that
 //                    overlap its rectangle with device atomics, so each item
-//                    is drawn exactly when the reference would draw it.  One
-//                    wave64 works on one 8x8 block at a time with lane = pixel
-//                    (Rasterizer.cpp:1095-1292).
+//                    is drawn exactly when the reference would draw it.  A wave64
+//                    takes 64 (quad, block) pairs at a time, a lane each, for
+//                    their coverage, then one 8x8 block at a time with lane =
+//                    pixel (Rasterizer.cpp:1095-1292).
 #include "rz_kernels.h"
 
 #include <hip/hip_runtime.h>
@@ -1419,8 +1420,7 @@ constexpr uint32_t kDoneVisibleOne = 0x10000u;
 // walked in draw order against the tile's depth and hiZ held in LDS, then the
 // tile is written back.  Shared by the single-view frame kernel (one
 // work-group per tile, gated query items) and the multi-view persistent
-// kernel (work-groups take (view, tile) units from a queue; items are never
-// gated, so no tile waits on another).
+// kernel (work-groups take (view, tile) units from a queue).
 struct TileJob {
   const ItemDesc* items;
   const ItemState* state;
