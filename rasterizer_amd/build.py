@@ -84,18 +84,20 @@ def build(verbose: bool = False) -> Path:
             *[str(BUILD / n) for n in objs], "-lpthread"]
     _run_all([link])
     os.replace(tmp, LIB)
-    # Test programs of the C++ drop-in headers (run by tests/test_gpu_sah.py
-    # and tests/test_gpu_dropin.py).
+    # Test programs: of the C++ drop-in headers (run by tests/test_gpu_sah.py
+    # and tests/test_gpu_dropin.py), and of the host side with a HIP runtime of
+    # its own (tests/test_host_runtime.py).
     bindir = ROOT / "tests" / "_bin"
     progs = []
-    for name in ("sah_dropin_check", "main_sequence_check"):
+    extra = {"host_runtime_check": ["-rdynamic", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{CSRC}"]}
+    for name in ("sah_dropin_check", "main_sequence_check", "host_runtime_check"):
         src = ROOT / "tests" / "cpp" / f"{name}.cpp"
         if src.exists():
             bindir.mkdir(exist_ok=True)
             progs.append(["g++", "-O2", "-std=c++17", "-msse4.1", f"-I{ROOT / 'include' / 'rasterizer_amd'}",
                           f"-I{ROOT / 'include'}", str(src), f"-L{LIBDIR}", "-lrasterizer_amd",
                           "-Wl,-rpath,$ORIGIN/../../rasterizer_amd/_lib", "-Wl,-rpath,/opt/rocm/lib",
-                          "-o", str(bindir / name)])
+                          *extra.get(name, []), "-o", str(bindir / name)])
     if progs:
         _run_all(progs)
     return LIB

@@ -186,6 +186,26 @@ static void free_context(rz_context* c) {
 
 static int noalloc_init(int device);
 
+// Pinned host memory that kernels read and write through *dev; coherent
+// (fine-grained), so that nothing of an earlier use is in a cache.
+template <typename T>
+static int host_alloc(T** host, T** dev, size_t count) {
+  *host = *dev = nullptr;
+  void* h = nullptr;
+  if (hipHostMalloc(&h, count * sizeof(T), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+    (void)hipGetLastError();
+    return RZ_ERR_OUT_OF_MEMORY;
+  }
+  void* d = nullptr;
+  if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+    (void)hipHostFree(h);
+    return RZ_ERR_DEVICE;
+  }
+  *host = static_cast<T*>(h);
+  *dev = static_cast<T*>(d);
+  return RZ_OK;
+}
+
 extern "C" int rz_create(uint32_t width, uint32_t height, rz_context** out) {
   if (!out) return RZ_ERR_INVALID_ARGUMENT;
   *out = nullptr;
@@ -225,6 +245,12 @@ extern "C" int rz_create(uint32_t width, uint32_t height, rz_context** out) {
       hipMemcpy(c->d_cov, tabs.covLanes, sizeof tabs.covLanes, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(c->d_rcp, tabs.rcp, sizeof tabs.rcp, hipMemcpyHostToDevice) != hipSuccess)
     return fail(RZ_ERR_DEVICE);
+  // Here, and not where it is first used: the blocking calls of a program that
+  // may not allocate any more (rz_draw_frame_noalloc) must not either, and must
+  // wait for the stream whatever happens.
+  const int words = host_alloc(&c->h_words, &c->words.out, 2);
+  if (words != RZ_OK) return fail(words);
+  c->words.err = c->d_err;
 
   // Pick the smallest tile whose grid fits co-resident on this device.
   bool placed = false;
@@ -340,33 +366,6 @@ extern "C" int rz_occluder_destroy(rz_occluder* o) {
   hipFree(o->d_packets);
   delete o;
   return RZ_OK;
-}
-
-// Pinned host memory that kernels read and write through *dev; coherent
-// (fine-grained), so that nothing of an earlier use is in a cache.
-template <typename T>
-static int host_alloc(T** host, T** dev, size_t count) {
-  *host = *dev = nullptr;
-  void* h = nullptr;
-  if (hipHostMalloc(&h, count * sizeof(T), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
-    (void)hipGetLastError();
-    return RZ_ERR_OUT_OF_MEMORY;
-  }
-  void* d = nullptr;
-  if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
-    (void)hipHostFree(h);
-    return RZ_ERR_DEVICE;
-  }
-  *host = static_cast<T*>(h);
-  *dev = static_cast<T*>(d);
-  return RZ_OK;
-}
-
-static int ensure_words(rz_context* c) {
-  if (c->h_words) return RZ_OK;
-  const int s = host_alloc(&c->h_words, &c->words.out, 2);
-  c->words.err = c->d_err;
-  return s;
 }
 
 // Folds every recorded profiling slot into the running sums.
@@ -741,8 +740,6 @@ static int finish(rz_context* c) {
 
 extern "C" int rz_sync(rz_context* ctx) {
   if (!ctx) return RZ_ERR_INVALID_ARGUMENT;
-  const int s = ensure_words(ctx);
-  if (s != RZ_OK) return s;
   RZ_HIP(launch_host_words(ctx->words, ctx->stream));
   return finish(ctx);
 }
@@ -802,15 +799,13 @@ static QueryParams query_params(rz_context* c, const float* bounds, uint32_t n, 
 extern "C" int rz_query(rz_context* ctx, const float boundsMin[4], const float boundsMax[4], int* visible,
                         int* needsClipping) {
   if (!ctx || !boundsMin || !boundsMax || !visible || !needsClipping) return RZ_ERR_INVALID_ARGUMENT;
-  int s = ensure_words(ctx);
-  if (s != RZ_OK) return s;
   QueryBox box;
   std::memcpy(box.lo, boundsMin, 16);
   std::memcpy(box.hi, boundsMax, 16);
   QueryParams q = query_params(ctx, nullptr, 1, nullptr, nullptr);
   q.words = ctx->words;
   RZ_HIP(launch_query_one(q, box, ctx->stream));
-  s = finish(ctx);
+  const int s = finish(ctx);
   if (s != RZ_OK) return s;
   const uint32_t code = static_cast<volatile uint32_t*>(ctx->h_words)[1];
   *visible = int(code & 1);
@@ -822,12 +817,10 @@ extern "C" int rz_query2d(rz_context* ctx, uint32_t minX, uint32_t maxX, uint32_
                           uint32_t maxZ, int* visible) {
   if (!ctx || !visible || minX > maxX || minY > maxY || maxX >= ctx->width || maxY >= ctx->height)
     return RZ_ERR_INVALID_ARGUMENT;
-  int s = ensure_words(ctx);
-  if (s != RZ_OK) return s;
   QueryParams q = query_params(ctx, nullptr, 0, nullptr, nullptr);
   q.words = ctx->words;
   RZ_HIP(launch_query2d(minX, maxX, minY, maxY, maxZ, q, ctx->stream));
-  s = finish(ctx);
+  const int s = finish(ctx);
   if (s != RZ_OK) return s;
   *visible = int(static_cast<volatile uint32_t*>(ctx->h_words)[1]);
   return RZ_OK;
@@ -837,8 +830,6 @@ extern "C" int rz_query_batch(rz_context* ctx, uint32_t n, const float* bounds, 
                               uint8_t* needsClipping) {
   if (!ctx || (n && (!bounds || !visible))) return RZ_ERR_INVALID_ARGUMENT;
   if (n == 0) return RZ_OK;
-  int s = ensure_words(ctx);
-  if (s != RZ_OK) return s;
   // Up to kHostQueries boxes the kernel reads the boxes from host memory and
   // writes the answers there: no copy is enqueued.
   const bool direct = n <= kHostQueries && ensure_query_host(ctx, n) == RZ_OK;
@@ -850,7 +841,7 @@ extern "C" int rz_query_batch(rz_context* ctx, uint32_t n, const float* bounds, 
     uint8_t* d_vis = ctx->d_hQuery + size_t(ctx->h_queryCap) * 32;
     q = query_params(ctx, reinterpret_cast<const float*>(ctx->d_hQuery), n, d_vis, d_vis + ctx->h_queryCap);
   } else {
-    s = ensure_queries(ctx, n);
+    const int s = ensure_queries(ctx, n);
     if (s != RZ_OK) return s;
     RZ_HIP(hipMemcpyAsync(ctx->d_qbounds, bounds, size_t(n) * 32, hipMemcpyHostToDevice, ctx->stream));
     q = query_params(ctx, ctx->d_qbounds, n, ctx->d_qvis, ctx->d_qclip);
@@ -864,7 +855,7 @@ extern "C" int rz_query_batch(rz_context* ctx, uint32_t n, const float* bounds, 
     RZ_HIP(hipMemcpyAsync(visible, ctx->d_qvis, n, hipMemcpyDeviceToHost, ctx->stream));
     if (needsClipping) RZ_HIP(hipMemcpyAsync(needsClipping, ctx->d_qclip, n, hipMemcpyDeviceToHost, ctx->stream));
   }
-  s = finish(ctx);
+  const int s = finish(ctx);
   if (direct) {
     std::memcpy(visible, h_vis, n);
     if (needsClipping) std::memcpy(needsClipping, h_vis + ctx->h_queryCap, n);
@@ -887,8 +878,6 @@ extern "C" int rz_readback_depth(rz_context* ctx, void* rgba) {
   if (!ctx || !rgba) return RZ_ERR_INVALID_ARGUMENT;
   const size_t px = size_t(ctx->width) * ctx->height;
   if (!ctx->d_rgba && dev_alloc(&ctx->d_rgba, px) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
-  const int s = ensure_words(ctx);
-  if (s != RZ_OK) return s;
   RZ_HIP(launch_readback(ctx->d_depth, ctx->d_hiz, ctx->width, ctx->height, ctx->bX, ctx->d_rgba, ctx->words,
                          ctx->stream));
   RZ_HIP(hipMemcpyAsync(rgba, ctx->d_rgba, px * 4, hipMemcpyDeviceToHost, ctx->stream));
@@ -898,8 +887,6 @@ extern "C" int rz_readback_depth(rz_context* ctx, void* rgba) {
 extern "C" int rz_readback_raw(rz_context* ctx, uint16_t* depth, uint16_t* hiz) {
   if (!ctx) return RZ_ERR_INVALID_ARGUMENT;
   const size_t nb = size_t(ctx->bX) * ctx->bY;
-  const int s = ensure_words(ctx);
-  if (s != RZ_OK) return s;
   RZ_HIP(launch_host_words(ctx->words, ctx->stream));
   if (depth) RZ_HIP(hipMemcpyAsync(depth, ctx->d_depth, nb * 128, hipMemcpyDeviceToHost, ctx->stream));
   if (hiz) RZ_HIP(hipMemcpyAsync(hiz, ctx->d_hiz, (nb + 8) * 2, hipMemcpyDeviceToHost, ctx->stream));

@@ -1,0 +1,191 @@
+// The C ABI's host side without a GPU: this program defines the HIP runtime
+// functions that librasterizer_amd.so calls (the program's definitions come
+// before the library's own dependencies), with device memory as host memory and
+// kernel launches that do nothing but are recorded.  It counts allocations,
+// checks that what is freed was allocated, and can make allocations fail.
+// Run with the name of a check; exits 0 when it holds (tests/test_host_runtime.py).
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <set>
+#include <vector>
+
+#include "rasterizer_amd.h"
+
+namespace {
+
+struct Runtime {
+  std::set<void*> device, pinned;
+  std::vector<size_t> deviceSizes, pinnedSizes;  // of every allocation asked for
+  int badFrees = 0;                              // of memory that is not allocated
+  int streamSyncs = 0;
+  int failDevice = -1, failPinned = -1;  // allocations that succeed before every further one fails (-1: all do)
+  int launches = 0;
+  dim3 grid;  // of the last launch
+};
+Runtime& rt() {
+  static Runtime r;
+  return r;
+}
+
+hipError_t allocate(std::set<void*>& live, std::vector<size_t>& sizes, int& fail, void** p, size_t bytes) {
+  sizes.push_back(bytes);
+  *p = nullptr;
+  if (fail == 0) return hipErrorOutOfMemory;
+  if (fail > 0) --fail;
+  *p = std::calloc(bytes ? bytes : 1, 1);  // untouched pages cost nothing
+  if (!*p) return hipErrorOutOfMemory;
+  live.insert(*p);
+  return hipSuccess;
+}
+hipError_t release(std::set<void*>& live, void* p) {
+  if (!p) return hipSuccess;
+  if (live.erase(p) == 0) {
+    ++rt().badFrees;
+    return hipErrorInvalidValue;
+  }
+  std::free(p);
+  return hipSuccess;
+}
+void copy(void* dst, const void* src, size_t n) { std::memmove(dst, src, n); }
+
+int object;  // what streams, events and graphs point to
+
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) { return allocate(rt().device, rt().deviceSizes, rt().failDevice, p, n); }
+hipError_t hipFree(void* p) { return release(rt().device, p); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  return allocate(rt().pinned, rt().pinnedSizes, rt().failPinned, p, n);
+}
+hipError_t hipHostFree(void* p) { return release(rt().pinned, p); }
+hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) { return *d = h, hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return copy(d, s, n), hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+  return copy(d, s, n), hipSuccess;
+}
+hipError_t hipMemset(void* d, int v, size_t n) { return std::memset(d, v, n), hipSuccess; }
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return std::memset(d, v, n), hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  return *s = reinterpret_cast<hipStream_t>(&object), hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return ++rt().streamSyncs, hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return *e = reinterpret_cast<hipEvent_t>(&object), hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 0.0f, hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+int hipGetStreamDeviceId(hipStream_t) { return 0; }
+hipError_t hipGetSymbolAddress(void** p, const void*) {
+  static void* symbol = std::calloc(size_t(64) << 20, 1);  // the draw's static device array
+  return *p = symbol, hipSuccess;
+}
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) {
+  return *n = 2, hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipLaunchKernel(const void*, dim3 grid, dim3, void**, size_t, hipStream_t) {
+  ++rt().launches;
+  rt().grid = grid;
+  return hipSuccess;
+}
+hipError_t hipLaunchCooperativeKernel(const void* f, dim3 g, dim3 b, void** a, unsigned s, hipStream_t st) {
+  return hipLaunchKernel(f, g, b, a, s, st);
+}
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3, size_t, hipStream_t) { return rt().grid = grid, hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shared, hipStream_t* stream) {
+  *grid = rt().grid;
+  *block = dim3(1);
+  *shared = 0;
+  *stream = nullptr;
+  return hipSuccess;
+}
+}
+
+namespace {
+
+int failures = 0;
+#define CHECK(cond)                                                     \
+  do {                                                                  \
+    if (!(cond)) {                                                      \
+      std::printf("line %d: %s does not hold\n", __LINE__, #cond);      \
+      ++failures;                                                       \
+    }                                                                   \
+  } while (0)
+
+rz_context* context(uint32_t w, uint32_t h) {
+  rz_context* c = nullptr;
+  CHECK(rz_create(w, h, &c) == RZ_OK);
+  return c;
+}
+
+// rz_sync and rz_readback_raw allocate nothing, on a fresh context too, and
+// wait for the stream when no memory can be had.
+void blocking_calls() {
+  rz_context* c = context(64, 64);
+  std::vector<uint16_t> depth(64 * 64), hiz(64 + 8);
+  const size_t device = rt().deviceSizes.size(), pinned = rt().pinnedSizes.size();
+  rt().failDevice = rt().failPinned = 0;
+  for (int i = 0; i < 2; ++i) {
+    int before = rt().streamSyncs;
+    CHECK(rz_sync(c) == RZ_OK);
+    CHECK(rt().streamSyncs > before);
+    before = rt().streamSyncs;
+    CHECK(rz_readback_raw(c, depth.data(), hiz.data()) == RZ_OK);
+    CHECK(rt().streamSyncs > before);
+    int visible = 0, clip = 0;
+    const float lo[4] = {0, 0, 0, 1}, hi[4] = {1, 1, 1, 1};
+    CHECK(rz_query(c, lo, hi, &visible, &clip) == RZ_OK);
+    CHECK(rz_query2d(c, 0, 7, 0, 7, 9, &visible) == RZ_OK);
+  }
+  CHECK(rt().deviceSizes.size() == device && rt().pinnedSizes.size() == pinned);
+  rt().failDevice = rt().failPinned = -1;
+  CHECK(rz_destroy(c) == RZ_OK);
+}
+
+// A context that cannot be made whole is not made, and nothing of it is left.
+void failed_creation() {
+  for (int n = 0;; ++n) {
+    rt().failPinned = n;
+    rz_context* c = nullptr;
+    const int s = rz_create(64, 64, &c);
+    rt().failPinned = -1;
+    if (s == RZ_OK) {
+      CHECK(n > 0);
+      CHECK(rz_destroy(c) == RZ_OK);
+      break;
+    }
+    CHECK(s == RZ_ERR_OUT_OF_MEMORY && !c);
+    CHECK(rt().device.empty() && rt().pinned.empty());
+  }
+}
+
+struct Check {
+  const char* name;
+  void (*run)();
+};
+const Check checks[] = {{"blocking_calls", blocking_calls}, {"failed_creation", failed_creation}};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  for (const Check& c : checks) {
+    if (argc > 1 && std::strcmp(argv[1], c.name) != 0) continue;
+    c.run();
+    CHECK(rt().badFrees == 0);
+    CHECK(rt().device.empty() && rt().pinned.empty());
+    std::printf("%s: %s\n", c.name, failures ? "failed" : "ok");
+    return failures ? 1 : 0;
+  }
+  std::printf("no such check\n");
+  return 2;
+}
