@@ -724,13 +724,15 @@ extern "C" int rz_set_wait_timeout(rz_context* ctx, uint64_t ticks) {
   return RZ_OK;
 }
 
-// Waits for the stream, whose last kernel writes the context's host words, then
-// reports and clears the device error word.
-static int finish(rz_context* c) {
+// Waits for the stream, then reports and clears the device error word: from the
+// context's host words, which the stream's last kernel writes, or, where no
+// kernel did (mirrored false), with a copy.
+static int finish(rz_context* c, bool mirrored = true) {
   RZ_HIP(hipStreamSynchronize(c->stream));
   const int s = flush_pending_status(c);
   if (s != RZ_OK) return s;
-  const uint32_t err = *static_cast<volatile uint32_t*>(c->h_words);
+  uint32_t err = *static_cast<volatile uint32_t*>(c->h_words);
+  if (!mirrored) RZ_HIP(hipMemcpy(&err, c->d_err, sizeof err, hipMemcpyDeviceToHost));
   if (err) {
     RZ_HIP(hipMemset(c->d_err, 0, sizeof(uint32_t)));
     return (err & kErrTimeout) ? RZ_ERR_TIMEOUT : RZ_ERR_DEVICE;
@@ -740,8 +742,10 @@ static int finish(rz_context* c) {
 
 extern "C" int rz_sync(rz_context* ctx) {
   if (!ctx) return RZ_ERR_INVALID_ARGUMENT;
-  RZ_HIP(launch_host_words(ctx->words, ctx->stream));
-  return finish(ctx);
+  // A launch that reports an error (which can be one that another HIP call
+  // left) keeps the call neither from waiting nor from its result.
+  const bool mirrored = launch_host_words(ctx->words, ctx->stream) == hipSuccess;
+  return finish(ctx, mirrored);
 }
 
 // Host memory of a batch of at most kHostQueries boxes: 32 bytes of box, then
@@ -887,10 +891,10 @@ extern "C" int rz_readback_depth(rz_context* ctx, void* rgba) {
 extern "C" int rz_readback_raw(rz_context* ctx, uint16_t* depth, uint16_t* hiz) {
   if (!ctx) return RZ_ERR_INVALID_ARGUMENT;
   const size_t nb = size_t(ctx->bX) * ctx->bY;
-  RZ_HIP(launch_host_words(ctx->words, ctx->stream));
+  const bool mirrored = launch_host_words(ctx->words, ctx->stream) == hipSuccess;
   if (depth) RZ_HIP(hipMemcpyAsync(depth, ctx->d_depth, nb * 128, hipMemcpyDeviceToHost, ctx->stream));
   if (hiz) RZ_HIP(hipMemcpyAsync(hiz, ctx->d_hiz, (nb + 8) * 2, hipMemcpyDeviceToHost, ctx->stream));
-  return finish(ctx);
+  return finish(ctx, mirrored);
 }
 
 extern "C" int rz_upload_raw(rz_context* ctx, const uint16_t* depth, const uint16_t* hiz) {

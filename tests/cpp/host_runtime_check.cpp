@@ -22,8 +22,8 @@ struct Runtime {
   int badFrees = 0;                              // of memory that is not allocated
   int streamSyncs = 0;
   int failDevice = -1, failPinned = -1;  // allocations that succeed before every further one fails (-1: all do)
-  int launches = 0;
-  dim3 grid;  // of the last launch
+  dim3 grid;                             // of the last launch
+  hipError_t lastError = hipSuccess;     // what the next hipGetLastError reports
 };
 Runtime& rt() {
   static Runtime r;
@@ -92,9 +92,12 @@ hipError_t hipGetSymbolAddress(void** p, const void*) {
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int, size_t) {
   return *n = 2, hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = rt().lastError;
+  rt().lastError = hipSuccess;
+  return e;
+}
 hipError_t hipLaunchKernel(const void*, dim3 grid, dim3, void**, size_t, hipStream_t) {
-  ++rt().launches;
   rt().grid = grid;
   return hipSuccess;
 }
@@ -169,11 +172,29 @@ void failed_creation() {
   }
 }
 
+// An error that another HIP call left behind is not theirs: they wait and give
+// their results.
+void error_left_behind() {
+  rz_context* c = context(64, 64);
+  std::vector<uint16_t> depth(64 * 64), hiz(64 + 8);
+  int before = rt().streamSyncs;
+  rt().lastError = hipErrorInvalidValue;
+  CHECK(rz_sync(c) == RZ_OK);
+  CHECK(rt().streamSyncs > before);
+  before = rt().streamSyncs;
+  rt().lastError = hipErrorInvalidValue;
+  CHECK(rz_readback_raw(c, depth.data(), hiz.data()) == RZ_OK);
+  CHECK(rt().streamSyncs > before);
+  CHECK(rz_destroy(c) == RZ_OK);
+}
+
 struct Check {
   const char* name;
   void (*run)();
 };
-const Check checks[] = {{"blocking_calls", blocking_calls}, {"failed_creation", failed_creation}};
+const Check checks[] = {{"blocking_calls", blocking_calls},
+                        {"error_left_behind", error_left_behind},
+                        {"failed_creation", failed_creation}};
 
 }  // namespace
 
