@@ -11,9 +11,10 @@
 namespace rzd {
 
 // Device memory handed out in 256-byte aligned parts, released in the reverse
-// order (Frame).  A call that needs more than is there gets further blocks;
-// after it they are given back and the next call allocates one block of the
-// size that was in use, and a block above kKeepDevice is not kept either.
+// order (Frame).  A call that needs more than is there gets further blocks; after
+// it they are given back and the next call allocates one block of the size that
+// was in use.  More than kKeepDevice is not kept, and the next call allocates so
+// much at once only when its first part or block is a fair share of it.
 // Used by one context's calls, on its stream, by one thread at a time, so a
 // part is only handed on to work that the stream orders behind its last use;
 // everything is freed with the context.
@@ -39,8 +40,10 @@ class Scratch {
     if (cur_ == nBlocks_) {
       if (nBlocks_ == kMaxBlocks) return nullptr;
       Block b;
-      if (nBlocks_ == 0 && want_ > bytes && hipMalloc(&b.base, want_) == hipSuccess) {
-        b.size = want_;
+      const bool alike = want_ <= kKeepDevice ? nBlocks_ == 0 : before_ + bytes >= want_ / 16;
+      const size_t more = alike && before_ < want_ ? want_ - before_ : 0;
+      if (more > bytes && hipMalloc(&b.base, more) == hipSuccess) {
+        b.size = more;
       } else {
         (void)hipGetLastError();
         if (hipMalloc(&b.base, bytes) != hipSuccess) {
@@ -54,7 +57,8 @@ class Scratch {
     }
     T* p = reinterpret_cast<T*>(static_cast<unsigned char*>(blocks_[cur_].base) + used_);
     used_ += bytes;
-    peak_ = peak_ > before_ + used_ ? peak_ : before_ + used_;
+    live_ += bytes;
+    peak_ = peak_ > live_ ? peak_ : live_;
     return p;
   }
 
@@ -79,11 +83,12 @@ class Scratch {
   // Parts taken while a Frame lives are released when it ends.
   class Frame {
    public:
-    explicit Frame(Scratch& s) : s_(s), cur_(s.cur_), used_(s.used_), before_(s.before_) { ++s_.depth_; }
+    explicit Frame(Scratch& s) : s_(s), cur_(s.cur_), used_(s.used_), before_(s.before_), live_(s.live_) { ++s_.depth_; }
     ~Frame() {
       s_.cur_ = cur_;
       s_.used_ = used_;
       s_.before_ = before_;
+      s_.live_ = live_;
       if (--s_.depth_ == 0) s_.trim();
     }
     Frame(const Frame&) = delete;
@@ -91,7 +96,7 @@ class Scratch {
 
    private:
     Scratch& s_;
-    size_t cur_, used_, before_;
+    size_t cur_, used_, before_, live_;
   };
 
  private:
@@ -102,7 +107,7 @@ class Scratch {
 
   void free_blocks() {
     for (size_t i = 0; i < nBlocks_; ++i) (void)hipFree(blocks_[i].base);  // waits for the work that uses it
-    nBlocks_ = cur_ = used_ = before_ = 0;
+    nBlocks_ = cur_ = used_ = before_ = live_ = 0;
   }
   void trim() {
     if (nBlocks_ > 1 || (nBlocks_ == 1 && blocks_[0].size > kKeepDevice)) free_blocks();
@@ -110,12 +115,14 @@ class Scratch {
     peak_ = 0;
   }
 
-  // A call takes at most 40 parts (rz_prepare_mesh_device).
+  // A call takes at most 46 parts (rz_prepare_mesh_device: 2 of its own, 11 of
+  // the decomposition, 4 of the scene, 24 of the SAH pass, 5 of the bake).
   static constexpr size_t kMaxBlocks = 64;
   Block blocks_[kMaxBlocks];
   size_t nBlocks_ = 0;
   size_t cur_ = 0, used_ = 0;  // the next part starts at blocks_[cur_].base + used_
   size_t before_ = 0;          // the sizes of the blocks before it
+  size_t live_ = 0;            // the parts handed out: one block would hold as much
   size_t peak_ = 0, want_ = 0;
   int depth_ = 0;
   void* host_ = nullptr;

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "rasterizer_amd.h"
+#include "rz_scratch.h"
 
 namespace {
 
@@ -188,13 +189,46 @@ void error_left_behind() {
   CHECK(rz_destroy(c) == RZ_OK);
 }
 
+// Scene preparation's working memory: what a call used is one block from the
+// next call on, unless it is more than is kept; a small call after such a one
+// allocates no more than it takes.
+void scratch() {
+  using rzd::Scratch;
+  {
+    Scratch s;
+    auto call = [&](size_t part, int parts) {
+      const size_t before = rt().deviceSizes.size();
+      Scratch::Frame frame(s);
+      for (int i = 0; i < parts; ++i) CHECK(s.take<unsigned char>(part) != nullptr);
+      return rt().deviceSizes.size() - before;
+    };
+    CHECK(call(1 << 20, 46) == 46);
+    CHECK(call(1 << 20, 46) == 1 && rt().deviceSizes.back() == size_t(46) << 20);
+    CHECK(call(1 << 20, 46) == 0);
+    CHECK(call(1000, 3) == 0);
+    CHECK(call(Scratch::kKeepDevice / 2, 5) == 5);
+    CHECK(rt().device.empty());  // too large to be kept
+    CHECK(call(Scratch::kKeepDevice / 2, 5) == 1 && rt().deviceSizes.back() == 5 * Scratch::kKeepDevice / 2);
+    CHECK(call(1000, 3) == 3);
+    for (size_t k = rt().deviceSizes.size() - 3; k < rt().deviceSizes.size(); ++k) CHECK(rt().deviceSizes[k] == 1024);
+    CHECK(call(Scratch::kKeepDevice / 2, 5) > 0);
+    CHECK(call(1000, 3) == 3);
+    CHECK(call(1000, 3) == 1);
+    rt().failDevice = 0;
+    Scratch::Frame frame(s);
+    CHECK(s.take<int>(100) != nullptr && s.take<int>(1 << 20) == nullptr);
+    rt().failDevice = -1;
+  }
+}
+
 struct Check {
   const char* name;
   void (*run)();
 };
 const Check checks[] = {{"blocking_calls", blocking_calls},
                         {"error_left_behind", error_left_behind},
-                        {"failed_creation", failed_creation}};
+                        {"failed_creation", failed_creation},
+                        {"scratch", scratch}};
 
 }  // namespace
 

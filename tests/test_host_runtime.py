@@ -14,7 +14,7 @@ from rasterizer_amd import build
 PROG = Path(__file__).resolve().parent / "_bin" / "host_runtime_check"
 
 
-@pytest.mark.parametrize("check", ["blocking_calls", "error_left_behind", "failed_creation"])
+@pytest.mark.parametrize("check", ["blocking_calls", "error_left_behind", "failed_creation", "scratch"])
 def test_host_runtime(check):
     if not PROG.exists():
         build.build()
