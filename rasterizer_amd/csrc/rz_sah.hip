@@ -623,7 +623,7 @@ __global__ void __launch_bounds__(256) scene_boxes_kernel(const float4* __restri
                                                           uint32_t* __restrict__ partials) {
   const uint32_t first = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
   SceneShare s;
-  for (uint32_t j = first; j < nPad; j += step) {
+  for (uint32_t j = first; j < nPad; j += step) {  // nPad is at most 2^28
     float4 mn = make_float4(INFINITY, INFINITY, INFINITY, INFINITY);
     float4 mx = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
 #pragma unroll
@@ -636,7 +636,7 @@ __global__ void __launch_bounds__(256) scene_boxes_kernel(const float4* __restri
     boxes[2 * size_t(j)] = mn;
     boxes[2 * size_t(j) + 1] = mx;
   }
-  for (uint32_t j = first; j < nBox; j += step) s.add(boxVertices[j]);
+  for (size_t j = first; j < nBox; j += step) s.add(boxVertices[j]);  // nBox can be up to 2^32 - 1
   reduce_share(s, partials + 9 * size_t(blockIdx.x));
 }
 
@@ -669,7 +669,8 @@ __global__ void __launch_bounds__(256) scene_gather_kernel(const float4* __restr
 hipError_t launch_scene_boxes(const float* vertices, uint32_t nQuads, uint32_t nPad, const float* boxVertices,
                               uint32_t nBox, float* boxes, uint32_t* partials, uint32_t* sceneKeys,
                               hipStream_t stream) {
-  const uint32_t parts = std::min(grid_of(std::max(nPad, boxVertices ? nBox : 0u)), kSceneParts);
+  const size_t items = std::max<size_t>(nPad, boxVertices ? nBox : 0u);
+  const uint32_t parts = uint32_t(std::min<size_t>((items + 255u) / 256u, kSceneParts));
   scene_boxes_kernel<<<parts, 256, 0, stream>>>(reinterpret_cast<const float4*>(vertices), nQuads, nPad,
                                                 reinterpret_cast<const float4*>(boxVertices), boxVertices ? nBox : 0u,
                                                 reinterpret_cast<float4*>(boxes), partials);

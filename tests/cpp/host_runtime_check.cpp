@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "rasterizer_amd.h"
+#include "rz_kernels.h"
 #include "rz_scratch.h"
 
 namespace {
@@ -24,6 +25,7 @@ struct Runtime {
   int streamSyncs = 0;
   int failDevice = -1, failPinned = -1;  // allocations that succeed before every further one fails (-1: all do)
   dim3 grid;                             // of the last launch
+  unsigned largestGrid = 0;
   hipError_t lastError = hipSuccess;     // what the next hipGetLastError reports
 };
 Runtime& rt() {
@@ -100,6 +102,7 @@ hipError_t hipGetLastError() {
 }
 hipError_t hipLaunchKernel(const void*, dim3 grid, dim3, void**, size_t, hipStream_t) {
   rt().grid = grid;
+  if (grid.x > rt().largestGrid) rt().largestGrid = grid.x;
   return hipSuccess;
 }
 hipError_t hipLaunchCooperativeKernel(const void* f, dim3 g, dim3 b, void** a, unsigned s, hipStream_t st) {
@@ -221,6 +224,17 @@ void scratch() {
   }
 }
 
+// The scene box over as many vertices as a call can have: its launches have
+// work-groups, no more than there are partial results.
+void scene_box_sizes() {
+  for (uint32_t n : {0u, 1u, 256u, 257u, 131072u, 131073u, 0xFFFE0001u, 0xFFFFFF01u, 0xFFFFFFFFu}) {
+    rt().largestGrid = 0;
+    CHECK(rzd::launch_scene_boxes(nullptr, 8, 8, reinterpret_cast<const float*>(&object), n, nullptr, nullptr, nullptr,
+                                  nullptr) == hipSuccess);
+    CHECK(rt().largestGrid == (n < 131072u ? n / 256u + (n % 256u != 0u || n == 0u) : rzd::kSceneParts));
+  }
+}
+
 struct Check {
   const char* name;
   void (*run)();
@@ -228,7 +242,8 @@ struct Check {
 const Check checks[] = {{"blocking_calls", blocking_calls},
                         {"error_left_behind", error_left_behind},
                         {"failed_creation", failed_creation},
-                        {"scratch", scratch}};
+                        {"scratch", scratch},
+                        {"scene_box_sizes", scene_box_sizes}};
 
 }  // namespace
 

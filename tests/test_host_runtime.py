@@ -14,7 +14,8 @@ from rasterizer_amd import build
 PROG = Path(__file__).resolve().parent / "_bin" / "host_runtime_check"
 
 
-@pytest.mark.parametrize("check", ["blocking_calls", "error_left_behind", "failed_creation", "scratch"])
+@pytest.mark.parametrize("check", ["blocking_calls", "error_left_behind", "failed_creation", "scratch",
+                                   "scene_box_sizes"])
 def test_host_runtime(check):
     if not PROG.exists():
         build.build()
