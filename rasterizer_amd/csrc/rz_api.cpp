@@ -929,12 +929,12 @@ extern "C" int rz_get_tables(rz_context* ctx, uint64_t* coverage4096, uint32_t* 
   if (!ctx) return RZ_ERR_INVALID_ARGUMENT;
   if (coverage4096) {
     // The device's words hold their bits in lane order.
-    std::vector<uint64_t> words(4096);
-    RZ_HIP(hipMemcpy(words.data(), ctx->d_cov, 4096 * 8, hipMemcpyDeviceToHost));
+    RZ_HIP(hipMemcpy(coverage4096, ctx->d_cov, 4096 * 8, hipMemcpyDeviceToHost));
     for (int i = 0; i < 4096; ++i) {
+      const uint64_t lanes = coverage4096[i];
       coverage4096[i] = 0;
       for (uint32_t lane = 0; lane < 64; ++lane)
-        coverage4096[i] |= ((words[size_t(i)] >> lane) & 1ull) << rzi::cov_bit_of_lane(lane);
+        coverage4096[i] |= ((lanes >> lane) & 1ull) << rzi::cov_bit_of_lane(lane);
     }
   }
   if (rcp4096) RZ_HIP(hipMemcpy(rcp4096, ctx->d_rcp, 4096 * 4, hipMemcpyDeviceToHost));

@@ -47,8 +47,9 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <memory>
+#include <new>
 #include <type_traits>
-#include <vector>
 
 #include "rasterizer_amd.h"
 #include "rz_kernels.h"
@@ -542,8 +543,9 @@ int sah_batches_run(hipStream_t stream, Scratch& scratch, uint32_t n, const floa
   }
   sah_emit_kernel<<<grid_of(n), 256, 0, stream>>>(level & 1u ? B.orders : A.orders, A.batchAxis, n, gran, d_indices);
   SAH_HIP(hipGetLastError());
-  std::vector<uint8_t> starts(nChunks);
-  SAH_HIP(hipMemcpyAsync(starts.data(), A.starts, nChunks, hipMemcpyDeviceToHost, stream));
+  const std::unique_ptr<uint8_t[]> starts(new (std::nothrow) uint8_t[nChunks]);
+  if (!starts) return RZ_ERR_OUT_OF_MEMORY;
+  SAH_HIP(hipMemcpyAsync(starts.get(), A.starts, nChunks, hipMemcpyDeviceToHost, stream));
   SAH_HIP(hipStreamSynchronize(stream));
   uint32_t count = 0;
   for (uint32_t c = 1; c < nChunks; ++c)

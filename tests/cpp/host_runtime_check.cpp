@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <set>
 #include <vector>
 
@@ -26,6 +27,8 @@ struct Runtime {
   int failDevice = -1, failPinned = -1;  // allocations that succeed before every further one fails (-1: all do)
   dim3 grid;                             // of the last launch
   unsigned largestGrid = 0;
+  size_t largestNew = ~size_t(0);        // operator new fails for more
+  bool zeroWords = false;                // copies of 16 bytes to the host read as zeros
   hipError_t lastError = hipSuccess;     // what the next hipGetLastError reports
 };
 Runtime& rt() {
@@ -54,9 +57,22 @@ hipError_t release(std::set<void*>& live, void* p) {
 }
 void copy(void* dst, const void* src, size_t n) { std::memmove(dst, src, n); }
 
+void copy_out(void* dst, const void* src, size_t n, hipMemcpyKind kind) {
+  copy(dst, src, n);
+  if (kind == hipMemcpyDeviceToHost && n == 16 && rt().zeroWords) std::memset(dst, 0, n);
+}
+
 int object;  // what streams, events and graphs point to
 
 }  // namespace
+
+void* operator new(size_t n) {
+  void* p = n > rt().largestNew ? nullptr : std::malloc(n ? n : 1);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) { return allocate(rt().device, rt().deviceSizes, rt().failDevice, p, n); }
@@ -67,8 +83,8 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
 hipError_t hipHostFree(void* p) { return release(rt().pinned, p); }
 hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) { return *d = h, hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return copy(d, s, n), hipSuccess; }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
-  return copy(d, s, n), hipSuccess;
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, hipStream_t) {
+  return copy_out(d, s, n, kind), hipSuccess;
 }
 hipError_t hipMemset(void* d, int v, size_t n) { return std::memset(d, v, n), hipSuccess; }
 hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return std::memset(d, v, n), hipSuccess; }
@@ -87,6 +103,11 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms =
 hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
 hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
+  std::memset(p, 0, sizeof *p);
+  std::strcpy(p->gcnArchName, "gfx950");
+  return hipSuccess;
+}
 int hipGetStreamDeviceId(hipStream_t) { return 0; }
 hipError_t hipGetSymbolAddress(void** p, const void*) {
   static void* symbol = std::calloc(size_t(64) << 20, 1);  // the draw's static device array
@@ -235,6 +256,25 @@ void scene_box_sizes() {
   }
 }
 
+// Host memory that cannot be had is a status, not an exception through the C ABI.
+void no_host_memory() {
+  rz_context* c = context(64, 64);
+  std::vector<uint64_t> cov(4096);
+  rt().largestNew = 4096;
+  CHECK(rz_get_tables(c, cov.data(), nullptr) == RZ_OK);
+  rt().largestNew = ~size_t(0);
+  const uint32_t n = 50000;
+  std::vector<float> boxes(size_t(n) * 8);  // from malloc: 16-byte aligned
+  std::vector<uint32_t> idx(n), offsets(n + 1);
+  uint32_t count = 0;
+  rt().zeroWords = true;  // the pass's words: no error, no open range
+  CHECK(rz_sah_batches(c, n, boxes.data(), 512, 8, idx.data(), offsets.data(), &count) == RZ_OK);
+  rt().largestNew = 4096;
+  CHECK(rz_sah_batches(c, n, boxes.data(), 512, 8, idx.data(), offsets.data(), &count) == RZ_ERR_OUT_OF_MEMORY);
+  rt().largestNew = ~size_t(0);
+  CHECK(rz_destroy(c) == RZ_OK);
+}
+
 struct Check {
   const char* name;
   void (*run)();
@@ -243,7 +283,8 @@ const Check checks[] = {{"blocking_calls", blocking_calls},
                         {"error_left_behind", error_left_behind},
                         {"failed_creation", failed_creation},
                         {"scratch", scratch},
-                        {"scene_box_sizes", scene_box_sizes}};
+                        {"scene_box_sizes", scene_box_sizes},
+                        {"no_host_memory", no_host_memory}};
 
 }  // namespace
 
