@@ -36,6 +36,14 @@ hipError_t dev_alloc(T** p, size_t count) {
   return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
 }
 
+// For buffers that are about to be allocated anew: if one of several cannot be
+// had, the context does not go on holding the others' old addresses.
+template <typename T>
+void dev_free(T** p) {
+  hipFree(*p);
+  *p = nullptr;
+}
+
 }  // namespace
 
 namespace rzi {
@@ -405,11 +413,11 @@ static int ensure_capacity(rz_context* c, uint32_t nItems, uint32_t nQuads) {
   }
   if (nItems > c->capItems) {
     const uint32_t cap = std::max<uint32_t>(nItems, std::max<uint32_t>(64, c->capItems * 2));
-    hipFree(c->d_items);
-    hipFree(c->d_state);
-    hipFree(c->d_done);
-    hipFree(c->d_visible);
-    hipFree(c->d_itemBox);
+    dev_free(&c->d_items);
+    dev_free(&c->d_state);
+    dev_free(&c->d_done);
+    dev_free(&c->d_visible);
+    dev_free(&c->d_itemBox);
     c->capItems = 0;
     if (dev_alloc(&c->d_items, cap) != hipSuccess || dev_alloc(&c->d_state, cap) != hipSuccess ||
         dev_alloc(&c->d_done, cap) != hipSuccess || dev_alloc(&c->d_visible, cap) != hipSuccess ||
@@ -419,10 +427,10 @@ static int ensure_capacity(rz_context* c, uint32_t nItems, uint32_t nQuads) {
   }
   if (nQuads > c->capQuads) {
     const uint32_t cap = std::max<uint32_t>(nQuads, std::max<uint32_t>(1024, c->capQuads + c->capQuads / 2));
-    hipFree(c->d_recs);
-    hipFree(c->d_bbox);
-    hipFree(c->d_groupBox);
-  hipFree(c->d_groupItem);
+    dev_free(&c->d_recs);
+    dev_free(&c->d_bbox);
+    dev_free(&c->d_groupBox);
+    dev_free(&c->d_groupItem);
     c->capQuads = 0;
     if (dev_alloc(&c->d_recs, cap) != hipSuccess || dev_alloc(&c->d_bbox, cap) != hipSuccess ||
         dev_alloc(&c->d_groupBox, (cap + 63) / 64) != hipSuccess ||
@@ -769,9 +777,9 @@ static int ensure_query_host(rz_context* c, uint32_t n) {
 static int ensure_queries(rz_context* c, uint32_t n) {
   if (n <= c->capQueries) return RZ_OK;
   RZ_HIP(hipStreamSynchronize(c->stream));
-  hipFree(c->d_qbounds);
-  hipFree(c->d_qvis);
-  hipFree(c->d_qclip);
+  dev_free(&c->d_qbounds);
+  dev_free(&c->d_qvis);
+  dev_free(&c->d_qclip);
   c->capQueries = 0;
   const uint32_t cap = std::max<uint32_t>(n, 1024);
   if (dev_alloc(&c->d_qbounds, size_t(cap) * 8) != hipSuccess || dev_alloc(&c->d_qvis, cap) != hipSuccess ||

@@ -275,6 +275,37 @@ void no_host_memory() {
   CHECK(rz_destroy(c) == RZ_OK);
 }
 
+// Buffers that grow and cannot: the call says so, what it freed is not freed
+// again, and the next call with memory works.
+void failed_growth() {
+  std::vector<uint32_t> packets(4 * 8 * 4);
+  std::vector<float> boxes(8 * 200000);
+  std::vector<uint8_t> visible(200000);
+  const float lo[4] = {0, 0, 0, 1}, hi[4] = {1, 1, 1, 1};
+  for (int n = 0; n < 12; ++n) {
+    rz_context* c = context(64, 64);
+    rz_occluder* o = nullptr;
+    CHECK(rz_occluder_create(c, packets.data(), 16, lo, hi, lo, hi, &o) == RZ_OK);
+    auto draw = [&](uint32_t count) {
+      std::vector<const rz_occluder*> items(count, o);
+      return rz_draw_frame(c, count, items.data(), nullptr);
+    };
+    auto query = [&](uint32_t count) { return rz_query_batch(c, count, boxes.data(), visible.data(), nullptr); };
+    CHECK(draw(3) == RZ_OK && query(150000) == RZ_OK);
+    rt().failDevice = n;
+    const int d = draw(1000), q = query(200000);
+    CHECK((d == RZ_OK || d == RZ_ERR_OUT_OF_MEMORY) && (q == RZ_OK || q == RZ_ERR_OUT_OF_MEMORY));
+    CHECK((d == RZ_OK && q == RZ_OK) == (n >= 12));
+    if (n % 2) {
+      rt().failDevice = -1;
+      CHECK(draw(2000) == RZ_OK && query(200000) == RZ_OK);
+    }
+    rt().failDevice = -1;
+    CHECK(rz_occluder_destroy(o) == RZ_OK && rz_destroy(c) == RZ_OK);
+    CHECK(rt().badFrees == 0 && rt().device.empty());
+  }
+}
+
 struct Check {
   const char* name;
   void (*run)();
@@ -284,7 +315,8 @@ const Check checks[] = {{"blocking_calls", blocking_calls},
                         {"failed_creation", failed_creation},
                         {"scratch", scratch},
                         {"scene_box_sizes", scene_box_sizes},
-                        {"no_host_memory", no_host_memory}};
+                        {"no_host_memory", no_host_memory},
+                        {"failed_growth", failed_growth}};
 
 }  // namespace
 
