@@ -253,7 +253,9 @@ int rz_prepare_mesh_device(rz_context* ctx, uint32_t nTriangles, const uint32_t*
  * the far vertex within 0.5 units of each other's plane (RSQRTPS-normalised
  * normals, as the reference), as a maximum matching grown greedily and then
  * by augmenting paths; a triangle left single becomes the degenerate quad
- * (i0, i2, i1, i0).  Writes 4 indices per quad to out (room for
+ * (i0, i2, i1, i0).  A triangle that repeats an index can be matched with
+ * itself and is then in no quad; no augmenting path leads through it, so that
+ * the search ends on every mesh.  Writes 4 indices per quad to out (room for
  * 4 * (nIndices / 3) words) and the number of words to *nOut; identical to
  * the reference's output, quad for quad.  vertices: nVertices x 4 floats
  * (xyzw); an index >= nVertices is RZ_ERR_INVALID_ARGUMENT. */

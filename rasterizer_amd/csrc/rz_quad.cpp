@@ -69,6 +69,10 @@ struct EdgeIndex {
 inline uint64_t edge_key(uint32_t a, uint32_t b) { return (uint64_t(a) << 32) | b; }
 
 // --- maximum matching (QuadDecomposition.cpp:28-309) ------------------------
+// A triangle that holds an edge and its reverse (two equal indices) is its own
+// neighbour, and the greedy pass can pair it with itself.  Grown into a search's
+// tree, such a vertex becomes its own parent, and no walk towards the root gets
+// past it: an edge whose walk comes there is left out (the search would not end).
 class Matcher {
  public:
   // Writes each vertex's partner, or -1, to mate[0 .. n).
@@ -169,8 +173,9 @@ class Matcher {
     if (token_[wb] != round_) {
       if (mate_[w] == -1) {
         path.push_back(w);  // :157-161
-        trace(v, root, path);
-        return true;
+        if (trace(v, root, path)) return true;
+        path.clear();
+        return false;
       }
       grow(v, w);
     } else if (depth_[wb] % 2 == 0) {
@@ -197,8 +202,9 @@ class Matcher {
   void shrink(int v, int w) {
     int a = v, b = w;
     while (b != a) {
-      if (depth_[a] > depth_[b]) a = parent_[a];
-      else b = parent_[b];
+      int& deeper = depth_[a] > depth_[b] ? a : b;
+      if (parent_[deeper] == deeper) return;  // matched to itself
+      deeper = parent_[deeper];
     }
     const int base = find(a);
     shrink_side(base, v, w);
@@ -218,10 +224,11 @@ class Matcher {
   }
 
   // Appends the tree path from s to t, expanding blossoms through their
-  // bridges (:223-252).
-  void trace(int s, int t, std::vector<int>& path) {
+  // bridges (:223-252); false when the walk comes to a vertex matched to itself.
+  bool trace(int s, int t, std::vector<int>& path) {
     while (s != t) {
       if (depth_[s] % 2 == 0) {
+        if (mate_[s] == s) return false;
         path.push_back(s);
         path.push_back(mate_[s]);
         s = parent_[mate_[s]];
@@ -230,11 +237,12 @@ class Matcher {
       const std::pair<int, int> br = bridge_[s];
       path.push_back(s);
       const size_t from = path.size();
-      trace(br.first, mate_[s], path);
+      if (!trace(br.first, mate_[s], path)) return false;
       std::reverse(path.begin() + std::ptrdiff_t(from), path.end());
       s = br.second;
     }
     path.push_back(s);
+    return true;
   }
 
   const uint32_t* start_;
