@@ -991,9 +991,13 @@ extern "C" int rz_bake_device(rz_context* ctx, uint32_t n, const uint32_t* verte
   if (tabs.rsqrtStatus != RZ_OK) return tabs.rsqrtStatus;
   const int status = ensure_rsqrt(ctx);
   if (status != RZ_OK) return status;
-  uint32_t largest = 0;
-  for (uint32_t i = 0; i < n; ++i) largest = std::max(largest, (vertexOffsets[i + 1] - vertexOffsets[i]) / 4);
-  const size_t quads = largest > kBakeLdsQuads ? vertexOffsets[n] / 4 : 0;
+  uint32_t largest = 0, ldsQuads = 0;
+  for (uint32_t i = 0; i < n; ++i) {
+    const uint32_t size = (vertexOffsets[i + 1] - vertexOffsets[i]) / 4;
+    largest = std::max(largest, size);
+    if (size <= kBakeLdsQuads) ldsQuads = std::max(ldsQuads, size);
+  }
+  const size_t quads = largest > ldsQuads ? vertexOffsets[n] / 4 : 0;
   Scratch::Frame frame(ctx->scratch);
   float* d_ref = ctx->scratch.take<float>(size_t(n) * 8);
   uint32_t* d_offsets = ctx->scratch.take<uint32_t>(size_t(n) + 1);
@@ -1002,6 +1006,7 @@ extern "C" int rz_bake_device(rz_context* ctx, uint32_t n, const uint32_t* verte
   p.packets = d_packets;
   p.bounds = d_bounds;
   p.rsqrt = ctx->d_rsqrt;
+  p.ldsQuads = ldsQuads;
   p.normals = ctx->scratch.take<float4>(quads);
   p.cluster = ctx->scratch.take<uint32_t>(quads);
   p.order = ctx->scratch.take<uint32_t>(quads);

@@ -37,14 +37,6 @@ __device__ __forceinline__ float wave_extreme(Ext e) {
 
 namespace {
 
-// An occluder's working set in LDS.
-struct BakeSmem {
-  float4 normals[kBakeLdsQuads];
-  float4 sorted[kBakeLdsQuads];  // the normals in cluster order
-  uint32_t order[kBakeLdsQuads];
-  uint32_t cluster[kBakeLdsQuads];
-};
-
 // One occluder by one wave.  N, order and C are per quad, in LDS (with the
 // normals in cluster order in M) or, for an occluder too large for that, in
 // the caller's scratch memory (M null).
@@ -203,19 +195,25 @@ __device__ __forceinline__ void bake_occluder(const BakeParams& p, uint32_t o, f
 // occluder's quads long (one wave per occluder, a few hundred occluders).
 // From LDS, over consecutive normals, 878 city occluders take 60 us; with
 // each seed's lane walking every quad's cluster and normal in global memory
-// they took 256.
+// they took 256.  The LDS is what the launch's largest such occluder needs (40
+// bytes a quad: the normals, the normals in cluster order, the order and the
+// clusters), so that small ones leave room for many waves on a CU: rz_bake_device
+// of 12,000 occluders of 8 quads takes 76 us, and 120 with room for 1,024 quads
+// each, which was slower than from global memory (104).
 __global__ void __launch_bounds__(64) rz_bake_kernel(BakeParams p) {
-  __shared__ BakeSmem sm;
-  const uint32_t o = blockIdx.x, v0 = p.offsets[o], quads = (p.offsets[o + 1] - v0) / 4;
-  if (quads <= kBakeLdsQuads)
-    bake_occluder(p, o, sm.normals, sm.sorted, sm.order, sm.cluster);
+  extern __shared__ float4 bakeLds[];
+  const uint32_t o = blockIdx.x, v0 = p.offsets[o], quads = (p.offsets[o + 1] - v0) / 4, n = p.ldsQuads;
+  uint32_t* words = reinterpret_cast<uint32_t*>(bakeLds + 2 * n);
+  if (quads <= n)
+    bake_occluder(p, o, bakeLds, bakeLds + n, words, words + n);
   else
     bake_occluder(p, o, p.normals + v0 / 4, nullptr, p.order + v0 / 4, p.cluster + v0 / 4);
 }
 
 hipError_t launch_bake(const BakeParams& p, uint32_t nOccluders, hipStream_t stream) {
   if (nOccluders == 0) return hipSuccess;
-  hipLaunchKernelGGL(rz_bake_kernel, dim3(nOccluders), dim3(64), 0, stream, p);
+  if (p.ldsQuads > kBakeLdsQuads) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(rz_bake_kernel, dim3(nOccluders), dim3(64), size_t(p.ldsQuads) * kBakeLdsBytes, stream, p);
   return hipGetLastError();
 }
 

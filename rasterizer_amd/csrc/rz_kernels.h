@@ -318,9 +318,11 @@ uint32_t mlp_forward_max_groups();
 // its reference box ref[8o .. 8o + 8) (min xyzw, max xyzw); packets get one
 // word per vertex at the same offsets, bounds 12 floats per occluder
 // (boundsMin, boundsMax, centre).  Scratch per quad (normals, cluster, order)
-// is used by occluders of more than kBakeLdsQuads quads only, and may be null
-// without any.
+// is used by occluders of more than ldsQuads quads only, and may be null
+// without any.  ldsQuads: at most kBakeLdsQuads, the quads that an occluder can
+// have to be baked in LDS.
 constexpr uint32_t kBakeLdsQuads = 1024;  // 40 KB of LDS an occluder, four to a CU
+constexpr uint32_t kBakeLdsBytes = 40;    // a quad
 struct BakeParams {
   const float* vertices;
   const uint32_t* offsets;
@@ -331,6 +333,7 @@ struct BakeParams {
   uint32_t* cluster;
   uint32_t* order;
   const uint32_t* rsqrt;  // 8192-entry host RSQRTPS table
+  uint32_t ldsQuads;
 };
 hipError_t launch_bake(const BakeParams& p, uint32_t nOccluders, hipStream_t stream);
 // SAH batching of n quad boxes on the stream (rz_sah.hip); an RZ_* status.
