@@ -148,19 +148,26 @@ __global__ void __launch_bounds__(kQdBlock) qd_adjacency_kernel(QdParams p) {
     }
     at[k] = j;
   }
-  while (true) {
-    uint32_t s = 0xFFFFFFFFu, from = 3u;
+  // The next entry of each list, or none, in registers: an edge that thousands
+  // of triangles share makes this the longest chain (3,000 triangles on one edge
+  // in both directions: rz_quad_decompose_device 4.5 ms with the three entries
+  // loaded again in each step, 3.3 ms so).
+  constexpr uint32_t kNone = 0xFFFFFFFFu;
+  uint32_t head[3];
+  auto load_head = [&](uint32_t k) {
+    head[k] = at[k] < p.nHalf && p.keys[at[k]] == rev[k] ? p.seqs[at[k]] : kNone;
+  };
 #pragma unroll
-    for (uint32_t k = 0; k < 3; ++k)
-      if (at[k] < p.nHalf && p.keys[at[k]] == rev[k] && p.seqs[at[k]] < s) {
-        s = p.seqs[at[k]];
-        from = k;
-      }
-    if (from == 3u) break;
+  for (uint32_t k = 0; k < 3; ++k) load_head(k);
+  while (true) {
+    const uint32_t s = min(head[0], min(head[1], head[2]));
+    if (s == kNone) break;
+    const uint32_t from = s == head[0] ? 0u : s == head[1] ? 1u : 2u;
 #pragma unroll
     for (uint32_t k = 0; k < 3; ++k)
       if (k == from) {
         ++at[k];
+        load_head(k);
         const uint32_t nb = s / 3u, kk = s - 3u * nb;
         const uint32_t* o = p.idx + 3u * size_t(nb);
         // The later triangle's edge runs from v[next3(k)] to v[k].
