@@ -54,8 +54,11 @@ struct ViewHost {
 // Bytes between a view's visible and clip flags in the answers array.
 size_t answers_stride(uint32_t n) { return (size_t(n) + 63) & ~size_t(63); }
 
-// Largest answers array that is mirrored in pinned host memory.
-constexpr size_t kMirrorBytes = size_t(256) << 20;
+// Pinned host memory through which answers come back: enough for 16 views of
+// 65,536 queries a copy.  Pinning costs the first read of a views object about
+// 0.25 ms a MiB: with all answers pinned it took 9.9 ms for 128 such views (3.8 in
+// two pageable copies a view), with this 3.6, and later reads 1.2 ms either way.
+constexpr size_t kMirrorBytes = size_t(2) << 20;
 
 template <typename T>
 hipError_t dev_alloc(T** p, size_t count) {
@@ -129,13 +132,15 @@ struct rz_views {
   uint32_t* d_nActive = nullptr;
   bool gated = false;   // query-gated draw loop per view (Main.cpp:192-206) instead of classify-then-draw
   bool cooperative = true;  // gated launches: cooperative dispatch (RZ_FRAME_LAUNCH=plain: plain)
-  // Every view's query answers in one device array, and its pinned mirror
-  // (allocated by the first read): views [fetchedFirst, fetchedEnd) hold the
-  // last step's answers there.
+  // Every view's query answers in one device array, and a pinned buffer
+  // (allocated by the first read) that holds the last step's answers of views
+  // [fetchedFirst, fetchedEnd); the last fetchedRun views before fetchedEnd were
+  // fetched one after another.
   uint8_t* d_answers = nullptr;
   size_t answerBytes = 0;
   uint8_t* h_answers = nullptr;
-  uint32_t fetchedFirst = 0, fetchedEnd = 0;
+  size_t mirrorBytes = 0;
+  uint32_t fetchedFirst = 0, fetchedEnd = 0, fetchedRun = 0;
   uint32_t* d_err = nullptr;  // device error word of gated waits
   uint32_t* h_err = nullptr;  // pinned, coherent: d_err as the last step's query kernel left it
   uint32_t* d_hErr = nullptr;  // h_err's device mapping
@@ -393,8 +398,6 @@ static int place_answers(rz_views* v) {
   v->answerBytes = 0;
   v->fetchedFirst = v->fetchedEnd = 0;
   for (ViewHost& h : v->views) h.answersN = 0;
-  if (v->h_answers) (void)hipHostFree(v->h_answers);
-  v->h_answers = nullptr;
   if (dev_alloc(&v->d_answers, std::max<size_t>(total, 1)) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
   v->answerBytes = total;
   size_t at = 0;
@@ -910,20 +913,41 @@ extern "C" int rz_views_read_raw(rz_views* v, uint32_t view, uint16_t* depth, ui
   return RZ_OK;
 }
 
-// The view's answers of the last (finished) step in the pinned mirror.  The
+// The pinned buffer of the answers, for as much as the views need of it; false
+// when it cannot be had.
+static bool ensure_mirror(rz_views* v) {
+  const size_t bytes = std::min(v->answerBytes, kMirrorBytes);
+  if (v->h_answers && v->mirrorBytes >= bytes) return true;
+  if (v->h_answers) (void)hipHostFree(v->h_answers);
+  v->h_answers = nullptr;
+  v->mirrorBytes = 0;
+  v->fetchedFirst = v->fetchedEnd = 0;
+  if (hipHostMalloc(reinterpret_cast<void**>(&v->h_answers), bytes) != hipSuccess) {
+    v->h_answers = nullptr;
+    (void)hipGetLastError();  // handled: copied without it
+    return false;
+  }
+  v->mirrorBytes = bytes;
+  return true;
+}
+
+// The view's answers of the last (finished) step in the pinned buffer.  The
 // first view read after a step is copied alone; a program that goes on to the
-// next views gets as many again with each copy (128 views in 8 copies), where
-// two blocking copies to pageable memory per view took longer than the step:
-// 128 views of 65,536 queries 8 ms against a 5.3 ms step.
+// next views gets as many with each copy as it has read so far (and as fit),
+// where two blocking copies to pageable memory per view took longer than the
+// step: 128 views of 65,536 queries 8 ms against a 5.3 ms step.
 static int fetch_answers(rz_views* v, uint32_t view) {
   if (view >= v->fetchedFirst && view < v->fetchedEnd) return RZ_OK;
   const uint32_t nv = uint32_t(v->views.size());
   const bool next = view == v->fetchedEnd && v->fetchedEnd > v->fetchedFirst;
-  const uint32_t end = std::min(nv, view + (next ? v->fetchedEnd - v->fetchedFirst : 1u));
-  const size_t from = v->views[view].answersAt, to = end < nv ? v->views[end].answersAt : v->answerBytes;
-  v->fetchedFirst = next ? v->fetchedFirst : view;
-  v->fetchedEnd = view;  // until the copy is complete
-  RZ_HIP(hipMemcpyAsync(v->h_answers + from, v->d_answers + from, to - from, hipMemcpyDeviceToHost, v->stream));
+  const size_t from = v->views[view].answersAt;
+  auto past = [&](uint32_t end) { return end < nv ? v->views[end].answersAt : v->answerBytes; };
+  uint32_t end = view + 1;
+  const uint32_t most = std::min(nv, view + (next ? v->fetchedRun : 1u));
+  while (end < most && past(end + 1) - from <= v->mirrorBytes) ++end;
+  v->fetchedFirst = v->fetchedEnd = view;  // until the copy is complete
+  v->fetchedRun = (next ? v->fetchedRun : 0u) + (end - view);
+  RZ_HIP(hipMemcpyAsync(v->h_answers, v->d_answers + from, past(end) - from, hipMemcpyDeviceToHost, v->stream));
   RZ_HIP(hipStreamSynchronize(v->stream));
   v->fetchedEnd = end;
   return RZ_OK;
@@ -933,28 +957,24 @@ extern "C" int rz_views_read_queries(rz_views* v, uint32_t view, uint8_t* visibl
   if (!v || view >= v->views.size()) return RZ_ERR_INVALID_ARGUMENT;
   RZ_HIP(hipStreamSynchronize(v->stream));
   const ViewHost& h = v->views[view];
-  const size_t n = h.nQueries;
+  const size_t n = h.nQueries, stride = answers_stride(h.nQueries);
   if (n == 0) return RZ_OK;
   if (h.answersN != h.nQueries) {  // no step has run with this many queries
     if (visible) std::memset(visible, 0, n);
     if (needsClipping) std::memset(needsClipping, 0, n);
     return RZ_OK;
   }
-  const size_t clipAt = h.answersAt + answers_stride(h.nQueries);
-  if (!v->h_answers && v->answerBytes <= kMirrorBytes &&
-      hipHostMalloc(reinterpret_cast<void**>(&v->h_answers), v->answerBytes) != hipSuccess) {
-    v->h_answers = nullptr;
-    (void)hipGetLastError();  // handled: copied without a mirror
-  }
-  if (!v->h_answers) {
-    if (visible) RZ_HIP(hipMemcpy(visible, v->d_answers + h.answersAt, n, hipMemcpyDeviceToHost));
-    if (needsClipping) RZ_HIP(hipMemcpy(needsClipping, v->d_answers + clipAt, n, hipMemcpyDeviceToHost));
+  if (2 * stride > kMirrorBytes || !ensure_mirror(v)) {
+    const uint8_t* at = v->d_answers + h.answersAt;
+    if (visible) RZ_HIP(hipMemcpy(visible, at, n, hipMemcpyDeviceToHost));
+    if (needsClipping) RZ_HIP(hipMemcpy(needsClipping, at + stride, n, hipMemcpyDeviceToHost));
     return RZ_OK;
   }
   const int s = fetch_answers(v, view);
   if (s != RZ_OK) return s;
-  if (visible) std::memcpy(visible, v->h_answers + h.answersAt, n);
-  if (needsClipping) std::memcpy(needsClipping, v->h_answers + clipAt, n);
+  const uint8_t* at = v->h_answers + (h.answersAt - v->views[v->fetchedFirst].answersAt);
+  if (visible) std::memcpy(visible, at, n);
+  if (needsClipping) std::memcpy(needsClipping, at + stride, n);
   return RZ_OK;
 }
 

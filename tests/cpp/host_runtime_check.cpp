@@ -306,6 +306,33 @@ void failed_growth() {
   }
 }
 
+// Answers of a step come back through a bounded pinned buffer, and without it
+// where it cannot be had.
+void view_answers() {
+  rz_context* c = context(64, 64);
+  const uint32_t size[3] = {64, 64, 64}, counts[3] = {1500000, 0, 700000};
+  std::vector<float> boxes(size_t(counts[0]) * 8);
+  std::vector<uint8_t> visible(counts[0]), clip(counts[0]);
+  rz_views* v = nullptr;
+  CHECK(rz_views_create(3, size, size, &v) == RZ_OK);
+  for (uint32_t k = 0; k < 3; ++k) CHECK(rz_views_set_queries(v, k, counts[k], boxes.data()) == RZ_OK);
+  CHECK(rz_views_run(v, 0) == RZ_OK && rz_views_sync(v, nullptr) == RZ_OK);
+  for (int pinned : {0, -1}) {
+    rt().failPinned = pinned;
+    rt().pinnedSizes.clear();
+    for (uint32_t k : {2u, 0u, 1u, 2u}) {
+      std::memset(visible.data(), 7, visible.size());
+      std::memset(clip.data(), 7, clip.size());
+      CHECK(rz_views_read_queries(v, k, visible.data(), clip.data()) == RZ_OK);
+      for (uint32_t i = 0; i < counts[k]; i += 997) CHECK(visible[i] == 0 && clip[i] == 0);
+      CHECK(counts[k] == counts[0] || (visible[counts[k]] == 7 && clip[counts[k]] == 7));
+    }
+    for (size_t n : rt().pinnedSizes) CHECK(n <= size_t(2) << 20);
+  }
+  rt().failPinned = -1;
+  CHECK(rz_views_destroy(v) == RZ_OK && rz_destroy(c) == RZ_OK);
+}
+
 struct Check {
   const char* name;
   void (*run)();
@@ -316,7 +343,8 @@ const Check checks[] = {{"blocking_calls", blocking_calls},
                         {"scratch", scratch},
                         {"scene_box_sizes", scene_box_sizes},
                         {"no_host_memory", no_host_memory},
-                        {"failed_growth", failed_growth}};
+                        {"failed_growth", failed_growth},
+                        {"view_answers", view_answers}};
 
 }  // namespace
 

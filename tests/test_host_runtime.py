@@ -15,7 +15,8 @@ PROG = Path(__file__).resolve().parent / "_bin" / "host_runtime_check"
 
 
 @pytest.mark.parametrize("check", ["blocking_calls", "error_left_behind", "failed_creation", "scratch",
-                                   "scene_box_sizes", "no_host_memory", "failed_growth"])
+                                   "scene_box_sizes", "no_host_memory", "failed_growth",
+                                   "view_answers"])
 def test_host_runtime(check):
     if not PROG.exists():
         build.build()
