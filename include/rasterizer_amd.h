@@ -295,10 +295,11 @@ int rz_profile_read(rz_context* ctx, double ms[4], uint32_t counts[2]);
  * tilesX*tilesY records of 22 u64 into out (when out is non-NULL and *count
  * is large enough) and sets *count to the number of records: total ticks,
  * ticks waiting on other tiles, waits (items undecided when the tile reached
- * them), ticks in local query2D work, query2D
- * contributions, ticks drawing (scan + draw), quads drawn, items touching the
- * tile, scan ticks, scan passes, tile load ticks, item-loop ticks, draw
- * ticks, (quad, block) pairs visited, of which rejected, of which written,
+ * them), ticks in local query2D work, query2D contributions, ticks drawing
+ * (scan + draw), quads drawn (a quad that every block already rejects is left
+ * out before; its pairs are visited and rejected ones all the same), items
+ * touching the tile, scan ticks, scan passes, tile load ticks, item-loop ticks,
+ * draw ticks, (quad, block) pairs visited, of which rejected, of which written,
  * draw ticks staging per-row folds, draw ticks in the per-block loops, chunks
  * drawn, fold additions staged, query partials evaluated ahead of their turn
  * and of those contributed early (ticks of the 100 MHz s_memrealtime clock). */
