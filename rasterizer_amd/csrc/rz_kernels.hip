@@ -254,7 +254,8 @@ __device__ bool query2d_wave(uint32_t minX, uint32_t maxX, uint32_t minY, uint32
 // Bound by latency (box, reciprocal table, tile minima, hiZ, pixels in turn)
 // and instructions: a city query's rectangle has some tens of blocks, so a
 // whole wave for each box in turn left most lanes idle.  A batch of 1,000,003
-// city boxes, together with launch_query's rule: 180 us before, 28 us now.
+// city boxes, together with launch_query's rule: 157 to 180 us before, 18 to 24 us
+// now, by where the camera stands (the table in launch_query is of one of them).
 template <bool WHOLE>
 __device__ bool query2d_boxes(const QueryPre& Q, bool test, const QueryBufs& B, uint32_t lane) {
   const uint32_t tx0 = Q.minX >> 6, ty0 = Q.minY >> 6;
@@ -1353,7 +1354,7 @@ __device__ __forceinline__ bool quad_touches_tile(const RecWords& R, int tbx0, i
 // the tile.  Only blocks with hiZ >= 2 count: their minimum only grows, so they
 // still reject it at its turn (a block at hiZ 0 could come to read as cleared).
 // Where most quads are hidden this spares them the staging and the draw's two
-// phases: a 4K frame of 12,000 icospheres 0.70 ms without, 0.50 ms with it.
+// phases: a 4K frame of 12,000 icospheres 0.71 ms without, 0.47 ms with it.
 // blocks: how many it may write.
 constexpr int kHiddenBlocks = 64;
 template <int TBX, int TBY>
@@ -1618,9 +1619,10 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
     // other waves are at a barrier meanwhile, and small items share scans and
     // draws.  (With the eight waves sharing every query2D and every poll, two
     // barriers an item, and each item scanned and drawn by itself, a 4K frame
-    // of 12,000 icospheres took 1.20 ms, and takes 0.72 ms; the raster launches
-    // of 20 and 128 city frames in flight took 0.83 and 3.09 ms, and take 0.78 and
-    // 3.01 ms, that of 64 mixed views 0.61 and 0.51 ms.)
+    // of 12,000 icospheres took 1.20 ms, with this 0.72 ms (0.41 ms with
+    // quad_hidden and the item boxes, which came after); the raster launches of 20
+    // and 128 city frames in flight 0.83 and 3.09 ms, with this 0.78 and 3.01 ms,
+    // that of 64 mixed views 0.61 and 0.51 ms.)
     bool arrived = true;  // at a block of 64 slots
     uint32_t upTo = 0;    // lane i: groups of the round's drawn items up to item block + i
     for (uint32_t k = 0;;) {
@@ -2691,15 +2693,15 @@ hipError_t launch_query(const QueryParams& p, hipStream_t stream) {
   // the whole wave, is the shortest chain.  Larger ones get as many boxes per
   // wave as fill the slots once, eight rectangles at a time: fewer leave most
   // lanes of the projection idle, more leave slots idle and make longer waves.
-  // Device batches of city boxes over the 1080p buffer, us per call:
+  // Device batches of city boxes over the 1080p buffer, us per call back to back:
   //   boxes      1 whole  4 whole  8 boxes  16    32    64
-  //   1,000      7.7      8.3      12.7
-  //   8,192      9.2      8.0      12.6
-  //   32,768     16.8     10.7     12.9
-  //   65,536     27       15.9     15.9     17    19    19
-  //   131,072    48       25       20.5     17.6  18.4  19.4
-  //   262,144                      33       22    18    20
-  //   1,000,003                    106      64    40    28
+  //   1,000      5.7      7.4      9.3      9.9   9.2   10.4
+  //   8,192      7.7      6.8      9.5      9.6   10.6  11.8
+  //   32,768     15.4     10.0     14.9     14.7  15.1  15.6
+  //   65,536     25.7     14.4     14.8     15.0  15.1  15.9
+  //   131,072    45.9     23.9     18.2     14.9  14.9  15.7
+  //   262,144    87.1     41.8     30.3     19.8  14.9  15.3
+  //   1,000,003  332      155      106      60.8  36.3  24.3
   constexpr uint32_t kWaves = 8192;
   auto go = [&](auto kernel, uint32_t bpw) {
     hipLaunchKernelGGL(kernel, dim3(groups(groups(p.n, bpw), 4)), dim3(256), 0, stream, p);
