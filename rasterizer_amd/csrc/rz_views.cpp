@@ -916,8 +916,9 @@ extern "C" int rz_views_read_raw(rz_views* v, uint32_t view, uint16_t* depth, ui
 // The pinned buffer of the answers, for as much as the views need of it; false
 // when it cannot be had.
 static bool ensure_mirror(rz_views* v) {
-  const size_t bytes = std::min(v->answerBytes, kMirrorBytes);
+  size_t bytes = std::min(v->answerBytes, kMirrorBytes);
   if (v->h_answers && v->mirrorBytes >= bytes) return true;
+  bytes = std::max(bytes, std::min(2 * v->mirrorBytes, kMirrorBytes));
   if (v->h_answers) (void)hipHostFree(v->h_answers);
   v->h_answers = nullptr;
   v->mirrorBytes = 0;

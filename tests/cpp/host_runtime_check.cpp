@@ -333,6 +333,31 @@ void view_answers() {
   CHECK(rz_views_destroy(v) == RZ_OK && rz_destroy(c) == RZ_OK);
 }
 
+// Batches and views' answers that grow from call to call seldom pin memory anew.
+void growing_calls() {
+  rz_context* c = context(64, 64);
+  std::vector<float> boxes(size_t(131072) * 8);
+  std::vector<uint8_t> visible(131072);
+  rt().pinnedSizes.clear();
+  for (uint32_t n = 500; n <= 131072; n += 500)
+    CHECK(rz_query_batch(c, n, boxes.data(), visible.data(), nullptr) == RZ_OK);
+  CHECK(rz_query_batch(c, 131072, boxes.data(), visible.data(), nullptr) == RZ_OK);
+  CHECK(rt().pinnedSizes.size() <= 9);
+  const uint32_t size = 64;
+  rz_views* v = nullptr;
+  CHECK(rz_views_create(1, &size, &size, &v) == RZ_OK);
+  const size_t before = rt().pinnedSizes.size();
+  uint32_t steps = 0;
+  for (uint32_t n = 1000; n <= 131072; n += 1000, ++steps) {
+    CHECK(rz_views_set_queries(v, 0, n, boxes.data()) == RZ_OK);
+    CHECK(rz_views_run(v, 0) == RZ_OK && rz_views_sync(v, nullptr) == RZ_OK);
+    CHECK(rz_views_read_queries(v, 0, visible.data(), nullptr) == RZ_OK);
+  }
+  // A changed number of queries makes a new plan, whose view table is pinned.
+  CHECK(rt().pinnedSizes.size() - before <= steps + 9);
+  CHECK(rz_views_destroy(v) == RZ_OK && rz_destroy(c) == RZ_OK);
+}
+
 struct Check {
   const char* name;
   void (*run)();
@@ -344,7 +369,8 @@ const Check checks[] = {{"blocking_calls", blocking_calls},
                         {"scene_box_sizes", scene_box_sizes},
                         {"no_host_memory", no_host_memory},
                         {"failed_growth", failed_growth},
-                        {"view_answers", view_answers}};
+                        {"view_answers", view_answers},
+                        {"growing_calls", growing_calls}};
 
 }  // namespace
 
