@@ -12,9 +12,10 @@ namespace rzd {
 
 // Device memory handed out in 256-byte aligned parts, released in the reverse
 // order (Frame).  A call that needs more than is there gets further blocks; after
-// it they are given back and the next call allocates one block of the size that
-// was in use.  More than kKeepDevice is not kept, and the next call allocates so
-// much at once only when its first part or block is a fair share of it.
+// it they are given back and the next call allocates one block of half as much
+// again as was in use, for calls that grow.  More than kKeepDevice is not kept,
+// and the next call allocates so much at once only when its first part or block is
+// a fair share of it.
 // Used by one context's calls, on its stream, by one thread at a time, so a
 // part is only handed on to work that the stream orders behind its last use;
 // everything is freed with the context.
@@ -67,15 +68,17 @@ class Scratch {
   void* host(size_t bytes) {
     if (bytes > kMaxHost) return nullptr;
     if (bytes > hostBytes_) {
+      const size_t twice = 2 * hostBytes_ < kMaxHost ? 2 * hostBytes_ : kMaxHost;  // pinning is slow: grow seldom
       if (host_) (void)hipHostFree(host_);
       host_ = nullptr;
       hostBytes_ = 0;
-      if (hipHostMalloc(&host_, bytes) != hipSuccess) {
+      const size_t size = bytes > twice ? bytes : twice;
+      if (hipHostMalloc(&host_, size) != hipSuccess) {
         (void)hipGetLastError();
         host_ = nullptr;
         return nullptr;
       }
-      hostBytes_ = bytes;
+      hostBytes_ = size;
     }
     return host_;
   }
@@ -110,8 +113,9 @@ class Scratch {
     nBlocks_ = cur_ = used_ = before_ = live_ = 0;
   }
   void trim() {
+    const size_t more = peak_ + peak_ / 2;
+    want_ = peak_ > kKeepDevice ? peak_ : more < kKeepDevice ? more : kKeepDevice;
     if (nBlocks_ > 1 || (nBlocks_ == 1 && blocks_[0].size > kKeepDevice)) free_blocks();
-    want_ = peak_;
     peak_ = 0;
   }
 

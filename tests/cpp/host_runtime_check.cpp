@@ -213,9 +213,9 @@ void error_left_behind() {
   CHECK(rz_destroy(c) == RZ_OK);
 }
 
-// Scene preparation's working memory: what a call used is one block from the
-// next call on, unless it is more than is kept; a small call after such a one
-// allocates no more than it takes.
+// Scene preparation's working memory: what a call used, and half as much again,
+// is one block from the next call on, unless it is more than is kept; a small call
+// after such a one allocates no more than it takes.
 void scratch() {
   using rzd::Scratch;
   {
@@ -227,8 +227,9 @@ void scratch() {
       return rt().deviceSizes.size() - before;
     };
     CHECK(call(1 << 20, 46) == 46);
-    CHECK(call(1 << 20, 46) == 1 && rt().deviceSizes.back() == size_t(46) << 20);
+    CHECK(call(1 << 20, 46) == 1 && rt().deviceSizes.back() == size_t(69) << 20);
     CHECK(call(1 << 20, 46) == 0);
+    for (int parts = 47; parts < 69; ++parts) CHECK(call(1 << 20, parts) == 0);  // growing calls
     CHECK(call(1000, 3) == 0);
     CHECK(call(Scratch::kKeepDevice / 2, 5) == 5);
     CHECK(rt().device.empty());  // too large to be kept
@@ -238,6 +239,10 @@ void scratch() {
     CHECK(call(Scratch::kKeepDevice / 2, 5) > 0);
     CHECK(call(1000, 3) == 3);
     CHECK(call(1000, 3) == 1);
+    rt().pinnedSizes.clear();
+    for (size_t bytes = 1000; bytes <= Scratch::kMaxHost; bytes += bytes / 16 + 100) CHECK(s.host(bytes) != nullptr);
+    CHECK(s.host(Scratch::kMaxHost) != nullptr && s.host(Scratch::kMaxHost + 1) == nullptr);
+    CHECK(rt().pinnedSizes.size() <= 18 && rt().pinnedSizes.back() == Scratch::kMaxHost);
     rt().failDevice = 0;
     Scratch::Frame frame(s);
     CHECK(s.take<int>(100) != nullptr && s.take<int>(1 << 20) == nullptr);
