@@ -18,6 +18,8 @@
 #include "rz_scratch.h"
 
 using namespace rzd;
+using rzi::dev_alloc;
+using rzi::host_alloc;
 
 namespace {
 
@@ -28,13 +30,6 @@ constexpr int kStagingSlots = 16;
 constexpr uint64_t kDrawsPerEvent = 8;
 constexpr int kProfSlots = 256;
 constexpr uint64_t kTimeoutTicks = 200000000ull;  // 2 s of the 100 MHz s_memrealtime clock
-
-template <typename T>
-hipError_t dev_alloc(T** p, size_t count) {
-  *p = nullptr;
-  if (count == 0) return hipSuccess;
-  return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
-}
 
 // For buffers that are about to be allocated anew: if one of several cannot be
 // had, the context does not go on holding the others' old addresses.
@@ -194,26 +189,6 @@ static void free_context(rz_context* c) {
 
 static int noalloc_init(int device);
 
-// Pinned host memory that kernels read and write through *dev; coherent
-// (fine-grained), so that nothing of an earlier use is in a cache.
-template <typename T>
-static int host_alloc(T** host, T** dev, size_t count) {
-  *host = *dev = nullptr;
-  void* h = nullptr;
-  if (hipHostMalloc(&h, count * sizeof(T), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
-    (void)hipGetLastError();
-    return RZ_ERR_OUT_OF_MEMORY;
-  }
-  void* d = nullptr;
-  if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
-    (void)hipHostFree(h);
-    return RZ_ERR_DEVICE;
-  }
-  *host = static_cast<T*>(h);
-  *dev = static_cast<T*>(d);
-  return RZ_OK;
-}
-
 extern "C" int rz_create(uint32_t width, uint32_t height, rz_context** out) {
   if (!out) return RZ_ERR_INVALID_ARGUMENT;
   *out = nullptr;
@@ -351,7 +326,7 @@ int occluder_create(rz_context* ctx, const uint32_t* packets, uint32_t packetCou
   std::memcpy(o->boundsMax, boundsMax, 16);
   o->d_packets = nullptr;
   if (packetCount) {
-    if (hipMalloc(reinterpret_cast<void**>(&o->d_packets), size_t(packetCount) * 32) != hipSuccess) {
+    if (dev_alloc(&o->d_packets, size_t(packetCount) * 8) != hipSuccess) {
       delete o;
       return RZ_ERR_OUT_OF_MEMORY;
     }
@@ -1203,8 +1178,10 @@ extern "C" int rz_profile_read(rz_context* ctx, double ms[4], uint32_t counts[2]
 
 extern "C" int rz_device_alloc(rz_context* ctx, size_t bytes, const void* init, void** devptr) {
   if (!ctx || !devptr || bytes == 0) return RZ_ERR_INVALID_ARGUMENT;
-  *devptr = nullptr;
-  if (hipMalloc(devptr, bytes) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
+  unsigned char* p = nullptr;
+  const bool ok = dev_alloc(&p, bytes) == hipSuccess;
+  *devptr = p;
+  if (!ok) return RZ_ERR_OUT_OF_MEMORY;
   const hipError_t e = init ? hipMemcpy(*devptr, init, bytes, hipMemcpyHostToDevice) : hipMemset(*devptr, 0, bytes);
   if (e != hipSuccess) {
     hipFree(*devptr);

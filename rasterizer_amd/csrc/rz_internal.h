@@ -59,6 +59,40 @@ namespace rzi {
 // is set (the C ABI itself only returns RZ_ERR_DEVICE).
 void report_hip_error(hipError_t error, const char* call, const char* file, int line);
 
+// Device memory for count elements (none for 0).  What failed is told by the
+// result alone: left in the runtime, it would be the next launch's error.
+template <typename T>
+hipError_t dev_alloc(T** p, size_t count) {
+  *p = nullptr;
+  if (count == 0) return hipSuccess;
+  void* d = nullptr;
+  const hipError_t e = hipMalloc(&d, count * sizeof(T));
+  if (e != hipSuccess) (void)hipGetLastError();
+  else *p = static_cast<T*>(d);
+  return e;
+}
+
+// Pinned host memory that kernels read and write through *dev; coherent
+// (fine-grained), so that nothing of an earlier use is in a cache.  An RZ_*
+// status.
+template <typename T>
+int host_alloc(T** host, T** dev, size_t count) {
+  *host = *dev = nullptr;
+  void* h = nullptr;
+  if (hipHostMalloc(&h, count * sizeof(T), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+    (void)hipGetLastError();
+    return RZ_ERR_OUT_OF_MEMORY;
+  }
+  void* d = nullptr;
+  if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+    (void)hipHostFree(h);
+    return RZ_ERR_DEVICE;
+  }
+  *host = static_cast<T*>(h);
+  *dev = static_cast<T*>(d);
+  return RZ_OK;
+}
+
 // The coverage table and this host's RCPPS table, built once per process.
 struct HostTables {
   int status = RZ_OK;

@@ -14,6 +14,8 @@
 #include "rz_kernels.h"
 
 using namespace rzd;
+using rzi::dev_alloc;
+using rzi::host_alloc;
 
 namespace {
 
@@ -53,9 +55,8 @@ int ensure_samples(rz_mlp* m, uint32_t n) {
   hipFree(m->d_ds);
   m->d_x = m->d_scores = m->d_ds = nullptr;
   m->capX = 0;
-  if (hipMalloc(reinterpret_cast<void**>(&m->d_x), size_t(n) * kMlpIn * 4) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&m->d_scores), size_t(n) * 4) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&m->d_ds), size_t(n) * 4) != hipSuccess)
+  if (dev_alloc(&m->d_x, size_t(n) * kMlpIn) != hipSuccess || dev_alloc(&m->d_scores, n) != hipSuccess ||
+      dev_alloc(&m->d_ds, n) != hipSuccess)
     return RZ_ERR_OUT_OF_MEMORY;
   m->capX = n;
   return RZ_OK;
@@ -66,7 +67,7 @@ int ensure_pairs(rz_mlp* m, uint32_t n) {
   hipFree(m->d_pairs);
   m->d_pairs = nullptr;
   m->capPairs = 0;
-  if (hipMalloc(reinterpret_cast<void**>(&m->d_pairs), size_t(n) * 8) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
+  if (dev_alloc(&m->d_pairs, size_t(n) * 2) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
   m->capPairs = n;
   return RZ_OK;
 }
@@ -75,23 +76,15 @@ int ensure_pairs(rz_mlp* m, uint32_t n) {
 // memory.
 int ensure_backward(rz_mlp* m, uint32_t n) {
   if (!m->h_result) {
-    void* h = nullptr;
-    if (hipHostMalloc(&h, (kMlpParams + 1) * sizeof(float), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
-      return RZ_ERR_OUT_OF_MEMORY;
-    void* d = nullptr;
-    if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
-      (void)hipHostFree(h);
-      return RZ_ERR_DEVICE;
-    }
-    m->h_result = static_cast<float*>(h);
-    m->d_hResult = static_cast<float*>(d);
+    const int s = host_alloc(&m->h_result, &m->d_hResult, kMlpParams + 1);
+    if (s != RZ_OK) return s;
   }
   const uint32_t rows = mlp_backward_rows(n);
   if (rows <= m->capPartial) return RZ_OK;
   hipFree(m->d_partial);
   m->d_partial = nullptr;
   m->capPartial = 0;
-  if (hipMalloc(reinterpret_cast<void**>(&m->d_partial), size_t(rows) * kMlpParams * sizeof(float)) != hipSuccess)
+  if (dev_alloc(&m->d_partial, size_t(rows) * kMlpParams) != hipSuccess)
     return RZ_ERR_OUT_OF_MEMORY;
   m->capPartial = rows;
   return RZ_OK;
@@ -149,12 +142,9 @@ extern "C" int rz_mlp_create(uint32_t seed, rz_mlp** out) {
   };
   if (hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) != hipSuccess) return fail(RZ_ERR_DEVICE);
   const size_t pb = kMlpParams * sizeof(float);
-  if (hipMalloc(reinterpret_cast<void**>(&m->d_w), pb) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&m->d_grad), pb) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&m->d_m), pb) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&m->d_v), pb) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&m->d_norm), 32 * sizeof(float)) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void**>(&m->d_loss), sizeof(float)) != hipSuccess)
+  if (dev_alloc(&m->d_w, kMlpParams) != hipSuccess || dev_alloc(&m->d_grad, kMlpParams) != hipSuccess ||
+      dev_alloc(&m->d_m, kMlpParams) != hipSuccess || dev_alloc(&m->d_v, kMlpParams) != hipSuccess ||
+      dev_alloc(&m->d_norm, 32) != hipSuccess || dev_alloc(&m->d_loss, 1) != hipSuccess)
     return fail(RZ_ERR_OUT_OF_MEMORY);
   // Glorot-uniform weights, zero biases, identity normalisation.
   std::vector<float> w(kMlpParams, 0.0f);

@@ -32,6 +32,8 @@ constexpr uint64_t kGatedTimeoutTicks = 200000000ull;  // 2 s of the 100 MHz s_m
 }
 
 using namespace rzd;
+using rzi::dev_alloc;
+using rzi::host_alloc;
 
 namespace {
 
@@ -59,13 +61,6 @@ size_t answers_stride(uint32_t n) { return (size_t(n) + 63) & ~size_t(63); }
 // 0.25 ms a MiB: with all answers pinned it took 9.9 ms for 128 such views (3.8 in
 // two pageable copies a view), with this 3.6, and later reads 1.2 ms either way.
 constexpr size_t kMirrorBytes = size_t(2) << 20;
-
-template <typename T>
-hipError_t dev_alloc(T** p, size_t count) {
-  *p = nullptr;
-  if (count == 0) return hipSuccess;
-  return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
-}
 
 }  // namespace
 
@@ -117,7 +112,7 @@ struct rz_views {
   uint64_t* d_sortKeysOut = nullptr;
   int sortEndBit = 32;
   uint32_t* d_drawn = nullptr;     // batches of drawn occluders (scored by the model), count in d_drawn[nBatches]
-  void* d_sortTemp = nullptr;
+  unsigned char* d_sortTemp = nullptr;
   size_t sortTempBytes = 0;
   int waves = 4;  // wave64s per raster work-group
   int tileB = 8;  // raster tile edge in 8x8 blocks (8 or 16; labelled steps use 8)
@@ -299,12 +294,9 @@ extern "C" int rz_views_create(uint32_t nViews, const uint32_t* widths, const ui
       dev_alloc(&v->d_queue, 1) != hipSuccess || dev_alloc(&v->d_err, 1) != hipSuccess)
     return fail(RZ_ERR_OUT_OF_MEMORY);
   if (hipMemset(v->d_err, 0, sizeof(uint32_t)) != hipSuccess) return fail(RZ_ERR_DEVICE);
-  if (hipHostMalloc(reinterpret_cast<void**>(&v->h_err), sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent) !=
-      hipSuccess)
-    return fail(RZ_ERR_OUT_OF_MEMORY);
+  const int pinned = host_alloc(&v->h_err, &v->d_hErr, 1);
+  if (pinned != RZ_OK) return fail(pinned);
   *v->h_err = 0;
-  if (hipHostGetDevicePointer(reinterpret_cast<void**>(&v->d_hErr), v->h_err, 0) != hipSuccess)
-    return fail(RZ_ERR_DEVICE);
   if (const char* mode = std::getenv("RZ_FRAME_LAUNCH")) v->cooperative = std::strcmp(mode, "plain") != 0;
   if (hipMemcpy(v->d_cov, tabs.covLanes, sizeof tabs.covLanes, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(v->d_rcp, tabs.rcp, sizeof tabs.rcp, hipMemcpyHostToDevice) != hipSuccess)
@@ -431,14 +423,10 @@ static int build_plan(rz_views* v) {
   uint64_t quads = 0;
   uint32_t units = 0, queries = 0, maxClear = 0;
   v->maxBlocks = 0;
-  if (hipHostMalloc(reinterpret_cast<void**>(&v->h_views), nv * sizeof(ViewDesc),
-                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
-    return RZ_ERR_OUT_OF_MEMORY;
-  {
-    void* mapped = nullptr;
-    RZ_HIP(hipHostGetDevicePointer(&mapped, v->h_views, 0));
-    v->d_hViews = static_cast<const ViewDesc*>(mapped);
-  }
+  ViewDesc* mapped = nullptr;
+  const int pinned = host_alloc(&v->h_views, &mapped, nv);
+  if (pinned != RZ_OK) return pinned;
+  v->d_hViews = mapped;
   for (uint32_t i = 0; i < nv; ++i) {
     ViewHost& h = v->views[i];
     ViewDesc& d = v->h_views[i];
@@ -553,9 +541,12 @@ static int build_plan(rz_views* v) {
   for (const ViewHost& h : v->views) v->f2b |= h.eye[3] != 0.0f;
   if (v->f2b && (v->model || v->batchOrder)) return RZ_ERR_INVALID_ARGUMENT;
   if (v->f2b) {
-    if (hipHostMalloc(reinterpret_cast<void**>(&v->h_eyes), size_t(nv) * 4 * sizeof(float)) != hipSuccess ||
-        dev_alloc(&v->d_eyes, size_t(nv) * 4) != hipSuccess)
+    if (hipHostMalloc(reinterpret_cast<void**>(&v->h_eyes), size_t(nv) * 4 * sizeof(float)) != hipSuccess) {
+      v->h_eyes = nullptr;
+      (void)hipGetLastError();
       return RZ_ERR_OUT_OF_MEMORY;
+    }
+    if (dev_alloc(&v->d_eyes, size_t(nv) * 4) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
   }
   {
     // Per-tile item lists: each unit gets room for all of its view's items
@@ -606,7 +597,7 @@ static int build_plan(rz_views* v) {
       return RZ_ERR_OUT_OF_MEMORY;
     RZ_HIP(rocprim::radix_sort_pairs(nullptr, bytes, v->d_sortKeys, v->d_sortKeysOut, v->d_itemIota,
                                               v->d_itemOrder, uint32_t(v->nItems), 0u, unsigned(v->sortEndBit), v->stream));
-    if (hipMalloc(&v->d_sortTemp, std::max<size_t>(bytes, 16)) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
+    if (dev_alloc(&v->d_sortTemp, std::max<size_t>(bytes, 16)) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
     v->sortTempBytes = bytes;
   }
   if (v->model) {
@@ -627,7 +618,7 @@ static int build_plan(rz_views* v) {
                                                 v->d_itemOrder, uint32_t(v->nItems), 0u, unsigned(v->sortEndBit), v->stream));
       bytes = std::max(bytes, itemBytes);
     }
-    if (hipMalloc(&v->d_sortTemp, std::max<size_t>(bytes, 16)) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
+    if (dev_alloc(&v->d_sortTemp, std::max<size_t>(bytes, 16)) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
     v->sortTempBytes = bytes;
   }
   if (v->batchOrder) {

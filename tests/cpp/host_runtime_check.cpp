@@ -39,7 +39,7 @@ Runtime& rt() {
 hipError_t allocate(std::set<void*>& live, std::vector<size_t>& sizes, int& fail, void** p, size_t bytes) {
   sizes.push_back(bytes);
   *p = nullptr;
-  if (fail == 0) return hipErrorOutOfMemory;
+  if (fail == 0) return rt().lastError = hipErrorOutOfMemory;
   if (fail > 0) --fail;
   *p = std::calloc(bytes ? bytes : 1, 1);  // untouched pages cost nothing
   if (!*p) return hipErrorOutOfMemory;
@@ -281,7 +281,7 @@ void no_host_memory() {
 }
 
 // Buffers that grow and cannot: the call says so, what it freed is not freed
-// again, and the next call with memory works.
+// again, and the next call with memory works and reports no error of this one.
 void failed_growth() {
   std::vector<uint32_t> packets(4 * 8 * 4);
   std::vector<float> boxes(8 * 200000);
@@ -306,9 +306,45 @@ void failed_growth() {
       CHECK(draw(2000) == RZ_OK && query(200000) == RZ_OK);
     }
     rt().failDevice = -1;
+    CHECK(rz_sync(c) == RZ_OK);
     CHECK(rz_occluder_destroy(o) == RZ_OK && rz_destroy(c) == RZ_OK);
     CHECK(rt().badFrees == 0 && rt().device.empty());
   }
+}
+
+// The same for a views object's plan and a model's buffers.
+void failed_plans() {
+  std::vector<uint32_t> packets(4 * 8 * 4);
+  std::vector<float> boxes(8 * 1000), x(16 * 1000), grad(5313);
+  const float lo[4] = {0, 0, 0, 1}, hi[4] = {1, 1, 1, 1}, eye[3] = {1, 2, 3};
+  const uint32_t size[2] = {64, 64}, pairs[2] = {0, 1};
+  rz_context* c = context(64, 64);
+  rz_occluder* o = nullptr;
+  CHECK(rz_occluder_create(c, packets.data(), 16, lo, hi, lo, hi, &o) == RZ_OK);
+  bool failed = true;
+  for (int n = 0; failed && n < 100; ++n)
+    for (int pinned = 0; pinned < 2; ++pinned) {
+      int& fail = pinned ? rt().failPinned : rt().failDevice;
+      rz_views* v = nullptr;
+      rz_mlp* m = nullptr;
+      CHECK(rz_views_create(2, size, size, &v) == RZ_OK && rz_mlp_create(1, &m) == RZ_OK);
+      for (uint32_t k = 0; k < 2; ++k)
+        CHECK(rz_views_set_occluders(v, k, 1, &o) == RZ_OK && rz_views_set_queries(v, k, 1000, boxes.data()) == RZ_OK &&
+              rz_views_set_eye(v, k, eye) == RZ_OK);
+      fail = n;
+      const int r = rz_views_run(v, 0);
+      fail = n;
+      const int g = rz_mlp_gradients(m, 1000, x.data(), 1, pairs, grad.data(), nullptr);
+      fail = -1;
+      CHECK((r == RZ_OK || r == RZ_ERR_OUT_OF_MEMORY) && (g == RZ_OK || g == RZ_ERR_OUT_OF_MEMORY));
+      CHECK(n > 0 || (r != RZ_OK && g != RZ_OK));
+      if (!pinned) failed = r != RZ_OK || g != RZ_OK;
+      CHECK(rz_views_run(v, 0) == RZ_OK && rz_views_sync(v, nullptr) == RZ_OK);
+      CHECK(rz_mlp_gradients(m, 1000, x.data(), 1, pairs, grad.data(), nullptr) == RZ_OK);
+      CHECK(rz_views_destroy(v) == RZ_OK && rz_mlp_destroy(m) == RZ_OK && rt().badFrees == 0);
+    }
+  CHECK(!failed);
+  CHECK(rz_occluder_destroy(o) == RZ_OK && rz_destroy(c) == RZ_OK);
 }
 
 // Answers of a step come back through a bounded pinned buffer, and without it
@@ -374,6 +410,7 @@ const Check checks[] = {{"blocking_calls", blocking_calls},
                         {"scene_box_sizes", scene_box_sizes},
                         {"no_host_memory", no_host_memory},
                         {"failed_growth", failed_growth},
+                        {"failed_plans", failed_plans},
                         {"view_answers", view_answers},
                         {"growing_calls", growing_calls}};
 

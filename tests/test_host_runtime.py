@@ -15,7 +15,7 @@ PROG = Path(__file__).resolve().parent / "_bin" / "host_runtime_check"
 
 
 @pytest.mark.parametrize("check", ["blocking_calls", "error_left_behind", "failed_creation", "scratch",
-                                   "scene_box_sizes", "no_host_memory", "failed_growth",
+                                   "scene_box_sizes", "no_host_memory", "failed_growth", "failed_plans",
                                    "view_answers", "growing_calls"])
 def test_host_runtime(check):
     if not PROG.exists():
