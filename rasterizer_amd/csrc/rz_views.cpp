@@ -391,6 +391,7 @@ static int place_answers(rz_views* v) {
   v->fetchedFirst = v->fetchedEnd = 0;
   for (ViewHost& h : v->views) h.answersN = 0;
   if (dev_alloc(&v->d_answers, std::max<size_t>(total, 1)) != hipSuccess) return RZ_ERR_OUT_OF_MEMORY;
+  RZ_HIP(hipMemsetAsync(v->d_answers, 0, std::max<size_t>(total, 1), v->stream));  // read as such if no step follows
   v->answerBytes = total;
   size_t at = 0;
   for (ViewHost& h : v->views) {

@@ -75,7 +75,11 @@ void operator delete(void* p) noexcept { std::free(p); }
 void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 extern "C" {
-hipError_t hipMalloc(void** p, size_t n) { return allocate(rt().device, rt().deviceSizes, rt().failDevice, p, n); }
+hipError_t hipMalloc(void** p, size_t n) {
+  const hipError_t e = allocate(rt().device, rt().deviceSizes, rt().failDevice, p, n);
+  if (e == hipSuccess && n <= size_t(1) << 20) std::memset(*p, 0xAB, n);  // device memory is not cleared
+  return e;
+}
 hipError_t hipFree(void* p) { return release(rt().device, p); }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   return allocate(rt().pinned, rt().pinnedSizes, rt().failPinned, p, n);
@@ -338,6 +342,10 @@ void failed_plans() {
       fail = -1;
       CHECK((r == RZ_OK || r == RZ_ERR_OUT_OF_MEMORY) && (g == RZ_OK || g == RZ_ERR_OUT_OF_MEMORY));
       CHECK(n > 0 || (r != RZ_OK && g != RZ_OK));
+      // No step has run: no box is visible.
+      std::vector<uint8_t> visible(1000, 7), clip(1000, 7);
+      CHECK(rz_views_read_queries(v, 1, visible.data(), clip.data()) == RZ_OK);
+      for (int k = 0; k < 1000; ++k) CHECK(visible[k] == 0 && clip[k] == 0);
       if (!pinned) failed = r != RZ_OK || g != RZ_OK;
       CHECK(rz_views_run(v, 0) == RZ_OK && rz_views_sync(v, nullptr) == RZ_OK);
       CHECK(rz_mlp_gradients(m, 1000, x.data(), 1, pairs, grad.data(), nullptr) == RZ_OK);
