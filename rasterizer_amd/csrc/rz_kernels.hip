@@ -1349,24 +1349,31 @@ __device__ __forceinline__ bool quad_touches_tile(const RecWords& R, int tbx0, i
   return !misses;
 }
 
+// The blocks that a quad whose block index did not wrap shares with the tile.
+__device__ __forceinline__ uint32_t quad_blocks(const RecWords& R, int tbx0, int tbx1, int tby0, int tby1, int bX,
+                                                float invBX) {
+  const int fb = int(R.w[3].w), minY = div_bx(fb, bX, invBX), minX = fb - minY * bX;
+  const int columns = min(tbx1, minX + int(R.w[4].x & 0xFFFFu) - 1) - max(tbx0, minX) + 1;
+  const int rows = min(tby1, minY + int(R.w[4].x >> 16) - 1) - max(tby0, minY) + 1;
+  return uint32_t(columns * rows);
+}
+
 // Whether every block that a quad may write in the tile already rejects it (hiZ
 // at or above its largest depth), for a quad of at most kHiddenBlocks blocks in
 // the tile.  Only blocks with hiZ >= 2 count: their minimum only grows, so they
 // still reject it at its turn (a block at hiZ 0 could come to read as cleared).
 // Where most quads are hidden this spares them the staging and the draw's two
 // phases: a 4K frame of 12,000 icospheres 0.71 ms without, 0.47 ms with it.
-// blocks: how many it may write.
 constexpr int kHiddenBlocks = 64;
 template <int TBX, int TBY>
 __device__ __forceinline__ bool quad_hidden(const RecWords& R, const TileSmem<TBX, TBY>& sm, int tbx0, int tbx1,
-                                            int tby0, int tby1, int bX, float invBX, uint32_t& blocks) {
+                                            int tby0, int tby1, int bX, float invBX) {
   const int fb = int(R.w[3].w), rangeX = int(R.w[4].x & 0xFFFFu), rangeY = int(R.w[4].x >> 16);
   const uint32_t maxZ = R.w[4].y >> 16;
   const int minY = div_bx(fb, bX, invBX), minX = fb - minY * bX;
   const int x0 = max(tbx0, minX) - tbx0, x1 = min(tbx1, minX + rangeX - 1) - tbx0;
   const int y0 = max(tby0, minY) - tby0, y1 = min(tby1, minY + rangeY - 1) - tby0;
   const int n = (x1 - x0 + 1) * (y1 - y0 + 1);
-  blocks = uint32_t(n);
   if (minX + rangeX > bX || n > kHiddenBlocks) return false;
   bool open = false;
   int x = x0, lb = y0 * TBX + x0;
@@ -1782,12 +1789,10 @@ __device__ __forceinline__ void process_tile(const TileJob& J, TileSmem<TBX, TBY
             quad = ((first >> 6) + g) * 64u + lane;
             if (quad >= first && quad < past) {
               const RecWords rec = load_rec(&J.recs[quad]);
-              uint32_t blocks = 0;
-              hit = quad_touches_tile(rec, tbx0, tbx1, tby0, tby1, bX, invBX);
-              if (hit && drew && quad_hidden<TBX, TBY>(rec, sm, tbx0, tbx1, tby0, tby1, bX, invBX, blocks)) {
-                hit = false;
-                hidden = blocks;
-              }
+              hit = quad_touches_tile(rec, tbx0, tbx1, tby0, tby1, bX, invBX) &&
+                    !(drew && quad_hidden<TBX, TBY>(rec, sm, tbx0, tbx1, tby0, tby1, bX, invBX));
+              if (STATS && !hit && quad_touches_tile(rec, tbx0, tbx1, tby0, tby1, bX, invBX))
+                hidden = quad_blocks(rec, tbx0, tbx1, tby0, tby1, bX, invBX);
             }
           }
           if (STATS) {
